@@ -9,7 +9,8 @@ Inputs are resident in HBM before the timed region.
 
 The JSON line carries:
   roofline      the dominant kernel (the dense JFA pass k_jfa_quad, passes
-                1 .. P-1; pass 0 is a scatter of the seeds): algorithmic
+                5 .. P-1; the first five run in one launch over residue
+                classes, k_jfa_lattice): algorithmic
                 bytes per launch (read + write of the int32 label map,
                 8 B/pixel) over its mean duration measured with HIP events
                 on the engine's stream, against the 8 TB/s HBM peak;

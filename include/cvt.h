@@ -138,9 +138,10 @@ int cvt_energy(cvt_ctx *ctx, double *energy, double *gradnorm);
 int cvt_synchronize(cvt_ctx *ctx);
 /* Runs `iterations` (1..1000) Lloyd steps eagerly with HIP events around
  * each phase and returns mean durations in ms: ms[0] one dense JFA pass (the
- * back-to-back sequence of passes 1 .. P-1 over P - 1), ms[1] the moment
- * kernel, ms[2] the first JFA pass (from the seed map), ms[3] update +
- * finalize, ms[4] the whole JFA, ms[5] the whole step,
+ * back-to-back sequence of the passes after the first launch over their
+ * count), ms[1] the moment kernel, ms[2] the first JFA launch (from the seed
+ * map: the first pass, or the first five where those run on residue classes),
+ * ms[3] update + finalize, ms[4] the whole JFA, ms[5] the whole step,
  * ms[6] the JFA pass count P, ms[7] the moment tile.
  * (No reference counterpart: the reference times stages with clock(),
  * source/main.cpp:181-242.) */

@@ -30,8 +30,11 @@ struct Ctx {
     uint32_t *seed = nullptr;      // seed map [H][W]
     bool seeds_valid = false;      // seed map holds the current sites
     uint32_t *lab[2] = {nullptr, nullptr};
-    uint32_t *first = nullptr;     // first JFA pass [H][W]: none except at the
-                                   // receivers of the current seeds while a JFA runs
+    uint32_t *first = nullptr;     // the JFA's first launch writes it [H][W]: the map
+                                   // after the lattice passes, or after a seed scatter
+                                   // (none except at the receivers of the current seeds
+                                   // while a JFA runs)
+    bool first_clean = true;       // `first` holds none everywhere between JFAs
     int final_buf = 0;             // lab[final_buf] = labels of the last JFA
     uint32_t *labels_map() const { return lab[final_buf]; }
     // a map the JFA's result does not live in (scratch for exports)
@@ -74,6 +77,7 @@ struct Ctx {
     ~Ctx();
     int enqueue_seed();
     void clear_seed_map();         // every pixel back to none()
+    void clean_first();            // `first` as the current sites' first launch needs it
     int enqueue_jfa(hipEvent_t after_first = nullptr);   // event recorded after pass 0
     int enqueue_moments();
     // defer: the update leaves its finalize (energy sums, history, stop rule,

@@ -2,10 +2,11 @@
 //
 // One cvt_ctx owns every device buffer of one grid for its whole life (the
 // reference allocates and frees about eleven N^2 buffers per gCVT call,
-// source/gcvt.cu:840-903).  A Lloyd iteration is P JFA launches (the first a
-// scatter of the seeds), one moment launch and one update launch (whose last
-// block also adds the energy partials and appends to the history); it is
-// captured once into a hipGraph
+// source/gcvt.cu:840-903).  A Lloyd iteration is the JFA's launches (the first
+// takes five passes where the grid and the site density allow it, and scatters
+// the seeds elsewhere), one moment launch and one update launch (whose energy
+// partials the next iteration's first launch adds and appends to the history);
+// it is captured once into a hipGraph
 // and replayed, so the host does no work per iteration and never
 // synchronises inside the loop (the reference copies the energy back every
 // 10th iteration, source/gcvt.cu:1080).
@@ -156,25 +157,47 @@ int Ctx::enqueue_jfa(hipEvent_t after_first)
     int step = jfa_first_step(W, H);
     const uint32_t *in = seed;
     int cur = 0;
-    // Pass 0 reads only the seed map: with three passes or more it scatters
-    // the seeds into `first`, which holds none except at their receivers
-    // (measured: 7.6 against 13.5 us at 2048^2, 6.9 against 7.8 at 512^2).
-    // Pass 1 resets the seed map it no longer needs, pass 2 resets `first`:
-    // both hold entries only around the seed pixels of sites [0, S) (the
+    // The first passes run on residue classes in one launch where the grid
+    // and the site density allow it (launch_jfa_lattice): it reads the seed
+    // map and writes `first` whole, and the launch after it resets the seed
+    // map, one store per seed pixel.
+    // Otherwise pass 0 reads only the seed map: with three passes or more it
+    // scatters the seeds into `first`, which holds none except at their
+    // receivers (measured: 7.6 against 13.5 us at 2048^2, 6.9 against 7.8 at
+    // 512^2).  Pass 1 resets the seed map it no longer needs, pass 2 resets
+    // `first`.
+    // Both maps hold entries only around the seed pixels of sites [0, S) (the
     // sites do not move during a JFA; compaction only shrinks the count).
-    const bool scatter = np >= 3;
+    const int done = jfa_lattice_passes(W, H, S);
+    const bool scatter = !done && np >= 3;
     const int step0 = step;
     // A deferred finalize of the previous iteration (the Lloyd iteration's
-    // site update leaves it pending) runs as one more workgroup of the seed
-    // scatter, or as its own launch when there is no scatter; either is a
+    // site update leaves it pending) runs as one more workgroup of the first
+    // launch, or as its own launch when that is a dense pass; either is a
     // no-op when nothing is pending.
     const FinalArgs fa = final_args(1, nullptr);
-    if (!scatter) enqueue_finalize();
-    // with a small site table the last five passes run fused (launch_jfa_tail)
-    const bool tail = use_tail && jfa_tail_ok(jplan, np);
-    for (int k = 0; k < np; ++k) {
-        if (tail && k == np - 5) {
-            launch_jfa_tail(stream, jplan, in, lab[cur], sites, W, H, dstate + ST_STOP);
+    // with a small site table the last passes run fused (launch_jfa_tail)
+    const int tail = use_tail ? jfa_tail_passes(jplan, np, done) : 0;
+    int k = 0;
+    if (done) {
+        // the JFA's last launch writes the map whose parity is the count of
+        // launches that follow; the other one is free
+        const int after = tail ? np - done - tail + 1 : np - done;
+        first_clean = false;
+        launch_jfa_lattice(stream, seed, first, lab[after & 1], sites, W, H, none(),
+                           dstate + ST_STOP, blockpart, dstate, &fa);
+        if (after_first) hipEventRecord(after_first, stream);
+        in = first;
+        step >>= done;
+        k = done;
+    } else if (!scatter) {
+        enqueue_finalize();
+    }
+    for (; k < np; ++k) {
+        if (tail && k == np - tail) {
+            const bool reset = done && k == done;
+            launch_jfa_tail(stream, jplan, tail, in, lab[cur], sites, W, H,
+                            reset ? seed : nullptr, none(), reset ? S : 0, dstate + ST_STOP);
             cur ^= 1;
             break;
         }
@@ -187,9 +210,9 @@ int Ctx::enqueue_jfa(hipEvent_t after_first)
             continue;
         }
         uint32_t *out = lab[cur];
-        uint32_t *clear = (k == 1) ? seed : (k == 2 && scatter) ? first : nullptr;
+        uint32_t *clear = (k == std::max(done, 1)) ? seed : (k == 2 && scatter) ? first : nullptr;
         launch_jfa_pass(stream, jplan, in, out, sites, W, H, step, clear, none(),
-                        clear ? S : 0, k == 2 ? step0 : 0, dstate + ST_STOP);
+                        clear ? S : 0, clear == first ? step0 : 0, dstate + ST_STOP);
         if (k == 0 && after_first) hipEventRecord(after_first, stream);
         in = out;
         cur ^= 1;
@@ -198,6 +221,14 @@ int Ctx::enqueue_jfa(hipEvent_t after_first)
     final_buf = cur ^ 1;
     seeds_valid = false;
     return hipGetLastError() == hipSuccess ? CVT_OK : fail(CVT_ERR_HIP, "jfa launch failed");
+}
+
+// `first` as the seed scatter needs it: the lattice launch leaves labels in it
+void Ctx::clean_first()
+{
+    if (first_clean || jfa_lattice_passes(W, H, S)) return;
+    hipLaunchKernelGGL(k_fill_u32, dim3(1024), dim3(256), 0, stream, first, none(), (long)W * H);
+    first_clean = true;
 }
 
 FinalArgs Ctx::final_args(int record, double *out_eg) const
@@ -331,8 +362,9 @@ int Ctx::lloyd_until(int max_iter, float omega, double rel_tol, int window, doub
                        window, ran);
     // A stop raised by the finalize inside a seed scatter can leave part of
     // that scatter's receivers in `first`, which holds none between JFAs:
-    // clear it.
-    hipLaunchKernelGGL(k_fill_u32, dim3(1024), dim3(256), 0, stream, first, none(), (long)W * H);
+    // clear it (the lattice launch writes all of it each time).
+    first_clean = false;
+    clean_first();
     int n = 0;
     if (hipMemcpyAsync(&n, ran, sizeof n, hipMemcpyDeviceToHost, stream) != hipSuccess ||
         hipStreamSynchronize(stream) != hipSuccess)
@@ -567,6 +599,7 @@ int cvt_set_sites(cvt_ctx *ctx, const float *xy, const uint8_t *fixed, int num_s
     const int oldS = c->S;
     c->S = num_sites;
     c->seeds_valid = false;
+    c->clean_first();
     c->enqueue_seed();
     if (c->tile_auto) {
         int rc = set_tile_internal(c, 0);
@@ -735,7 +768,8 @@ int cvt_profile(cvt_ctx *ctx, int iterations, float omega, double *ms)
     if (iterations < 1 || iterations > 1000 || !ms)
         return fail(CVT_ERR_ARG, "iterations %d (1..1000)", iterations);
     const int np = jfa_num_passes(c->W, c->H);
-    // five events per iteration bracket the phases (the first JFA pass, the
+    const int nd = np - std::max(1, jfa_lattice_passes(c->W, c->H, c->S));   // dense passes
+    // five events per iteration bracket the phases (the first JFA launch, the
     // other passes, moments, update); nothing in between, so the passes run
     // back to back as in a graph replay
     constexpr int NE = 5;
@@ -769,7 +803,7 @@ int cvt_profile(cvt_ctx *ctx, int iterations, float omega, double *ms)
     for (auto &e : ev) hipEventDestroy(e);
     if (rc) return rc;
     c->labels_fresh = true;
-    ms[0] = np > 1 ? acc[1] / ((double)iterations * (np - 1)) : acc[0] / iterations;
+    ms[0] = np > 1 ? acc[1] / ((double)iterations * nd) : acc[0] / iterations;
     ms[2] = np > 1 ? acc[0] / iterations : 0.0;
     ms[1] = acc[2] / iterations;
     ms[3] = acc[3] / iterations;

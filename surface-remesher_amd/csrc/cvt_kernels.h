@@ -4,10 +4,11 @@
 //   rho      fp32 [H][W]      density, unnormalised (scaled by rho_scale = 2^-k
 //                             in-kernel so that every scaled value is <= 1)
 //   seed     uint32 [H][W]    seed map: label of the site on that pixel, `none`
-//                             elsewhere; read by JFA pass 0, cleared by pass 1,
-//                             re-seeded by the site update
-//   first    uint32 [H][W]    output of JFA pass 0 (the seeds scattered to
-//                             their receivers); `none` elsewhere between JFAs
+//                             elsewhere; read by the JFA's first launch, cleared
+//                             by the next, re-seeded by the site update
+//   first    uint32 [H][W]    output of the JFA's first launch: the map after the
+//                             passes on residue classes, or the seeds scattered
+//                             to their receivers (`none` elsewhere between JFAs)
 //   lab[2]   uint32 [H][W]    JFA ping-pong label maps
 //   sites    float2 [capS+1]  site table, pixel units; sites[capS] = (inf, inf)
 //                             is the sentinel

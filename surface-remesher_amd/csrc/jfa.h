@@ -45,14 +45,29 @@ void launch_jfa_pass(hipStream_t st, const JfaPlan &plan, const uint32_t *in, ui
                      const float2 *sites, int W, int H, int step, uint32_t *clear, uint32_t none,
                      int nclear = 0, int rstep = 0, const int *stop = nullptr);
 
-// The last five passes (steps 8, 4, 2, 1, 1) fused into one launch over
-// 32 x 32 tiles with a 16-pixel halo staged in LDS, for plans whose site
-// table is staged whole in a 16 or 40 KB array and JFAs of eight passes or
-// more: out = those five passes applied to `in` (the step-16 map), bit for
-// bit.  `stop` as in launch_jfa_pass.
-bool jfa_tail_ok(const JfaPlan &plan, int passes);
-void launch_jfa_tail(hipStream_t st, const JfaPlan &plan, const uint32_t *in, uint32_t *out,
-                     const float2 *sites, int W, int H, const int *stop = nullptr);
+// The last passes (five: steps 8, 4, 2, 1, 1; or the last three or four of
+// them) fused into one launch over 32 x 32 tiles with a halo staged in LDS,
+// for plans whose site table is staged whole in a 16 or 40 KB array and JFAs
+// of eight passes or more: how many such a JFA takes with `done` passes run
+// by launch_jfa_lattice (0: none), and the launch: out = those passes applied
+// to `in`, bit for bit.  With a non-null clear that map is reset to `none` at
+// the seed pixels of sites [0, nclear).  `stop` as in launch_jfa_pass.
+int jfa_tail_passes(const JfaPlan &plan, int passes, int done);
+void launch_jfa_tail(hipStream_t st, const JfaPlan &plan, int passes, const uint32_t *in,
+                     uint32_t *out, const float2 *sites, int W, int H, uint32_t *clear,
+                     uint32_t none, int nclear, const int *stop = nullptr);
+
+// The first passes of a JFA in one launch over residue classes
+// (jfa_lattice.hip): how many a map of W x H pixels and S sites takes that way
+// (0: none), and the launch, which reads the seed map and writes the map after
+// those passes to `out`, every pixel of it.  scratch: a map that nothing else
+// reads or writes meanwhile.  The seed map is left as it is.  stop, blockpart,
+// dstate and fa as in launch_jfa_seed_pass.
+int jfa_lattice_passes(int W, int H, int S);
+void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out, uint32_t *scratch,
+                        const float2 *sites, int W, int H, uint32_t none,
+                        const int *stop = nullptr, const double *blockpart = nullptr,
+                        int *dstate = nullptr, const FinalArgs *fa = nullptr);
 
 // The first pass from a seed map (labels only at the seed pixels of sites
 // [0, S), none elsewhere), computed from the seeds into a map `out` that

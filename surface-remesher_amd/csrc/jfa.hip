@@ -866,8 +866,9 @@ __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa
 }
 
 // ---------------------------------------------------------------------------
-// Fused tail: the last five passes (steps 8, 4, 2, 1 and the extra 1) of one
-// map in one launch, for site tables that fit in LDS beside the tile.  Each
+// Fused tail: the last passes (steps 8, 4, 2, 1 and the extra 1, or the last
+// three or four of these) of one map in one launch, for site tables that fit
+// in LDS beside the tile.  Each
 // workgroup owns a kTailT x kTailT tile of the output.  It loads the tile and
 // a kTailHalo-pixel halo of the step-16 map into LDS and runs the five
 // passes there, each over the tile grown by the steps still to come (8, 4,
@@ -875,7 +876,7 @@ __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa
 // it.  Taps off the grid are redirected to the pixel's own row or column,
 // as in the dense pass, so the grid edges need no halo.  Each pixel takes
 // the (d, label) minimum over its nine taps with the dense pass's distance
-// formula: the map equals five dense passes bit for bit.
+// formula: the map equals the dense passes bit for bit.
 // ---------------------------------------------------------------------------
 static constexpr int kTailT = 32, kTailHalo = 16, kTailP = kTailT + 2 * kTailHalo;
 
@@ -883,8 +884,9 @@ template <int ENTRIES>
 __global__ __launch_bounds__(1024) void k_jfa_tail(const uint32_t *__restrict__ in,
                                                    uint32_t *__restrict__ out,
                                                    const float2 *__restrict__ sites, int table_f4,
-                                                   int W, int H, int tilesX,
-                                                   const int *__restrict__ stop)
+                                                   int W, int H, int tilesX, int skip,
+                                                   uint32_t *__restrict__ clear, uint32_t none,
+                                                   int nclear, const int *__restrict__ stop)
 {
     // the site table at LDS byte 0, then the two tile buffers
     __shared__ float4 lds_all[ENTRIES / 2 + kTailP * kTailP / 2];
@@ -894,10 +896,19 @@ __global__ __launch_bounds__(1024) void k_jfa_tail(const uint32_t *__restrict__ 
     const int tY = blockIdx.x / tilesX, tX = blockIdx.x - tY * tilesX;
     const int X0 = tX * kTailT, Y0 = tY * kTailT;
     const int bx = X0 - kTailHalo, by = Y0 - kTailHalo;   // the buffers' origin on the grid
-    const int halt = stop_word(stop);
+    SparseReset pro;
+    pro.halt = stop_word(stop);
+    pro.clear = clear;
+    pro.sites = sites;
+    pro.W = W;
+    pro.H = H;
+    pro.nclear = nclear;
+    pro.rstep = 0;
+    pro.none = none;
     {
-        const int x0 = max(bx, 0), x1 = min(X0 + kTailT + kTailHalo, W);
-        const int y0 = max(by, 0), y1 = min(Y0 + kTailT + kTailHalo, H);
+        const int halo = kTailHalo >> skip;
+        const int x0 = max(X0 - halo, 0), x1 = min(X0 + kTailT + halo, W);
+        const int y0 = max(Y0 - halo, 0), y1 = min(Y0 + kTailT + halo, H);
         const int w = x1 - x0, n = w * (y1 - y0);
         for (int i = tid; i < n; i += nt) {
             const int r = i / w, x = x0 + (i - r * w), y = y0 + r;
@@ -910,10 +921,10 @@ __global__ __launch_bounds__(1024) void k_jfa_tail(const uint32_t *__restrict__ 
     tab.n4 = table_f4;
     tab.base = 0;
     tab.stage();                     // ends with a barrier: buf0 is complete too
-    if (halt) return;
+    if (pro()) return;
     uint32_t *cur = buf0, *nxt = buf1;
 #pragma unroll 1
-    for (int k = 0; k < 5; ++k) {
+    for (int k = skip; k < 5; ++k) {
         const int s = k == 0 ? 8 : k == 1 ? 4 : k == 2 ? 2 : 1;
         const int g = k == 0 ? 8 : k == 1 ? 4 : k == 2 ? 2 : k == 3 ? 1 : 0;   // halo after
         const int x0 = max(X0 - g, 0), x1 = min(X0 + kTailT + g, W);
@@ -947,23 +958,26 @@ __global__ __launch_bounds__(1024) void k_jfa_tail(const uint32_t *__restrict__ 
     }
 }
 
-bool jfa_tail_ok(const JfaPlan &p, int passes)
+int jfa_tail_passes(const JfaPlan &p, int passes, int done)
 {
-    // the dense passes 1 and 2 (which reset the seed and first-pass maps)
-    // stay before the tail; the table fits beside the tile buffers
-    return passes >= 8 && (p.lds_entries == 2048 || p.lds_entries == 5120);
+    // without the lattice launch (done == 0) the dense passes 1 and 2, which
+    // reset the seed and first-pass maps, stay before the tail; the table
+    // fits beside the tile buffers
+    if (passes < 8 || (p.lds_entries != 2048 && p.lds_entries != 5120)) return 0;
+    return std::min(5, passes - done);
 }
 
-void launch_jfa_tail(hipStream_t st, const JfaPlan &p, const uint32_t *in, uint32_t *out,
-                     const float2 *sites, int W, int H, const int *stop)
+void launch_jfa_tail(hipStream_t st, const JfaPlan &p, int passes, const uint32_t *in,
+                     uint32_t *out, const float2 *sites, int W, int H, uint32_t *clear,
+                     uint32_t none, int nclear, const int *stop)
 {
     const int tx = (W + kTailT - 1) / kTailT, ty = (H + kTailT - 1) / kTailT;
     if (p.lds_entries == 2048)
         hipLaunchKernelGGL(k_jfa_tail<2048>, dim3(tx * ty), dim3(1024), 0, st, in, out, sites,
-                           p.table_f4, W, H, tx, stop);
+                           p.table_f4, W, H, tx, 5 - passes, clear, none, nclear, stop);
     else
         hipLaunchKernelGGL(k_jfa_tail<5120>, dim3(tx * ty), dim3(1024), 0, st, in, out, sites,
-                           p.table_f4, W, H, tx, stop);
+                           p.table_f4, W, H, tx, 5 - passes, clear, none, nclear, stop);
 }
 
 // ---------------------------------------------------------------------------

@@ -183,8 +183,9 @@ class Engine:
 
     def profile(self, iterations: int = 5, omega: float = 1.0) -> dict:
         """Eager Lloyd steps timed per phase with HIP events (ms); jfa_pass is
-        one dense JFA pass (passes 1 .. P-1, mean), jfa_first the first pass
-        (from the seed map)."""
+        one dense JFA pass (the passes after the first launch, mean),
+        jfa_first the first launch (from the seed map: one pass, or the first
+        five)."""
         ms = np.zeros(8, np.float64)
         call("cvt_profile", self._h, int(iterations), float(omega), _out_ptr(ms, np.float64, 8))
         return {"jfa_pass": ms[0], "jfa_first": ms[2], "moments": ms[1], "update": ms[3],

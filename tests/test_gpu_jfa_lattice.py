@@ -1,0 +1,81 @@
+"""The first five JFA passes on residue classes (csrc/jfa_lattice.hip): the
+label map equals the oracle's JFA bit for bit at the edges of the launch's
+rule and of its mask path."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def labels(W, H, xy):
+    import cvtamd
+    with cvtamd.Engine(W, H, len(xy)) as e:
+        e.set_sites(xy)
+        e.voronoi()
+        return e.labels()
+
+
+def random_sites(seed, W, H, S):
+    g = np.random.default_rng(seed)
+    return (g.random((S, 2)) * [W, H]).astype(np.float32)
+
+
+@pytest.mark.parametrize("W,H,S", [
+    (65, 65, 20),        # the smallest first step (64) that takes it
+    (128, 33, 20),       # the shortest side it takes, one lattice row of some classes
+    (129, 128, 80),      # a first step of 128 with one column beyond it
+    (255, 257, 300),     # odd in both sides, the last row and column ragged
+    (513, 300, 700),     # first step 512 on a grid barely above it
+    (1022, 768, 3900),   # width 2 mod 4 near the rule's 200 pixels per site
+    (2048, 1030, 10000), # sixteen-wave groups, ragged rows
+    (4096, 2051, 9000),  # eight-wave groups
+    (512, 512, 1),       # one site
+])
+def test_labels_equal_oracle(gpu, orc, W, H, S):
+    xy = random_sites(W + H + S, W, H, S)
+    assert np.array_equal(labels(W, H, xy), orc.jfa(W, H, xy))
+
+
+@pytest.mark.parametrize("n,per", [(512, 16), (512, 17), (512, 18), (2048, 17), (1024, 400)])
+def test_classes_at_and_past_the_mask_capacity(gpu, orc, n, per):
+    """`per` seeds in one residue class (16 fit a wave's masks; with 17 and
+    more the class takes the dense evaluation), the rest spread"""
+    first = 1 << ((n - 1).bit_length() - 1)
+    s = first // 16
+    g = np.random.default_rng(per)
+    cell = g.choice((n // s) ** 2, per, replace=False)
+    # pixels (5 mod s, 3 mod s), in a random label order
+    one = np.stack([s * (cell % (n // s)) + 5.5, s * (cell // (n // s)) + 3.25], 1)
+    xy = np.concatenate([one, g.random((n * n // 400, 2)) * n]).astype(np.float32)
+    xy = xy[g.permutation(len(xy))]
+    assert np.array_equal(labels(n, n, xy), orc.jfa(n, n, xy))
+
+
+def test_shared_pixels_ties_and_off_grid_sites(gpu, orc):
+    """equal sites, sites sharing a pixel, exact distance ties (sites on pixel
+    corners of a coarse grid) and sites off the grid"""
+    n = 256
+    a = np.arange(8, n, 32, dtype=np.float32)
+    grid = np.stack(np.meshgrid(a, a), -1).reshape(-1, 2)
+    xy = np.concatenate([grid, grid[::3], grid[::5] + np.float32(0.5),
+                         np.array([[-40, 30], [300, 300], [10, -200], [256, 256]], np.float32)])
+    xy = xy[np.random.default_rng(1).permutation(len(xy))].astype(np.float32)
+    assert np.array_equal(labels(n, n, xy), orc.jfa(n, n, xy))
+
+
+def test_site_counts_on_either_side_of_the_rule(gpu, orc):
+    """one engine, site sets that take the lattice launch, the seed scatter
+    and the lattice launch again: the maps the two keep between runs agree"""
+    import cvtamd
+    n = 256
+    with cvtamd.Engine(n, n, 4000) as e:
+        e.set_density(np.ones((n, n), np.float32))
+        for S in (300, 4000, 200, 330, 2000):
+            xy = random_sites(S, n, n, S)
+            e.set_sites(xy)
+            e.voronoi()
+            assert np.array_equal(e.labels(), orc.jfa(n, n, xy)), S
+            e.lloyd_until(9, target=1e30)
+            e.lloyd(3)
+            e.voronoi()
+            assert np.array_equal(e.labels(), orc.jfa(n, n, e.sites())), S
