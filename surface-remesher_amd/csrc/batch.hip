@@ -7,9 +7,9 @@
 // own sentinel at site_off + cap).  Labels are byte offsets into the whole
 // site table, so one label space serves all patches.
 //
-// One Lloyd iteration of the whole batch is Pmax JFA passes (patches run
-// their passes right-aligned; a pass is one launch per step class present in
-// it), one moment launch over the tiles of every patch, one update launch
+// One Lloyd iteration of the whole batch is Pmax JFA passes (the first five of
+// most patches in one launch over residue classes, the others one launch per
+// step class present in the pass; patches run their passes right-aligned), one moment launch over the tiles of every patch, one update launch
 // over the site blocks of every patch and one finalize launch (one block per
 // patch); it is captured once into a hipGraph.  Each patch's results equal a
 // single-patch run on the same inputs bit for bit: labels, moments (integer
@@ -166,7 +166,8 @@ struct Batch {
     int np = 0;
     std::vector<BatchPatch> hp;
     std::vector<BatchUnit> units;
-    std::vector<int> tile_patch, blk_patch;
+    std::vector<int> tile_patch, blk_patch, lat_patch;
+    std::vector<char> first_clean;   // the patch's part of `first` holds its `none`
     std::vector<char> have_density;
     std::vector<double> escale;
     long total_pix = 0;
@@ -176,10 +177,10 @@ struct Batch {
     hipStream_t stream = nullptr, own_stream = nullptr;
     BatchPatch *d_patch = nullptr;
     BatchUnit *d_units = nullptr;
-    int *d_tile_patch = nullptr, *d_blk_patch = nullptr;
+    int *d_tile_patch = nullptr, *d_blk_patch = nullptr, *d_lat_patch = nullptr;
     float *rho = nullptr;
     uint32_t *seed = nullptr, *lab0 = nullptr, *lab1 = nullptr;
-    uint32_t *first = nullptr;     // the seed scatter's output, `none` between JFAs
+    uint32_t *first = nullptr;     // output of the lattice launch and of the seed scatter
     int *d_site_patch = nullptr;   // patch of each site slot (-1: padding, sentinel)
     float2 *sites = nullptr;
     uint8_t *fixed = nullptr;
@@ -203,7 +204,7 @@ struct Batch {
         if (graph) (void)hipGraphDestroy(graph);
         void *b[] = {d_patch, d_units, d_tile_patch, d_blk_patch, rho, seed, lab0, lab1, sites,
                      fixed, slots, ovf, ovf_head, blockpart, hist, d_escale, hist_len, dstate,
-                     dflags, first, d_site_patch};
+                     dflags, first, d_site_patch, d_lat_patch};
         for (void *p : b)
             if (p) (void)hipFree(p);
         if (own_stream) (void)hipStreamDestroy(own_stream);
@@ -269,6 +270,28 @@ int Batch::plan()
         nblk += P.nblk;
         blk_patch.insert(blk_patch.end(), (size_t)P.nblk, p);
     }
+    // the patches whose first passes run on residue classes; the others need
+    // their part of `first` clean
+    lat_patch.clear();
+    for (int p = 0; p < np; ++p) {
+        BatchPatch &P = hp[p];
+        P.done = jfa_batch_lattice_passes(P.W, P.H, P.S);
+        P.lat_off = (int)lat_patch.size();
+        if (P.done) {
+            lat_patch.insert(lat_patch.end(), (size_t)jfa_batch_lattice_groups(P.W, P.H), p);
+            first_clean[p] = 0;
+        } else if (!first_clean[p]) {
+            hipLaunchKernelGGL(k_fill_u32, dim3(256), dim3(256), 0, stream, first + P.pix_off,
+                               8u * (uint32_t)(P.site_off + P.cap), (long)P.W * P.H);
+            first_clean[p] = 1;
+        }
+    }
+    if (d_lat_patch) (void)hipFree(d_lat_patch);
+    d_lat_patch = nullptr;
+    if (hipMalloc(&d_lat_patch, sizeof(int) * std::max<size_t>(1, lat_patch.size())) != hipSuccess)
+        return fail(CVT_ERR_NOMEM, "batch work tables");
+    (void)hipMemcpy(d_lat_patch, lat_patch.data(), sizeof(int) * lat_patch.size(),
+                    hipMemcpyHostToDevice);
     if (d_units) (void)hipFree(d_units);
     if (d_tile_patch) (void)hipFree(d_tile_patch);
     if (d_blk_patch) (void)hipFree(d_blk_patch);
@@ -318,7 +341,7 @@ unsigned Batch::pass_modes(int k) const
     unsigned m = 0;
     for (const BatchPatch &P : hp) {
         const int local = k - (pmax - P.passes);
-        if (local < 0) continue;
+        if (local < 0 || local < P.done) continue;
         if (local == 0 && P.passes >= 3) {
             m |= 8u;
             continue;
@@ -331,6 +354,8 @@ unsigned Batch::pass_modes(int k) const
 
 void Batch::enqueue_jfa()
 {
+    launch_jfa_batch_lattice(stream, d_patch, d_lat_patch, (int)lat_patch.size(), seed, first, lab0,
+                             sites);
     for (int k = 0; k < pmax; ++k) {
         const unsigned modes = pass_modes(k);
         if (modes & 8u)
@@ -393,6 +418,7 @@ int cvt_batch_create(cvt_batch **out, int num_patches, const int *widths, const 
     b->np = num_patches;
     b->hp.resize(num_patches);
     b->have_density.assign(num_patches, 0);
+    b->first_clean.assign(num_patches, 1);
     b->escale.assign(num_patches, 0.0);
     long pix = 0;
     int soff = 0, maxcap = 0;

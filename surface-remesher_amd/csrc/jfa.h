@@ -92,7 +92,9 @@ struct BatchPatch {
     int tile, tiles_x, tiles_y, tile_off;   // moment tiles
     int blk_off, nblk;         // update blocks [blk_off, blk_off + nblk)
     float rho_scale;           // 2^-k
-    float pad;
+    int done;                  // passes run by the lattice launch (0: none)
+    int lat_off;               // its first workgroup of that launch
+    int pad;
 };
 // a workgroup's share of a JFA pass: part b of the nb parts of one patch,
 // either its rows [y0, y1) (bands) or the b-th share of the pass's runs
@@ -105,11 +107,15 @@ struct BatchUnit {
 // lds_bytes) is staged in LDS.  One launch per step class in `modes` (bit 0:
 // step >= 4, bit 1: step 1, bit 2: step 2); a unit runs in the launch of its
 // patch's class.
-// A patch of three passes or more starts with a scatter of its seeds into
-// `first` (launch_jfa_batch_seeds, at the batched pass where its own pass 0
-// falls; its units skip that pass), reads `first` in its pass 1, which
-// resets the seed map at its seed pixels, and resets `first` at the seeds'
-// receivers in pass 2: both maps hold their patch's `none` between JFAs.
+// A patch whose first `done` passes run on residue classes
+// (launch_jfa_batch_lattice, before every batched pass) reads `first` in its
+// pass `done`, which resets the seed map at its seed pixels.  Any other patch
+// of three passes or more starts with a scatter of its seeds into `first`
+// (launch_jfa_batch_seeds, at the batched pass where its own pass 0 falls; its
+// units skip that pass), reads `first` in its pass 1, which resets the seed
+// map at its seed pixels, and resets `first` at the seeds' receivers in pass
+// 2: its part of `first` holds its `none` between JFAs, as every patch's part
+// of the seed map does.
 void launch_jfa_batch(hipStream_t st, const BatchPatch *patches, const BatchUnit *units, int nunits,
                       uint32_t *seed, uint32_t *first, uint32_t *lab0, uint32_t *lab1,
                       const float2 *sites, int pass, int pmax, size_t lds_bytes, unsigned modes);
@@ -118,5 +124,14 @@ void launch_jfa_batch(hipStream_t st, const BatchPatch *patches, const BatchUnit
 void launch_jfa_batch_seeds(hipStream_t st, const BatchPatch *patches, const int *site_patch,
                             int total_sites, const uint32_t *seed, uint32_t *first,
                             const float2 *sites, int pass, int pmax);
+
+// The passes on residue classes of every patch with done > 0: workgroups
+// [lat_off, lat_off + jfa_batch_lattice_groups) are the patch's, group_patch
+// names the patch of each.  jfa_batch_lattice_passes: the `done` of a patch.
+int jfa_batch_lattice_passes(int W, int H, int S);
+int jfa_batch_lattice_groups(int W, int H);
+void launch_jfa_batch_lattice(hipStream_t st, const BatchPatch *patches, const int *group_patch,
+                              int groups, const uint32_t *seed, uint32_t *first, uint32_t *scratch,
+                              const float2 *sites);
 
 }  // namespace cvt

@@ -1000,24 +1000,25 @@ __global__ __launch_bounds__(1024) void k_jfa_batch(const BatchPatch *__restrict
     const BatchUnit u = units[blockIdx.x];
     const BatchPatch P = patches[u.patch];
     const int local = pass - (pmax - P.passes);
-    if (local < 0) return;                                   // uniform per block
-    const bool scatter = P.passes >= 3;
+    if (local < P.done || local < 0) return;                 // uniform per block
+    const bool scatter = !P.done && P.passes >= 3;
     if (scatter && local == 0) return;                       // the seed scatter's pass
+    const int begin = P.done ? P.done : 1;                   // reads `first`, resets the seed map
     const int step = (local < P.passes - 1) ? (P.first_step >> local) : 1;
     if ((step == 1 ? STEP_1 : step == 2 ? STEP_2 : STEP_ANY) != MODE) return;
     uint32_t *bufs[2] = {lab0 + P.pix_off, lab1 + P.pix_off};
     const uint32_t *in = (local == 0)                 ? seed + P.pix_off
-                         : (local == 1 && scatter) ? first + P.pix_off
+                         : (local == begin && (scatter || P.done)) ? first + P.pix_off
                                                    : bufs[(local - 1) & 1];
     uint32_t *out = bufs[local & 1];
-    uint32_t *clear = (local == 1 && !scatter) ? seed + P.pix_off : nullptr;
+    uint32_t *clear = (local == 1 && !scatter && !P.done) ? seed + P.pix_off : nullptr;
     const uint32_t none = 8u * (uint32_t)(P.site_off + P.cap);
-    if (scatter && (local == 1 || local == 2)) {
-        // this unit's share of the sparse reset: the seed pixels (pass 1) or
-        // the seeds' receivers at the first step (pass 2); neither map is
-        // read or written by this pass
-        uint32_t *map = (local == 1 ? seed : first) + P.pix_off;
-        const int R = local == 2 ? 9 : 1;
+    if ((scatter && local == 2) || (local == begin && (scatter || P.done))) {
+        // this unit's share of the sparse reset: the seed pixels (the first
+        // dense pass) or the seeds' receivers at the first step (pass 2 after
+        // a scatter); neither map is read or written by this pass
+        uint32_t *map = (local == begin ? seed : first) + P.pix_off;
+        const int R = local == begin ? 1 : 9;
         const int s0 = (int)((long)P.S * u.b / u.nb), s1 = (int)((long)P.S * (u.b + 1) / u.nb);
         for (int t = threadIdx.x; t < R * (s1 - s0); t += blockDim.x) {
             const int i = s0 + t / R, r = t - R * (t / R);
@@ -1294,7 +1295,7 @@ __global__ __launch_bounds__(256) void k_jfa_batch_seeds(const BatchPatch *__res
     const int pid = site_patch[gi];
     if (pid < 0) return;
     const BatchPatch P = patches[pid];
-    if (pass - (pmax - P.passes) != 0 || P.passes < 3 || gi - P.site_off >= P.S) return;
+    if (pass - (pmax - P.passes) != 0 || P.done || P.passes < 3 || gi - P.site_off >= P.S) return;
     const int W = P.W, H = P.H, step = P.first_step;
     const float2 s = sites[gi];
     const int qx = seed_pixel(s.x, W), qy = seed_pixel(s.y, H);

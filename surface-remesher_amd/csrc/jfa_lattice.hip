@@ -420,6 +420,14 @@ __device__ __forceinline__ void lattice_group(LatLds<NW> &L, const uint32_t *see
     }
 }
 
+// blocks go to the 8 XCDs round robin: each XCD takes a contiguous stretch of
+// the n groups, so that groups sharing cache lines share an L2
+__device__ __forceinline__ int lattice_unit(int b, int n)
+{
+    const int q8 = n >> 3, r8 = n & 7, xcd = b & 7;
+    return xcd * q8 + min(xcd, r8) + (b >> 3);
+}
+
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_jfa_lattice(
     const uint32_t *seed, uint32_t *out, uint32_t *scratch, const float2 *__restrict__ sites, int W,
@@ -434,21 +442,39 @@ __global__ __launch_bounds__(64 * NW) void k_jfa_lattice(
         if (nb > 0 && threadIdx.x < 256) cvt_finalize_block(blockpart, nb, dstate, fa, red_e, red_g);
         return;
     }
-    // blocks go to the 8 XCDs round robin: each XCD takes a contiguous
-    // stretch of groups, so that groups sharing cache lines share an L2
-    const int n = (int)gridDim.x - fin, b = (int)blockIdx.x - fin;
-    const int q8 = n >> 3, r8 = n & 7, xcd = b & 7;
-    const int u = xcd * q8 + min(xcd, r8) + (b >> 3);
+    const int u = lattice_unit((int)blockIdx.x - fin, (int)gridDim.x - fin);
     const int gx = s / NW;
     const int ry = u / gx, rx0 = NW * (u - gx * ry);
     if (rx0 >= W) return;
     lattice_group<NW>(L, seed, out, scratch, sites, W, H, s, rx0, ry, none, stop);
 }
 
-int jfa_lattice_passes(int W, int H, int S)
+static constexpr int kBatchNW = 8;   // classes per workgroup of the batched launch
+
+__global__ __launch_bounds__(64 * kBatchNW) void k_jfa_batch_lattice(
+    const BatchPatch *__restrict__ patches, const int *__restrict__ group_patch,
+    const uint32_t *seed, uint32_t *first, uint32_t *scratch, const float2 *__restrict__ sites)
+{
+    __shared__ LatLds<kBatchNW> L;
+    const BatchPatch P = patches[group_patch[blockIdx.x]];
+    const int s = P.first_step / 16, gx = s / kBatchNW;
+    const int u = lattice_unit((int)blockIdx.x - P.lat_off, gx * s);
+    const int ry = u / gx, rx0 = kBatchNW * (u - gx * ry);
+    if (rx0 >= P.W) return;
+    lattice_group<kBatchNW>(L, seed + P.pix_off, first + P.pix_off, scratch + P.pix_off, sites,
+                            P.W, P.H, s, rx0, ry, 8u * (uint32_t)(P.site_off + P.cap), nullptr);
+}
+
+static int first_step(int W, int H)
 {
     int first = 1;
     while (2 * first < std::max(W, H)) first *= 2;
+    return first;
+}
+
+int jfa_lattice_passes(int W, int H, int S)
+{
+    const int first = first_step(W, H);
     // steps of 64 and more (a group of four classes is a quad of pixels), a
     // shorter side of at least half the first step (a class is 32 points long
     // and a wave's work does not shrink with its width), and few enough seeds
@@ -462,13 +488,10 @@ void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out, uin
                         const float2 *sites, int W, int H, uint32_t none, const int *stop,
                         const double *blockpart, int *dstate, const FinalArgs *fa)
 {
-    int first = 1;
-    while (2 * first < std::max(W, H)) first *= 2;
-    const int s = first / 16, fin = fa ? 1 : 0;
-    const int rows = std::min(s, H);
+    const int s = first_step(W, H) / 16, fin = fa ? 1 : 0;
     const FinalArgs f = fa ? *fa : FinalArgs();
 #define CVT_LATTICE(NW)                                                                        \
-    hipLaunchKernelGGL(k_jfa_lattice<NW>, dim3(s / NW * rows + fin), dim3(64 * NW), 0, st, seed, \
+    hipLaunchKernelGGL(k_jfa_lattice<NW>, dim3(s / NW * s + fin), dim3(64 * NW), 0, st, seed, \
                        out, scratch, sites, W, H, s, none, stop, fin, blockpart, dstate, f)
     // s^2 classes, one per wave.  Wide groups write whole cache lines, narrow
     // ones spread the waves over the CUs and wait for fewer others.  Measured
@@ -481,6 +504,27 @@ void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out, uin
     else
         CVT_LATTICE(4);
 #undef CVT_LATTICE
+}
+
+// (a first step of 128 or more: a workgroup's eight classes lie in one stride)
+int jfa_batch_lattice_passes(int W, int H, int S)
+{
+    return first_step(W, H) >= 16 * kBatchNW ? jfa_lattice_passes(W, H, S) : 0;
+}
+
+int jfa_batch_lattice_groups(int W, int H)
+{
+    const int s = first_step(W, H) / 16;
+    return s / kBatchNW * s;
+}
+
+void launch_jfa_batch_lattice(hipStream_t st, const BatchPatch *patches, const int *group_patch,
+                              int groups, const uint32_t *seed, uint32_t *first, uint32_t *scratch,
+                              const float2 *sites)
+{
+    if (groups > 0)
+        hipLaunchKernelGGL(k_jfa_batch_lattice, dim3(groups), dim3(64 * kBatchNW), 0, st, patches,
+                           group_patch, seed, first, scratch, sites);
 }
 
 }  // namespace cvt

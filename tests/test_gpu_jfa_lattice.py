@@ -79,3 +79,26 @@ def test_site_counts_on_either_side_of_the_rule(gpu, orc):
             e.lloyd(3)
             e.voronoi()
             assert np.array_equal(e.labels(), orc.jfa(n, n, e.sites())), S
+
+
+def test_batch_of_patches_on_both_sides_of_the_rule(gpu, orc):
+    """patches with and without the lattice launch in one batch (first steps of
+    32 .. 1024, ragged sides, dense and sparse sites), then other site counts
+    that swap them"""
+    import cvtamd
+    sizes = [(64, 64), (128, 100), (132, 150), (260, 300), (520, 512), (1100, 700), (300, 256)]
+    few = [20, 60, 90, 350, 1200, 3500, 3000]
+    many = [20, 60, 700, 3500, 1200, 3800, 300]
+    with cvtamd.Batch(sizes, [max(a, b) for a, b in zip(few, many)]) as b:
+        for counts in (few, many, few):
+            xys = [random_sites(k + n, w, h, n) for k, ((w, h), n) in enumerate(zip(sizes, counts))]
+            for k, ((w, h), xy) in enumerate(zip(sizes, xys)):
+                b.set_density(k, np.ones((h, w), np.float32))
+                b.set_sites(k, xy)
+            b.voronoi()
+            for k, ((w, h), xy) in enumerate(zip(sizes, xys)):
+                assert np.array_equal(b.labels(k), orc.jfa(w, h, xy)), (counts, k)
+            b.lloyd(2)
+            b.voronoi()
+            for k, (w, h) in enumerate(sizes):
+                assert np.array_equal(b.labels(k), orc.jfa(w, h, b.sites(k))), (counts, k)
