@@ -530,33 +530,27 @@ int cvt_set_density(cvt_ctx *ctx, const float *density)
     const long n = (long)c->W * c->H;
     HIPCHK(hipMemcpyAsync(c->rho, density, sizeof(float) * n, hipMemcpyDefault, c->stream),
            "density upload");
-    int zero = 0;
-    HIPCHK(hipMemcpyAsync(c->dflags + FLAG_BAD, &zero, sizeof zero, hipMemcpyHostToDevice, c->stream),
-           "flag reset");
-    const int nb = 1024;
-    hipLaunchKernelGGL(k_density_stats, dim3(nb), dim3(256), 0, c->stream, c->rho, n, c->scratch,
-                       c->dflags);
-    std::vector<float> bm(nb);
-    int bad = 0;
-    HIPCHK(hipMemcpyAsync(bm.data(), c->scratch, sizeof(float) * nb, hipMemcpyDeviceToHost, c->stream),
-           "density stats");
-    HIPCHK(hipMemcpyAsync(&bad, c->dflags + FLAG_BAD, sizeof bad, hipMemcpyDeviceToHost, c->stream),
-           "density flag");
+    uint32_t *stats = reinterpret_cast<uint32_t *>(c->scratch), st[2];
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->stream, stats, 0u, 2L);
+    hipLaunchKernelGGL(k_density_max, dim3(density_max_blocks(n)), dim3(1024),
+                       0, c->stream, c->rho, n, stats);
+    HIPCHK(hipMemcpyAsync(st, stats, sizeof st, hipMemcpyDeviceToHost, c->stream), "density stats");
     HIPCHK(hipStreamSynchronize(c->stream), "density stats");
-    if (bad) {
+    if (st[1]) {
         c->have_density = false;
         return fail(CVT_ERR_ARG, "density holds a negative, NaN or infinite value");
     }
-    float mx = 0.0f;
-    for (float v : bm) mx = std::max(mx, v);
+    float mx;
+    memcpy(&mx, &st[0], sizeof mx);
     // rho' = rho * 2^-rho_exp <= 1 keeps the fixed-point moment sums in range
     int ex = 0;
     if (mx > 0.0f) {
         frexp((double)mx, &ex);   // mx in [2^(ex-1), 2^ex)
     }
+    // (the captured iterations hold the scale, not the values)
+    if (c->rho_exp != ex) c->graph_valid = false;
     c->rho_exp = ex;
     c->have_density = true;
-    c->graph_valid = false;
     return CVT_OK;
 }
 
