@@ -14,14 +14,15 @@ namespace cvt {
 // 160 KB) when it fits, or, for larger tables, lds_entries = -20480: the
 // first 20478 entries and a zero entry in LDS, the rest gathered from global
 // memory;
-// otherwise one pixel per lane.
+// otherwise one pixel per lane.  tail_entries: the array (16 or 40 KB) that
+// launch_jfa_tail stages the table in, at any width; 0 when it is larger.
 // runs_mask < 0 (JFA_AUTO): runs where every wave of the launch gets one,
 // bands of rows elsewhere; otherwise bit k set = runs at step 2^k, clear =
 // bands (the labels do not depend on it).
 enum { JFA_AUTO = -1 };
 struct JfaPlan {
     bool quad = false, lds = false;
-    int grid = 0, threads = 0, table_f4 = 0, lds_entries = 0;
+    int grid = 0, threads = 0, table_f4 = 0, lds_entries = 0, tail_entries = 0;
     size_t lds_bytes = 0;
     int runs_mask = JFA_AUTO, blocks_per_cu = 0;
 };
@@ -47,8 +48,8 @@ void launch_jfa_pass(hipStream_t st, const JfaPlan &plan, const uint32_t *in, ui
 
 // The last passes (five: steps 8, 4, 2, 1, 1; or the last three or four of
 // them) fused into one launch over 32 x 32 tiles with a halo staged in LDS,
-// for plans whose site table is staged whole in a 16 or 40 KB array and JFAs
-// of eight passes or more: how many such a JFA takes with `done` passes run
+// for plans whose site table fits a 16 or 40 KB array and JFAs of eight passes
+// or more: how many such a JFA takes with `done` passes run
 // by launch_jfa_lattice (0: none), and the launch: out = those passes applied
 // to `in`, bit for bit.  With a non-null clear that map is reset to `none` at
 // the seed pixels of sites [0, nclear).  `stop` as in launch_jfa_pass.

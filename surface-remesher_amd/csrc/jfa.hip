@@ -963,7 +963,7 @@ int jfa_tail_passes(const JfaPlan &p, int passes, int done)
     // without the lattice launch (done == 0) the dense passes 1 and 2, which
     // reset the seed and first-pass maps, stay before the tail; the table
     // fits beside the tile buffers
-    if (passes < 8 || (p.lds_entries != 2048 && p.lds_entries != 5120)) return 0;
+    if (passes < 8 || p.tail_entries == 0) return 0;
     return std::min(5, passes - done);
 }
 
@@ -972,7 +972,7 @@ void launch_jfa_tail(hipStream_t st, const JfaPlan &p, int passes, const uint32_
                      uint32_t none, int nclear, const int *stop)
 {
     const int tx = (W + kTailT - 1) / kTailT, ty = (H + kTailT - 1) / kTailT;
-    if (p.lds_entries == 2048)
+    if (p.tail_entries == 2048)
         hipLaunchKernelGGL(k_jfa_tail<2048>, dim3(tx * ty), dim3(1024), 0, st, in, out, sites,
                            p.table_f4, W, H, tx, 5 - passes, clear, none, nclear, stop);
     else
@@ -1116,6 +1116,9 @@ JfaPlan plan_jfa(int W, int H, int capS, int runs_mask, int blocks_per_cu)
     p.table_f4 = (capS + 2) / 2;
     const int entries = 2 * p.table_f4;
     p.lds_entries = 0;
+    p.tail_entries = entries <= kLdsEntries[0]   ? kLdsEntries[0]
+                     : entries <= kLdsEntries[1] ? kLdsEntries[1]
+                                                 : 0;
     if (p.quad) {
         for (int e : kLdsEntries)
             if (entries <= e) { p.lds_entries = e; break; }

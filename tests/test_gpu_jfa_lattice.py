@@ -102,3 +102,17 @@ def test_batch_of_patches_on_both_sides_of_the_rule(gpu, orc):
             b.voronoi()
             for k, (w, h) in enumerate(sizes):
                 assert np.array_equal(b.labels(k), orc.jfa(w, h, b.sites(k))), (counts, k)
+
+
+@pytest.mark.parametrize("W,H,S", [
+    (65, 70, 2000),      # no lattice launch: dense passes, then five fused
+    (130, 129, 90),      # lattice, then the last four fused
+    (127, 66, 40),       # lattice, then the last three fused
+    (301, 33, 2047),     # the largest 16 KB table
+    (517, 260, 2048),    # the smallest 40 KB table
+    (1021, 530, 5118),   # the largest 40 KB table
+    (1021, 530, 5119),   # too large for the fused passes
+])
+def test_fused_tail_at_widths_not_a_multiple_of_four(gpu, orc, W, H, S):
+    xy = random_sites(7 * W + S, W, H, S)
+    assert np.array_equal(labels(W, H, xy), orc.jfa(W, H, xy))
