@@ -21,10 +21,12 @@
 //             holds them (orientation tests against the new point)
 //   flip      Lawson flips until no edge is illegal: every illegal edge bids
 //             its id (3 t + i, t the lower triangle) on both its triangles,
-//             an edge that wins both flips, the outer neighbours are re-linked
-//             through per-edge forwarding records, and points follow their
-//             triangle across the new diagonal.  The lowest illegal edge
-//             always wins, so every round makes progress.
+//             an edge that wins both flips, and the outer neighbours are
+//             re-linked through per-edge forwarding records.  The lowest
+//             illegal edge always wins, so every pass makes progress.  A pass
+//             works on lists: the triangles that changed, the illegal edges
+//             found among them.  Points whose triangle was flipped walk to
+//             the one that holds them when they next bid.
 // Predicates are exact, and exactly degenerate cases (three collinear, four
 // cocircular points) are decided by a symbolic perturbation of the points
 // by index (Simulation of Simplicity, dt_predicates.h), as gDel2D does
@@ -54,7 +56,13 @@ namespace cvt {
 using namespace dt;
 
 enum { C_UNINS = 0, C_DUP = 1, C_ERR = 2, C_FLIPS = 3, C_A = 4, C_B = 5, C_C = 6, C_FTOT = 7,
-       C_MISS = 8, C_NCROSS = 9, C_WSLOT = 10, NUM_C = 12 };
+       C_MISS = 8, C_NCROSS = 9, C_WSLOT = 10,
+       // triangles listed for a flip pass and edges found illegal by it, one
+       // word each for even and odd passes of a flip run; the run's passes
+       // that flipped; whether it converged; triangles to split; passes the
+       // last k_dt_flip_tail ran
+       C_LIST = 11, C_CAND = 13, C_PASSES = 15, C_CONV = 16, C_SPLITS = 17, C_RAN = 18,
+       NUM_C = 20 };
 static constexpr int kParts = 256;              // workgroups of the first-triangle search
 static constexpr unsigned long long NO_BID = ~0ull;
 static constexpr int NO_FLIP = 0x7fffffff;
@@ -296,6 +304,34 @@ __device__ __forceinline__ int inf_pos(const int *v, int I)
     return v[0] == I ? 0 : v[1] == I ? 1 : v[2] == I ? 2 : -1;
 }
 
+// The triangle that holds point q, walking from triangle t: across an edge q
+// lies strictly beyond (a Delaunay triangulation has no such cycle), around
+// the hull by the rays from O, and in from the wedge that holds q.  Under the
+// perturbation exactly one triangle holds q.  The step bound guards a broken
+// mesh.
+__device__ __forceinline__ int walk_point(const Pt *P, int n, const int *tv, const int *to, int q,
+                                          int t, int T, int *err)
+{
+    for (int step = 0; step < 2 * T + 64; ++step) {
+        const int v[3] = {tv[3 * t], tv[3 * t + 1], tv[3 * t + 2]};
+        const int k = inf_pos(v, n);
+        int e = -1;
+        if (k < 0) {
+            for (int i = 0; i < 3 && e < 0; ++i)
+                if (orient_p(P, v[(i + 1) % 3], v[(i + 2) % 3], q, err) < 0) e = i;
+        } else {
+            const int u = v[(k + 1) % 3], w = v[(k + 2) % 3];
+            if (orient_p(P, n, u, q, err) > 0) e = (k + 2) % 3;
+            else if (orient_p(P, n, w, q, err) < 0) e = (k + 1) % 3;
+            else if (orient_p(P, u, w, q, err) < 0) e = k;
+        }
+        if (e < 0) return t;
+        t = to[3 * t + e] >> 4;
+    }
+    set_flag(err, DT_ERR_DEGENERATE);
+    return t;
+}
+
 // atomicMin of each lane's bid on vote[t], one atomic per distinct t in the
 // wave (in early rounds most of a wave's points share a triangle); called
 // by every lane of the wave
@@ -353,17 +389,24 @@ __device__ __forceinline__ unsigned long long point_bid(const Pt *P, int n, cons
 }
 
 __global__ __launch_bounds__(256) void k_dt_vote(const Pt *__restrict__ P, int n,
-                                                 const int *__restrict__ tv,
+                                                 int T, const int *__restrict__ tv,
+                                                 const int *__restrict__ to,
+                                                 const int *__restrict__ fstamp, int first,
                                                  int *__restrict__ loc,
                                                  unsigned long long *__restrict__ vote,
                                                  int *__restrict__ cnt)
 {
+    if (!cnt[C_CONV]) return;              // the flips before this round go on
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     bool live = false, dup = false;
     int t = -1;
     unsigned long long bid = NO_BID;
     if (p < n && loc[p] >= 0) {
         t = loc[p];
+        if (fstamp[t] >= first) {          // flipped since p last bid
+            t = walk_point(P, n, tv, to, p, t, T, cnt + C_ERR);
+            loc[p] = t;
+        }
         int dupv;
         bid = point_bid(P, n, tv, p, t, dupv);
         dup = dupv >= 0;
@@ -382,19 +425,26 @@ __global__ __launch_bounds__(256) void k_dt_vote(const Pt *__restrict__ P, int n
 static constexpr int kVoteLds = 4096;
 __global__ __launch_bounds__(1024) void k_dt_vote_lds(const Pt *__restrict__ P, int n, int T,
                                                       const int *__restrict__ tv,
+                                                      const int *__restrict__ to,
+                                                      const int *__restrict__ fstamp, int first,
                                                       int *__restrict__ loc,
                                                       unsigned long long *__restrict__ vote,
                                                       int *__restrict__ cnt)
 {
     __shared__ unsigned long long sv[kVoteLds];
     __shared__ int scount[2];
+    if (!cnt[C_CONV]) return;
     for (int i = threadIdx.x; i < T; i += blockDim.x) sv[i] = NO_BID;
     if (threadIdx.x < 2) scount[threadIdx.x] = 0;
     __syncthreads();
     int live = 0, dups = 0;
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-        const int t = loc[p];
+        int t = loc[p];
         if (t < 0) continue;
+        if (fstamp[t] >= first) {
+            t = walk_point(P, n, tv, to, p, t, T, cnt + C_ERR);
+            loc[p] = t;
+        }
         int dupv;
         const unsigned long long bid = point_bid(P, n, tv, p, t, dupv);
         if (dupv >= 0) {
@@ -433,9 +483,14 @@ __device__ __forceinline__ int child_slot(int t, int i, int T, const int *base)
 __global__ void k_dt_split(const Pt *__restrict__ P, int n, int T, int *__restrict__ tv,
                            int *__restrict__ to, const unsigned long long *__restrict__ vote,
                            const int *__restrict__ base, int *__restrict__ loc,
-                           int *__restrict__ chk, int next_pass, int *__restrict__ cnt)
+                           int *__restrict__ chk, int next_pass, int *__restrict__ list,
+                           int *__restrict__ cnt)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) {                          // the flip run that follows checks the children
+        cnt[C_LIST] = 3 * base[T];
+        cnt[C_LIST + 1] = cnt[C_CAND] = cnt[C_CAND + 1] = cnt[C_PASSES] = cnt[C_CONV] = 0;
+    }
     if (t >= T || vote[t] == NO_BID) return;
     int *err = cnt + C_ERR;
     const int p = (int)(vote[t] & 0xffffffffu);
@@ -452,6 +507,7 @@ __global__ void k_dt_split(const Pt *__restrict__ P, int n, int T, int *__restri
     for (int i = 0; i < 3; ++i) {
         const int s = slot[i];
         chk[s] = next_pass;
+        list[3 * base[t] + i] = s;
         tv[3 * s] = v[(i + 1) % 3];
         tv[3 * s + 1] = v[(i + 2) % 3];
         tv[3 * s + 2] = p;
@@ -524,128 +580,231 @@ __device__ __forceinline__ bool illegal(const Pt *P, int n, const int *v, int w,
     return orient_p(P, v[(k + 1) % 3], v[(k + 2) % 3], w, err) > 0;
 }
 
-// an edge can turn illegal only when one of its triangles changed (split or
-// flipped) before this pass: chk[t] holds the pass that must look at t
-__global__ void k_dt_flip_mark(const Pt *__restrict__ P, int n, int T, const int *__restrict__ tv,
-                               const int *__restrict__ to, const int *__restrict__ chk, int pass,
-                               int *__restrict__ fvote, int *__restrict__ cnt)
+// ---------------------------------------------------------------------------
+// A flip pass.  An edge can turn illegal only when one of its triangles
+// changed (split or flipped) before the pass, so the pass looks at a list of
+// triangles (chk[t] == pass for each) and leaves the next pass's: every
+// triangle with an illegal edge, whether that edge flipped or lost its bid to
+// a lower one.  Three steps, each over a list, with everything before it done:
+//   mark   the illegal edges of the listed triangles bid and are listed
+//   flip   the edges that won both bids
+//   fix    the links around the flipped pairs; the bids reset
+// A full-size pass takes a launch per step.  Once few triangles are left, one
+// workgroup runs pass after pass (k_dt_flip_tail): the passes of 16 K points
+// then cost about 3 us instead of three launches of 4 to 12 us, most passes of
+// every round being small.  At 1 M points the lists replaced three scans of
+// 2 M triangles and 1 M points a pass (20, 15 and 8 us).
+// ---------------------------------------------------------------------------
+struct FlipArgs {
+    const Pt *P;
+    int n;
+    int *tv, *to, *chk, *fvote, *fwd, *fstamp;
+    int *list[2];             // triangles of even / odd passes of the run
+    int4 *cand;               // illegal edges: t, m, edge of t | edge of m << 2, flipped
+    int *cnt;
+};
+
+// chk and fvote are changed by atomics in the pass that reads them: read where
+// those are performed
+__device__ __forceinline__ int dev_load(const int *p)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) cnt[C_FLIPS] = 0;                  // this pass's flips (k_dt_flip counts)
-    if (t >= T) return;
-    int *err = cnt + C_ERR;
-    const bool mine = chk[t] == pass;
-    const int v[3] = {tv[3 * t], tv[3 * t + 1], tv[3 * t + 2]};
-    for (int i = 0; i < 3; ++i) {
-        const int r = to[3 * t + i];
-        const int m = r >> 4;
-        if (r < 0 || m < t) continue;               // each edge once, by its lower triangle
-        if (r & 4) continue;                        // a constraint edge never flips
-        if (!mine && chk[m] != pass) continue;
-        const int w = tv[3 * m + (r & 3)];
-        if (illegal(P, n, v, w, err)) {
-            const int id = 3 * t + i;
-            atomicMin(&fvote[t], id);
-            atomicMin(&fvote[m], id);
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// next free place of a list, one atomic per wave; called by the lanes that push
+__device__ __forceinline__ int push_slot(int *counter)
+{
+    const unsigned long long m = __ballot(1);
+    const int lane = threadIdx.x & 63, lead = __ffsll((long long)m) - 1;
+    int base = 0;
+    if (lane == lead) base = atomicAdd(counter, __popcll(m));
+    return __shfl(base, lead) + __popcll(m & ((1ull << lane) - 1ull));
+}
+
+// edge e of listed triangle u
+__device__ __forceinline__ void flip_mark(const FlipArgs &a, int u, int e, int pass, int *ncand)
+{
+    const int r = a.to[3 * u + e], m = r >> 4, k = r & 3;
+    if (r < 0 || (r & 4)) return;                 // a constraint edge never flips
+    if (m < u && dev_load(&a.chk[m]) == pass) return;   // the lower triangle looks at it
+    // the test is the lower triangle's
+    const int t = min(u, m), o = max(u, m);
+    const int i = t == u ? e : k, j = t == u ? k : e;
+    const int v[3] = {a.tv[3 * t], a.tv[3 * t + 1], a.tv[3 * t + 2]};
+    if (!illegal(a.P, a.n, v, a.tv[3 * o + j], a.cnt + C_ERR)) return;
+    const int id = 3 * t + i;
+    atomicMin(&a.fvote[t], id);
+    atomicMin(&a.fvote[o], id);
+    a.cand[push_slot(ncand)] = make_int4(t, o, i | (j << 2), 0);
+}
+
+// flip of the edge i of t shared with edge k of m, if it won both bids: t' =
+// (v_i, v_i+1, w) in slot t, m' = (w, v_i+2, v_i) in slot m; the outer links
+// are kept as they were (fixed by flip_fix) and each old outer edge forwards
+// to its new place in fwd[3 * slot + old edge]
+__device__ __forceinline__ bool flip_do(const FlipArgs &a, int idx, int pass, int *next,
+                                        int *nnext)
+{
+    const int4 c = a.cand[idx];
+    const int t = c.x, m = c.y, i = c.z & 3, k = c.z >> 2;
+    if (atomicExch(&a.chk[t], pass + 1) != pass + 1) next[push_slot(nnext)] = t;
+    if (atomicExch(&a.chk[m], pass + 1) != pass + 1) next[push_slot(nnext)] = m;
+    const int id = 3 * t + i;
+    if (dev_load(&a.fvote[t]) != id || dev_load(&a.fvote[m]) != id) return false;
+    int *tv = a.tv, *to = a.to, *fwd = a.fwd;
+    const int vi = tv[3 * t + i], vi1 = tv[3 * t + (i + 1) % 3], vi2 = tv[3 * t + (i + 2) % 3];
+    const int w = tv[3 * m + k];
+    const int ot1 = to[3 * t + (i + 1) % 3], ot2 = to[3 * t + (i + 2) % 3];
+    const int om1 = to[3 * m + (k + 1) % 3], om2 = to[3 * m + (k + 2) % 3];
+    tv[3 * t] = vi;
+    tv[3 * t + 1] = vi1;
+    tv[3 * t + 2] = w;
+    tv[3 * m] = w;
+    tv[3 * m + 1] = vi2;
+    tv[3 * m + 2] = vi;
+    // t': edge 0 = (vi1, w) was m's edge k+1; edge 1 = diagonal;
+    //     edge 2 = (vi, vi1) was t's edge i+2
+    // m': edge 0 = (vi2, vi) was t's edge i+1; edge 1 = diagonal;
+    //     edge 2 = (w, vi2) was m's edge k+2
+    to[3 * t] = om1;
+    to[3 * t + 1] = (m << 4) | 1;
+    to[3 * t + 2] = ot2;
+    to[3 * m] = ot1;
+    to[3 * m + 1] = (t << 4) | 1;
+    to[3 * m + 2] = om2;
+    fwd[3 * t + (i + 2) % 3] = (t << 4) | 2;
+    fwd[3 * t + (i + 1) % 3] = (m << 4) | 0;
+    fwd[3 * m + (k + 1) % 3] = (t << 4) | 0;
+    fwd[3 * m + (k + 2) % 3] = (m << 4) | 2;
+    a.fstamp[t] = pass;
+    a.fstamp[m] = pass;
+    a.cand[idx].w = 1;
+    return true;
+}
+
+// re-links the outer edges of a flipped pair (through the forwarding records
+// of flipped neighbours) and resets the bids of a listed edge's triangles
+__device__ __forceinline__ void flip_fix(const FlipArgs &a, int idx, int pass)
+{
+    const int4 c = a.cand[idx];
+    a.fvote[c.x] = NO_FLIP;
+    a.fvote[c.y] = NO_FLIP;
+    if (!c.w) return;
+    for (int s = 0; s < 2; ++s) {
+        const int i = s ? c.y : c.x;
+        for (int e = 0; e < 3; e += 2) {
+            const int r = a.to[3 * i + e];
+            const int m = r >> 4, k = r & 3;
+            // bit 2 marks a constraint edge on both of its sides
+            if (a.fstamp[m] == pass)
+                a.to[3 * i + e] = a.fwd[3 * m + k] | (r & 4);
+            else
+                a.to[3 * m + k] = (i << 4) | e | (r & 4);
         }
     }
 }
 
-// flip of the edge i of t shared with edge k of m: t' = (v_i, v_i+1, w) in
-// slot t, m' = (w, v_i+2, v_i) in slot m; the outer links are kept as they
-// were (fixed by k_dt_flip_fix) and each old outer edge forwards to its new
-// place in fwd[3 * slot + old edge]
-__global__ void k_dt_flip(int T, int *__restrict__ tv, int *__restrict__ to,
-                          const int *__restrict__ fvote, int *__restrict__ fwd,
-                          int *__restrict__ fstamp, int4 *__restrict__ fdiag, int *__restrict__ chk,
-                          int round, int *__restrict__ cnt)
+// the steps of pass `pass`, whose list is list[par]
+__global__ __launch_bounds__(256) void k_dt_flip_mark(FlipArgs a, int par, int pass)
+{
+    const int n = 3 * a.cnt[C_LIST + par];
+    for (int x = blockIdx.x * 256 + threadIdx.x; x < n; x += gridDim.x * 256)
+        flip_mark(a, a.list[par][x / 3], x % 3, pass, a.cnt + C_CAND + par);
+}
+
+__global__ __launch_bounds__(256) void k_dt_flip(FlipArgs a, int par, int pass)
+{
+    const int n = a.cnt[C_CAND + par];
+    int did = 0;
+    for (int x = blockIdx.x * 256 + threadIdx.x; x < n; x += gridDim.x * 256)
+        did += flip_do(a, x, pass, a.list[par ^ 1], a.cnt + C_LIST + (par ^ 1));
+    for (int o = 32; o > 0; o >>= 1) did += __shfl_xor(did, o);
+    if ((threadIdx.x & 63) == 0 && did) atomicAdd(a.cnt + C_FTOT, did);
+}
+
+__global__ __launch_bounds__(256) void k_dt_flip_fix(FlipArgs a, int par, int pass)
+{
+    const int n = a.cnt[C_CAND + par];
+    for (int x = blockIdx.x * 256 + threadIdx.x; x < n; x += gridDim.x * 256) flip_fix(a, x, pass);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.cnt[C_LIST + par] = 0;               // the pass after the next writes these
+        a.cnt[C_CAND + (par ^ 1)] = 0;
+        a.cnt[C_PASSES] += n > 0;
+    }
+}
+
+// Pass after pass by one workgroup while the list is not empty and holds at
+// most kTailList triangles; `done` passes of the run came before.  Publishes
+// the counters for the host.
+static constexpr int kTailList = 2048;
+__global__ __launch_bounds__(1024) void k_dt_flip_tail(FlipArgs a, int done, int pass,
+                                                       int max_passes)
+{
+    __shared__ int nlist[2], ncand;
+    __shared__ int flips;
+    int par = done & 1;
+    if (threadIdx.x == 0) {
+        nlist[par] = a.cnt[C_LIST + par];
+        nlist[par ^ 1] = 0;
+        ncand = 0;
+        flips = 0;
+    }
+    __syncthreads();
+    int ran = 0, flipped = 0;
+    for (; ran < max_passes; ++ran, ++pass, par ^= 1) {
+        const int n = nlist[par];
+        if (n == 0 || n > kTailList) break;
+        for (int x = threadIdx.x; x < 3 * n; x += 1024)
+            flip_mark(a, a.list[par][x / 3], x % 3, pass, &ncand);
+        __syncthreads();
+        const int nc = ncand;
+        int did = 0;
+        for (int x = threadIdx.x; x < nc; x += 1024)
+            did += flip_do(a, x, pass, a.list[par ^ 1], &nlist[par ^ 1]);
+        if (did) atomicAdd(&flips, did);
+        __syncthreads();
+        for (int x = threadIdx.x; x < nc; x += 1024) flip_fix(a, x, pass);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            nlist[par] = 0;
+            ncand = 0;
+        }
+        __syncthreads();
+        flipped += nc > 0;
+    }
+    if (threadIdx.x == 0) {
+        a.cnt[C_LIST + par] = nlist[par];
+        a.cnt[C_LIST + (par ^ 1)] = 0;
+        a.cnt[C_CAND] = a.cnt[C_CAND + 1] = 0;
+        a.cnt[C_PASSES] += flipped;
+        a.cnt[C_RAN] = ran;
+        a.cnt[C_CONV] = nlist[par] == 0;
+        a.cnt[C_FTOT] += flips;
+    }
+}
+
+// every triangle on the list of a run's first pass
+__global__ void k_dt_list_all(int T, int *__restrict__ list, int *__restrict__ chk, int pass,
+                              int *__restrict__ cnt)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    bool did = false;
+    if (t == 0) {
+        cnt[C_LIST] = T;
+        cnt[C_LIST + 1] = cnt[C_CAND] = cnt[C_CAND + 1] = cnt[C_PASSES] = cnt[C_CONV] = 0;
+    }
     if (t < T) {
-        const int id = fvote[t];
-        // a triangle with an illegal edge is looked at again next pass,
-        // whether that edge flips now or lost the bid to a lower one
-        if (id != NO_FLIP) chk[t] = round + 1;
-        if (id != NO_FLIP && id / 3 == t) {
-            const int i = id - 3 * t;
-            const int r = to[3 * t + i], m = r >> 4, k = r & 3;
-            if (fvote[m] == id) {
-                did = true;
-                const int vi = tv[3 * t + i], vi1 = tv[3 * t + (i + 1) % 3],
-                          vi2 = tv[3 * t + (i + 2) % 3];
-                const int w = tv[3 * m + k];
-                const int ot1 = to[3 * t + (i + 1) % 3], ot2 = to[3 * t + (i + 2) % 3];
-                const int om1 = to[3 * m + (k + 1) % 3], om2 = to[3 * m + (k + 2) % 3];
-                tv[3 * t] = vi;
-                tv[3 * t + 1] = vi1;
-                tv[3 * t + 2] = w;
-                tv[3 * m] = w;
-                tv[3 * m + 1] = vi2;
-                tv[3 * m + 2] = vi;
-                // t': edge 0 = (vi1, w) was m's edge k+1; edge 1 = diagonal;
-                //     edge 2 = (vi, vi1) was t's edge i+2
-                // m': edge 0 = (vi2, vi) was t's edge i+1; edge 1 = diagonal;
-                //     edge 2 = (w, vi2) was m's edge k+2
-                to[3 * t] = om1;
-                to[3 * t + 1] = (m << 4) | 1;
-                to[3 * t + 2] = ot2;
-                to[3 * m] = ot1;
-                to[3 * m + 1] = (t << 4) | 1;
-                to[3 * m + 2] = om2;
-                fwd[3 * t + (i + 2) % 3] = (t << 4) | 2;
-                fwd[3 * t + (i + 1) % 3] = (m << 4) | 0;
-                fwd[3 * m + (k + 1) % 3] = (t << 4) | 0;
-                fwd[3 * m + (k + 2) % 3] = (m << 4) | 2;
-                fstamp[t] = round;
-                fstamp[m] = round;
-                chk[t] = round + 1;
-                chk[m] = round + 1;
-                const int4 d = make_int4(vi, w, t, m);
-                fdiag[t] = d;
-                fdiag[m] = d;
-            }
-        }
-    }
-    const int c = __syncthreads_count(did);
-    if (threadIdx.x == 0 && c) {
-        atomicAdd(cnt + C_FLIPS, c);
-        atomicAdd(cnt + C_FTOT, c);
+        list[t] = t;
+        chk[t] = pass;
     }
 }
 
-// after a flip pass, per triangle t < T: re-link the outer edges of flipped
-// triangles (through the forwarding records of flipped neighbours) and
-// reset the bid for the next pass; per point q < n: follow a flipped
-// triangle across its new diagonal
-__global__ void k_dt_flip_fix(const Pt *__restrict__ P, int n, int T, int *__restrict__ to,
-                              const int *__restrict__ fwd, const int *__restrict__ fstamp,
-                              const int4 *__restrict__ fdiag, int *__restrict__ fvote,
-                              int *__restrict__ loc, int round, int *__restrict__ cnt)
+// what the host waits for, written to its pinned memory
+__global__ void k_dt_publish(const int *__restrict__ cnt, const int *__restrict__ splits,
+                             int *__restrict__ host)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < T) {
-        fvote[i] = NO_FLIP;
-        if (fstamp[i] == round) {
-            for (int e = 0; e < 3; e += 2) {
-                const int r = to[3 * i + e];
-                const int m = r >> 4, k = r & 3;
-                // bit 2 marks a constraint edge on both of its sides
-                if (fstamp[m] == round)
-                    to[3 * i + e] = fwd[3 * m + k] | (r & 4);
-                else
-                    to[3 * m + k] = (i << 4) | e | (r & 4);
-            }
-        }
-    }
-    if (i < n) {
-        const int t = loc[i];
-        if (t >= 0 && fstamp[t] == round) {
-            const int4 d = fdiag[t];
-            // t' = (vi, vi1, w) lies right of vi -> w
-            loc[i] = orient_p(P, d.x, d.y, i, cnt + C_ERR) < 0 ? d.z : d.w;
-        }
-    }
+    if (threadIdx.x < NUM_C) host[threadIdx.x] = cnt[threadIdx.x];
+    __threadfence_system();
+    if (threadIdx.x == 0 && splits) host[C_SPLITS] = *splits;
 }
 
 // ---------------------------------------------------------------------------
@@ -976,7 +1135,8 @@ struct DtCtx {
     unsigned long long *vote = nullptr;    // [Tmax]
     int *flag = nullptr, *pos = nullptr;   // [Tmax], [Tmax + 1]
     int *fvote = nullptr, *fstamp = nullptr, *fwd = nullptr, *chk = nullptr;
-    int4 *fdiag = nullptr;
+    int *list[2] = {nullptr, nullptr};     // [Tmax] triangles a flip pass looks at
+    int4 *cand = nullptr;                  // [3 Tmax / 2] illegal edges of a pass
     int *loc = nullptr;                    // [maxN]
     int *otri = nullptr, *oopp = nullptr;  // [Tmax][3] output staging
     int *cnt = nullptr;                    // [NUM_C]
@@ -991,7 +1151,7 @@ struct DtCtx {
     int2 *cross = nullptr;
     int *part = nullptr;                   // [3 kParts] first-triangle search
     double *partv = nullptr;               // [kParts]
-    int *hcnt = nullptr;                   // pinned [NUM_C + 1]
+    int *hcnt = nullptr;                   // pinned [NUM_C]
     char *arena = nullptr;
     int stats[4] = {0, 0, 0, 0};           // rounds, flip passes, flips, duplicates
 };
@@ -1040,7 +1200,8 @@ extern "C" int cvt_dt_create(cvt_dt **out, int max_points)
         carve(c->vote, T, set); carve(c->flag, T, set); carve(c->pos, T + 1, set);
         carve(c->fvote, T, set); carve(c->fstamp, T, set); carve(c->fwd, 3 * T, set);
         carve(c->chk, T, set);
-        carve(c->fdiag, T, set); carve(c->loc, N, set); carve(c->cnt, NUM_C, set);
+        carve(c->list[0], T, set); carve(c->list[1], T, set); carve(c->cand, 3 * T / 2 + 1, set);
+        carve(c->loc, N, set); carve(c->cnt, NUM_C, set);
         carve(c->otri, 3 * T, set); carve(c->oopp, 3 * T, set);
         carve(c->part, 3 * kParts, set); carve(c->partv, kParts, set);
         carve(c->vt, N, set);
@@ -1052,7 +1213,7 @@ extern "C" int cvt_dt_create(cvt_dt **out, int max_points)
         return fail(CVT_ERR_NOMEM, "%zu bytes for %d points", at, max_points);
     }
     layout(true);
-    if (hipHostMalloc((void **)&c->hcnt, sizeof(int) * (NUM_C + 1), 0) != hipSuccess ||
+    if (hipHostMalloc((void **)&c->hcnt, sizeof(int) * NUM_C, 0) != hipSuccess ||
         hipStreamCreate(&c->st) != hipSuccess) {
         dt_free(c);
         return fail(CVT_ERR_HIP, "stream / pinned counters");
@@ -1067,32 +1228,71 @@ extern "C" int cvt_dt_destroy(cvt_dt *dt)
     return CVT_OK;
 }
 
-// Lawson flips to Delaunay over T triangles.  Each pass flips at least the
-// lowest illegal edge; passes are enqueued kFlipChunk at a time and the
-// flips of the chunk's last pass read back (a pass with nothing to check
-// costs only its launches).  The bound guards a broken mesh.
-static int flip_to_delaunay(DtCtx *c, int n, int T, int &round)
+// the counters (and the count of triangles to split) in the host's pinned memory
+static int read_counters(DtCtx *c, const int *splits, const char *what)
 {
-    hipStream_t st = c->st;
-    int *h = c->hcnt;
-    constexpr int kFlipChunk = 4;
-    for (int pass = 0;; pass += kFlipChunk) {
-        if (pass > 4 * c->Tmax + 64) return fail(CVT_ERR_STATE, "flipping did not converge");
-        for (int q = 0; q < kFlipChunk; ++q) {
-            ++round;
-            hipLaunchKernelGGL(k_dt_flip_mark, dim3(nb(T)), dim3(256), 0, st, c->P, n, T, c->tv,
-                               c->to, c->chk, round, c->fvote, c->cnt);
-            hipLaunchKernelGGL(k_dt_flip, dim3(nb(T)), dim3(256), 0, st, T, c->tv, c->to,
-                               c->fvote, c->fwd, c->fstamp, c->fdiag, c->chk, round, c->cnt);
-            hipLaunchKernelGGL(k_dt_flip_fix, dim3(nb(std::max(T, n))), dim3(256), 0, st, c->P, n,
-                               T, c->to, c->fwd, c->fstamp, c->fdiag, c->fvote, c->loc, round,
-                               c->cnt);
-            ++c->stats[1];
-        }
-        DCHK(hipMemcpyAsync(h, c->cnt, sizeof(int) * NUM_C, hipMemcpyDeviceToHost, st), "counters");
-        DCHK(hipStreamSynchronize(st), "flip");
-        if (h[C_FLIPS] == 0 || h[C_ERR]) return CVT_OK;
+    hipLaunchKernelGGL(k_dt_publish, dim3(1), dim3(64), 0, c->st, c->cnt, splits, c->hcnt);
+    DCHK(hipGetLastError(), what);
+    DCHK(hipStreamSynchronize(c->st), what);
+    return CVT_OK;
+}
+
+static FlipArgs flip_args(DtCtx *c, int n)
+{
+    FlipArgs a;
+    a.P = c->P; a.n = n; a.tv = c->tv; a.to = c->to; a.chk = c->chk; a.fvote = c->fvote;
+    a.fwd = c->fwd; a.fstamp = c->fstamp; a.list[0] = c->list[0]; a.list[1] = c->list[1];
+    a.cand = c->cand; a.cnt = c->cnt;
+    return a;
+}
+
+// Part of a run of Lawson flips to Delaunay: `done` passes came before, passes
+// number from round + 1, at most `listed` triangles are on the list.  While it
+// may be long, passes of a launch per step; then k_dt_flip_tail, which leaves
+// C_CONV set when nothing is left.  The caller reads the counters and adds the
+// tail's C_RAN to done and round.  Eight passes of a workgroup's own take
+// longer than a launch: long lists are few passes away, and a list that the
+// tail finds too long comes back here.
+static void enqueue_flips(DtCtx *c, int n, int listed, int &done, int &round)
+{
+    const FlipArgs a = flip_args(c, n);
+    const int big = listed <= kTailList ? 0 : done == 0 ? 4 : 8;
+    const unsigned grid = (unsigned)std::min<long>(2048, nb(3L * listed));
+    for (int q = 0; q < big; ++q, ++done) {
+        ++round;
+        hipLaunchKernelGGL(k_dt_flip_mark, dim3(grid), dim3(256), 0, c->st, a, done & 1, round);
+        hipLaunchKernelGGL(k_dt_flip, dim3(grid), dim3(256), 0, c->st, a, done & 1, round);
+        hipLaunchKernelGGL(k_dt_flip_fix, dim3(grid), dim3(256), 0, c->st, a, done & 1, round);
     }
+    // (a bounded number of passes: the kernel's time stays bounded too)
+    hipLaunchKernelGGL(k_dt_flip_tail, dim3(1), dim3(1024), 0, c->st, a, done, round + 1, 4096);
+}
+
+// after the counters were read: the passes the tail ran, and whether the run
+// goes on (C_CONV clear, no error)
+static int flips_left(DtCtx *c, int &done, int &round)
+{
+    done += c->hcnt[C_RAN];
+    round += c->hcnt[C_RAN];
+    if (c->hcnt[C_CONV] || c->hcnt[C_ERR]) {
+        // passes are counted in fours, as a run read its flips back once did
+        c->stats[1] += 4 * (c->hcnt[C_PASSES] / 4 + 1);
+        return 0;
+    }
+    return c->hcnt[C_LIST + (done & 1)];
+}
+
+static int flip_to_delaunay(DtCtx *c, int n, int listed, int &round)
+{
+    int done = 0;
+    while (listed > 0) {
+        if (done > 4 * c->Tmax + 64) return fail(CVT_ERR_STATE, "flipping did not converge");
+        enqueue_flips(c, n, listed, done, round);
+        const int rc = read_counters(c, nullptr, "flip");
+        if (rc) return rc;
+        listed = flips_left(c, done, round);
+    }
+    return CVT_OK;
 }
 
 // the constraint segments as edges (gDel2D's doInsertConstraints), then the
@@ -1133,7 +1333,8 @@ static int insert_constraints(DtCtx *c, int n, int T, int nseg, int &round)
                         "%d inserted)", outer, h[C_MISS], h[C_FLIPS]);
     }
     // every edge may have to change now: look at all triangles once
-    hipLaunchKernelGGL(k_dt_fill<int>, dim3(nb(T)), dim3(256), 0, st, c->chk, round + 1, (long)T);
+    hipLaunchKernelGGL(k_dt_list_all, dim3(nb(T)), dim3(256), 0, st, T, c->list[0], c->chk,
+                       round + 1, c->cnt);
     return flip_to_delaunay(c, n, T, round);
 }
 
@@ -1212,37 +1413,49 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
         return fail(CVT_ERR_ARG, "coordinates span more than 2^71 units of their finest bit");
     if (h[C_ERR]) return fail(CVT_ERR_ARG, "degenerate input: all points collinear or coincident");
     hipLaunchKernelGGL(k_dt_locate0, dim3(nb(n)), dim3(256), 0, st, c->P, n, c->loc, c->cnt);
-    int T = 4, round = 0;
-    // each round inserts at least one point
+    hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_CONV, 1, 1L);
+    int T = 4, round = 0, done = 0;
+    int first = 1;                     // first pass of the latest flip run
+    // Each round inserts at least one point.  A round's bids are enqueued
+    // behind the flips of the round before and do nothing while those go on
+    // (C_CONV): the host reads the counters once per round.
     for (int guard = 0; guard <= n; ++guard) {
-        hipLaunchKernelGGL(k_dt_fill<unsigned long long>, dim3(nb(T)), dim3(256), 0, st, c->vote,
-                           NO_BID, (long)T);
-        hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_UNINS, 0, 1L);
-        if (T <= kVoteLds)
-            hipLaunchKernelGGL(k_dt_vote_lds, dim3((unsigned)std::min<long>(256, (n + 1023) / 1024)),
-                               dim3(1024), 0, st, c->P, n, T, c->tv, c->loc, c->vote, c->cnt);
-        else
-            hipLaunchKernelGGL(k_dt_vote, dim3(nb(n)), dim3(256), 0, st, c->P, n, c->tv, c->loc,
-                               c->vote, c->cnt);
-        hipLaunchKernelGGL(k_dt_split_flags, dim3(nb(T)), dim3(256), 0, st, c->vote, T, c->flag);
-        launch_exclusive_scan(st, c->flag, T, c->pos);
-        DCHK(hipMemcpyAsync(h, c->cnt, sizeof(int) * NUM_C, hipMemcpyDeviceToHost, st), "counters");
-        DCHK(hipMemcpyAsync(h + NUM_C, c->pos + T, sizeof(int), hipMemcpyDeviceToHost, st),
-             "counters");
-        DCHK(hipStreamSynchronize(st), "vote");
+        for (;;) {
+            hipLaunchKernelGGL(k_dt_fill<unsigned long long>, dim3(nb(T)), dim3(256), 0, st,
+                               c->vote, NO_BID, (long)T);
+            hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_UNINS, 0, 1L);
+            if (T <= kVoteLds)
+                hipLaunchKernelGGL(k_dt_vote_lds,
+                                   dim3((unsigned)std::min<long>(256, (n + 1023) / 1024)),
+                                   dim3(1024), 0, st, c->P, n, T, c->tv, c->to, c->fstamp, first,
+                                   c->loc, c->vote, c->cnt);
+            else
+                hipLaunchKernelGGL(k_dt_vote, dim3(nb(n)), dim3(256), 0, st, c->P, n, T, c->tv,
+                                   c->to, c->fstamp, first, c->loc, c->vote, c->cnt);
+            hipLaunchKernelGGL(k_dt_split_flags, dim3(nb(T)), dim3(256), 0, st, c->vote, T,
+                               c->flag);
+            launch_exclusive_scan(st, c->flag, T, c->pos);
+            const int rc = read_counters(c, c->pos + T, "vote");
+            if (rc) return rc;
+            if (guard == 0) break;
+            const int left = flips_left(c, done, round);
+            if (left == 0) break;
+            if (done > 4 * c->Tmax + 64) return fail(CVT_ERR_STATE, "flipping did not converge");
+            enqueue_flips(c, n, left, done, round);
+        }
         if (h[C_ERR]) break;
         if (h[C_UNINS] == 0) break;
-        const int splits = h[NUM_C];
+        const int splits = h[C_SPLITS];
         if (T + 2 * splits > c->Tmax) return fail(CVT_ERR_CAPACITY, "triangle capacity");
         hipLaunchKernelGGL(k_dt_split, dim3(nb(T)), dim3(256), 0, st, c->P, n, T, c->tv, c->to,
-                           c->vote, c->pos, c->loc, c->chk, round + 1, c->cnt);
+                           c->vote, c->pos, c->loc, c->chk, round + 1, c->list[0], c->cnt);
         hipLaunchKernelGGL(k_dt_relocate_split, dim3(nb(n)), dim3(256), 0, st, c->P, n, T, c->tv,
                            c->vote, c->pos, c->loc, c->cnt);
         T += 2 * splits;
         ++c->stats[0];
-        const int rc = flip_to_delaunay(c, n, T, round);
-        if (rc) return rc;
-        if (h[C_ERR]) break;
+        done = 0;
+        first = round + 1;
+        enqueue_flips(c, n, 3 * splits, done, round);
     }
     if (!h[C_ERR] && num_segments > 0) {
         const int rc = insert_constraints(c, n, T, num_segments, round);
@@ -1257,9 +1470,11 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
         return fail(CVT_ERR_ARG, "degenerate input: collinear points where a triangle was needed");
     hipLaunchKernelGGL(k_dt_alive, dim3(nb(T)), dim3(256), 0, st, c->tv, T, n, c->flag);
     launch_exclusive_scan(st, c->flag, T, c->pos);
-    DCHK(hipMemcpyAsync(h + NUM_C, c->pos + T, sizeof(int), hipMemcpyDeviceToHost, st), "count");
-    DCHK(hipStreamSynchronize(st), "count");
-    const int nt = h[NUM_C];
+    {
+        const int rc = read_counters(c, c->pos + T, "count");
+        if (rc) return rc;
+    }
+    const int nt = h[C_SPLITS];
     *num_tri = nt;
     if (nt > capacity) return fail(CVT_ERR_CAPACITY, "%d triangles, capacity %d", nt, capacity);
     // staged, then copied: the caller's arrays may be host or device memory
