@@ -37,8 +37,8 @@ class Delaunay:
             n = points.shape[0]
         pp, keep = _ptr(points, np.float64)
         cap = max(2 * n, 1)
-        tri = np.zeros((cap, 3), np.int32)
-        opp = np.zeros((cap, 3), np.int32) if want_opp else None
+        tri = np.empty((cap, 3), np.int32)
+        opp = np.empty((cap, 3), np.int32) if want_opp else None
         nt = C.c_int(0)
         po = opp.ctypes.data_as(C.c_void_p) if want_opp else None
         if segments is None:
@@ -50,7 +50,9 @@ class Delaunay:
             call("cvt_dt_compute_constrained", self._h, pp, int(n), ps, int(m),
                  tri.ctypes.data_as(C.c_void_p), po, cap, C.byref(nt))
         k = nt.value
-        return tri[:k].copy(), (opp[:k].copy() if want_opp else None)
+        # (the unused rows, two and one per hull point, stay behind the result;
+        # on an error nothing is returned)
+        return tri[:k], (opp[:k] if want_opp else None)
 
     def stats(self) -> dict:
         s = np.zeros(4, np.int32)
