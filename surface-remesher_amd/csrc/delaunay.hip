@@ -71,15 +71,42 @@ struct Pt {
     double x, y;
 };
 
+// The points as the kernels hold them, in the order of kSortMin below, and the
+// caller's index of each (null: the caller's order).  Whatever an index
+// decides (ties, the perturbation, which duplicate is kept) is decided by the
+// caller's, so the result does not depend on the order.
+struct Pts {
+    const Pt *p;
+    const int *ids;
+    __device__ __forceinline__ const Pt &operator[](int i) const { return p[i]; }
+    __device__ __forceinline__ int id(int i) const { return ids ? ids[i] : i; }
+};
+
 // orientation of indexed points under the perturbation (never 0 for
 // distinct points)
-__device__ __forceinline__ int orient_p(const Pt *P, int a, int b, int c, int *err)
+__device__ __forceinline__ int orient_p(Pts P, int a, int b, int c, int *err)
 {
-    return orient2d_sos(P[a].x, P[a].y, P[b].x, P[b].y, P[c].x, P[c].y, a, b, c, err);
+    const int o = orient2d(P[a].x, P[a].y, P[b].x, P[b].y, P[c].x, P[c].y, err);
+    if (o) return o;
+    int idx[3] = {P.id(a), P.id(b), P.id(c)};
+    double x[6] = {P[a].x, P[a].y, P[b].x, P[b].y, P[c].x, P[c].y};
+    const int par = sort_by_index<3>(idx, x);
+    return par * orient_sos(x);
+}
+
+// in-circle test under the perturbation
+__device__ __forceinline__ int incircle_p(Pts P, int a, int b, int c, int d, int *err)
+{
+    const int o = incircle(P[a].x, P[a].y, P[b].x, P[b].y, P[c].x, P[c].y, P[d].x, P[d].y, err);
+    if (o) return o;
+    int idx[4] = {P.id(a), P.id(b), P.id(c), P.id(d)};
+    double x[8] = {P[a].x, P[a].y, P[b].x, P[b].y, P[c].x, P[c].y, P[d].x, P[d].y};
+    const int par = sort_by_index<4>(idx, x);
+    return par * incircle_sos(x, err);
 }
 
 // the exact, unperturbed orientation
-__device__ __forceinline__ int orient_x(const Pt *P, int a, int b, int c, int *err)
+__device__ __forceinline__ int orient_x(Pts P, int a, int b, int c, int *err)
 {
     return orient2d(P[a].x, P[a].y, P[b].x, P[b].y, P[c].x, P[c].y, err);
 }
@@ -104,21 +131,125 @@ __global__ void k_dt_fill(T *__restrict__ p, T v, long n)
         p[i] = v;
 }
 
+// ---------------------------------------------------------------------------
+// The order of the points.  A caller's order is random in space as a rule, and
+// every test of a triangle gathers its points: from kSortMin points up they
+// are kept sorted by the cells of a 2^b x 2^b grid over their bounding box,
+// the cells along a Z curve (a counting sort; the order within a cell is
+// arbitrary).  gDel2D sorts its input as well (GDel2DInput's noSort switches
+// it off, source/gDel2D/gDel2D/GpuDelaunay.h:28-64).
+// ---------------------------------------------------------------------------
+static constexpr int kSortMin = 65536;
+
+// part[4 b ..]: min x, min y, -max x, -max y of workgroup b's finite points
+__global__ __launch_bounds__(256) void k_dt_bounds(const Pt *__restrict__ in, int n,
+                                                   double *__restrict__ part)
+{
+    __shared__ double r[4][256];
+    double m[4] = {1e308, 1e308, 1e308, 1e308};
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const Pt p = in[i];
+        if (!isfinite(p.x) || !isfinite(p.y)) continue;
+        m[0] = fmin(m[0], p.x);
+        m[1] = fmin(m[1], p.y);
+        m[2] = fmin(m[2], -p.x);
+        m[3] = fmin(m[3], -p.y);
+    }
+    for (int k = 0; k < 4; ++k) r[k][threadIdx.x] = m[k];
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s)
+            for (int k = 0; k < 4; ++k)
+                r[k][threadIdx.x] = fmin(r[k][threadIdx.x], r[k][threadIdx.x + s]);
+        __syncthreads();
+    }
+    if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = r[threadIdx.x][0];
+}
+
+// the bounds of all kParts workgroups, by every thread of a workgroup
+__device__ __forceinline__ void all_bounds(const double *part, double (&lo)[2], double (&scale)[2],
+                                           int cells)
+{
+    __shared__ double r[4][kParts];
+    for (int i = threadIdx.x; i < kParts; i += blockDim.x)
+        for (int k = 0; k < 4; ++k) r[k][i] = part[4 * i + k];
+    __syncthreads();
+    for (int s = kParts / 2; s > 0; s >>= 1) {
+        for (int i = threadIdx.x; i < s; i += blockDim.x)
+            for (int k = 0; k < 4; ++k) r[k][i] = fmin(r[k][i], r[k][i + s]);
+        __syncthreads();
+    }
+    for (int k = 0; k < 2; ++k) {
+        const double w = -r[2 + k][0] - r[k][0];
+        lo[k] = r[k][0];
+        scale[k] = w > 0.0 && w < 1e300 ? cells / w : 0.0;
+    }
+}
+
+__device__ __forceinline__ unsigned spread_bits(unsigned v)   // bit i to bit 2 i
+{
+    v = (v | (v << 8)) & 0x00ff00ffu;
+    v = (v | (v << 4)) & 0x0f0f0f0fu;
+    v = (v | (v << 2)) & 0x33333333u;
+    return (v | (v << 1)) & 0x55555555u;
+}
+
+// cell of each point and its rank among the cell's points
+__global__ __launch_bounds__(256) void k_dt_cells(const Pt *__restrict__ in, int n,
+                                                  const double *__restrict__ part, int cells,
+                                                  int *__restrict__ cell, int *__restrict__ rank,
+                                                  int *__restrict__ count)
+{
+    double lo[2], scale[2];
+    all_bounds(part, lo, scale, cells);
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const Pt p = in[i];
+        const double top = (double)(cells - 1);
+        // (NaN compares false: cell 0)
+        const double fx = (p.x - lo[0]) * scale[0], fy = (p.y - lo[1]) * scale[1];
+        const unsigned x = fx >= 0.0 ? (unsigned)fmin(fx, top) : 0u;
+        const unsigned y = fy >= 0.0 ? (unsigned)fmin(fy, top) : 0u;
+        const int c = (int)(spread_bits(x) | (spread_bits(y) << 1));
+        cell[i] = c;
+        rank[i] = atomicAdd(&count[c], 1);
+    }
+}
+
+__global__ void k_dt_place(const Pt *__restrict__ in, int n, const int *__restrict__ cell,
+                           const int *__restrict__ rank, const int *__restrict__ start,
+                           Pt *__restrict__ out, int *__restrict__ ids, int *__restrict__ place)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) ids[n] = n;                    // O
+    if (i >= n) return;
+    const int k = start[cell[i]] + rank[i];
+    out[k] = in[i];
+    ids[k] = i;
+    place[i] = k;
+}
+
+// the segments' ends from the caller's indices to the points' places
+__global__ void k_dt_place_segments(int *__restrict__ seg, int m, const int *__restrict__ place)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < m) seg[i] = place[seg[i]];
+}
+
 // first triangle: a = lowest x (then y, then index), b = highest, c = the
 // point farthest from the line ab (approximate distance, ties by index);
 // each search is a per-workgroup pass over the points and a one-workgroup
 // pass over the kParts partial results
-__device__ __forceinline__ bool pt_before(const Pt *P, int i, int j)   // (x, y, index) order
+__device__ __forceinline__ bool pt_before(Pts P, int i, int j)   // (x, y, index) order
 {
     if (j < 0) return true;
     if (i < 0) return false;
     if (P[i].x != P[j].x) return P[i].x < P[j].x;
     if (P[i].y != P[j].y) return P[i].y < P[j].y;
-    return i < j;
+    return P.id(i) < P.id(j);
 }
 
 // block-wide: (a, b) = first and last candidates; reduce pairs in LDS
-__device__ void reduce_ab(const Pt *P, int &a, int &b)
+__device__ void reduce_ab(Pts P, int &a, int &b)
 {
     __shared__ int sa[256], sb[256];
     sa[threadIdx.x] = a;
@@ -137,7 +268,7 @@ __device__ void reduce_ab(const Pt *P, int &a, int &b)
     b = sb[0];
 }
 
-__global__ __launch_bounds__(256) void k_dt_ab_part(const Pt *__restrict__ P, int n,
+__global__ __launch_bounds__(256) void k_dt_ab_part(Pts P, int n,
                                                     int *__restrict__ part, int *__restrict__ cnt)
 {
     int a = -1, b = -1;
@@ -158,7 +289,7 @@ __global__ __launch_bounds__(256) void k_dt_ab_part(const Pt *__restrict__ P, in
     }
 }
 
-__global__ __launch_bounds__(256) void k_dt_ab_final(const Pt *__restrict__ P,
+__global__ __launch_bounds__(256) void k_dt_ab_final(Pts P,
                                                      const int *__restrict__ part,
                                                      int *__restrict__ cnt)
 {
@@ -171,7 +302,7 @@ __global__ __launch_bounds__(256) void k_dt_ab_final(const Pt *__restrict__ P,
 }
 
 // block-wide: the largest v, ties by the lower index
-__device__ void reduce_far(double &v, int &c)
+__device__ void reduce_far(Pts P, double &v, int &c)
 {
     __shared__ double sv[256];
     __shared__ int sc[256];
@@ -183,7 +314,7 @@ __device__ void reduce_far(double &v, int &c)
             const double v2 = sv[threadIdx.x + s];
             const int c2 = sc[threadIdx.x + s];
             if (c2 >= 0 && (sc[threadIdx.x] < 0 || v2 > sv[threadIdx.x] ||
-                            (v2 == sv[threadIdx.x] && c2 < sc[threadIdx.x]))) {
+                            (v2 == sv[threadIdx.x] && P.id(c2) < P.id(sc[threadIdx.x])))) {
                 sv[threadIdx.x] = v2;
                 sc[threadIdx.x] = c2;
             }
@@ -194,7 +325,7 @@ __device__ void reduce_far(double &v, int &c)
     c = sc[0];
 }
 
-__global__ __launch_bounds__(256) void k_dt_c_part(const Pt *__restrict__ P, int n,
+__global__ __launch_bounds__(256) void k_dt_c_part(Pts P, int n,
                                                    const int *__restrict__ cnt,
                                                    double *__restrict__ partv,
                                                    int *__restrict__ partc)
@@ -206,28 +337,28 @@ __global__ __launch_bounds__(256) void k_dt_c_part(const Pt *__restrict__ P, int
         const double ux = P[b].x - P[a].x, uy = P[b].y - P[a].y;
         for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
             const double v = fabs(ux * (P[i].y - P[a].y) - uy * (P[i].x - P[a].x));
-            if (v > best || (v == best && i < c)) { best = v; c = i; }
+            if (v > best || (v == best && c >= 0 && P.id(i) < P.id(c))) { best = v; c = i; }
         }
     }
-    reduce_far(best, c);
+    reduce_far(P, best, c);
     if (threadIdx.x == 0) {
         partv[blockIdx.x] = best;
         partc[blockIdx.x] = c;
     }
 }
 
-__global__ __launch_bounds__(256) void k_dt_c_final(const double *__restrict__ partv,
+__global__ __launch_bounds__(256) void k_dt_c_final(Pts P, const double *__restrict__ partv,
                                                     const int *__restrict__ partc,
                                                     int *__restrict__ cnt)
 {
     double v = partv[threadIdx.x];
     int c = partc[threadIdx.x];
-    reduce_far(v, c);
+    reduce_far(P, v, c);
     if (threadIdx.x == 0) cnt[C_C] = c;
 }
 
 // the four triangles of the first triangle on the sphere, and O
-__global__ void k_dt_init(Pt *__restrict__ P, int n, int *__restrict__ tv, int *__restrict__ to,
+__global__ void k_dt_init(Pts P, Pt *out, int n, int *__restrict__ tv, int *__restrict__ to,
                           int *__restrict__ cnt)
 {
     int *err = cnt + C_ERR;
@@ -248,7 +379,7 @@ __global__ void k_dt_init(Pt *__restrict__ P, int n, int *__restrict__ tv, int *
     Pt O;
     O.x = (P[a].x + P[b].x + P[c].x) / 3.0;
     O.y = (P[a].y + P[b].y + P[c].y) / 3.0;
-    P[n] = O;
+    out[n] = O;                            // (the array of P)
     if (orient_x(P, a, b, n, err) <= 0 || orient_x(P, b, c, n, err) <= 0 ||
         orient_x(P, c, a, n, err) <= 0) {
         set_flag(err, DT_ERR_DEGENERATE);                  // a sliver first triangle
@@ -269,7 +400,7 @@ __global__ void k_dt_init(Pt *__restrict__ P, int n, int *__restrict__ tv, int *
 }
 
 // every other point to T0 or to the wedge of T1..T3 that holds it
-__global__ void k_dt_locate0(const Pt *__restrict__ P, int n, int *__restrict__ loc,
+__global__ void k_dt_locate0(Pts P, int n, int *__restrict__ loc,
                              int *__restrict__ cnt)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -309,7 +440,7 @@ __device__ __forceinline__ int inf_pos(const int *v, int I)
 // the hull by the rays from O, and in from the wedge that holds q.  Under the
 // perturbation exactly one triangle holds q.  The step bound guards a broken
 // mesh.
-__device__ __forceinline__ int walk_point(const Pt *P, int n, const int *tv, const int *to, int q,
+__device__ __forceinline__ int walk_point(Pts P, int n, const int *tv, const int *to, int q,
                                           int t, int T, int *err)
 {
     for (int step = 0; step < 2 * T + 64; ++step) {
@@ -332,15 +463,17 @@ __device__ __forceinline__ int walk_point(const Pt *P, int n, const int *tv, con
     return t;
 }
 
-// atomicMin of each lane's bid on vote[t], one atomic per distinct t in the
-// wave (in early rounds most of a wave's points share a triangle); called
-// by every lane of the wave
+// atomicMin of each lane's bid on vote[t]: one atomic for the points of the
+// first lane's triangle and one for those of the first lane's left (in early
+// rounds most of a wave's points share a triangle or two), then one per point
+// (later a wave's points lie in as many triangles: reducing each in turn took
+// 56 us a round at 1 M points); called by every lane of the wave
 __device__ __forceinline__ void wave_min_bid(unsigned long long *vote, int t,
                                              unsigned long long bid, bool active)
 {
     const int lane = threadIdx.x & 63;
     unsigned long long pending = __ballot(active);
-    while (pending) {
+    for (int round = 0; round < 2 && pending; ++round) {
         const int leader = __ffsll((long long)pending) - 1;
         const int t0 = __shfl(t, leader);
         const bool mine = active && t == t0;
@@ -353,11 +486,12 @@ __device__ __forceinline__ void wave_min_bid(unsigned long long *vote, int t,
         pending &= ~__ballot(mine);
         active = active && !mine;
     }
+    if (active) atomicMin(&vote[t], bid);
 }
 
 // the bid of point p on its triangle (NO_BID, and dupv = the vertex, when p
 // duplicates one of the triangle's vertices)
-__device__ __forceinline__ unsigned long long point_bid(const Pt *P, int n, const int *tv, int p,
+__device__ __forceinline__ unsigned long long point_bid(Pts P, int n, const int *tv, int p,
                                                         int t, int &dupv)
 {
     const int v[3] = {tv[3 * t], tv[3 * t + 1], tv[3 * t + 2]};
@@ -385,10 +519,10 @@ __device__ __forceinline__ unsigned long long point_bid(const Pt *P, int n, cons
         key = (float)(1.0 / (1.0 + (d + 1e-6) / (1.0 + fabs(2.0 * t - 1.0))));
     }
     if (!(key >= 0.0f)) key = 3.0e38f;
-    return ((unsigned long long)__float_as_uint(key) << 32) | (unsigned)p;
+    return ((unsigned long long)__float_as_uint(key) << 32) | (unsigned)P.id(p);
 }
 
-__global__ __launch_bounds__(256) void k_dt_vote(const Pt *__restrict__ P, int n,
+__global__ __launch_bounds__(256) void k_dt_vote(Pts P, int n,
                                                  int T, const int *__restrict__ tv,
                                                  const int *__restrict__ to,
                                                  const int *__restrict__ fstamp, int first,
@@ -423,7 +557,7 @@ __global__ __launch_bounds__(256) void k_dt_vote(const Pt *__restrict__ P, int n
 // non-empty entries to the global minimum (one global atomic per triangle
 // per workgroup instead of one per wave)
 static constexpr int kVoteLds = 4096;
-__global__ __launch_bounds__(1024) void k_dt_vote_lds(const Pt *__restrict__ P, int n, int T,
+__global__ __launch_bounds__(1024) void k_dt_vote_lds(Pts P, int n, int T,
                                                       const int *__restrict__ tv,
                                                       const int *__restrict__ to,
                                                       const int *__restrict__ fstamp, int first,
@@ -473,6 +607,14 @@ __global__ void k_dt_split_flags(const unsigned long long *__restrict__ vote, in
     if (t < T) flag[t] = vote[t] != NO_BID;
 }
 
+// the point whose bid won; place: where the point of each caller's index is
+// kept (null: at it)
+__device__ __forceinline__ int winner(unsigned long long bid, const int *place)
+{
+    const int id = (int)(bid & 0xffffffffu);
+    return place ? place[id] : id;
+}
+
 __device__ __forceinline__ int child_slot(int t, int i, int T, const int *base)
 {
     return i == 0 ? t : T + 2 * base[t] + (i - 1);
@@ -480,11 +622,11 @@ __device__ __forceinline__ int child_slot(int t, int i, int T, const int *base)
 
 // 1 -> 3 split of every triangle with a bid: child i = (v[i+1], v[i+2], p)
 // takes slot t (i = 0) or T + 2 rank + i - 1, its edge 2 is the parent's edge i
-__global__ void k_dt_split(const Pt *__restrict__ P, int n, int T, int *__restrict__ tv,
+__global__ void k_dt_split(Pts P, int n, int T, int *__restrict__ tv,
                            int *__restrict__ to, const unsigned long long *__restrict__ vote,
                            const int *__restrict__ base, int *__restrict__ loc,
-                           int *__restrict__ chk, int next_pass, int *__restrict__ list,
-                           int *__restrict__ cnt)
+                           const int *__restrict__ place, int *__restrict__ chk, int next_pass,
+                           int *__restrict__ list, int *__restrict__ cnt)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {                          // the flip run that follows checks the children
@@ -493,7 +635,7 @@ __global__ void k_dt_split(const Pt *__restrict__ P, int n, int T, int *__restri
     }
     if (t >= T || vote[t] == NO_BID) return;
     int *err = cnt + C_ERR;
-    const int p = (int)(vote[t] & 0xffffffffu);
+    const int p = winner(vote[t], place);
     const int v[3] = {tv[3 * t], tv[3 * t + 1], tv[3 * t + 2]};
     const int o[3] = {to[3 * t], to[3 * t + 1], to[3 * t + 2]};
     for (int i = 0; i < 3; ++i) {
@@ -525,11 +667,11 @@ __global__ void k_dt_split(const Pt *__restrict__ P, int n, int T, int *__restri
 }
 
 // the other points of a split triangle to the child that holds them
-__global__ void k_dt_relocate_split(const Pt *__restrict__ P, int n, int T,
+__global__ void k_dt_relocate_split(Pts P, int n, int T,
                                     const int *__restrict__ tv,
                                     const unsigned long long *__restrict__ vote,
                                     const int *__restrict__ base, int *__restrict__ loc,
-                                    int *__restrict__ cnt)
+                                    const int *__restrict__ place, int *__restrict__ cnt)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     bool dup = false;
@@ -537,7 +679,7 @@ __global__ void k_dt_relocate_split(const Pt *__restrict__ P, int n, int T,
         const int t = loc[q];
         if (t >= 0 && vote[t] != NO_BID) {
             int *err = cnt + C_ERR;
-            const int p = (int)(vote[t] & 0xffffffffu);
+            const int p = winner(vote[t], place);
             const int c1 = child_slot(t, 1, T, base);
             // child 0 = (v1, v2, p), child 1 = (v2, v0, p)
             const int v[3] = {tv[3 * c1 + 1], tv[3 * t], tv[3 * t + 1]};
@@ -570,13 +712,12 @@ __global__ void k_dt_relocate_split(const Pt *__restrict__ P, int n, int T,
 
 // w strictly inside the circumcircle of t (for t with the infinite vertex:
 // strictly beyond its finite edge)
-__device__ __forceinline__ bool illegal(const Pt *P, int n, const int *v, int w, int *err)
+__device__ __forceinline__ bool illegal(Pts P, int n, const int *v, int w, int *err)
 {
     if (w == n) return false;
     const int k = inf_pos(v, n);
     if (k < 0)
-        return incircle_sos(P[v[0]].x, P[v[0]].y, P[v[1]].x, P[v[1]].y, P[v[2]].x, P[v[2]].y,
-                            P[w].x, P[w].y, v[0], v[1], v[2], w, err) > 0;
+        return incircle_p(P, v[0], v[1], v[2], w, err) > 0;
     return orient_p(P, v[(k + 1) % 3], v[(k + 2) % 3], w, err) > 0;
 }
 
@@ -596,7 +737,7 @@ __device__ __forceinline__ bool illegal(const Pt *P, int n, const int *v, int w,
 // 2 M triangles and 1 M points a pass (20, 15 and 8 us).
 // ---------------------------------------------------------------------------
 struct FlipArgs {
-    const Pt *P;
+    Pts P;
     int n;
     int *tv, *to, *chk, *fvote, *fwd, *fstamp;
     int *list[2];             // triangles of even / odd passes of the run
@@ -621,8 +762,30 @@ __device__ __forceinline__ int push_slot(int *counter)
     return __shfl(base, lead) + __popcll(m & ((1ull << lane) - 1ull));
 }
 
+// Entries of a global list gathered by one workgroup in LDS and added with one
+// atomic per flush.  (With an atomic per wave, the waves of a full pass queued
+// on the list's counter: the mark step took 48 us a pass at 1 M points, 13.5
+// this way, the flip step 20 and 12.)
+template <typename E, int CAP> struct PushBuf {
+    E e[CAP];
+    int n, base;
+};
+
+template <typename E, int CAP>
+__device__ __forceinline__ void push_flush(PushBuf<E, CAP> &b, E *list, int *counter)
+{
+    __syncthreads();
+    if (threadIdx.x == 0 && b.n) b.base = atomicAdd(counter, b.n);
+    __syncthreads();
+    for (int i = threadIdx.x; i < b.n; i += blockDim.x) list[b.base + i] = b.e[i];
+    __syncthreads();
+    if (threadIdx.x == 0) b.n = 0;
+    __syncthreads();
+}
+
 // edge e of listed triangle u
-__device__ __forceinline__ void flip_mark(const FlipArgs &a, int u, int e, int pass, int *ncand)
+__device__ __forceinline__ void flip_mark(const FlipArgs &a, int u, int e, int pass, int4 *cand,
+                                          int *ncand)
 {
     const int r = a.to[3 * u + e], m = r >> 4, k = r & 3;
     if (r < 0 || (r & 4)) return;                 // a constraint edge never flips
@@ -635,7 +798,7 @@ __device__ __forceinline__ void flip_mark(const FlipArgs &a, int u, int e, int p
     const int id = 3 * t + i;
     atomicMin(&a.fvote[t], id);
     atomicMin(&a.fvote[o], id);
-    a.cand[push_slot(ncand)] = make_int4(t, o, i | (j << 2), 0);
+    cand[push_slot(ncand)] = make_int4(t, o, i | (j << 2), 0);
 }
 
 // flip of the edge i of t shared with edge k of m, if it won both bids: t' =
@@ -707,19 +870,41 @@ __device__ __forceinline__ void flip_fix(const FlipArgs &a, int idx, int pass)
 // the steps of pass `pass`, whose list is list[par]
 __global__ __launch_bounds__(256) void k_dt_flip_mark(FlipArgs a, int par, int pass)
 {
+    __shared__ PushBuf<int4, 1024> b;
+    if (threadIdx.x == 0) b.n = 0;
+    __syncthreads();
     const int n = 3 * a.cnt[C_LIST + par];
-    for (int x = blockIdx.x * 256 + threadIdx.x; x < n; x += gridDim.x * 256)
-        flip_mark(a, a.list[par][x / 3], x % 3, pass, a.cnt + C_CAND + par);
+    for (int x0 = blockIdx.x * 256; x0 < n; x0 += gridDim.x * 256) {
+        const int x = x0 + threadIdx.x;
+        if (x < n) flip_mark(a, a.list[par][x / 3], x % 3, pass, b.e, &b.n);
+        // (read between barriers: the next step's pushes change it)
+        __syncthreads();
+        const int have = b.n;
+        __syncthreads();
+        if (have > 1024 - 256) push_flush(b, a.cand, a.cnt + C_CAND + par);
+    }
+    push_flush(b, a.cand, a.cnt + C_CAND + par);
 }
 
 __global__ __launch_bounds__(256) void k_dt_flip(FlipArgs a, int par, int pass)
 {
+    __shared__ PushBuf<int, 2048> b;
+    __shared__ int flips;
+    if (threadIdx.x == 0) b.n = flips = 0;
+    __syncthreads();
     const int n = a.cnt[C_CAND + par];
     int did = 0;
-    for (int x = blockIdx.x * 256 + threadIdx.x; x < n; x += gridDim.x * 256)
-        did += flip_do(a, x, pass, a.list[par ^ 1], a.cnt + C_LIST + (par ^ 1));
-    for (int o = 32; o > 0; o >>= 1) did += __shfl_xor(did, o);
-    if ((threadIdx.x & 63) == 0 && did) atomicAdd(a.cnt + C_FTOT, did);
+    for (int x0 = blockIdx.x * 256; x0 < n; x0 += gridDim.x * 256) {
+        const int x = x0 + threadIdx.x;
+        if (x < n) did += flip_do(a, x, pass, b.e, &b.n);
+        __syncthreads();
+        const int have = b.n;
+        __syncthreads();
+        if (have > 2048 - 512) push_flush(b, a.list[par ^ 1], a.cnt + C_LIST + (par ^ 1));
+    }
+    if (did) atomicAdd(&flips, did);
+    push_flush(b, a.list[par ^ 1], a.cnt + C_LIST + (par ^ 1));
+    if (threadIdx.x == 0 && flips) atomicAdd(a.cnt + C_FTOT, flips);
 }
 
 __global__ __launch_bounds__(256) void k_dt_flip_fix(FlipArgs a, int par, int pass)
@@ -755,7 +940,7 @@ __global__ __launch_bounds__(1024) void k_dt_flip_tail(FlipArgs a, int done, int
         const int n = nlist[par];
         if (n == 0 || n > kTailList) break;
         for (int x = threadIdx.x; x < 3 * n; x += 1024)
-            flip_mark(a, a.list[par][x / 3], x % 3, pass, &ncand);
+            flip_mark(a, a.list[par][x / 3], x % 3, pass, a.cand, &ncand);
         __syncthreads();
         const int nc = ncand;
         int did = 0;
@@ -857,7 +1042,7 @@ __device__ __forceinline__ int kept_vertex(const int *loc, int v)
 // one thread per segment: marks it when present (ncr = 0), else lists the
 // edges it crosses from a to b (ncr of them; -1 beyond kCavMax).  a is the
 // end of lower degree (the turn around it is the shorter), kept in sa.
-__global__ void k_dt_walk(const Pt *__restrict__ P, int n, int T, const int *__restrict__ tv,
+__global__ void k_dt_walk(Pts P, int n, int T, const int *__restrict__ tv,
                           int *__restrict__ to, const int *__restrict__ vt,
                           const int *__restrict__ deg, const int *__restrict__ loc,
                           const int *__restrict__ seg, int nseg, int2 *__restrict__ cross,
@@ -970,7 +1155,7 @@ __global__ void k_dt_claim(const int *__restrict__ to, const int2 *__restrict__ 
 
 // apexes for the chain ch[0 .. len) over the base (ch[0], ch[len-1]), the
 // chain on the base's left: appends counterclockwise triangles to nt
-__device__ int triangulate_chain(const Pt *P, const int *ch, int len, int *nt, int cnt0,
+__device__ int triangulate_chain(Pts P, const int *ch, int len, int *nt, int cnt0,
                                  int *stack, int *err)
 {
     int sp = 0, nn = cnt0;
@@ -982,9 +1167,7 @@ __device__ int triangulate_chain(const Pt *P, const int *ch, int len, int *nt, i
         int c = i0 + 1;
         for (int i = i0 + 2; i < i1; ++i) {
             const int p = ch[i0], q = ch[i1], r = ch[c], x = ch[i];
-            if (incircle_sos(P[p].x, P[p].y, P[q].x, P[q].y, P[r].x, P[r].y, P[x].x, P[x].y, p,
-                             q, r, x, err) > 0)
-                c = i;
+            if (incircle_p(P, p, q, r, x, err) > 0) c = i;
         }
         nt[3 * nn] = ch[i0];
         nt[3 * nn + 1] = ch[i1];
@@ -1000,7 +1183,7 @@ __device__ int triangulate_chain(const Pt *P, const int *ch, int len, int *nt, i
 
 // one thread per segment that holds its claims: the cavity replaced by the
 // segment and the triangulations of its two sides
-__global__ void k_dt_cavity(const Pt *__restrict__ P, int n, int *__restrict__ tv,
+__global__ void k_dt_cavity(Pts P, int n, int *__restrict__ tv,
                             int *__restrict__ to, const int *__restrict__ loc,
                             const int *__restrict__ seg, const int2 *__restrict__ cross,
                             const int *__restrict__ ncr, int nseg, int round,
@@ -1100,7 +1283,7 @@ __global__ void k_dt_alive(const int *__restrict__ tv, int T, int n, int *__rest
     if (t < T) flag[t] = tv[3 * t] != n && tv[3 * t + 1] != n && tv[3 * t + 2] != n;
 }
 
-__global__ void k_dt_output(const int *__restrict__ tv, const int *__restrict__ to, int T, int n,
+__global__ void k_dt_output(Pts P, const int *__restrict__ tv, const int *__restrict__ to, int T, int n,
                             const int *__restrict__ flag, const int *__restrict__ pos,
                             int *__restrict__ tri, int *__restrict__ opp)
 {
@@ -1108,7 +1291,7 @@ __global__ void k_dt_output(const int *__restrict__ tv, const int *__restrict__ 
     if (t >= T || !flag[t]) return;
     const int j = pos[t];
     for (int e = 0; e < 3; ++e) {
-        tri[3 * j + e] = tv[3 * t + e];
+        tri[3 * j + e] = P.id(tv[3 * t + e]);
         if (opp) {
             const int r = to[3 * t + e], m = r >> 4;
             opp[3 * j + e] = flag[m] ? (pos[m] << 4) | (r & 7) : -1;
@@ -1131,6 +1314,12 @@ struct DtCtx {
     int maxN = 0, Tmax = 0;
     hipStream_t st = nullptr;
     Pt *P = nullptr;                       // [maxN + 1]; point n is O
+    Pt *in = nullptr;                      // [maxN] the caller's points, to be sorted
+    int *ids = nullptr, *place = nullptr;  // [maxN + 1], [maxN] (see Pts, winner)
+    double *bounds = nullptr;              // [4 kParts]
+    bool sorted = false;
+    Pts pts() const { return Pts{P, sorted ? ids : nullptr}; }
+    const int *places() const { return sorted ? place : nullptr; }
     int *tv = nullptr, *to = nullptr;      // [Tmax][3]
     unsigned long long *vote = nullptr;    // [Tmax]
     int *flag = nullptr, *pos = nullptr;   // [Tmax], [Tmax + 1]
@@ -1196,7 +1385,9 @@ extern "C" int cvt_dt_create(cvt_dt **out, int max_points)
     };
     auto layout = [&](bool set) {
         at = 0;
-        carve(c->P, N + 1, set); carve(c->tv, 3 * T, set); carve(c->to, 3 * T, set);
+        carve(c->P, N + 1, set); carve(c->in, N, set); carve(c->ids, N + 1, set);
+        carve(c->place, N, set); carve(c->bounds, 4 * kParts, set);
+        carve(c->tv, 3 * T, set); carve(c->to, 3 * T, set);
         carve(c->vote, T, set); carve(c->flag, T, set); carve(c->pos, T + 1, set);
         carve(c->fvote, T, set); carve(c->fstamp, T, set); carve(c->fwd, 3 * T, set);
         carve(c->chk, T, set);
@@ -1240,7 +1431,7 @@ static int read_counters(DtCtx *c, const int *splits, const char *what)
 static FlipArgs flip_args(DtCtx *c, int n)
 {
     FlipArgs a;
-    a.P = c->P; a.n = n; a.tv = c->tv; a.to = c->to; a.chk = c->chk; a.fvote = c->fvote;
+    a.P = c->pts(); a.n = n; a.tv = c->tv; a.to = c->to; a.chk = c->chk; a.fvote = c->fvote;
     a.fwd = c->fwd; a.fstamp = c->fstamp; a.list[0] = c->list[0]; a.list[1] = c->list[1];
     a.cand = c->cand; a.cnt = c->cnt;
     return a;
@@ -1308,13 +1499,13 @@ static int insert_constraints(DtCtx *c, int n, int T, int nseg, int &round)
         hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_MISS, 0, 1L);
         hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_FLIPS, 0, 1L);
         hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_WSLOT, 0, 1L);
-        hipLaunchKernelGGL(k_dt_walk, dim3(nb(nseg)), dim3(256), 0, st, c->P, n, T, c->tv, c->to,
+        hipLaunchKernelGGL(k_dt_walk, dim3(nb(nseg)), dim3(256), 0, st, c->pts(), n, T, c->tv, c->to,
                            c->vt, c->deg, c->loc, c->seg, nseg, c->cross, c->ncr, c->sa, c->cnt);
         hipLaunchKernelGGL(k_dt_fill<unsigned long long>, dim3(nb(T)), dim3(256), 0, st, c->own,
                            ~0ull, (long)T);
         hipLaunchKernelGGL(k_dt_claim, dim3(nb(nseg)), dim3(256), 0, st, c->to, c->cross, c->ncr,
                            nseg, outer, c->own);
-        hipLaunchKernelGGL(k_dt_cavity, dim3((nseg + 63) / 64), dim3(64), 0, st, c->P, n, c->tv,
+        hipLaunchKernelGGL(k_dt_cavity, dim3((nseg + 63) / 64), dim3(64), 0, st, c->pts(), n, c->tv,
                            c->to, c->loc, c->seg, c->cross, c->ncr, nseg, outer, c->own, c->sa,
                            c->ws, std::min(nseg, kWsSlots), c->cnt);
         DCHK(hipMemcpyAsync(h, c->cnt, sizeof(int) * NUM_C, hipMemcpyDeviceToHost, st), "counters");
@@ -1391,7 +1582,27 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
     hipStream_t st = c->st;
     int *h = c->hcnt;
     for (int i = 0; i < 4; ++i) c->stats[i] = 0;
-    DCHK(hipMemcpyAsync(c->P, points, sizeof(Pt) * n, hipMemcpyDefault, st), "point upload");
+    c->sorted = n >= kSortMin;
+    DCHK(hipMemcpyAsync(c->sorted ? c->in : c->P, points, sizeof(Pt) * n, hipMemcpyDefault, st),
+         "point upload");
+    if (c->sorted) {
+        // about four points per cell; the cells' work arrays lie in buffers
+        // that the triangulation has no use for yet
+        int cells = 64;
+        while (4L * cells * cells * 4 <= n && cells < 4096) cells *= 2;
+        int *cell = c->fvote, *rank = c->fstamp, *count = c->list[0], *start = c->list[1];
+        hipLaunchKernelGGL(k_dt_bounds, dim3(kParts), dim3(256), 0, st, c->in, n, c->bounds);
+        hipLaunchKernelGGL(k_dt_fill<int>, dim3(nb((long)cells * cells)), dim3(256), 0, st, count, 0,
+                           (long)cells * cells);
+        hipLaunchKernelGGL(k_dt_cells, dim3(512), dim3(256), 0, st, c->in, n, c->bounds, cells,
+                           cell, rank, count);
+        launch_exclusive_scan(st, count, cells * cells, start);
+        hipLaunchKernelGGL(k_dt_place, dim3(nb(n)), dim3(256), 0, st, c->in, n, cell, rank, start,
+                           c->P, c->ids, c->place);
+        if (num_segments > 0)
+            hipLaunchKernelGGL(k_dt_place_segments, dim3(nb(2L * num_segments)), dim3(256), 0, st,
+                               c->seg, 2 * num_segments, c->place);
+    }
     hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt, 0, (long)NUM_C);
     hipLaunchKernelGGL(k_dt_fill<int>, dim3(nb(c->Tmax)), dim3(256), 0, st, c->fstamp, -1,
                        (long)c->Tmax);
@@ -1399,20 +1610,20 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
                        (long)c->Tmax);
     hipLaunchKernelGGL(k_dt_fill<int>, dim3(nb(c->Tmax)), dim3(256), 0, st, c->fvote, NO_FLIP,
                        (long)c->Tmax);
-    hipLaunchKernelGGL(k_dt_ab_part, dim3(kParts), dim3(256), 0, st, c->P, n, c->part, c->cnt);
-    hipLaunchKernelGGL(k_dt_ab_final, dim3(1), dim3(kParts), 0, st, c->P, c->part, c->cnt);
-    hipLaunchKernelGGL(k_dt_c_part, dim3(kParts), dim3(256), 0, st, c->P, n, c->cnt, c->partv,
+    hipLaunchKernelGGL(k_dt_ab_part, dim3(kParts), dim3(256), 0, st, c->pts(), n, c->part, c->cnt);
+    hipLaunchKernelGGL(k_dt_ab_final, dim3(1), dim3(kParts), 0, st, c->pts(), c->part, c->cnt);
+    hipLaunchKernelGGL(k_dt_c_part, dim3(kParts), dim3(256), 0, st, c->pts(), n, c->cnt, c->partv,
                        c->part + 2 * kParts);
-    hipLaunchKernelGGL(k_dt_c_final, dim3(1), dim3(kParts), 0, st, c->partv, c->part + 2 * kParts,
+    hipLaunchKernelGGL(k_dt_c_final, dim3(1), dim3(kParts), 0, st, c->pts(), c->partv, c->part + 2 * kParts,
                        c->cnt);
-    hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(1), 0, st, c->P, n, c->tv, c->to, c->cnt);
+    hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(1), 0, st, c->pts(), c->P, n, c->tv, c->to, c->cnt);
     DCHK(hipMemcpyAsync(h, c->cnt, sizeof(int) * NUM_C, hipMemcpyDeviceToHost, st), "check");
     DCHK(hipStreamSynchronize(st), "first triangle");
     if (h[C_ERR] & DT_ERR_INPUT) return fail(CVT_ERR_ARG, "a point is not finite");
     if (h[C_ERR] & DT_ERR_RANGE)
         return fail(CVT_ERR_ARG, "coordinates span more than 2^71 units of their finest bit");
     if (h[C_ERR]) return fail(CVT_ERR_ARG, "degenerate input: all points collinear or coincident");
-    hipLaunchKernelGGL(k_dt_locate0, dim3(nb(n)), dim3(256), 0, st, c->P, n, c->loc, c->cnt);
+    hipLaunchKernelGGL(k_dt_locate0, dim3(nb(n)), dim3(256), 0, st, c->pts(), n, c->loc, c->cnt);
     hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_CONV, 1, 1L);
     int T = 4, round = 0, done = 0;
     int first = 1;                     // first pass of the latest flip run
@@ -1427,10 +1638,11 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
             if (T <= kVoteLds)
                 hipLaunchKernelGGL(k_dt_vote_lds,
                                    dim3((unsigned)std::min<long>(256, (n + 1023) / 1024)),
-                                   dim3(1024), 0, st, c->P, n, T, c->tv, c->to, c->fstamp, first,
+                                   dim3(1024), 0, st, c->pts(), n, T, c->tv, c->to, c->fstamp,
+                                   first,
                                    c->loc, c->vote, c->cnt);
             else
-                hipLaunchKernelGGL(k_dt_vote, dim3(nb(n)), dim3(256), 0, st, c->P, n, T, c->tv,
+                hipLaunchKernelGGL(k_dt_vote, dim3(nb(n)), dim3(256), 0, st, c->pts(), n, T, c->tv,
                                    c->to, c->fstamp, first, c->loc, c->vote, c->cnt);
             hipLaunchKernelGGL(k_dt_split_flags, dim3(nb(T)), dim3(256), 0, st, c->vote, T,
                                c->flag);
@@ -1447,10 +1659,10 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
         if (h[C_UNINS] == 0) break;
         const int splits = h[C_SPLITS];
         if (T + 2 * splits > c->Tmax) return fail(CVT_ERR_CAPACITY, "triangle capacity");
-        hipLaunchKernelGGL(k_dt_split, dim3(nb(T)), dim3(256), 0, st, c->P, n, T, c->tv, c->to,
-                           c->vote, c->pos, c->loc, c->chk, round + 1, c->list[0], c->cnt);
-        hipLaunchKernelGGL(k_dt_relocate_split, dim3(nb(n)), dim3(256), 0, st, c->P, n, T, c->tv,
-                           c->vote, c->pos, c->loc, c->cnt);
+        hipLaunchKernelGGL(k_dt_split, dim3(nb(T)), dim3(256), 0, st, c->pts(), n, T, c->tv, c->to,
+                           c->vote, c->pos, c->loc, c->places(), c->chk, round + 1, c->list[0], c->cnt);
+        hipLaunchKernelGGL(k_dt_relocate_split, dim3(nb(n)), dim3(256), 0, st, c->pts(), n, T, c->tv,
+                           c->vote, c->pos, c->loc, c->places(), c->cnt);
         T += 2 * splits;
         ++c->stats[0];
         done = 0;
@@ -1478,7 +1690,7 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
     *num_tri = nt;
     if (nt > capacity) return fail(CVT_ERR_CAPACITY, "%d triangles, capacity %d", nt, capacity);
     // staged, then copied: the caller's arrays may be host or device memory
-    hipLaunchKernelGGL(k_dt_output, dim3(nb(T)), dim3(256), 0, st, c->tv, c->to, T, n, c->flag,
+    hipLaunchKernelGGL(k_dt_output, dim3(nb(T)), dim3(256), 0, st, c->pts(), c->tv, c->to, T, n, c->flag,
                        c->pos, c->otri, opp ? c->oopp : nullptr);
     DCHK(hipGetLastError(), "output launch");
     if (nt > 0) {
