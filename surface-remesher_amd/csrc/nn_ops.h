@@ -7,34 +7,43 @@
 
 namespace cvt {
 
-// 3x3 conv, padding 1: out = act(bias + conv(in, w)); w [9][Cout][Cin] bf16;
-// Cin % 32 == 0, Cout % 32 == 0
-void nn_conv3x3(hipStream_t s, const uint16_t *in, const uint16_t *w, const float *bias,
-                uint16_t *out, int N, int H, int W, int Cin, int Cout, int relu);
-// weight gradient dw[9][Cout][Cin] (+= when accumulate) of out-gradient g;
-// work holds nn_dw_splits(M, Cin, Cout) * 9 * Cout * Cin floats
-void nn_conv3x3_dw(hipStream_t s, const uint16_t *in, const uint16_t *g, float *dw, float *work,
-                   int N, int H, int W, int Cin, int Cout, int accumulate);
-int nn_dw_splits(long M, int Cin, int Cout);
-// db[c] = sum_m g[m][c]; work holds nn_colsum_splits(M) * C floats.  With
-// relu_y, g is first masked in place by the ReLU derivative of the layer's
-// output relu_y (g = 0 where relu_y <= 0).
-// splits of the column sum over M rows (its workspace holds splits * C floats)
-int nn_colsum_splits(long M);
-void nn_colsum(hipStream_t s, uint16_t *g, long M, int C, float *db, float *work,
-               const uint16_t *relu_y);
+// 3x3 convolution, padding 1, of N images of H x W pixels:
+// out = act(bias + conv(in, w)), Cin and Cout multiples of 32.
+struct NnConv {
+    // input channels: c0 of in0 (a multiple of 32; at half resolution and
+    // upsampled to nearest when up), then Cin - c0 of in1
+    const uint16_t *in0;
+    int c0, up;
+    const uint16_t *in1;
+    const uint16_t *w;        // bf16 in the order of nn_weights_bf16
+    const float *bias;        // or null
+    int relu;
+    uint16_t *out;
+    uint16_t *pool;           // or null: the 2x2 average of out (H, W even)
+    // the first c_low output channels (a multiple of 32) are summed 2x2 into
+    // low (H / 2, W / 2, c_low) and out holds the others: the gradient of an
+    // input with `up` (H, W even)
+    uint16_t *low;
+    int c_low;
+    // or null: a layer's ReLU output; low (when c_low) or out is zero where
+    // it is not positive
+    const uint16_t *mask;
+};
+void nn_conv3x3(hipStream_t s, const NnConv &p, int N, int H, int W, int Cin, int Cout);
+// gradients dw[9][Cout][Cin] and then db[Cout] of the convolution p (its
+// inputs) from the out-gradient g; work holds
+// nn_dw_max_splits(Cin, Cout) * Cout * (9 * Cin + 1) floats
+void nn_conv3x3_dw(hipStream_t s, const NnConv &p, const uint16_t *g, float *dw_db, float *work,
+                   int N, int H, int W, int Cin, int Cout);
+int nn_dw_max_splits(int Cin, int Cout);
 // fp32 weights -> bf16 forward copy and flipped/transposed data-gradient copy
 void nn_weights_bf16(hipStream_t s, const float *w, int Cin, int Cout, uint16_t *wf, uint16_t *wb);
-void nn_avgpool2(hipStream_t s, const uint16_t *in, uint16_t *out, int N, int H, int W, int C);
-void nn_avgpool2_bwd(hipStream_t s, const uint16_t *gout, uint16_t *gin, int N, int H, int W, int C,
-                     int accumulate);
-// (N, H, W, C1) low upsampled x2 into channels [0, C1), skip (N, 2H, 2W, C2)
-// into [C1, C1 + C2)
-void nn_up_concat(hipStream_t s, const uint16_t *low, const uint16_t *skip, uint16_t *out, int N,
-                  int H, int W, int C1, int C2);
-void nn_up_concat_bwd(hipStream_t s, const uint16_t *gout, uint16_t *glow, uint16_t *gskip, int N,
-                      int H, int W, int C1, int C2, int acc_skip);
-// 1x1 head NN_HEAD_C -> 2 (fp32 out); dwh_db = [dwh (2C), dbh (2)]; work
+// gradient of the 2x2 average
+// with mask (a ReLU output shaped as gin), gin = 0 where mask <= 0
+void nn_avgpool2_bwd(hipStream_t s, const uint16_t *gout, uint16_t *gin, const uint16_t *mask,
+                     int N, int H, int W, int C, int accumulate);
+// 1x1 head NN_HEAD_C -> 2 (fp32 out); its backward masks gx by x > 0 (x is a
+// ReLU output); dwh_db = [dwh (2C), dbh (2)]; work
 // nn_head_splits(M) * (2C + 2) floats
 constexpr int NN_HEAD_C = 32;
 int nn_head_splits(long M);

@@ -19,371 +19,16 @@
 namespace cvt {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 __device__ __forceinline__ float bf2f(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
 __device__ __forceinline__ uint16_t f2bf(float f)
 {
-    // round to nearest even (no NaN inputs in this network)
-    const uint32_t u = __float_as_uint(f);
-    const uint32_t r = u + 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(r >> 16);
+    return __builtin_bit_cast(uint16_t, (__bf16)f);   // to nearest even, in hardware
 }
 
-// Implicit-GEMM 3x3 convolution, NHWC bf16, fp32 accumulation on MFMA:
-// out[m][co] = act(bias[co] + sum_tap sum_ci in[m + off(tap)][ci] * w[tap][co][ci])
-// A block computes 128 pixels x BN output channels (4 waves x 32 pixels;
-// each wave 2 x BN/16 MFMA tiles of 16 x 16); the reduction runs over
-// (tap, 32-channel slice) stages, double-buffered in LDS with the next
-// stage's global loads issued before the current stage's MFMAs.
-// grid (ceil(M / 128), Cout / BN), block 256; Cin % 32 == 0, Cout % BN == 0.
-template <int BN>
-__global__ __launch_bounds__(256) void k_conv3x3_t(const uint16_t *__restrict__ in,
-                                                   const uint16_t *__restrict__ w,
-                                                   const float *__restrict__ bias,
-                                                   uint16_t *__restrict__ out, int N, int H, int W,
-                                                   int Cin, int Cout, int relu)
-{
-    constexpr int BM = 128, LK = 40;               // pixels per block, LDS row pitch (bf16)
-    __shared__ uint16_t sA[2][BM * LK];
-    __shared__ uint16_t sB[2][BN * LK];
-    const long M = (long)N * H * W;
-    const long m0 = (long)blockIdx.x * BM;
-    const int co0 = blockIdx.y * BN;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    // A staging: pixel am = t / 2, channels [16 * (t % 2), +16): two 16-byte words
-    const int am = t >> 1, ahalf = t & 1;
-    const long m = m0 + am;
-    int an = 0, ay = 0, ax = 0;
-    if (m < M) {
-        an = (int)(m / ((long)H * W));
-        const int r = (int)(m - (long)an * H * W);
-        ay = r / W;
-        ax = r - ay * W;
-    }
-    // B staging: output channel bco = t / 4, 8 channels at 8 * (t % 4)
-    const bool bstage = t < BN * 4;
-    const int bco = t >> 2, bpart = t & 3;
-    const int nci = Cin / 32, nstage = 9 * nci;
-    uint4 va0, va1, vb;
-    auto load = [&](int st) {
-        const int tap = st / nci, ci0 = (st - tap * nci) * 32;
-        const int yy = ay + tap / 3 - 1, xx = ax + tap % 3 - 1;
-        va0 = va1 = make_uint4(0, 0, 0, 0);
-        if (m < M && yy >= 0 && yy < H && xx >= 0 && xx < W) {
-            const uint4 *src = reinterpret_cast<const uint4 *>(
-                in + (((long)an * H + yy) * W + xx) * Cin + ci0 + 16 * ahalf);
-            va0 = src[0];
-            va1 = src[1];
-        }
-        if (bstage)
-            vb = *reinterpret_cast<const uint4 *>(w + ((long)tap * Cout + co0 + bco) * Cin + ci0 +
-                                                  8 * bpart);
-    };
-    auto store = [&](int buf) {
-        uint4 *da = reinterpret_cast<uint4 *>(&sA[buf][am * LK + 16 * ahalf]);
-        da[0] = va0;
-        da[1] = va1;
-        if (bstage) *reinterpret_cast<uint4 *>(&sB[buf][bco * LK + 8 * bpart]) = vb;
-    };
-    f32x4 acc[2][BN / 16];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int b = 0; b < BN / 16; ++b) acc[i][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    load(0);
-    store(0);
-    __syncthreads();
-    int buf = 0;
-    for (int st = 0; st < nstage; ++st) {
-        const bool more = st + 1 < nstage;
-        if (more) load(st + 1);
-        bf16x8 a[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            a[i] = *reinterpret_cast<const bf16x8 *>(
-                &sA[buf][(wave * 32 + i * 16 + (lane & 15)) * LK + 8 * (lane >> 4)]);
-#pragma unroll
-        for (int b = 0; b < BN / 16; ++b) {
-            const bf16x8 bb = *reinterpret_cast<const bf16x8 *>(
-                &sB[buf][(b * 16 + (lane & 15)) * LK + 8 * (lane >> 4)]);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bb, acc[i][b], 0, 0, 0);
-        }
-        if (more) store(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
-    }
-#pragma unroll
-    for (int b = 0; b < BN / 16; ++b) {
-        const int co = co0 + b * 16 + (lane & 15);
-        const float bv = bias ? bias[co] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const long mm = m0 + wave * 32 + i * 16 + 4 * (lane >> 4) + e;
-                if (mm < M) {
-                    float v = acc[i][b][e] + bv;
-                    if (relu) v = fmaxf(v, 0.0f);
-                    out[mm * Cout + co] = f2bf(v);
-                }
-            }
-    }
-}
-
-// Weight-gradient partials of TG taps on a BCO x BCI tile of (co, ci):
-// part[split][tap][co][ci] = sum over the split's pixels m of
-// g[m][co] * in[m + off(tap)][ci].  grid (9 / TG * Cout/BCO * Cin/BCI,
-// splits), block 256; TG = 3 takes the three taps of one kernel row, which
-// share the g tile and read the same input rows.  The reduction runs over
-// pixels in stages of KM; each stage's g tile and TG tap-shifted input tiles
-// are staged in LDS transposed to [channel][pixel] (the MFMA operands take 8
-// consecutive pixels per lane): a staging item is 4 pixels x 4 channels,
-// written as 4 eight-byte rows, dealt to the 256 threads in turn.  Each wave
-// then runs KM / 32 MFMA k-steps on each of its tiles, in pixel order, so
-// the sums depend on neither KM nor TG.  The next stage's loads are issued
-// before this stage's MFMAs (two LDS buffers, one barrier per stage).
-// Requires W % 4 == 0 and chunk % 4 == 0.
-template <int BCO, int BCI, int KM, int TG>
-__global__ __launch_bounds__(256) void k_conv3x3_dw2(const uint16_t *__restrict__ in,
-                                                     const uint16_t *__restrict__ g,
-                                                     float *__restrict__ part, int N, int H, int W,
-                                                     int Cin, int Cout, long chunk)
-{
-    constexpr int LP = KM + 8;                     // LDS row pitch (bf16)
-    constexpr int NTT = (BCO / 16) * (BCI / 16);   // 16x16 output tiles per tap
-    constexpr int TPW = TG * NTT / 4;              // tiles per wave
-    constexpr int NGI = (KM / 4) * (BCO / 4);      // g items per stage
-    constexpr int NXT = (KM / 4) * (BCI / 4);      // input items per tap and stage
-    constexpr int IG = (NGI + 255) / 256, IX = (TG * NXT + 255) / 256;
-    static_assert(TPW * 4 == TG * NTT, "tiles must fill the waves");
-    __shared__ uint16_t sG[2][BCO * LP];
-    __shared__ uint16_t sX[2][TG][BCI * LP];
-    const int nco = Cout / BCO, nci = Cin / BCI;
-    const int bx = blockIdx.x;
-    const int tap0 = (bx / (nco * nci)) * TG;
-    const int co0 = ((bx / nci) % nco) * BCO, ci0 = (bx % nci) * BCI;
-    const long M = (long)N * H * W;
-    const long mb = (long)blockIdx.y * chunk, me = min(M, mb + chunk);
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    // g item it: pixel group it / (BCO / 4), channel group it % (BCO / 4);
-    // input item it: tap tap0 + it / NXT, then the same split of it % NXT
-    uint2 vg[IG][4], vx[IX][4];
-    auto load = [&](long mc) {
-#pragma unroll
-        for (int r = 0; r < IG; ++r) {
-            const int it = t + 256 * r, ch = 4 * (it % (BCO / 4));
-            const long m = mc + 4 * (it / (BCO / 4));
-#pragma unroll
-            for (int p = 0; p < 4; ++p)
-                vg[r][p] = (it < NGI && m + p < me)
-                               ? *reinterpret_cast<const uint2 *>(g + (m + p) * Cout + co0 + ch)
-                               : make_uint2(0, 0);
-        }
-#pragma unroll
-        for (int r = 0; r < IX; ++r) {
-            const int it = t + 256 * r, j = it / NXT, rest = it % NXT;
-            const int ch = 4 * (rest % (BCI / 4));
-            const long m = mc + 4 * (rest / (BCI / 4));   // 4 pixels of one row
-#pragma unroll
-            for (int p = 0; p < 4; ++p) vx[r][p] = make_uint2(0, 0);
-            if (j >= TG || m >= me) continue;
-            const int tap = tap0 + j, ky = tap / 3 - 1, kx = tap % 3 - 1;
-            const int n = (int)(m / ((long)H * W));
-            const int rr = (int)(m - (long)n * H * W);
-            const int y = rr / W, x = rr - (rr / W) * W;
-            const int yy = y + ky;
-            if (yy < 0 || yy >= H) continue;
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const int xx = x + p + kx;
-                if (m + p < me && xx >= 0 && xx < W)
-                    vx[r][p] = *reinterpret_cast<const uint2 *>(
-                        in + (((long)n * H + yy) * W + xx) * Cin + ci0 + ch);
-            }
-        }
-    };
-    // channel q of an item: its values at the 4 pixels, one 8-byte row piece
-    auto put = [&](uint16_t *dst, const uint2 (&v)[4], int ch, int pg) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t e0 = ((q < 2 ? v[0].x : v[0].y) >> (16 * (q & 1))) & 0xffffu;
-            const uint32_t e1 = ((q < 2 ? v[1].x : v[1].y) >> (16 * (q & 1))) & 0xffffu;
-            const uint32_t e2 = ((q < 2 ? v[2].x : v[2].y) >> (16 * (q & 1))) & 0xffffu;
-            const uint32_t e3 = ((q < 2 ? v[3].x : v[3].y) >> (16 * (q & 1))) & 0xffffu;
-            *reinterpret_cast<uint2 *>(&dst[(ch + q) * LP + 4 * pg]) =
-                make_uint2(e0 | (e1 << 16), e2 | (e3 << 16));
-        }
-    };
-    auto store = [&](int buf) {
-#pragma unroll
-        for (int r = 0; r < IG; ++r) {
-            const int it = t + 256 * r;
-            if (it < NGI) put(sG[buf], vg[r], 4 * (it % (BCO / 4)), it / (BCO / 4));
-        }
-#pragma unroll
-        for (int r = 0; r < IX; ++r) {
-            const int it = t + 256 * r, j = it / NXT, rest = it % NXT;
-            if (j < TG) put(sX[buf][j], vx[r], 4 * (rest % (BCI / 4)), rest / (BCI / 4));
-        }
-    };
-    f32x4 acc[TPW];
-#pragma unroll
-    for (int k = 0; k < TPW; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    int buf = 0;
-    load(mb);
-    store(0);
-    __syncthreads();
-    for (long mc = mb; mc < me; mc += KM) {
-        const bool more = mc + KM < me;
-        if (more) load(mc + KM);
-#pragma unroll
-        for (int kk = 0; kk < KM / 32; ++kk)
-#pragma unroll
-            for (int k = 0; k < TPW; ++k) {
-                const int tile = wave + 4 * k, j = tile / NTT, rem = tile % NTT;
-                const int tco = rem / (BCI / 16), tci = rem % (BCI / 16);
-                const bf16x8 a = *reinterpret_cast<const bf16x8 *>(
-                    &sG[buf][(tco * 16 + (lane & 15)) * LP + 32 * kk + 8 * (lane >> 4)]);
-                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(
-                    &sX[buf][j][(tci * 16 + (lane & 15)) * LP + 32 * kk + 8 * (lane >> 4)]);
-                acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[k], 0, 0, 0);
-            }
-        if (more) store(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
-    }
-    const long tap_sz = (long)Cout * Cin;
-#pragma unroll
-    for (int k = 0; k < TPW; ++k) {
-        const int tile = wave + 4 * k, j = tile / NTT, rem = tile % NTT;
-        const int tco = rem / (BCI / 16), tci = rem % (BCI / 16);
-        float *dst = part + (long)blockIdx.y * 9 * tap_sz + (long)(tap0 + j) * tap_sz;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int co = co0 + tco * 16 + 4 * (lane >> 4) + e;
-            const int ci = ci0 + tci * 16 + (lane & 15);
-            dst[(long)co * Cin + ci] = acc[k][e];
-        }
-    }
-}
-
-// out[c] = sum_s part[s][c] for few columns and many splits: one block per
-// column, threads take every 256th split, then a fixed-order tree
-__global__ __launch_bounds__(256) void k_sum_cols(const float *__restrict__ part, int splits, int C,
-                                                  float *__restrict__ out)
-{
-    __shared__ float red[256];
-    const int c = blockIdx.x;
-    float acc = 0.0f;
-    for (int k = threadIdx.x; k < splits; k += 256) acc += part[(long)k * C + c];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = red[0];
-}
-
-// out[i] = sum_s part[s][i] in a fixed order (deterministic): block 256
-// takes 64 consecutive i; its four waves sum the splits s = q, q + 4, ...
-// (q = wave) in order, then the four sums are added in wave order.
-// grid ceil(n / 64).
-__global__ __launch_bounds__(256) void k_sum_splits(const float *__restrict__ part, int splits,
-                                                    long n, float *__restrict__ out,
-                                                    int accumulate)
-{
-    __shared__ float red[4][64];
-    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const long i = (long)blockIdx.x * 64 + lane;
-    float s = 0.0f;
-    if (i < n) {
-#pragma unroll 8
-        for (int k = q; k < splits; k += 4) s += part[(long)k * n + i];
-    }
-    red[q][lane] = s;
-    __syncthreads();
-    if (q == 0 && i < n) {
-        const float t = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
-        out[i] = accumulate ? out[i] + t : t;
-    }
-}
-
-// per-split column sums of g [M][C] (bf16, C % 8 == 0, C <= 256) ->
-// part[split][C]: a thread owns 8 consecutive channels (one 16-byte load per
-// row) and every (256 / (C / 8))-th row of the split; the threads of one
-// channel group are then added in thread order (deterministic).  With RELU,
-// g is first masked in place by the ReLU derivative of the layer's output y
-// (g = 0 where y <= 0), the backward of the activation, and the masked
-// values are summed.
-template <bool RELU>
-__global__ __launch_bounds__(256) void k_colsum(uint16_t *__restrict__ g,
-                                                const uint16_t *__restrict__ y, long M, int C,
-                                                long chunk, float *__restrict__ part)
-{
-    __shared__ float red[256][9];
-    const long mb = (long)blockIdx.x * chunk, me = min(M, mb + chunk);
-    const int cg = C >> 3;                    // channel groups of 8
-    const int rows = 256 / cg;                // rows per block step
-    const int t = threadIdx.x;
-    const int grp = t % cg, r0 = t / cg;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (r0 < rows) {
-        for (long m = mb + r0; m < me; m += rows) {
-            uint4 *gp = reinterpret_cast<uint4 *>(g + m * C + grp * 8);
-            const uint4 v = *gp;
-            uint32_t w[4] = {v.x, v.y, v.z, v.w};
-            if constexpr (RELU) {
-                const uint4 yv = *reinterpret_cast<const uint4 *>(y + m * C + grp * 8);
-                const uint32_t yw[4] = {yv.x, yv.y, yv.z, yv.w};
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (!(__uint_as_float(yw[k] << 16) > 0.0f)) w[k] &= 0xffff0000u;
-                    if (!(__uint_as_float(yw[k] & 0xffff0000u) > 0.0f)) w[k] &= 0x0000ffffu;
-                }
-                *gp = make_uint4(w[0], w[1], w[2], w[3]);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                acc[2 * k] += __uint_as_float(w[k] << 16);
-                acc[2 * k + 1] += __uint_as_float(w[k] & 0xffff0000u);
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) red[t][k] = acc[k];
-    __syncthreads();
-    if (t < C) {
-        const int cgp = t >> 3, k = t & 7;
-        float s = 0.0f;
-        for (int r = 0; r < rows; ++r) s += red[r * cg + cgp][k];
-        part[(long)blockIdx.x * C + t] = s;
-    }
-}
-
-// fp32 master [9][Cout][Cin] -> bf16 forward copy (same layout) and the
-// flipped, transposed copy for the data gradient: [9][Cin][Cout], tap -> 8 - tap
-__global__ void k_weights_bf16(const float *__restrict__ w, int Cin, int Cout,
-                               uint16_t *__restrict__ wf, uint16_t *__restrict__ wb)
-{
-    const long n = 9L * Cin * Cout;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int tap = (int)(i / ((long)Cin * Cout));
-    const int r = (int)(i - (long)tap * Cin * Cout);
-    const int co = r / Cin, ci = r - (r / Cin) * Cin;
-    const uint16_t v = f2bf(w[i]);
-    wf[i] = v;
-    wb[((long)(8 - tap) * Cin + ci) * Cout + co] = v;
-}
-
-// g *= (y > 0)
-// Elementwise layers work on 8 channels (one 16-byte word) per thread with
-// 32-bit indices: channel counts are multiples of 8 and every tensor of the
-// network has fewer than 2^31 elements.
 __device__ __forceinline__ void unpack8(const uint4 &v, float f[8])
 {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -395,37 +40,568 @@ __device__ __forceinline__ void unpack8(const uint4 &v, float f[8])
 }
 __device__ __forceinline__ uint4 pack8(const float f[8])
 {
-    uint32_t w[4];
+    bf16x8 v;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) w[k] = (uint32_t)f2bf(f[2 * k]) | ((uint32_t)f2bf(f[2 * k + 1]) << 16);
+    for (int k = 0; k < 8; ++k) v[k] = (__bf16)f[k];
+    const u32x4 w = __builtin_bit_cast(u32x4, v);
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// 2x2 average pool, NHWC (H, W even)
-__global__ void k_avgpool2(const uint16_t *__restrict__ in, uint16_t *__restrict__ out, int N,
-                           int H, int W, int C)
+// g where the layer's output y > 0, else 0: the derivative of the ReLU
+__device__ __forceinline__ uint4 relu_mask(uint4 g, const uint4 &y)
 {
-    const int Ho = H / 2, Wo = W / 2, C8 = C / 8;
-    const int n8 = N * Ho * Wo * C8;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n8) return;
-    const int c8 = i % C8;
-    const int p = i / C8;
-    const int x = p % Wo, y = (p / Wo) % Ho, b = p / (Wo * Ho);
-    const uint4 *src = reinterpret_cast<const uint4 *>(in);
-    const int base = ((b * H + 2 * y) * W + 2 * x) * C8 + c8;
-    float f0[8], f1[8], f2[8], f3[8], o[8];
-    unpack8(src[base], f0);
-    unpack8(src[base + C8], f1);
-    unpack8(src[base + W * C8], f2);
-    unpack8(src[base + W * C8 + C8], f3);
+    uint32_t w[4] = {g.x, g.y, g.z, g.w};
+    const uint32_t yw[4] = {y.x, y.y, y.z, y.w};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) o[k] = 0.25f * (f0[k] + f1[k] + f2[k] + f3[k]);
-    reinterpret_cast<uint4 *>(out)[i] = pack8(o);
+    for (int k = 0; k < 4; ++k) {
+        if (!(__uint_as_float(yw[k] << 16) > 0.0f)) w[k] &= 0xffff0000u;
+        if (!(__uint_as_float(yw[k] & 0xffff0000u) > 0.0f)) w[k] &= 0x0000ffffu;
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Implicit-GEMM 3x3 convolution, NHWC bf16, fp32 accumulation on MFMA:
+// out[m][co] = act(bias[co] + sum_tap sum_ci in[m + off(tap)][ci] * w[tap][co][ci])
+// A wave computes a strip of 16 x R pixels (columns x rows) of 32 output
+// channels; the block's WX x WY strips share one input window in LDS.  Every
+// sum runs over the taps in order and, within a tap, over 32-channel slices,
+// whatever the tile: the rounding of a layer does not depend on the batch.
+// The weights are stored in the order of the MFMA's row operand
+// (k_weights_bf16) and come straight from memory to registers.  The channels
+// of a lane's two row operands interleave by fours, so that a lane ends with
+// eight consecutive channels of its pixel: one 16-byte store.
+// The input channels come from in0 (the first c0, read at half resolution
+// when `up`: the nearest upsampling of a decoder level) and then in1, so a
+// skip concatenation needs no tensor of its own.
+// The items (tile, 32-channel group) of one tile run on one XCD, next to each
+// other: `per` tiles to each of the 8 XCDs.
+struct ConvShape {
+    int H, W, Cin, Cout, tilesX, tilesY, tiles;
+};
+
+// the source of channel slice sl of image n, as a buffer that reads zero
+// outside, and byte offset / pitch of its pixels
+struct ConvSource {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int pitch, row, sh;                            // bytes per pixel, pixels per row
+};
+__device__ __forceinline__ ConvSource conv_source(const NnConv &p, const ConvShape &q, int n, int sl)
+{
+    const int ci0 = 32 * sl;
+    const bool first = ci0 < p.c0;
+    const int C = first ? p.c0 : q.Cin - p.c0, sh = first ? p.up : 0;
+    const int Hs = q.H >> sh, Ws = q.W >> sh;
+    const uint16_t *src = (first ? p.in0 + ci0 : p.in1 + (ci0 - p.c0)) + (long)n * Hs * Ws * C;
+    ConvSource c;
+    c.rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)src, 0, 2 * Hs * Ws * C, 0x00020000);
+    c.pitch = 2 * C;
+    c.row = Ws;
+    c.sh = sh;
+    return c;
+}
+// 8 channels from byte o of pixel (yy, xx), zero outside the image
+__device__ __forceinline__ u32x4 conv_load(const ConvSource &c, const ConvShape &q, int yy, int xx, int o)
+{
+    const bool in = (uint32_t)yy < (uint32_t)q.H && (uint32_t)xx < (uint32_t)q.W;
+    return __builtin_amdgcn_raw_buffer_load_b128(
+        c.rsrc, in ? (uint32_t)(((yy >> c.sh) * c.row + (xx >> c.sh)) * c.pitch + o) : ~0u, 0, 0);
+}
+
+// bias, activation and stores of a strip: column x, rows y0 .. of image n,
+// channels co .. co + 7 of this lane
+template <int R, int NT>
+__device__ __forceinline__ void conv_store(const NnConv &p, const ConvShape &q, const f32x4 (&acc)[R][NT],
+                                           int n, int y0, int x, int co, int b0 = 0)
+{
+    static_assert(R % 2 == 0, "rows in pairs");
+    float bv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bv[e] = p.bias ? p.bias[co + e] : 0.0f;
+    const bool low = co < p.c_low;                 // uniform: c_low is a multiple of 32
+    const int Co = q.Cout - p.c_low, Cl = low ? p.c_low : q.Cout;
+    const long o0 = ((long)(n * q.H + y0) * q.W + x) * Co + co - p.c_low;
+#pragma unroll
+    for (int r = 0; r < R; r += 2) {
+        uint4 w[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] = acc[r + j][b0 + (e >> 2)][e & 3] + bv[e];
+                if (p.relu) v[e] = fmaxf(v[e], 0.0f);
+            }
+            w[j] = pack8(v);
+            if (low || x >= q.W || y0 + r + j >= q.H) continue;
+            const long o = o0 + (long)(r + j) * q.W * Co;
+            uint4 u = w[j];
+            if (p.mask && !p.c_low) u = relu_mask(u, *reinterpret_cast<const uint4 *>(p.mask + o));
+            *reinterpret_cast<uint4 *>(p.out + o) = u;
+        }
+        if (!low && !p.pool) continue;
+        // 2x2 sums of the rounded values, the right column from the next lane
+        float f[2][8], v[8];
+        unpack8(w[0], f[0]);
+        unpack8(w[1], f[1]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float g[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                g[j] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f[j][e]), 0xb1,
+                                                                  0xf, 0xf, true));
+            v[e] = f[0][e] + g[0] + f[1][e] + g[1];
+            if (!low) v[e] *= 0.25f;
+        }
+        if (x >= q.W || y0 + r >= q.H || (x & 1)) continue;
+        const long o = ((long)(n * (q.H / 2) + (y0 + r) / 2) * (q.W / 2) + x / 2) * Cl + co;
+        uint4 u = pack8(v);
+        if (low && p.mask) u = relu_mask(u, *reinterpret_cast<const uint4 *>(p.mask + o));
+        *reinterpret_cast<uint4 *>((low ? p.low : p.pool) + o) = u;
+    }
+}
+
+// Convolution of NS slices whose weights stay in registers while the block
+// walks over its tiles (one channel group per block).  The pixels of one
+// window row at one column offset and slice are one MFMA operand, read once
+// and multiplied with the weights of the three vertical taps into three rows
+// of sums: 3 (R + 2) LDS reads for 18 R MFMAs per slice.  The next tile's
+// window is loaded meanwhile.
+// block 64 WX WY, grid 8 J, J a multiple of Cout / 32.
+template <int R, int WX, int WY, int NS>
+__global__ __launch_bounds__(64 * WX * WY, NS == 1 ? 2 : 1) void k_conv3x3_keep(const NnConv p,
+                                                                              const ConvShape q)
+{
+    constexpr int GT = 64 * WX * WY;
+    constexpr int PX = 16 * WX + 2, PY = R * WY + 2;
+    constexpr int LK = 40, SL = PX * PY * LK;      // LDS pitch of a pixel, a slice (bf16)
+    constexpr int NA = (PX * PY * 4 + GT - 1) / GT;   // 16-byte loads per thread and slice
+    __shared__ uint16_t sA[NS * SL];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wx = wave % WX, wy = wave / WX;
+    const int NC = q.Cout >> 5, per = (q.tiles + 7) >> 3, J = (gridDim.x >> 3) / NC;
+    const int tile0 = (blockIdx.x & 7) * per, mine = min(per, q.tiles - tile0);
+    const int cg = (blockIdx.x >> 3) % NC;
+    int k = (blockIdx.x >> 3) / NC;
+    if (k >= mine) return;
+
+    int wpos[NA];                                  // window row << 8 | column of the loads
+#pragma unroll
+    for (int r = 0; r < NA; ++r) {
+        const int px = (t + GT * r) >> 2;
+        wpos[r] = (px / PX) << 8 | px % PX;
+    }
+    u32x4 va[NS][NA];
+    auto load_window = [&](int kk) {
+        const int tile = tile0 + kk;
+        const int x0 = (tile % q.tilesX) * (16 * WX) - 1;
+        const int y0 = ((tile / q.tilesX) % q.tilesY) * (R * WY) - 1, n = tile / (q.tilesX * q.tilesY);
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl) {
+            const ConvSource c = conv_source(p, q, n, sl);
+#pragma unroll
+            for (int r = 0; r < NA; ++r)
+                va[sl][r] = conv_load(c, q, y0 + (wpos[r] >> 8), x0 + (wpos[r] & 255), 16 * (t & 3));
+        }
+    };
+    load_window(k);
+    bf16x8 wr[9][NS][2];
+#pragma unroll
+    for (int i = 0; i < 18 * NS; ++i)
+        wr[i / (2 * NS)][(i >> 1) % NS][i & 1] =
+            *reinterpret_cast<const bf16x8 *>(p.w + ((long)cg * (18 * NS) + i) * 512 + 8 * lane);
+    const uint16_t *sx = &sA[(wy * R * PX + 16 * wx + (lane & 15)) * LK + 8 * (lane >> 4)];
+    for (; k < mine; k += J) {
+        __syncthreads();
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl)
+#pragma unroll
+            for (int r = 0; r < NA; ++r) {
+                const int i = t + GT * r;
+                if (i < PX * PY * 4)
+                    *reinterpret_cast<u32x4 *>(&sA[sl * SL + (i >> 2) * LK + 8 * (i & 3)]) = va[sl][r];
+            }
+        __syncthreads();
+        if (k + J < mine) load_window(k + J);
+        f32x4 acc[R][2];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[r][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // window operands (row, column offset, slice) are read D ahead
+        constexpr int D = 3, NX = 3 * (R + 2) * NS;
+        bf16x8 xr[D + 1];
+        auto read = [&](int j) {
+            xr[j % (D + 1)] = *reinterpret_cast<const bf16x8 *>(
+                sx + j % NS * SL + (j / (3 * NS) * PX + j / NS % 3) * LK);
+        };
+#pragma unroll
+        for (int j = 0; j < D; ++j) read(j);
+#pragma unroll
+        for (int j = 0; j < NX; ++j) {
+            if (j + D < NX) read(j + D);
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) {
+                const int o = j / (3 * NS) - dy;
+                if (o < 0 || o >= R) continue;
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    acc[o][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        wr[3 * dy + j / NS % 3][j % NS][b], xr[j % (D + 1)], acc[o][b], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int tile = tile0 + k;
+        conv_store<R, 2>(p, q, acc, tile / (q.tilesX * q.tilesY),
+                         ((tile / q.tilesX) % q.tilesY) * (R * WY) + wy * R,
+                         (tile % q.tilesX) * (16 * WX) + 16 * wx + (lane & 15), 32 * cg + 8 * (lane >> 4));
+    }
+}
+
+// Convolution of any number of channels to 16 NT of them: the window of all
+// slices lies in LDS, loaded at once, and the weights of a step (tap, slice)
+// come WD steps ahead of their use: R LDS reads and R NT MFMAs per step.  An
+// LDS pixel is 64 bytes, its four 16-byte parts permuted by the column so that
+// 16 lanes of adjacent pixels meet distinct banks.
+// block 64 WX WY, grid 8 * (tiles / 8) * Cout / (16 NT), LDS (16 WX + 2) (R WY
+// + 2) 64 bytes per slice.
+template <int R, int WX, int WY, int NT, int WD>
+__global__ __launch_bounds__(64 * WX * WY, NT > 2 ? 1 : 2) void k_conv3x3(const NnConv p,
+                                                                        const ConvShape q)
+{
+    static_assert(9 % WD == 0 && WD % 3 == 0, "the rings turn with the steps");
+    constexpr int GT = 64 * WX * WY;
+    constexpr int PX = 16 * WX + 2, PY = R * WY + 2, SL = PX * PY * 32;
+    constexpr int NA = (PX * PY * 4 + GT - 1) / GT;
+    extern __shared__ __attribute__((aligned(16))) uint16_t conv_lds[];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wx = wave % WX, wy = wave / WX;
+    const int NC = q.Cout / (16 * NT), ns = q.Cin >> 5, per = (q.tiles + 7) >> 3;
+    const int k = blockIdx.x >> 3, cg = k % NC;
+    const int tile = (blockIdx.x & 7) * per + k / NC;
+    if (k / NC >= per || tile >= q.tiles) return;
+    const int x0 = (tile % q.tilesX) * (16 * WX), y0 = ((tile / q.tilesX) % q.tilesY) * (R * WY);
+    const int n = tile / (q.tilesX * q.tilesY);
+
+    bf16x8 wr[WD][NT];
+    const uint16_t *wp = p.w + (long)cg * (NT / 2) * ns * (18 * 512) + 8 * lane;
+    auto load_weights = [&](bf16x8 (&f)[NT], int st) {
+#pragma unroll
+        for (int b = 0; b < NT; ++b)
+            f[b] = *reinterpret_cast<const bf16x8 *>(wp + ((b >> 1) * ns * 18 + 2 * st + (b & 1)) * 512);
+    };
+#pragma unroll
+    for (int i = 0; i < WD; ++i) load_weights(wr[i], i);
+    // slices whose loads are in flight together, as registers allow
+    constexpr int NB = R == 2 || NT > 2 ? 7 : 4;
+    for (int sl = 0; sl < ns; sl += NB) {
+        u32x4 va[NB][NA];
+#pragma unroll
+        for (int h = 0; h < NB; ++h) {
+            if (sl + h >= ns) break;
+            const ConvSource c = conv_source(p, q, n, sl + h);
+#pragma unroll
+            for (int r = 0; r < NA; ++r) {
+                const int px = (t + GT * r) >> 2, row = px / PX;
+                va[h][r] = conv_load(c, q, row < PY ? y0 - 1 + row : -1, x0 - 1 + px % PX, 16 * (t & 3));
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < NB; ++h) {
+            if (sl + h >= ns) break;
+#pragma unroll
+            for (int r = 0; r < NA; ++r) {
+                const int i = t + GT * r, px = i >> 2;
+                if (i < PX * PY * 4)
+                    *reinterpret_cast<u32x4 *>(
+                        &conv_lds[(sl + h) * SL + px * 32 + 8 * ((i & 3) ^ (((px % PX) >> 2) & 3))]) = va[h][r];
+            }
+        }
+    }
+    f32x4 acc[R][NT];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) acc[r][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    const int col0 = 16 * wx + (lane & 15);
+    // step st = tap * ns + sl, operands two steps ahead
+    bf16x8 xr[3][R];
+    int tap = 0, sl = 0;                           // of the next read
+    auto read_step = [&](bf16x8 (&x)[R]) {
+        const int col = col0 + tap % 3;
+        const uint16_t *a = conv_lds + sl * SL + (wy * R * PX + (tap / 3) * PX + col) * 32 +
+                            8 * ((lane >> 4) ^ ((col >> 2) & 3));
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[r] = *reinterpret_cast<const bf16x8 *>(a + r * PX * 32);
+        if (++sl == ns) {
+            sl = 0;
+            tap = min(tap + 1, 8);
+        }
+    };
+    const int steps = 9 * ns;
+    read_step(xr[0]);
+    read_step(xr[1]);
+    for (int st = 0; st < steps; st += 9) {
+#pragma unroll
+        for (int u = 0; u < 9; ++u) {
+            read_step(xr[(u + 2) % 3]);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int b = 0; b < NT; ++b)
+                    acc[r][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u % WD][b], xr[u % 3][r],
+                                                                        acc[r][b], 0, 0, 0);
+            load_weights(wr[u % WD], min(st + u + WD, steps - 1));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < NT; b += 2)
+        conv_store<R, NT>(p, q, acc, n, y0 + wy * R, x0 + col0, 16 * (NT * cg + b) + 8 * (lane >> 4), b);
+}
+
+// eight bf16 of one channel at eight consecutive pixels, for 16 channels and
+// 32 pixels per wave, from two transposing LDS reads of a [pixel][channel]
+// tile: of each 16 lanes, lane i reads four channels of pixel i / 4 and
+// receives channel i of the four pixels
+__device__ __forceinline__ bf16x8 read_pixels(const uint16_t *lo, const uint16_t *hi)
+{
+    typedef __attribute__((address_space(3))) bf16x4 lds4;
+    const bf16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4 *)(bf16x4 *)lo);
+    const bf16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4 *)(bf16x4 *)hi);
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// Weight-gradient partials of a 32 x 32 block of (co, ci), all nine taps:
+// part[split][tap][co][ci] = sum over the split's pixels m of
+// g[m][co] * in[m + off(tap)][ci], followed in each split by the bias
+// partials [co], the sums of g[m][co] (from the blocks of ci = 0 ..).
+// The reduction runs over pixels, 32 of one image row per MFMA step.  A block
+// walks over 32 x 2R pixel tiles; g and the input window of a tile are staged
+// in LDS as they lie in memory, and the transposing LDS reads deliver 8
+// consecutive pixels of a channel at any column offset, so every tap reads
+// the one window.  Wave w takes 16 output channels (w & 1) of R rows (w / 2):
+// a window row's six operands (3 column offsets, 2 x 16 input channels) meet
+// the g operands of the three rows it is a vertical neighbour of, 18 MFMAs
+// for 14 reads; 72 sums per lane stay in registers over the whole split.  The
+// next tile's loads run during a tile's MFMAs.  Pixels outside the image read
+// as zero.  LDS rows are 64 bytes per pixel; the two 32-byte halves swap every
+// eight columns, which keeps the 32 lanes of a read phase on distinct banks.
+// Input channels come as in k_conv3x3.  grid Cout / 32 * Cin / 32 * splits, the
+// splits a multiple of 8: the blocks of one split run on one XCD, next to each
+// other, so its pixels are read from memory once.
+// Bound by memory on large images: 16 images of 256^2, 32 -> 32 channels, 35 us
+// for 134 MB (128 us when each tap read its own shifted tile, transposed by
+// eight-byte pieces), 96 -> 32 63 us (346 us); the bias gradient was a pass of
+// its own over g, 31 us.
+template <int R>
+__global__ __launch_bounds__(256, 2) void k_conv3x3_dw(const NnConv p, const uint16_t *__restrict__ g,
+                                                       float *__restrict__ part, int H, int W,
+                                                       int Cin, int Cout, int tilesX, int tilesY,
+                                                       int tiles, int splits)
+{
+    constexpr int TH = 2 * R, PX = 34, PY = TH + 2;
+    constexpr int NX = (PX * PY * 4 + 255) / 256, NG = TH * 32 * 4 / 256;
+    constexpr int RED = 2 * 64 * 72 * 4;           // bytes of the final sum over row sets
+    constexpr int LDS = (PX * PY + TH * 32) * 64;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[LDS > RED ? LDS : RED];
+    uint16_t *sX = reinterpret_cast<uint16_t *>(lds), *sG = sX + PX * PY * 32;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nci = Cin >> 5, P = (Cout >> 5) * nci;
+    const int k = blockIdx.x >> 3, pair = k % P;
+    const int split = (k / P) * 8 + (blockIdx.x & 7);
+    const int co0 = 32 * (pair / nci), ci0 = 32 * (pair % nci);
+    const int tb = (int)((long)tiles * split / splits), te = (int)((long)tiles * (split + 1) / splits);
+    const int cot = wave & 1, rs = wave >> 1;
+    const bool first = ci0 < p.c0;
+    const uint16_t *src = first ? p.in0 + ci0 : p.in1 + (ci0 - p.c0);
+    const int C = first ? p.c0 : Cin - p.c0, sh = first ? p.up : 0, Hs = H >> sh, Ws = W >> sh;
+
+    // window loads: LDS position | column << 16 | row << 24
+    int wpos[NX];
+#pragma unroll
+    for (int r = 0; r < NX; ++r) {
+        const int px = (t + 256 * r) >> 2, col = px % PX, row = px / PX;
+        wpos[r] = (px * 32 + 8 * ((t & 3) ^ (2 * ((col >> 3) & 1)))) | col << 16 | row << 24;
+    }
+    u32x4 vx[NX], vg[NG];
+    auto load = [&](int tile) {
+        const int x0 = (tile % tilesX) * 32, y0 = ((tile / tilesX) % tilesY) * TH;
+        const int n = tile / (tilesX * tilesY);
+        const auto rx = __builtin_amdgcn_make_buffer_rsrc((void *)(src + (long)n * Hs * Ws * C), 0,
+                                                          2 * Hs * Ws * C, 0x00020000);
+        const auto rg = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(g + (long)n * H * W * Cout + co0), 0, 2 * H * W * Cout, 0x00020000);
+#pragma unroll
+        for (int r = 0; r < NX; ++r) {
+            const int yy = y0 - 1 + (wpos[r] >> 24), xx = x0 - 1 + ((wpos[r] >> 16) & 255);
+            const uint32_t o = 2 * ((yy >> sh) * Ws + (xx >> sh)) * C + 16 * (t & 3);
+            vx[r] = __builtin_amdgcn_raw_buffer_load_b128(
+                rx, (uint32_t)yy < (uint32_t)H && (uint32_t)xx < (uint32_t)W ? o : ~0u, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < NG; ++r) {
+            const int yy = y0 + 2 * r + (t >> 7), xx = x0 + ((t >> 2) & 31);
+            const uint32_t o = 2 * (yy * W + xx) * Cout + 16 * (t & 3);
+            vg[r] = __builtin_amdgcn_raw_buffer_load_b128(rg, yy < H && xx < W ? o : ~0u, 0, 0);
+        }
+    };
+    // LDS positions of this lane's reads: column offset dx, pixel half h; the
+    // second 16 channels are at ^ 16
+    const int pc = 8 * (lane >> 4) + ((lane & 15) >> 2), cc = 4 * (lane & 3);
+    int ax[3][2], ag[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int col = pc + 4 * h;
+        ag[h] = (rs * R * 32 + col) * 32 + 16 * (cot ^ ((col >> 3) & 1)) + cc;
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+            ax[dx][h] = (rs * R * PX + col + dx) * 32 + 16 * (((col + dx) >> 3) & 1) + cc;
+    }
+    f32x4 acc[9][2], accb = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[i][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+    if (tb < te) load(tb);
+    for (int tile = tb; tile < te; ++tile) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < NX; ++r)
+            if (NX * 256 == PX * PY * 4 || t + 256 * r < PX * PY * 4)
+                *reinterpret_cast<u32x4 *>(&sX[wpos[r] & 0xffff]) = vx[r];
+#pragma unroll
+        for (int r = 0; r < NG; ++r)
+            *reinterpret_cast<u32x4 *>(
+                &sG[((t + 256 * r) >> 2) * 32 + 8 * ((t & 3) ^ (2 * ((t >> 5) & 1)))]) = vg[r];
+        __syncthreads();
+        if (tile + 1 < te) load(tile + 1);
+        // operands are read D steps (of a window row and column offset) ahead
+        constexpr int D = 1, NQ = 3 * (R + 2);
+        bf16x8 gv[4], xv[D + 1][2];
+        auto read_step = [&](int q) {
+            const int r = q / 3, dx = q % 3;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                xv[q % (D + 1)][b] = read_pixels(sX + ((ax[dx][0] ^ (16 * b)) + r * PX * 32),
+                                                 sX + ((ax[dx][1] ^ (16 * b)) + r * PX * 32));
+            if (dx == 0 && r < R) gv[r % 4] = read_pixels(sG + ag[0] + r * 1024, sG + ag[1] + r * 1024);
+        };
+#pragma unroll
+        for (int q = 0; q < D; ++q) read_step(q);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int r = q / 3, dx = q % 3;
+            if (q + D < NQ) read_step(q + D);
+            if (dx == 0 && r < R)
+                accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gv[r % 4], ones, accb, 0, 0, 0);
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) {
+                if (r - dy < 0 || r - dy >= R) continue;
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    acc[3 * dy + dx][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        gv[(r - dy) % 4], xv[q % (D + 1)][b], acc[3 * dy + dx][b], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // the two row sets' sums
+    float *red = reinterpret_cast<float *>(lds);
+    __syncthreads();
+    if (rs == 1) {
+#pragma unroll
+        for (int i = 0; i < 72; ++i)
+            red[(cot * 72 + i) * 64 + lane] = acc[i >> 3][(i >> 2) & 1][i & 3];
+    }
+    __syncthreads();
+    if (rs == 0) {
+        const long sz = (long)Cout * Cin;
+        const int co = co0 + 16 * cot + 4 * (lane >> 4), ci = ci0 + (lane & 15);
+        float *dst = part + split * (9 * sz + Cout) + (long)co * Cin + ci;
+#pragma unroll
+        for (int i = 0; i < 72; ++i)
+            dst[(i >> 3) * sz + (long)(i & 3) * Cin + 16 * ((i >> 2) & 1)] =
+                acc[i >> 3][(i >> 2) & 1][i & 3] + red[(cot * 72 + i) * 64 + lane];
+    }
+    if (ci0 == 0) {
+        __syncthreads();
+        if (rs == 1 && (lane & 15) == 0) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) red[16 * cot + 4 * (lane >> 4) + e] = accb[e];
+        }
+        __syncthreads();
+        if (rs == 0 && (lane & 15) == 0) {
+            const int c = 16 * cot + 4 * (lane >> 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                part[split * Cout * (9L * Cin + 1) + 9L * Cout * Cin + co0 + c + e] =
+                    accb[e] + red[c + e];
+        }
+    }
+}
+
+// out[i] = sum_s part[s][i] in a fixed order (deterministic): a block of 512
+// takes 32 consecutive i; its sixteen half waves sum the splits s = q, q + 16,
+// ... (q = half wave) in order, then the sums are added in order.
+// grid ceil(n / 32).
+__global__ __launch_bounds__(512) void k_sum_splits(const float *__restrict__ part, int splits,
+                                                    long n, float *__restrict__ out)
+{
+    __shared__ float red[16][32];
+    const int lane = threadIdx.x & 31, q = threadIdx.x >> 5;
+    const long i = (long)blockIdx.x * 32 + lane;
+    float s = 0.0f;
+    if (i < n) {
+#pragma unroll 8
+        for (int k = q; k < splits; k += 16) s += part[(long)k * n + i];
+    }
+    red[q][lane] = s;
+    __syncthreads();
+    if (q == 0 && i < n) {
+#pragma unroll
+        for (int j = 1; j < 16; ++j) s += red[j][lane];
+        out[i] = s;
+    }
+}
+
+// fp32 master [9][Cout][Cin] -> bf16 forward copy (same layout) and the
+// flipped, transposed copy for the data gradient: [9][Cin][Cout], tap -> 8 - tap
+// position of a convolution weight in k_conv3x3's operand order: blocks
+// [Cout / 32][9 taps][Cin / 32][2 row operands][64 lanes][8 channels of ci];
+// lane l, operand b holds row co = 8 ((l & 15) / 4) + 4 b + l % 4 of its
+// 32-channel block and columns ci = 8 (l / 16) ..
+__device__ __forceinline__ long conv_weight_index(int tap, int co, int ci, int Cin)
+{
+    const int c = co & 31, i = ci & 31;
+    const int lane = (c >> 3) * 4 + (c & 3) + 16 * (i >> 3), b = (c >> 2) & 1;
+    return ((((long)(co >> 5) * 9 + tap) * (Cin >> 5) + (ci >> 5)) * 2 + b) * 512 + lane * 8 + (i & 7);
+}
+
+__global__ void k_weights_bf16(const float *__restrict__ w, int Cin, int Cout,
+                               uint16_t *__restrict__ wf, uint16_t *__restrict__ wb)
+{
+    const long n = 9L * Cin * Cout;
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int tap = (int)(i / ((long)Cin * Cout));
+    const int r = (int)(i - (long)tap * Cin * Cout);
+    const int co = r / Cin, ci = r - (r / Cin) * Cin;
+    const uint16_t v = f2bf(w[i]);
+    wf[conv_weight_index(tap, co, ci, Cin)] = v;
+    wb[conv_weight_index(8 - tap, ci, co, Cout)] = v;
+}
+
+// gradient of the 2x2 average pool, NHWC (H, W even), 8 channels (one 16-byte
+// word) per thread with 32-bit indices: channel counts are multiples of 8 and
+// every tensor of the network has fewer than 2^31 such words
 __global__ void k_avgpool2_bwd(const uint16_t *__restrict__ gout, uint16_t *__restrict__ gin,
-                               int N, int H, int W, int C, int accumulate)
+                               const uint16_t *__restrict__ mask, int N, int H, int W, int C,
+                               int accumulate)
 {
     const int C8 = C / 8;
     const int n8 = N * H * W * C8;
@@ -445,64 +621,9 @@ __global__ void k_avgpool2_bwd(const uint16_t *__restrict__ gout, uint16_t *__re
 #pragma unroll
         for (int k = 0; k < 8; ++k) o[k] = 0.25f * v[k];
     }
-    reinterpret_cast<uint4 *>(gin)[i] = pack8(o);
-}
-
-// nearest 2x upsample of a (N, H, W, C1) tensor into channels [0, C1) of a
-// (N, 2H, 2W, C1 + C2) tensor, and copy of skip (N, 2H, 2W, C2) into [C1, C1+C2)
-__global__ void k_up_concat(const uint16_t *__restrict__ low, const uint16_t *__restrict__ skip,
-                            uint16_t *__restrict__ out, int N, int H, int W, int C1, int C2)
-{
-    const int Ho = 2 * H, Wo = 2 * W, C8 = (C1 + C2) / 8, L8 = C1 / 8, S8 = C2 / 8;
-    const int n8 = N * Ho * Wo * C8;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n8) return;
-    const int c8 = i % C8;
-    const int p = i / C8;
-    const int x = p % Wo, y = (p / Wo) % Ho, b = p / (Wo * Ho);
-    reinterpret_cast<uint4 *>(out)[i] =
-        (c8 < L8) ? reinterpret_cast<const uint4 *>(low)[((b * H + y / 2) * W + x / 2) * L8 + c8]
-                  : reinterpret_cast<const uint4 *>(skip)[p * S8 + (c8 - L8)];
-}
-
-// gradient of k_up_concat: 2x2 sums into the low tensor, and the skip part
-// added into the skip gradient (accumulate) or written
-__global__ void k_up_concat_bwd(const uint16_t *__restrict__ gout, uint16_t *__restrict__ glow,
-                                uint16_t *__restrict__ gskip, int N, int H, int W, int C1, int C2,
-                                int acc_skip)
-{
-    const int Ho = 2 * H, Wo = 2 * W, C8 = (C1 + C2) / 8, L8 = C1 / 8, S8 = C2 / 8;
-    const int nl = N * H * W * L8;
-    const int ns = N * Ho * Wo * S8;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint4 *go = reinterpret_cast<const uint4 *>(gout);
-    if (i < nl) {
-        const int c8 = i % L8;
-        const int p = i / L8;
-        const int x = p % W, y = (p / W) % H, b = p / (W * H);
-        const int o = ((b * Ho + 2 * y) * Wo + 2 * x) * C8 + c8;
-        float f0[8], f1[8], f2[8], f3[8], r[8];
-        unpack8(go[o], f0);
-        unpack8(go[o + C8], f1);
-        unpack8(go[o + Wo * C8], f2);
-        unpack8(go[o + Wo * C8 + C8], f3);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) r[k] = f0[k] + f1[k] + f2[k] + f3[k];
-        reinterpret_cast<uint4 *>(glow)[i] = pack8(r);
-    }
-    if (i < ns) {
-        const int c8 = i % S8;
-        const int p = i / S8;
-        float v[8];
-        unpack8(go[p * C8 + L8 + c8], v);
-        if (acc_skip) {
-            float g0[8];
-            unpack8(reinterpret_cast<const uint4 *>(gskip)[i], g0);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = g0[k] + v[k];
-        }
-        reinterpret_cast<uint4 *>(gskip)[i] = pack8(v);
-    }
+    uint4 w = pack8(o);
+    if (mask) w = relu_mask(w, reinterpret_cast<const uint4 *>(mask)[i]);
+    reinterpret_cast<uint4 *>(gin)[i] = w;
 }
 
 // 1x1 head, one pixel per thread: f[m] = bh + sum_c x[m][c] * wh[.][c], the
@@ -533,55 +654,53 @@ __global__ void k_head_fwd(const uint16_t *__restrict__ x, const float *__restri
 }
 
 // head gradients: gx[m][c] = sum_j gf[m][j] wh[j][c]; per-split partials of
-// dwh[j][c] = sum_m gf[m][j] x[m][c] and dbh[j] = sum_m gf[m][j].  A thread
-// takes every 256th pixel of the block's split (16-byte loads and stores of
-// the pixel's channels), then each partial is summed by a fixed butterfly
-// over the wave and the four waves in order (deterministic).
+// dwh[j][c] = sum_m gf[m][j] x[m][c] and dbh[j] = sum_m gf[m][j]; gx is zero
+// where x, a ReLU output, is not positive.  A thread takes eight channels (one
+// 16-byte load and store, adjacent over the wave) of every 64th pixel of the
+// block's split, then each partial is summed by a fixed butterfly over the
+// wave and the four waves in order (deterministic).  Bound by memory: 134 MB
+// for 16 images of 256^2 in 25 us (42 us with a whole pixel per thread).
 __global__ __launch_bounds__(256) void k_head_bwd(const uint16_t *__restrict__ x,
                                                   const float *__restrict__ gf,
                                                   const float *__restrict__ wh,
                                                   uint16_t *__restrict__ gx, float *__restrict__ part,
                                                   long M, long chunk)
 {
-    constexpr int C = NN_HEAD_C, NP = 2 * C + 2;
+    constexpr int C = NN_HEAD_C, NP = 2 * C + 2, Q = C / 8;
     __shared__ float red[4][NP];
     const long mb = (long)blockIdx.x * chunk, me = min(M, mb + chunk);
-    float accw[NP];
+    const int q = threadIdx.x % Q;                 // this thread's 8 channels
+    float w0[8], w1[8], acc[18];
 #pragma unroll
-    for (int k = 0; k < NP; ++k) accw[k] = 0.0f;
-    for (long m = mb + threadIdx.x; m < me; m += 256) {
-        const float g0 = gf[2 * m], g1 = gf[2 * m + 1];
-        const uint4 *src = reinterpret_cast<const uint4 *>(x + m * C);
-        uint4 *dst = reinterpret_cast<uint4 *>(gx + m * C);
+    for (int e = 0; e < 8; ++e) {
+        w0[e] = wh[8 * q + e];
+        w1[e] = wh[C + 8 * q + e];
+    }
 #pragma unroll
-        for (int q = 0; q < C / 8; ++q) {
-            const uint4 u = src[q];
-            const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
-            uint32_t o[4];
+    for (int k = 0; k < 18; ++k) acc[k] = 0.0f;
+    for (long m = mb + threadIdx.x / Q; m < me; m += 256 / Q) {
+        const float2 gm = *reinterpret_cast<const float2 *>(gf + 2 * m);
+        const uint4 u = *reinterpret_cast<const uint4 *>(x + m * C + 8 * q);
+        float v[8], o[8];
+        unpack8(u, v);
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const int c = 8 * q + e;
-                const float v0 = bf2f((uint16_t)(wd[e >> 1] & 0xffffu));
-                const float v1 = bf2f((uint16_t)(wd[e >> 1] >> 16));
-                o[e >> 1] = (uint32_t)f2bf(g0 * wh[c] + g1 * wh[C + c]) |
-                            ((uint32_t)f2bf(g0 * wh[c + 1] + g1 * wh[C + c + 1]) << 16);
-                accw[c] += g0 * v0;
-                accw[C + c] += g1 * v0;
-                accw[c + 1] += g0 * v1;
-                accw[C + c + 1] += g1 * v1;
-            }
-            dst[q] = make_uint4(o[0], o[1], o[2], o[3]);
+        for (int e = 0; e < 8; ++e) {
+            o[e] = gm.x * w0[e] + gm.y * w1[e];
+            acc[e] += gm.x * v[e];
+            acc[8 + e] += gm.y * v[e];
         }
-        accw[2 * C] += g0;
-        accw[2 * C + 1] += g1;
+        *reinterpret_cast<uint4 *>(gx + m * C + 8 * q) = relu_mask(pack8(o), u);
+        acc[16] += gm.x;
+        acc[17] += gm.y;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-    for (int k = 0; k < NP; ++k) {
-        float v = accw[k];
+    for (int k = 0; k < 18; ++k) {
+        float v = acc[k];
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if (lane == 0) red[wave][k] = v;
+        for (int o = 32; o >= Q; o >>= 1) v += __shfl_xor(v, o, 64);
+        const int c = k < 8 ? 8 * q + k : k < 16 ? C + 8 * q + k - 8 : 2 * C + k - 16;
+        if (lane < Q && (k < 16 || q == 0)) red[wave][c] = v;
     }
     __syncthreads();
     if (threadIdx.x < NP) {
@@ -779,70 +898,111 @@ __global__ void k_prepare_finish(const float *__restrict__ count, int R, int C, 
 // ---------------------------------------------------------------------------
 static inline unsigned nblk(long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-void nn_conv3x3(hipStream_t s, const uint16_t *in, const uint16_t *w, const float *bias,
-                uint16_t *out, int N, int H, int W, int Cin, int Cout, int relu)
+// The tile of a convolution.  Bound by memory on large images, by the latency
+// of its loads on one; us per call for (channels, side, images):
+//   32 -> 32, 256, 16    31 in 32 x 16 tiles            (73 tap by tap)
+//              256, 4    12.1, 32 x 8 11.4, 16 x 8 14.4
+//              256, 1     7.9,         6.2         6.2
+//   64 -> 64, 128, 16    30.6 weights three steps ahead, 34 nine (they take the
+//                        registers of a third block), 32 kept   (59)
+//   96 -> 96,  64, 16    20.0 nine ahead, 21.4 three, 22.7 kept (33)
+//   96 -> 32, 256, 16    73 kept, 93 nine ahead                 (183 and 55
+//                        for the concatenated tensor)
+//   160 -> 64, 128, 16   67 for 64 channels at once, 84 for 32  (117 + 24)
+//               128, 4   18.6                        22.4
+//   224 -> 96, 64, 16    31 for 96 channels at once, 47 for 32  (69 + 9)
+//               64, 4    26                          17.6
+//   96 -> 96,  64, 1      8.4 in 32 x 8 tiles, 6.8 in 16 x 4    (13.5)
+//   64 -> 64, 128, 4     10.3                  16
+// (in brackets a kernel that staged each tap of 128 pixels by itself).  So the
+// largest tile and the most channels at once that still give most of the 256
+// CUs a block.  Blocks that keep their weights: two per CU, or one where those
+// of three slices take the registers; each then walks its tiles and loads
+// ahead (16 images forward, one slice: 0.47 ms, 0.55 with half the blocks).
+void nn_conv3x3(hipStream_t s, const NnConv &p, int N, int H, int W, int Cin, int Cout)
 {
-    const long M = (long)N * H * W;
-    if (Cout % 64 == 0)
-        hipLaunchKernelGGL(k_conv3x3_t<64>, dim3(nblk(M, 128), Cout / 64), dim3(256), 0, s, in, w,
-                           bias, out, N, H, W, Cin, Cout, relu);
+    const int NC = Cout / 32;
+    auto shape = [&](int tw, int th) {
+        const int tx = (W + tw - 1) / tw, ty = (H + th - 1) / th;
+        return ConvShape{H, W, Cin, Cout, tx, ty, N * tx * ty};
+    };
+    auto tiles = [&](int tw, int th) { return (long)shape(tw, th).tiles; };
+#define NN_KEEP(R, WX, WY, NS)                                                                     \
+    {                                                                                              \
+        const ConvShape q = shape(16 * WX, R * WY);                                                \
+        const int per = (q.tiles + 7) / 8, most = std::max(1, (NS == 1 ? 64 : 32) / NC);           \
+        hipLaunchKernelGGL((k_conv3x3_keep<R, WX, WY, NS>), dim3(8 * NC * std::min(per, most)),    \
+                           dim3(64 * WX * WY), 0, s, p, q);                                        \
+    }
+#define NN_CONV(R, WX, WY, NT, WD)                                                                 \
+    {                                                                                              \
+        const ConvShape q = shape(16 * WX, R * WY);                                                \
+        const int per = (q.tiles + 7) / 8;                                                         \
+        hipLaunchKernelGGL((k_conv3x3<R, WX, WY, NT, WD>), dim3(8 * per * (2 * NC / NT)),          \
+                           dim3(64 * WX * WY), (16 * WX + 2) * (R * WY + 2) * 2 * Cin, s, p, q);   \
+    }
+    const long t8 = tiles(32, 8);
+    if (Cin == 32 && tiles(32, 16) * NC >= 384)
+        NN_KEEP(8, 2, 2, 1)
+    else if (Cin == 32 && t8 * NC >= 192)
+        NN_KEEP(4, 2, 2, 1)
+    else if (Cin == 32)
+        NN_KEEP(2, 1, 4, 1)
+    else if (Cin == 96 && t8 * NC >= 1024)
+        NN_KEEP(4, 2, 2, 3)
+    else if (Cin >= 128 && Cout % 96 == 0 && t8 * (Cout / 96) >= 192)
+        NN_CONV(4, 2, 2, 6, 9)
+    else if (Cin >= 128 && Cout % 64 == 0 && t8 * (Cout / 64) >= 192)
+        NN_CONV(4, 2, 2, 4, 9)
+    else if (t8 * NC < 256)
+        NN_CONV(2, 1, 2, 2, 9)
+    else if (Cin == 64)
+        NN_CONV(4, 2, 2, 2, 3)
     else
-        hipLaunchKernelGGL(k_conv3x3_t<32>, dim3(nblk(M, 128), Cout / 32), dim3(256), 0, s, in, w,
-                           bias, out, N, H, W, Cin, Cout, relu);
+        NN_CONV(4, 2, 2, 2, 9)
+#undef NN_CONV
+#undef NN_KEEP
 }
 
-// pixel splits of a weight gradient: about 8192 blocks per launch, at most
-// 256 splits and at least 1024 pixels per split
-int nn_dw_splits(long M, int Cin, int Cout)
+// rows of a wave in the weight gradient: tiles of 32 x 16 pixels, or 32 x 4
+// for so few pixels that the larger ones leave most blocks without one.  A
+// training step of 1 / 4 / 16 samples of 256^2 takes 436 / 689 / 1527 us with
+// the line at 16384 pixels, 449 / 703 / 1544 at 65536 and 460 / 710 / 1548 at
+// 131072.
+static int dw_rows(int N, int H, int W)
 {
-    const int bco = (Cout % 64 == 0) ? 64 : 32, bci = (Cin % 64 == 0) ? 64 : 32;
-    const long per_split = 9L * (Cout / bco) * (Cin / bci);
-    const long want = std::max<long>(1, 8192 / per_split);
-    return (int)std::max<long>(1, std::min<long>({256, want, M / 1024}));
+    return (long)N * H * W >= 16384 ? 8 : 2;
 }
 
-void nn_conv3x3_dw(hipStream_t s, const uint16_t *in, const uint16_t *g, float *dw, float *work,
-                   int N, int H, int W, int Cin, int Cout, int accumulate)
+static int dw_tiles(int N, int H, int W)
 {
-    const long M = (long)N * H * W;
-    const int splits = nn_dw_splits(M, Cin, Cout);
-    const int bco = (Cout % 64 == 0) ? 64 : 32, bci = (Cin % 64 == 0) ? 64 : 32;
-    // 64 pixels per stage; a kernel row of three taps per block, but one tap
-    // for the 64 x 64 tile (LDS for four blocks per CU)
-    const long chunk = ((M + splits - 1) / splits + 63) / 64 * 64;
-    const int tg = (bco == 64 && bci == 64) ? 1 : 3;
-    const dim3 grid(9 / tg * (Cout / bco) * (Cin / bci), splits);
-    if (bco == 64 && bci == 64)
-        hipLaunchKernelGGL((k_conv3x3_dw2<64, 64, 64, 1>), grid, dim3(256), 0, s, in, g, work, N, H,
-                           W, Cin, Cout, chunk);
-    else if (bco == 64)
-        hipLaunchKernelGGL((k_conv3x3_dw2<64, 32, 64, 3>), grid, dim3(256), 0, s, in, g, work, N, H,
-                           W, Cin, Cout, chunk);
-    else if (bci == 64)
-        hipLaunchKernelGGL((k_conv3x3_dw2<32, 64, 64, 3>), grid, dim3(256), 0, s, in, g, work, N, H,
-                           W, Cin, Cout, chunk);
-    else
-        hipLaunchKernelGGL((k_conv3x3_dw2<32, 32, 64, 3>), grid, dim3(256), 0, s, in, g, work, N, H,
-                           W, Cin, Cout, chunk);
-    const long n = 9L * Cout * Cin;
-    hipLaunchKernelGGL(k_sum_splits, dim3(nblk(n, 64)), dim3(256), 0, s, work, splits, n, dw,
-                       accumulate);
+    const int th = 2 * dw_rows(N, H, W);
+    return N * ((H + th - 1) / th) * ((W + 31) / 32);
 }
 
-int nn_colsum_splits(long M) { return (int)std::min<long>(1024, std::max<long>(1, M / 1024)); }
-
-void nn_colsum(hipStream_t s, uint16_t *g, long M, int C, float *db, float *work,
-               const uint16_t *relu_y)
+// most pixel splits of a weight gradient: two blocks per CU (in eights: a
+// block for each XCD); a 16-sample training step takes 1.71 ms with 512
+// blocks, 1.80 with 256 and 1.79 with 768
+int nn_dw_max_splits(int Cin, int Cout)
 {
-    const int splits = nn_colsum_splits(M);
-    const long chunk = (M + splits - 1) / splits;
-    if (relu_y)
-        hipLaunchKernelGGL(k_colsum<true>, dim3(splits), dim3(256), 0, s, g, relu_y, M, C, chunk,
-                           work);
+    return 8 * std::max(1, 512 / (8 * (Cin / 32) * (Cout / 32)));
+}
+
+
+void nn_conv3x3_dw(hipStream_t s, const NnConv &p, const uint16_t *g, float *dw_db, float *work,
+                   int N, int H, int W, int Cin, int Cout)
+{
+    const int tiles = dw_tiles(N, H, W);
+    const int splits = std::min(nn_dw_max_splits(Cin, Cout), 8 * ((tiles + 7) / 8));
+    const int P = (Cin / 32) * (Cout / 32), tx = (W + 31) / 32;
+    const long n = Cout * (9L * Cin + 1);
+    if (dw_rows(N, H, W) == 8)
+        hipLaunchKernelGGL((k_conv3x3_dw<8>), dim3(P * splits), dim3(256), 0, s, p, g, work, H, W,
+                           Cin, Cout, tx, (H + 15) / 16, tiles, splits);
     else
-        hipLaunchKernelGGL(k_colsum<false>, dim3(splits), dim3(256), 0, s, g, nullptr, M, C, chunk,
-                           work);
-    hipLaunchKernelGGL(k_sum_cols, dim3(C), dim3(256), 0, s, work, splits, C, db);
+        hipLaunchKernelGGL((k_conv3x3_dw<2>), dim3(P * splits), dim3(256), 0, s, p, g, work, H, W,
+                           Cin, Cout, tx, (H + 3) / 4, tiles, splits);
+    hipLaunchKernelGGL(k_sum_splits, dim3(nblk(n, 32)), dim3(512), 0, s, work, splits, n, dw_db);
 }
 
 void nn_weights_bf16(hipStream_t s, const float *w, int Cin, int Cout, uint16_t *wf, uint16_t *wb)
@@ -850,32 +1010,11 @@ void nn_weights_bf16(hipStream_t s, const float *w, int Cin, int Cout, uint16_t 
     hipLaunchKernelGGL(k_weights_bf16, dim3(nblk(9L * Cin * Cout)), dim3(256), 0, s, w, Cin, Cout, wf, wb);
 }
 
-void nn_avgpool2(hipStream_t s, const uint16_t *in, uint16_t *out, int N, int H, int W, int C)
+void nn_avgpool2_bwd(hipStream_t s, const uint16_t *gout, uint16_t *gin, const uint16_t *mask,
+                     int N, int H, int W, int C, int accumulate)
 {
-    hipLaunchKernelGGL(k_avgpool2, dim3(nblk((long)N * (H / 2) * (W / 2) * C / 8)), dim3(256), 0, s, in,
-                       out, N, H, W, C);
-}
-
-void nn_avgpool2_bwd(hipStream_t s, const uint16_t *gout, uint16_t *gin, int N, int H, int W, int C,
-                     int accumulate)
-{
-    hipLaunchKernelGGL(k_avgpool2_bwd, dim3(nblk((long)N * H * W * C / 8)), dim3(256), 0, s, gout, gin, N,
-                       H, W, C, accumulate);
-}
-
-void nn_up_concat(hipStream_t s, const uint16_t *low, const uint16_t *skip, uint16_t *out, int N,
-                  int H, int W, int C1, int C2)
-{
-    hipLaunchKernelGGL(k_up_concat, dim3(nblk((long)N * 4 * H * W * (C1 + C2) / 8)), dim3(256), 0, s,
-                       low, skip, out, N, H, W, C1, C2);
-}
-
-void nn_up_concat_bwd(hipStream_t s, const uint16_t *gout, uint16_t *glow, uint16_t *gskip, int N,
-                      int H, int W, int C1, int C2, int acc_skip)
-{
-    const long n = std::max((long)N * H * W * C1, (long)N * 4 * H * W * C2) / 8;
-    hipLaunchKernelGGL(k_up_concat_bwd, dim3(nblk(n)), dim3(256), 0, s, gout, glow, gskip, N, H, W,
-                       C1, C2, acc_skip);
+    hipLaunchKernelGGL(k_avgpool2_bwd, dim3(nblk((long)N * H * W * C / 8)), dim3(256), 0, s, gout, gin,
+                       mask, N, H, W, C, accumulate);
 }
 
 void nn_head_fwd(hipStream_t s, const uint16_t *x, const float *wh, const float *bh, float *f,
@@ -893,8 +1032,7 @@ void nn_head_bwd(hipStream_t s, const uint16_t *x, const float *gf, const float 
     const long chunk = (M + splits - 1) / splits;
     constexpr long NP = 2 * NN_HEAD_C + 2;
     hipLaunchKernelGGL(k_head_bwd, dim3(splits), dim3(256), 0, s, x, gf, wh, gx, work, M, chunk);
-    hipLaunchKernelGGL(k_sum_splits, dim3(nblk(NP, 64)), dim3(256), 0, s, work, splits, NP, dwh_db,
-                       0);
+    hipLaunchKernelGGL(k_sum_splits, dim3(nblk(NP, 32)), dim3(512), 0, s, work, splits, NP, dwh_db);
 }
 
 void nn_sample_loss(hipStream_t s, const float *field, int R, const float *uv, const float *target,

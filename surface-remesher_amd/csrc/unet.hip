@@ -58,7 +58,6 @@ struct UNet {
     uint16_t *x0 = nullptr;                 // input (maxb, R, R, IN_C)
     uint16_t *a[14], *ga[14];
     uint16_t *pool[3], *gpool[3];           // p1 (R/2, 32), p2 (R/4, 64), p3 (R/8, 96)
-    uint16_t *up[3], *gup[3];               // u3 (R/4, 224), u2 (R/2, 160), u1 (R, 96)
     float *field = nullptr, *gfield = nullptr;
     float *work = nullptr;
     long work_n = 0;
@@ -88,7 +87,7 @@ UNet::~UNet()
         bufs.push_back(wf[l]); bufs.push_back(wb[l]); bufs.push_back(a[l]); bufs.push_back(ga[l]);
     }
     for (int k = 0; k < 3; ++k) {
-        bufs.push_back(pool[k]); bufs.push_back(gpool[k]); bufs.push_back(up[k]); bufs.push_back(gup[k]);
+        bufs.push_back(pool[k]); bufs.push_back(gpool[k]);
     }
     for (void *b : bufs)
         if (b) (void)hipFree(b);
@@ -101,72 +100,90 @@ void UNet::upload_bf16()
         nn_weights_bf16(stream, p + woff[l], SPEC[l].cin, SPEC[l].cout, wf[l], wb[l]);
 }
 
+// convolution l over `in` or, for a decoder level's first one, over low
+// (upsampled) ++ in
+static NnConv conv_input(int l, const uint16_t *in, const uint16_t *low)
+{
+    NnConv c = {};
+    c.in0 = low ? low : in;
+    c.c0 = low ? SPEC[l].cin - SPEC[l].cout : SPEC[l].cin;
+    c.up = low != nullptr;
+    c.in1 = low ? in : nullptr;
+    return c;
+}
+
 void UNet::forward(int nb)
 {
-    const int R0 = res(0), R1 = res(1), R2 = res(2), R3 = res(3);
-    auto conv = [&](int l, const uint16_t *in) {
+    auto conv = [&](int l, const uint16_t *in, const uint16_t *low, uint16_t *pool) {
         const int r = res(SPEC[l].level);
-        nn_conv3x3(stream, in, wf[l], p + boff[l], a[l], nb, r, r, SPEC[l].cin, SPEC[l].cout, 1);
+        NnConv c = conv_input(l, in, low);
+        c.w = wf[l];
+        c.bias = p + boff[l];
+        c.relu = 1;
+        c.out = a[l];
+        c.pool = pool;
+        nn_conv3x3(stream, c, nb, r, r, SPEC[l].cin, SPEC[l].cout);
     };
-    conv(0, x0);
-    conv(1, a[0]);
-    nn_avgpool2(stream, a[1], pool[0], nb, R0, R0, 32);
-    conv(2, pool[0]);
-    conv(3, a[2]);
-    nn_avgpool2(stream, a[3], pool[1], nb, R1, R1, 64);
-    conv(4, pool[1]);
-    conv(5, a[4]);
-    nn_avgpool2(stream, a[5], pool[2], nb, R2, R2, 96);
-    conv(6, pool[2]);
-    conv(7, a[6]);
-    nn_up_concat(stream, a[7], a[5], up[0], nb, R3, R3, 128, 96);
-    conv(8, up[0]);
-    conv(9, a[8]);
-    nn_up_concat(stream, a[9], a[3], up[1], nb, R2, R2, 96, 64);
-    conv(10, up[1]);
-    conv(11, a[10]);
-    nn_up_concat(stream, a[11], a[1], up[2], nb, R1, R1, 64, 32);
-    conv(12, up[2]);
-    conv(13, a[12]);
+    conv(0, x0, nullptr, nullptr);
+    conv(1, a[0], nullptr, pool[0]);
+    conv(2, pool[0], nullptr, nullptr);
+    conv(3, a[2], nullptr, pool[1]);
+    conv(4, pool[1], nullptr, nullptr);
+    conv(5, a[4], nullptr, pool[2]);
+    conv(6, pool[2], nullptr, nullptr);
+    conv(7, a[6], nullptr, nullptr);
+    conv(8, a[5], a[7], nullptr);
+    conv(9, a[8], nullptr, nullptr);
+    conv(10, a[3], a[9], nullptr);
+    conv(11, a[10], nullptr, nullptr);
+    conv(12, a[1], a[11], nullptr);
+    conv(13, a[12], nullptr, nullptr);
     nn_head_fwd(stream, a[13], p + whoff, p + bhoff, field, npix(0, nb));
 }
 
 void UNet::backward(int nb)
 {
-    const int R0 = res(0), R1 = res(1), R2 = res(2), R3 = res(3);
+    const int R0 = res(0), R1 = res(1), R2 = res(2);
     // head: gfield -> ga[13], dwh, dbh
     nn_head_bwd(stream, a[13], gfield, p + whoff, ga[13], g + whoff, work, npix(0, nb));
-    // one conv layer: mask the output gradient by ReLU' and take the bias
-    // gradient (one pass), the weight gradient, then the input gradient into
-    // gin (if any)
-    auto layer = [&](int l, const uint16_t *in, uint16_t *gin) {
+    // one conv layer: the weight and bias gradients, then the input gradients
+    // into gin and glow (if any).  Gradients are masked by ReLU' where they
+    // are written last: here by mask, the output of the layer that made the
+    // input (the upsampled one of a decoder level).
+    auto layer = [&](int l, const uint16_t *in, const uint16_t *low, const uint16_t *mask,
+                     uint16_t *gin, uint16_t *glow) {
         const ConvSpec &c = SPEC[l];
         const int r = res(c.level);
-        const long m = npix(c.level, nb);
-        nn_colsum(stream, ga[l], m, c.cout, g + boff[l], work, a[l]);
-        nn_conv3x3_dw(stream, in, ga[l], g + woff[l], work, nb, r, r, c.cin, c.cout, 0);
-        if (gin) nn_conv3x3(stream, ga[l], wb[l], nullptr, gin, nb, r, r, c.cout, c.cin, 0);
+        const NnConv f = conv_input(l, in, low);
+        nn_conv3x3_dw(stream, f, ga[l], g + woff[l], work, nb, r, r, c.cin, c.cout);
+        if (!gin) return;
+        NnConv d = {};
+        d.in0 = ga[l];
+        d.c0 = c.cout;
+        d.w = wb[l];
+        d.out = gin;
+        d.low = glow;
+        d.c_low = low ? f.c0 : 0;
+        d.mask = mask;
+        nn_conv3x3(stream, d, nb, r, r, c.cout, c.cin);
     };
-    layer(13, a[12], ga[12]);
-    layer(12, up[2], gup[2]);
-    nn_up_concat_bwd(stream, gup[2], ga[11], ga[1], nb, R1, R1, 64, 32, 0);
-    layer(11, a[10], ga[10]);
-    layer(10, up[1], gup[1]);
-    nn_up_concat_bwd(stream, gup[1], ga[9], ga[3], nb, R2, R2, 96, 64, 0);
-    layer(9, a[8], ga[8]);
-    layer(8, up[0], gup[0]);
-    nn_up_concat_bwd(stream, gup[0], ga[7], ga[5], nb, R3, R3, 128, 96, 0);
-    layer(7, a[6], ga[6]);
-    layer(6, pool[2], gpool[2]);
-    nn_avgpool2_bwd(stream, gpool[2], ga[5], nb, R2, R2, 96, 1);
-    layer(5, a[4], ga[4]);
-    layer(4, pool[1], gpool[1]);
-    nn_avgpool2_bwd(stream, gpool[1], ga[3], nb, R1, R1, 64, 1);
-    layer(3, a[2], ga[2]);
-    layer(2, pool[0], gpool[0]);
-    nn_avgpool2_bwd(stream, gpool[0], ga[1], nb, R0, R0, 32, 1);
-    layer(1, a[0], ga[0]);
-    layer(0, x0, nullptr);
+    layer(13, a[12], nullptr, a[12], ga[12], nullptr);
+    layer(12, a[1], a[11], a[11], ga[1], ga[11]);
+    layer(11, a[10], nullptr, a[10], ga[10], nullptr);
+    layer(10, a[3], a[9], a[9], ga[3], ga[9]);
+    layer(9, a[8], nullptr, a[8], ga[8], nullptr);
+    layer(8, a[5], a[7], a[7], ga[5], ga[7]);
+    layer(7, a[6], nullptr, a[6], ga[6], nullptr);
+    layer(6, pool[2], nullptr, nullptr, gpool[2], nullptr);
+    nn_avgpool2_bwd(stream, gpool[2], ga[5], a[5], nb, R2, R2, 96, 1);
+    layer(5, a[4], nullptr, a[4], ga[4], nullptr);
+    layer(4, pool[1], nullptr, nullptr, gpool[1], nullptr);
+    nn_avgpool2_bwd(stream, gpool[1], ga[3], a[3], nb, R1, R1, 64, 1);
+    layer(3, a[2], nullptr, a[2], ga[2], nullptr);
+    layer(2, pool[0], nullptr, nullptr, gpool[0], nullptr);
+    nn_avgpool2_bwd(stream, gpool[0], ga[1], a[1], nb, R0, R0, 32, 1);
+    layer(1, a[0], nullptr, a[0], ga[0], nullptr);
+    layer(0, x0, nullptr, nullptr, nullptr, nullptr);
 }
 
 }  // namespace cvt
@@ -188,7 +205,7 @@ int cvt_unet_create(cvt_unet **out, int R, int max_batch, unsigned long long see
     memset(u->wf, 0, sizeof u->wf); memset(u->wb, 0, sizeof u->wb);
     memset(u->a, 0, sizeof u->a); memset(u->ga, 0, sizeof u->ga);
     memset(u->pool, 0, sizeof u->pool); memset(u->gpool, 0, sizeof u->gpool);
-    memset(u->up, 0, sizeof u->up); memset(u->gup, 0, sizeof u->gup);
+   
     u->R = R;
     u->maxb = max_batch;
     long off = 0;
@@ -218,22 +235,18 @@ int cvt_unet_create(cvt_unet **out, int R, int max_batch, unsigned long long see
         alloc((void **)&u->ga[l], 2 * an);
     }
     alloc((void **)&u->x0, 2 * u->npix(0, B) * IN_C);
-    const int pc[3] = {32, 64, 96}, uc[3] = {224, 160, 96}, ul[3] = {2, 1, 0};
+    const int pc[3] = {32, 64, 96};
     for (int k = 0; k < 3; ++k) {
         alloc((void **)&u->pool[k], 2 * u->npix(k + 1, B) * pc[k]);
         alloc((void **)&u->gpool[k], 2 * u->npix(k + 1, B) * pc[k]);
-        alloc((void **)&u->up[k], 2 * u->npix(ul[k], B) * uc[k]);
-        alloc((void **)&u->gup[k], 2 * u->npix(ul[k], B) * uc[k]);
     }
     alloc((void **)&u->field, sizeof(float) * 2 * u->npix(0, B));
     alloc((void **)&u->gfield, sizeof(float) * 2 * u->npix(0, B));
     // split-K workspace: the largest conv weight gradient and the head partials
     long wn = (long)nn_head_splits(u->npix(0, B)) * (2 * HEAD_C + 2);
     for (int l = 0; l < 14; ++l)
-        wn = std::max({wn,
-                       (long)nn_dw_splits(u->npix(SPEC[l].level, B), SPEC[l].cin, SPEC[l].cout) * 9L *
-                           SPEC[l].cin * SPEC[l].cout,
-                       (long)nn_colsum_splits(u->npix(SPEC[l].level, B)) * SPEC[l].cout});
+        wn = std::max(wn, (long)nn_dw_max_splits(SPEC[l].cin, SPEC[l].cout) * SPEC[l].cout *
+                              (9L * SPEC[l].cin + 1));
     u->work_n = wn;
     alloc((void **)&u->work, sizeof(float) * wn);
     alloc((void **)&u->count, sizeof(float) * R * R);
