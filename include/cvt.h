@@ -212,6 +212,12 @@ int cvt_rasterize(const double *points, const double *weight, int num_point, con
 int cvt_rasterize_noalloc(const double *points, const double *weight, int num_point,
                           const int *triangle, int num_tri, float *density, double scale, int n);
 
+/* Gives back the device memory that cvt_rasterize, cvt_locate_points and
+ * cvt_vertex_weights keep from call to call: at most four blocks and 64 MB
+ * per device (larger ones are freed by the call that needed them).  Blocks in
+ * use by a call of another thread stay with it. */
+int cvt_release_scratch(void);
+
 /* CDT input points (the site scan of delaunayInput, source/delaunay.h:48-58):
  * pixels (x, y) whose label is their own coordinates and whose mask byte is
  * 0 (mask may be null), in the reference's order (x outer, y inner), as

@@ -28,11 +28,10 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <type_traits>
-#include <vector>
 
 #include "../../include/cvt.h"
 #include "cvt_engine.h"
+#include "mesh_scratch.h"
 
 namespace cvt {
 
@@ -46,6 +45,33 @@ struct BinGrid {
     int G;
 };
 
+// a double as an unsigned key in the same order (NaN excluded), never 0
+__device__ __forceinline__ unsigned long long order_key(double v)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    return (b >> 63) ? ~b : b | (1ull << 63);
+}
+__device__ __forceinline__ double from_key(unsigned long long k)
+{
+    return __longlong_as_double((long long)((k >> 63) ? k & ~(1ull << 63) : ~k));
+}
+
+// square bins over the vertex box (no vertex, a zero-size or a non-finite
+// box: one bin).  bb: the largest keys of -x, -y (as complements), x and y,
+// 0 where no vertex had one.
+__device__ __forceinline__ BinGrid bin_grid(const unsigned long long *__restrict__ bb, int G)
+{
+    BinGrid g;
+    const double x0 = bb[0] ? from_key(~bb[0]) : INFINITY, y0 = bb[1] ? from_key(~bb[1]) : INFINITY;
+    const double x1 = bb[2] ? from_key(bb[2]) : -INFINITY, y1 = bb[3] ? from_key(bb[3]) : -INFINITY;
+    const double ex = x1 - x0, ey = y1 - y0, ext = ex < ey ? ey : ex;
+    g.ox = isfinite(x0) ? x0 : 0.0;
+    g.oy = isfinite(y0) ? y0 : 0.0;
+    g.inv = (ext > 0.0 && isfinite(ext)) ? (double)G / ext : 0.0;
+    g.G = g.inv == 0.0 ? 1 : G;
+    return g;
+}
+
 // bin of a coordinate: monotone in v (so a point inside a box maps inside the
 // box's bin range) and clamped to the grid, NaN to bin 0
 __device__ __forceinline__ int bin_of(double v, double o, double inv, int G)
@@ -55,80 +81,72 @@ __device__ __forceinline__ int bin_of(double v, double o, double inv, int G)
     return (int)floor(t);
 }
 
-// source/recover.h:30-53: w1, w2 from the dot products of v0 = p2 - p1,
-// v1 = p3 - p1, v2 = q - p1; a zero denominator gives -1 weights
-__device__ __forceinline__ void rec_bary(double x1, double y1, double x2, double y2, double x3,
-                                         double y3, double x0, double y0, double &w0,
-                                         double &w1, double &w2)
-{
-    const double v0x = x2 - x1, v0y = y2 - y1;
-    const double v1x = x3 - x1, v1y = y3 - y1;
-    const double v2x = x0 - x1, v2y = y0 - y1;
-    const double d00 = v0x * v0x + v0y * v0y;
-    const double d01 = v0x * v1x + v0y * v1y;
-    const double d11 = v1x * v1x + v1y * v1y;
-    const double d20 = v2x * v0x + v2y * v0y;
-    const double d21 = v2x * v1x + v2y * v1y;
-    const double den = d00 * d11 - d01 * d01;
-    if (den == 0) { w0 = w1 = w2 = -1; return; }
-    w1 = (d11 * d20 - d01 * d21) / den;
-    w2 = (d00 * d21 - d01 * d20) / den;
-    w0 = 1.0 - w1 - w2;
-}
-
-// bounding box of the vertices (one workgroup): bb = {xmin, ymin, xmax, ymax}
+// bounding box of the vertices as order keys (bb zeroed by the caller)
 __global__ __launch_bounds__(256) void k_vertex_bounds(const double *__restrict__ uv, int nv,
-                                                       double *__restrict__ bb)
+                                                       unsigned long long *__restrict__ bb)
 {
-    __shared__ double r[4][256];
-    double a = INFINITY, b = INFINITY, c = -INFINITY, d = -INFINITY;
-    for (int i = threadIdx.x; i < nv; i += 256) {
+    __shared__ double r[4][4];
+    double m[4] = {INFINITY, INFINITY, -INFINITY, -INFINITY};
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < nv; i += gridDim.x * 256) {
         const double x = uv[2 * i], y = uv[2 * i + 1];
-        a = fmin(a, x); b = fmin(b, y); c = fmax(c, x); d = fmax(d, y);
+        m[0] = fmin(m[0], x); m[1] = fmin(m[1], y); m[2] = fmax(m[2], x); m[3] = fmax(m[3], y);
     }
-    r[0][threadIdx.x] = a; r[1][threadIdx.x] = b; r[2][threadIdx.x] = c; r[3][threadIdx.x] = d;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            r[0][threadIdx.x] = fmin(r[0][threadIdx.x], r[0][threadIdx.x + o]);
-            r[1][threadIdx.x] = fmin(r[1][threadIdx.x], r[1][threadIdx.x + o]);
-            r[2][threadIdx.x] = fmax(r[2][threadIdx.x], r[2][threadIdx.x + o]);
-            r[3][threadIdx.x] = fmax(r[3][threadIdx.x], r[3][threadIdx.x + o]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        for (int o = 32; o > 0; o >>= 1) {
+            const double v = __shfl_xor(m[c], o, 64);
+            m[c] = c < 2 ? fmin(m[c], v) : fmax(m[c], v);
         }
-        __syncthreads();
+        if ((threadIdx.x & 63) == 0) r[c][threadIdx.x >> 6] = m[c];
     }
-    if (threadIdx.x < 4) bb[threadIdx.x] = r[threadIdx.x][0];
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c >= 4) return;
+    const double lo = fmin(fmin(r[c][0], r[c][1]), fmin(r[c][2], r[c][3]));
+    const double hi = fmax(fmax(r[c][0], r[c][1]), fmax(r[c][2], r[c][3]));
+    atomicMax(&bb[c], c < 2 ? ~order_key(lo) : order_key(hi));
 }
 
-// per face: index validation, the conservative bin box and the
-// ill-conditioned flag
+// the corners of a face, in one 48-byte record: a query reads a candidate
+// face with one gather behind its list entry
+struct FaceXY {
+    double x1, y1, x2, y2, x3, y3;
+};
+
+// per face: index validation, the corner record, the conservative bin box
+// and its (face, bin) pairs counted per bin.  Faces to test everywhere are
+// appended to alw in any order (a query keeps the lowest-index hit).
+// status: {a face indexes outside, pairs beyond the list, faces in alw}
 __global__ void k_face_boxes(const double *__restrict__ uv, int nv, const int *__restrict__ tri,
-                             int nf, BinGrid g, FaceBox *__restrict__ box,
-                             uint8_t *__restrict__ always, int *__restrict__ bad)
+                             int nf, const unsigned long long *__restrict__ bb, int G,
+                             FaceXY *__restrict__ xy, FaceBox *__restrict__ box,
+                             int *__restrict__ alw, int *__restrict__ count,
+                             int *__restrict__ status)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nf) return;
     const int a = tri[3 * i], b = tri[3 * i + 1], c = tri[3 * i + 2];
     FaceBox bx = {1, 0, 1, 0};
-    always[i] = 0;
     if ((unsigned)a >= (unsigned)nv || (unsigned)b >= (unsigned)nv || (unsigned)c >= (unsigned)nv) {
-        *bad = 1;
+        status[0] = 1;
         box[i] = bx;
         return;
     }
     const double x1 = uv[2 * a], y1 = uv[2 * a + 1];
     const double x2 = uv[2 * b], y2 = uv[2 * b + 1];
     const double x3 = uv[2 * c], y3 = uv[2 * c + 1];
+    xy[i] = FaceXY{x1, y1, x2, y2, x3, y3};
     const double v0x = x2 - x1, v0y = y2 - y1, v1x = x3 - x1, v1y = y3 - y1;
     const double d00 = v0x * v0x + v0y * v0y, d11 = v1x * v1x + v1y * v1y;
     const double d01 = v0x * v1x + v0y * v1y;
     const double den = d00 * d11 - d01 * d01;
     if (den == 0) { box[i] = bx; return; }          // holds no point
     if (!(den > 1e-12 * d00 * d11)) {                // thin or non-finite: test everywhere
-        always[i] = 1;
+        alw[atomicAdd(&status[2], 1)] = i;
         box[i] = bx;
         return;
     }
+    const BinGrid g = bin_grid(bb, G);
     const double xmin = fmin(x1, fmin(x2, x3)), xmax = fmax(x1, fmax(x2, x3));
     const double ymin = fmin(y1, fmin(y2, y3)), ymax = fmax(y1, fmax(y2, y3));
     const double eps = 1e-9 * fmax(xmax - xmin, ymax - ymin) + 1e-300;
@@ -137,27 +155,21 @@ __global__ void k_face_boxes(const double *__restrict__ uv, int nv, const int *_
     bx.y0 = bin_of(ymin - eps, g.oy, g.inv, g.G);
     bx.y1 = bin_of(ymax + eps, g.oy, g.inv, g.G);
     box[i] = bx;
+    for (int y = bx.y0; y <= bx.y1; ++y)
+        for (int x = bx.x0; x <= bx.x1; ++x) atomicAdd(&count[y * g.G + x], 1);
 }
 
-// (face, bin) pairs: count per bin
-__global__ void k_bin_count(const FaceBox *__restrict__ box, int nf, int G,
-                            int *__restrict__ count)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nf) return;
-    const FaceBox b = box[i];
-    for (int y = b.y0; y <= b.y1; ++y)
-        for (int x = b.x0; x <= b.x1; ++x) atomicAdd(&count[y * G + x], 1);
-}
-
-// Exclusive prefix sum of n counts into start[0 .. n], in three launches
-// over tiles of 4096 counts (1024 threads x 4 consecutive counts):
+// Exclusive prefix sum of n counts into start[0 .. n] over tiles of 4096
+// counts (1024 threads x 4 consecutive counts).  Up to kScanOne counts one
+// workgroup walks over the tiles (k_scan_one: 4.5 us for 6 000 counts, where
+// three launches take 7.4 us and their gaps; 11 us for 16 384, where they take
+// 8.2); beyond that in three launches:
 //   k_scan_tiles        each tile's total, parked in start[tile * 4096];
 //   k_scan_tile_totals  one workgroup turns the parked totals into the tiles'
 //                       offsets in place and writes start[n];
 //   k_scan_apply        each tile reads its offset, then writes its starts
 //                       (its first entry, the parked offset, last).
-constexpr int kScanTile = 4096;
+constexpr int kScanTile = 4096, kScanOne = 8192;
 
 // exclusive prefix sum over a 1024-thread workgroup of one value per thread;
 // total receives the workgroup's sum (lds: 32 ints)
@@ -244,14 +256,43 @@ __global__ __launch_bounds__(1024) void k_scan_apply(const int *__restrict__ cou
         }
 }
 
-// (face, bin) pairs: each face writes its index into the lists of its bins
-__global__ void k_bin_fill(const FaceBox *__restrict__ box, int nf, int G,
+__global__ __launch_bounds__(1024) void k_scan_one(const int *__restrict__ count, int n,
+                                                   int *__restrict__ start)
+{
+    __shared__ int lds[32];
+    int carry = 0;
+    for (int tile0 = 0; tile0 < n; tile0 += kScanTile) {
+        const long base = tile0 + 4 * (long)threadIdx.x;
+        const int4 c = tile_counts(count, base, n);
+        int total;
+        int run = carry + wg_exclusive_scan(c.x + c.y + c.z + c.w, lds, total);
+        const int v[4] = {c.x, c.y, c.z, c.w};
+        for (int k = 0; k < 4; ++k)
+            if (base + k < n) {
+                start[base + k] = run;
+                run += v[k];
+            }
+        carry += total;
+    }
+    if (threadIdx.x == 0) start[n] = carry;
+}
+
+// (face, bin) pairs: each face writes its index into the lists of its bins;
+// with more pairs than the list holds, nothing but the flag
+__global__ void k_bin_fill(const FaceBox *__restrict__ box, int nf,
+                           const unsigned long long *__restrict__ bb, int grid,
                            const int *__restrict__ start, int *__restrict__ cursor,
-                           int *__restrict__ list)
+                           int *__restrict__ list, int cap, int *__restrict__ status)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nf) return;
+    if (start[grid * grid] > cap) {
+        if (i == 0) status[1] = 1;
+        return;
+    }
     const FaceBox b = box[i];
+    if (b.x0 > b.x1) return;
+    const int G = bin_grid(bb, grid).G;
     for (int y = b.y0; y <= b.y1; ++y)
         for (int x = b.x0; x <= b.x1; ++x) {
             const int bin = y * G + x;
@@ -260,37 +301,80 @@ __global__ void k_bin_fill(const FaceBox *__restrict__ box, int nf, int G,
 }
 
 // one thread per query point: the lowest-index face of its bin list and of
-// the "always" list that holds it; face -1 when none does
-__global__ __launch_bounds__(256) void k_locate(const double *__restrict__ uv,
+// the "always" list that holds it; face -1 when none does.  Candidates are
+// decided by the signs of the weights' numerators, and the weights divided
+// out once, for the hit.  kAtOnce candidates are read together.  host, pinned,
+// receives the status and the number of pairs.
+// Bound by the latency of list entry -> face record: 49152 points in an
+// 11858-face mesh 13 us (17 us with indices and corners as separate gathers
+// and two divisions per candidate; 15 us with eight at a time).
+constexpr int kAtOnce = 4;
+__global__ __launch_bounds__(256) void k_locate(const FaceXY *__restrict__ xy,
                                                 const double *__restrict__ p3,
                                                 const int *__restrict__ tri,
                                                 const int *__restrict__ list,
                                                 const int *__restrict__ start,
-                                                const int *__restrict__ alw, int nalw, BinGrid g,
+                                                const int *__restrict__ alw,
+                                                const unsigned long long *__restrict__ bb, int G,
                                                 const double *__restrict__ q, int nq,
                                                 int *__restrict__ face, double *__restrict__ w,
-                                                double *__restrict__ out3)
+                                                double *__restrict__ out3,
+                                                const int *__restrict__ status,
+                                                int *__restrict__ host)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nq) return;
+    if (k == 0) {
+        host[0] = status[0];
+        host[1] = status[1];
+        host[2] = start[G * G];
+    }
+    if (k >= nq || status[0] || status[1]) return;
+    const int nalw = status[2];
     const double x = q[2 * k], y = q[2 * k + 1];
     int hit = -1;
-    double w0 = -1, w1 = -1, w2 = -1;
+    double h1 = 0.0, h2 = 0.0, hd = 1.0;
     // a non-finite point is in no face
     if (isfinite(x) && isfinite(y)) {
+        const BinGrid g = bin_grid(bb, G);
         const int bin = bin_of(y, g.oy, g.inv, g.G) * g.G + bin_of(x, g.ox, g.inv, g.G);
         const int a = start[bin], n = start[bin + 1] - a;
-        for (int j = 0; j < n + nalw; ++j) {
-            const int i = (j < n) ? list[a + j] : alw[j - n];
-            if (hit >= 0 && i > hit) continue;      // a lower-index hit is known
-            const int p0 = tri[3 * i], p1 = tri[3 * i + 1], p2 = tri[3 * i + 2];
-            double b0, b1, b2;
-            rec_bary(uv[2 * p0], uv[2 * p0 + 1], uv[2 * p1], uv[2 * p1 + 1], uv[2 * p2],
-                     uv[2 * p2 + 1], x, y, b0, b1, b2);
-            if (b0 < 0 || b1 < 0 || b2 < 0) continue;
-            hit = i;
-            w0 = b0; w1 = b1; w2 = b2;
+        for (int j0 = 0; j0 < n + nalw; j0 += kAtOnce) {
+            int id[kAtOnce];
+            FaceXY f[kAtOnce];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                const int j = min(j0 + u, n + nalw - 1);
+                id[u] = (j < n) ? list[a + j] : alw[j - n];
+            }
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) f[u] = xy[id[u]];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                // a lower-index hit is known (or the list ended: its last again)
+                if (hit >= 0 && id[u] >= hit) continue;
+                const double v0x = f[u].x2 - f[u].x1, v0y = f[u].y2 - f[u].y1;
+                const double v1x = f[u].x3 - f[u].x1, v1y = f[u].y3 - f[u].y1;
+                const double v2x = x - f[u].x1, v2y = y - f[u].y1;
+                const double d00 = v0x * v0x + v0y * v0y;
+                const double d01 = v0x * v1x + v0y * v1y;
+                const double d11 = v1x * v1x + v1y * v1y;
+                const double d20 = v2x * v0x + v2y * v0y;
+                const double d21 = v2x * v1x + v2y * v1y;
+                const double den = d00 * d11 - d01 * d01;
+                const double n1 = d11 * d20 - d01 * d21, n2 = d00 * d21 - d01 * d20;
+                if (den == 0) continue;
+                const int in = inside_sign(n1, n2, den);
+                if (in == 0 || (in < 0 && !inside_exact(n1, n2, den))) continue;
+                hit = id[u];
+                h1 = n1; h2 = n2; hd = den;
+            }
         }
+    }
+    double w0 = -1, w1 = -1, w2 = -1;
+    if (hit >= 0) {
+        w1 = h1 / hd;
+        w2 = h2 / hd;
+        w0 = 1.0 - w1 - w2;
     }
     face[k] = hit;
     if (w) {
@@ -312,26 +396,47 @@ __global__ __launch_bounds__(256) void k_locate(const double *__restrict__ uv,
     }
 }
 
+__global__ __launch_bounds__(256) void k_zero(uint4 *__restrict__ p, long n)
+{
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = make_uint4(0, 0, 0, 0);
+}
+
+void launch_zero(hipStream_t st, void *p, size_t bytes)
+{
+    const long n = (long)(bytes / 16);
+    if (n > 0)
+        hipLaunchKernelGGL(k_zero, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+                           static_cast<uint4 *>(p), n);
+}
+
 void launch_exclusive_scan(hipStream_t st, const int *count, int n, int *start)
 {
+    if (n <= kScanOne) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, st, count, n, start);
+        return;
+    }
     const int ntiles = (int)(((long)n + kScanTile - 1) / kScanTile);
-    if (ntiles > 0)
-        hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(1024), 0, st, count, n, start);
+    hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(1024), 0, st, count, n, start);
     hipLaunchKernelGGL(k_scan_tile_totals, dim3(1), dim3(1024), 0, st, start, n, ntiles);
-    if (ntiles > 0)
-        hipLaunchKernelGGL(k_scan_apply, dim3(ntiles), dim3(1024), 0, st, count, n, start);
+    hipLaunchKernelGGL(k_scan_apply, dim3(ntiles), dim3(1024), 0, st, count, n, start);
 }
 
 }  // namespace cvt
 
 using namespace cvt;
 
-#define LCHK(call, what)                                                               \
-    do {                                                                               \
-        hipError_t e_ = (call);                                                        \
-        if (e_ != hipSuccess) { rc = fail(CVT_ERR_HIP, "%s: %s", what, hipGetErrorString(e_)); goto done; } \
+#define LCHK(call, what)                                                                  \
+    do {                                                                                  \
+        hipError_t e_ = (call);                                                           \
+        if (e_ != hipSuccess) return fail(CVT_ERR_HIP, "%s: %s", what, hipGetErrorString(e_)); \
     } while (0)
 
+// One pass over the mesh and one over the queries, with one wait at the end:
+// the bin grid stays on the device, and the lists get room for the pairs of
+// an ordinary mesh (four to six per face); a mesh with more (long, slanted
+// faces) is seen at the wait, and its lists are filled again with room for
+// all.  Arguments in memory of the device are used where they are.
 extern "C" int cvt_locate_points(const double *uv, const double *p3, int nv, const int *tri,
                                  int nf, const double *q, int nq, int *face, double *w,
                                  double *out3)
@@ -344,96 +449,96 @@ extern "C" int cvt_locate_points(const double *uv, const double *p3, int nv, con
     if (nq == 0) return CVT_OK;
     // about two faces per bin, at most 1024 x 1024 bins
     const int G = std::max(1, std::min(1024, (int)ceil(sqrt((double)std::max(nf, 1) / 2.0))));
-    int rc = CVT_OK;
     hipStream_t st = nullptr;   // the legacy default stream, as the reference's calls use
-    double *d_uv = nullptr, *d_p3 = nullptr, *d_q = nullptr, *d_w = nullptr, *d_out3 = nullptr,
-           *d_bb = nullptr;
-    int *d_tri = nullptr, *d_list = nullptr, *d_count = nullptr, *d_start = nullptr,
-        *d_cursor = nullptr, *d_alw = nullptr, *d_bad = nullptr, *d_face = nullptr;
+    const size_t nva = (size_t)std::max(nv, 1), nfa = (size_t)std::max(nf, 1), nb = (size_t)G * G;
+    const size_t n1 = (size_t)nq, b_uv = 16 * nva, b_tri = 12 * nfa, b_q = 16 * n1, b_p3 = 24 * nva;
+    // outputs written in place must not meet an input, or one copied before
+    auto clear_of = [&](const void *o, size_t bytes) {
+        return !overlap(o, bytes, uv, b_uv) && !overlap(o, bytes, tri, b_tri) &&
+               !overlap(o, bytes, q, b_q) && !(out3 && overlap(o, bytes, p3, b_p3));
+    };
+    const bool own_uv = nv > 0 && in_place(uv, 8), own_tri = nf > 0 && in_place(tri, 4);
+    const bool own_q = in_place(q, 8), own_p3 = out3 && nv > 0 && in_place(p3, 8);
+    const bool own_face = in_place(face, 4) && clear_of(face, 4 * n1);
+    const bool own_w = w && in_place(w, 8) && clear_of(w, 24 * n1) && !overlap(w, 24 * n1, face, 4 * n1);
+    const bool own_out3 = out3 && in_place(out3, 8) && clear_of(out3, 24 * n1) &&
+                          !overlap(out3, 24 * n1, face, 4 * n1) && !overlap(out3, 24 * n1, w, 24 * n1);
+    double *d_uv = nullptr, *d_p3 = nullptr, *d_q = nullptr, *d_w = nullptr, *d_out3 = nullptr;
+    int *d_tri = nullptr, *d_list = nullptr, *d_count = nullptr, *d_cursor = nullptr,
+        *d_start = nullptr, *d_alw = nullptr, *d_status = nullptr, *d_face = nullptr;
+    unsigned long long *d_bb = nullptr;
     FaceBox *d_box = nullptr;
-    uint8_t *d_always = nullptr;
-    char *arena = nullptr;
-    int bad = 0, nalw = 0, total = 0, nbins = 0;
-    double bb[4] = {0, 0, 0, 0};
-    BinGrid g;
-    std::vector<uint8_t> always;
-    std::vector<int> alw;
-    const size_t nva = (size_t)std::max(nv, 1), nfa = (size_t)std::max(nf, 1);
-    const size_t nb = (size_t)G * G;
-    // the call's fixed-size buffers in one allocation, each at a 256-byte
-    // boundary (the bin lists, sized by the count, get their own)
-    size_t at = 0;
-    auto carve = [&](auto *&p, size_t n) {
-        at = (at + 255) & ~(size_t)255;
-        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(arena + at);
-        at += n * sizeof(*p);
-    };
+    FaceXY *d_xy = nullptr;
+    size_t cap = std::min<size_t>(8 * nfa + 1024, INT32_MAX);
+    MeshScratch mem;
+    Carver carve;
+    size_t zeroed = 0;
     auto layout = [&]() {
-        at = 0;
-        carve(d_uv, 2 * nva); carve(d_tri, 3 * nfa); carve(d_q, 2 * (size_t)nq);
-        carve(d_face, (size_t)nq); carve(d_box, nfa); carve(d_always, nfa); carve(d_alw, nfa);
-        carve(d_count, nb); carve(d_cursor, nb); carve(d_start, nb + 1); carve(d_bad, 1);
-        carve(d_bb, 4);
-        if (w) carve(d_w, 3 * (size_t)nq);
-        if (out3) { carve(d_out3, 3 * (size_t)nq); carve(d_p3, 3 * nva); }
+        carve.base = mem.base();
+        carve.at = 0;
+        carve(d_bb, 4);                          // zeroed from here
+        carve(d_status, 4); carve(d_count, nb); carve(d_cursor, nb);
+        zeroed = (carve.at + 255) & ~(size_t)255;
+        carve(d_start, nb + 1); carve(d_box, nfa); carve(d_xy, nfa); carve(d_alw, nfa);
+        if (!own_uv) carve(d_uv, 2 * nva);
+        if (!own_tri) carve(d_tri, 3 * nfa);
+        if (!own_q) carve(d_q, 2 * n1);
+        if (!own_face) carve(d_face, n1);
+        if (w && !own_w) carve(d_w, 3 * n1);
+        if (out3 && !own_out3) carve(d_out3, 3 * n1);
+        if (out3 && !own_p3) carve(d_p3, 3 * nva);
+        carve(d_list, cap);
     };
     layout();
-    LCHK(hipMalloc(&arena, at), "alloc");
+    LCHK(mem.take(carve.at), "alloc");
     layout();
-    if (out3 && nv > 0)
-        LCHK(hipMemcpyAsync(d_p3, p3, sizeof(double) * 3 * nv, hipMemcpyDefault, st), "upload");
-    if (nv > 0) LCHK(hipMemcpyAsync(d_uv, uv, sizeof(double) * 2 * nv, hipMemcpyDefault, st), "upload");
-    if (nf > 0) LCHK(hipMemcpyAsync(d_tri, tri, sizeof(int) * 3 * nf, hipMemcpyDefault, st), "upload");
-    LCHK(hipMemcpyAsync(d_q, q, sizeof(double) * 2 * nq, hipMemcpyDefault, st), "upload");
-    LCHK(hipMemsetAsync(d_bad, 0, sizeof(int), st), "memset");
-    if (nv > 0) {
-        hipLaunchKernelGGL(k_vertex_bounds, dim3(1), dim3(256), 0, st, d_uv, nv, d_bb);
-        LCHK(hipMemcpyAsync(bb, d_bb, sizeof(bb), hipMemcpyDeviceToHost, st), "bounds");
-    }
-    LCHK(hipStreamSynchronize(st), "bounds");
-    {
-        // square bins over the vertex box (a zero-size or non-finite box: one bin)
-        const double ext = std::max(bb[2] - bb[0], bb[3] - bb[1]);
-        g.G = G;
-        g.ox = std::isfinite(bb[0]) ? bb[0] : 0.0;
-        g.oy = std::isfinite(bb[1]) ? bb[1] : 0.0;
-        g.inv = (ext > 0.0 && std::isfinite(ext)) ? (double)G / ext : 0.0;
-        if (g.inv == 0.0) g.G = 1;
-    }
-    nbins = g.G * g.G;
-    LCHK(hipMemsetAsync(d_count, 0, sizeof(int) * nbins, st), "memset");
-    LCHK(hipMemsetAsync(d_cursor, 0, sizeof(int) * nbins, st), "memset");
-    if (nf > 0) {
-        hipLaunchKernelGGL(k_face_boxes, dim3((nf + 255) / 256), dim3(256), 0, st, d_uv, nv, d_tri,
-                           nf, g, d_box, d_always, d_bad);
-        hipLaunchKernelGGL(k_bin_count, dim3((nf + 255) / 256), dim3(256), 0, st, d_box, nf, g.G,
-                           d_count);
-    }
-    launch_exclusive_scan(st, d_count, nbins, d_start);
-    LCHK(hipMemcpyAsync(&total, d_start + nbins, sizeof(int), hipMemcpyDeviceToHost, st), "total");
-    LCHK(hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, st), "flag");
-    always.resize(std::max(nf, 1));
-    if (nf > 0) LCHK(hipMemcpyAsync(always.data(), d_always, nf, hipMemcpyDeviceToHost, st), "flags");
-    LCHK(hipStreamSynchronize(st), "boxes");
-    if (bad) { rc = fail(CVT_ERR_ARG, "a face indexes a vertex outside [0, %d)", nv); goto done; }
-    for (int i = 0; i < nf; ++i)
-        if (always[i]) alw.push_back(i);
-    nalw = (int)alw.size();
-    if (nalw) LCHK(hipMemcpyAsync(d_alw, alw.data(), sizeof(int) * nalw, hipMemcpyHostToDevice, st), "upload");
-    LCHK(hipMalloc(&d_list, sizeof(int) * (size_t)std::max(total, 1)), "alloc");
+    if (own_uv) d_uv = const_cast<double *>(uv);
+    else if (nv > 0) LCHK(hipMemcpyAsync(d_uv, uv, 16 * (size_t)nv, hipMemcpyDefault, st), "upload");
+    if (own_tri) d_tri = const_cast<int *>(tri);
+    else if (nf > 0) LCHK(hipMemcpyAsync(d_tri, tri, 12 * (size_t)nf, hipMemcpyDefault, st), "upload");
+    if (own_q) d_q = const_cast<double *>(q);
+    else LCHK(hipMemcpyAsync(d_q, q, b_q, hipMemcpyDefault, st), "upload");
+    if (own_p3) d_p3 = const_cast<double *>(p3);
+    else if (out3 && nv > 0)
+        LCHK(hipMemcpyAsync(d_p3, p3, 24 * (size_t)nv, hipMemcpyDefault, st), "upload");
+    if (own_face) d_face = face;
+    if (own_w) d_w = w;
+    if (own_out3) d_out3 = out3;
+    const dim3 gf((nf + 255) / 256), blk(256);
+    launch_zero(st, d_bb, zeroed);
+    if (nv > 0)
+        hipLaunchKernelGGL(k_vertex_bounds, dim3(std::min(64, (nv + 255) / 256)), blk, 0, st, d_uv,
+                           nv, d_bb);
     if (nf > 0)
-        hipLaunchKernelGGL(k_bin_fill, dim3((nf + 255) / 256), dim3(256), 0, st, d_box, nf, g.G,
-                           d_start, d_cursor, d_list);
-    hipLaunchKernelGGL(k_locate, dim3((nq + 255) / 256), dim3(256), 0, st, d_uv, d_p3, d_tri,
-                       d_list, d_start, d_alw, nalw, g, d_q, nq, d_face, d_w, d_out3);
-    LCHK(hipGetLastError(), "locate launch");
-    LCHK(hipMemcpyAsync(face, d_face, sizeof(int) * nq, hipMemcpyDefault, st), "download");
-    if (w) LCHK(hipMemcpyAsync(w, d_w, sizeof(double) * 3 * nq, hipMemcpyDefault, st), "download");
-    if (out3)
-        LCHK(hipMemcpyAsync(out3, d_out3, sizeof(double) * 3 * nq, hipMemcpyDefault, st), "download");
-    LCHK(hipStreamSynchronize(st), "locate");
-done:
-    if (d_list) (void)hipFree(d_list);
-    if (arena) (void)hipFree(arena);
-    return rc;
+        hipLaunchKernelGGL(k_face_boxes, gf, blk, 0, st, d_uv, nv, d_tri, nf, d_bb, G, d_xy, d_box,
+                           d_alw, d_count, d_status);
+    launch_exclusive_scan(st, d_count, (int)nb, d_start);
+    MeshScratch more;
+    int *host = mem.status();
+    for (int round = 0; round < 2; ++round) {
+        if (nf > 0)
+            hipLaunchKernelGGL(k_bin_fill, gf, blk, 0, st, d_box, nf, d_bb, G, d_start, d_cursor,
+                               d_list, (int)cap, d_status);
+        hipLaunchKernelGGL(k_locate, dim3((nq + 255) / 256), blk, 0, st, d_xy, d_p3, d_tri, d_list,
+                           d_start, d_alw, d_bb, G, d_q, nq, d_face, d_w, d_out3, d_status, host);
+        LCHK(hipGetLastError(), "locate launch");
+        LCHK(hipStreamSynchronize(st), "locate");
+        if (host[0]) {
+            mem.idle();
+            return fail(CVT_ERR_ARG, "a face indexes a vertex outside [0, %d)", nv);
+        }
+        if (!host[1]) break;
+        cap = (size_t)host[2];
+        LCHK(more.take(sizeof(int) * cap), "alloc");
+        d_list = reinterpret_cast<int *>(more.base());
+        LCHK(hipMemsetAsync(d_status + 1, 0, sizeof(int), st), "reset");
+    }
+    if (!own_face) LCHK(hipMemcpyAsync(face, d_face, 4 * n1, hipMemcpyDefault, st), "download");
+    if (w && !own_w) LCHK(hipMemcpyAsync(w, d_w, 24 * n1, hipMemcpyDefault, st), "download");
+    if (out3 && !own_out3)
+        LCHK(hipMemcpyAsync(out3, d_out3, 24 * n1, hipMemcpyDefault, st), "download");
+    if (!own_face || (w && !own_w) || (out3 && !own_out3)) LCHK(hipStreamSynchronize(st), "locate");
+    mem.idle();
+    more.idle();
+    return CVT_OK;
 }

@@ -1,0 +1,144 @@
+// mesh_scratch.cpp -- the store of mesh_scratch.h.
+#include "mesh_scratch.h"
+
+#include <stdint.h>
+
+#include <algorithm>
+#include <mutex>
+#include <vector>
+
+#include "../../include/cvt.h"
+#include "cvt_engine.h"
+
+namespace cvt {
+
+namespace {
+
+struct Block {
+    int device;
+    char *dev;
+    size_t bytes;
+    int *pinned;
+};
+
+std::mutex g_mutex;
+std::vector<Block> &store()
+{
+    // never destroyed: the runtime may be gone before a static's destructor
+    static std::vector<Block> *s = new std::vector<Block>();
+    return *s;
+}
+
+void drop(const Block &b)
+{
+    (void)hipFree(b.dev);
+    (void)hipHostFree(b.pinned);
+}
+
+}  // namespace
+
+void release_scratch()
+{
+    std::vector<Block> all;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        all.swap(store());
+    }
+    for (const Block &b : all) drop(b);
+}
+
+hipError_t MeshScratch::take(size_t bytes)
+{
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        std::vector<Block> &s = store();
+        auto best = s.end();
+        for (auto i = s.begin(); i != s.end(); ++i)
+            if (i->device == device && i->bytes >= bytes && (best == s.end() || i->bytes < best->bytes))
+                best = i;
+        if (best != s.end()) {
+            device_ = device;
+            dev_ = best->dev;
+            bytes_ = best->bytes;
+            pinned_ = best->pinned;
+            s.erase(best);
+            return hipSuccess;
+        }
+    }
+    // whole megabytes, so that a slightly larger mesh fits the same block
+    const size_t mb = (size_t)1 << 20, want = std::max(mb, (bytes + mb - 1) / mb * mb);
+    void *p = nullptr, *h = nullptr;
+    e = hipMalloc(&p, want);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        release_scratch();
+        e = hipMalloc(&p, want);
+        if (e != hipSuccess) return e;
+    }
+    e = hipHostMalloc(&h, sizeof(int) * kStatusWords, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        return e;
+    }
+    device_ = device;
+    dev_ = static_cast<char *>(p);
+    bytes_ = want;
+    pinned_ = static_cast<int *>(h);
+    return hipSuccess;
+}
+
+MeshScratch::~MeshScratch()
+{
+    if (!dev_) return;
+    if (!idle_) (void)hipStreamSynchronize(nullptr);
+    Block b{device_, dev_, bytes_, pinned_};
+    Block out{};
+    try {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        std::vector<Block> &s = store();
+        s.push_back(b);
+        b.dev = nullptr;
+        size_t held = 0, count = 0;
+        auto least = s.end();
+        for (auto i = s.begin(); i != s.end(); ++i)
+            if (i->device == device_) {
+                held += i->bytes;
+                ++count;
+                if (least == s.end() || i->bytes < least->bytes) least = i;
+            }
+        // over the bounds: too many bytes, this block leaves; too many blocks,
+        // the smallest
+        if (held > kScratchBytes || count > (size_t)kScratchBlocks) {
+            auto i = held > kScratchBytes ? s.end() - 1 : least;
+            out = *i;
+            s.erase(i);
+        }
+    } catch (...) {
+        if (b.dev) out = b;
+    }
+    if (out.dev) drop(out);
+}
+
+bool in_place(const void *p, size_t align)
+{
+    if (!p || (uintptr_t)p % align) return false;
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    int device = 0;
+    return hipGetDevice(&device) == hipSuccess && a.type == hipMemoryTypeDevice && a.device == device;
+}
+
+}  // namespace cvt
+
+extern "C" int cvt_release_scratch(void)
+{
+    cvt::clear_error();
+    cvt::release_scratch();
+    return CVT_OK;
+}

@@ -33,10 +33,10 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <type_traits>
 
 #include "../../include/cvt.h"
 #include "cvt_engine.h"
+#include "mesh_scratch.h"
 
 namespace cvt {
 
@@ -122,34 +122,62 @@ __device__ void heap_sort(int *a, int n)
 }
 
 // one thread per vertex: its corners in face order, both area sums, the
-// weight, and the running maximum of the weights at or below the cap
+// weight, and the running maximum of the weights at or below the cap.  A list
+// of up to kFewCorners keys is sorted by insertion in LDS (6 000 vertices 8 us,
+// 14.5 us with every list heap-sorted in memory and an atomic per vertex).
+constexpr int kFewCorners = 16;
 __global__ __launch_bounds__(256) void k_vertex_weight(const int *__restrict__ start,
                                                        int *__restrict__ list,
                                                        const double *__restrict__ a3,
                                                        const double *__restrict__ a2, int nv,
                                                        double *__restrict__ weight,
-                                                       unsigned long long *__restrict__ mx)
+                                                       unsigned long long *__restrict__ mx,
+                                                       const int *__restrict__ bad)
 {
+    __shared__ int keys[kFewCorners * 256];        // [corner][thread]
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-    const int b = start[v], n = start[v + 1] - b;
-    heap_sort(list + b, n);
-    double s3 = 0.0, s2 = 0.0;
-    for (int k = 0; k < n; ++k) {
-        const int f = list[b + k] / 3;
-        s3 += a3[f];
-        s2 += a2[f];
+    double top = 0.0;                              // of this thread's weight, if below the cap
+    if (v < nv && !*bad) {
+        const int b = start[v], n = start[v + 1] - b;
+        double s3 = 0.0, s2 = 0.0;
+        if (n <= kFewCorners) {
+            int *own = keys + threadIdx.x;
+            for (int k = 0; k < n; ++k) {
+                const int x = list[b + k];
+                int j = k;
+                for (; j > 0 && own[256 * (j - 1)] > x; --j) own[256 * j] = own[256 * (j - 1)];
+                own[256 * j] = x;
+            }
+            for (int k = 0; k < n; ++k) {
+                const int f = own[256 * k] / 3;
+                s3 += a3[f];
+                s2 += a2[f];
+            }
+        } else {
+            heap_sort(list + b, n);
+            for (int k = 0; k < n; ++k) {
+                const int f = list[b + k] / 3;
+                s3 += a3[f];
+                s2 += a2[f];
+            }
+        }
+        const double w = s3 / s2;
+        weight[v] = w;
+        if (w <= kWeightCap) top = w;
     }
-    const double w = s3 / s2;
-    weight[v] = w;
-    if (w <= kWeightCap) atomicMax(mx, (unsigned long long)__double_as_longlong(w));
+    for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
+    if ((threadIdx.x & 63) == 0 && top > 0.0)
+        atomicMax(mx, (unsigned long long)__double_as_longlong(top));
 }
 
 __global__ __launch_bounds__(256) void k_weight_cap(double *__restrict__ weight, int nv,
-                                                    const unsigned long long *__restrict__ mx)
+                                                    const unsigned long long *__restrict__ mx,
+                                                    const int *__restrict__ bad,
+                                                    int *__restrict__ host)
 {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
+    if (v == 0) host[0] = *bad;
+    if (v >= nv || *bad) return;
     if (weight[v] > kWeightCap) weight[v] = __longlong_as_double((long long)*mx);
 }
 
@@ -157,10 +185,10 @@ __global__ __launch_bounds__(256) void k_weight_cap(double *__restrict__ weight,
 
 using namespace cvt;
 
-#define WCHK(call, what)                                                               \
-    do {                                                                               \
-        hipError_t e_ = (call);                                                        \
-        if (e_ != hipSuccess) { rc = fail(CVT_ERR_HIP, "%s: %s", what, hipGetErrorString(e_)); goto done; } \
+#define WCHK(call, what)                                                                  \
+    do {                                                                                  \
+        hipError_t e_ = (call);                                                           \
+        if (e_ != hipSuccess) return fail(CVT_ERR_HIP, "%s: %s", what, hipGetErrorString(e_)); \
     } while (0)
 
 extern "C" int cvt_vertex_weights(const double *uv, const double *p3, int nv, const int *tri,
@@ -173,55 +201,65 @@ extern "C" int cvt_vertex_weights(const double *uv, const double *p3, int nv, co
     if (nv == 0 && nf > 0) return fail(CVT_ERR_ARG, "faces without vertices");
     if (nv == 0) return CVT_OK;
     if ((long)nf * 3 > INT32_MAX) return fail(CVT_ERR_ARG, "too many faces");
-    int rc = CVT_OK, bad = 0;
     hipStream_t st = nullptr;   // the legacy default stream, as the reference's calls use
+    const size_t nfa = (size_t)std::max(nf, 1), nvs = (size_t)nv;
+    // arguments in memory of the device are used where they are (the weights
+    // if they meet no input)
+    const bool own_uv = in_place(uv, 8), own_p3 = in_place(p3, 8);
+    const bool own_tri = nf > 0 && in_place(tri, 4);
+    const bool own_w = in_place(weight, 8) && !overlap(weight, 8 * nvs, uv, 16 * nvs) &&
+                       !overlap(weight, 8 * nvs, p3, 24 * nvs) &&
+                       !overlap(weight, 8 * nvs, tri, 12 * (size_t)nf);
     double *d_uv = nullptr, *d_p3 = nullptr, *d_a3 = nullptr, *d_a2 = nullptr, *d_w = nullptr;
     int *d_tri = nullptr, *d_count = nullptr, *d_start = nullptr, *d_cursor = nullptr,
         *d_list = nullptr, *d_bad = nullptr;
     unsigned long long *d_mx = nullptr;
-    char *arena = nullptr;
-    const size_t nfa = (size_t)std::max(nf, 1), nvs = (size_t)nv;
-    // every buffer of the call in one allocation, each at a 256-byte boundary
-    size_t at = 0;
-    auto carve = [&](auto *&p, size_t n) {
-        at = (at + 255) & ~(size_t)255;
-        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(arena + at);
-        at += n * sizeof(*p);
-    };
+    MeshScratch mem;
+    Carver carve;
+    size_t zeroed = 0;
     auto layout = [&]() {
-        at = 0;
-        carve(d_uv, 2 * nvs); carve(d_p3, 3 * nvs); carve(d_w, nvs);
-        carve(d_tri, 3 * nfa); carve(d_a3, nfa); carve(d_a2, nfa); carve(d_list, 3 * nfa);
-        carve(d_count, nvs); carve(d_cursor, nvs); carve(d_start, nvs + 1);
-        carve(d_bad, 1); carve(d_mx, 1);
+        carve.base = mem.base();
+        carve.at = 0;
+        carve(d_mx, 1);                          // zeroed from here
+        carve(d_bad, 1); carve(d_count, nvs); carve(d_cursor, nvs);
+        zeroed = (carve.at + 255) & ~(size_t)255;
+        carve(d_start, nvs + 1); carve(d_a3, nfa); carve(d_a2, nfa); carve(d_list, 3 * nfa);
+        if (!own_uv) carve(d_uv, 2 * nvs);
+        if (!own_p3) carve(d_p3, 3 * nvs);
+        if (!own_tri) carve(d_tri, 3 * nfa);
+        if (!own_w) carve(d_w, nvs);
     };
     layout();
-    WCHK(hipMalloc(&arena, at), "alloc");
+    WCHK(mem.take(carve.at), "alloc");
     layout();
-    WCHK(hipMemcpyAsync(d_uv, uv, sizeof(double) * 2 * nv, hipMemcpyDefault, st), "upload");
-    WCHK(hipMemcpyAsync(d_p3, p3, sizeof(double) * 3 * nv, hipMemcpyDefault, st), "upload");
-    if (nf > 0) WCHK(hipMemcpyAsync(d_tri, tri, sizeof(int) * 3 * nf, hipMemcpyDefault, st), "upload");
-    WCHK(hipMemsetAsync(d_count, 0, sizeof(int) * nv, st), "memset");
-    WCHK(hipMemsetAsync(d_cursor, 0, sizeof(int) * nv, st), "memset");
-    WCHK(hipMemsetAsync(d_bad, 0, sizeof(int), st), "memset");
-    WCHK(hipMemsetAsync(d_mx, 0, sizeof(unsigned long long), st), "memset");
+    if (own_uv) d_uv = const_cast<double *>(uv);
+    else WCHK(hipMemcpyAsync(d_uv, uv, 16 * nvs, hipMemcpyDefault, st), "upload");
+    if (own_p3) d_p3 = const_cast<double *>(p3);
+    else WCHK(hipMemcpyAsync(d_p3, p3, 24 * nvs, hipMemcpyDefault, st), "upload");
+    if (own_tri) d_tri = const_cast<int *>(tri);
+    else if (nf > 0) WCHK(hipMemcpyAsync(d_tri, tri, 12 * (size_t)nf, hipMemcpyDefault, st), "upload");
+    if (own_w) d_w = weight;
+    const dim3 gf((nf + 255) / 256), gv((nv + 255) / 256), blk(256);
+    launch_zero(st, d_mx, zeroed);
     if (nf > 0)
-        hipLaunchKernelGGL(k_face_areas, dim3((nf + 255) / 256), dim3(256), 0, st, d_uv, d_p3, nv,
-                           d_tri, nf, d_a3, d_a2, d_count, d_bad);
+        hipLaunchKernelGGL(k_face_areas, gf, blk, 0, st, d_uv, d_p3, nv, d_tri, nf, d_a3, d_a2,
+                           d_count, d_bad);
     launch_exclusive_scan(st, d_count, nv, d_start);
     if (nf > 0)
-        hipLaunchKernelGGL(k_corner_fill, dim3((nf + 255) / 256), dim3(256), 0, st, d_tri, nv,
-                           nf, d_start, d_cursor, d_list);
-    hipLaunchKernelGGL(k_vertex_weight, dim3((nv + 255) / 256), dim3(256), 0, st, d_start, d_list,
-                       d_a3, d_a2, nv, d_w, d_mx);
-    hipLaunchKernelGGL(k_weight_cap, dim3((nv + 255) / 256), dim3(256), 0, st, d_w, nv, d_mx);
+        hipLaunchKernelGGL(k_corner_fill, gf, blk, 0, st, d_tri, nv, nf, d_start, d_cursor, d_list);
+    hipLaunchKernelGGL(k_vertex_weight, gv, blk, 0, st, d_start, d_list, d_a3, d_a2, nv, d_w, d_mx,
+                       d_bad);
+    hipLaunchKernelGGL(k_weight_cap, gv, blk, 0, st, d_w, nv, d_mx, d_bad, mem.status());
     WCHK(hipGetLastError(), "weights launch");
-    WCHK(hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, st), "flag");
     WCHK(hipStreamSynchronize(st), "weights");
-    if (bad) { rc = fail(CVT_ERR_ARG, "a face indexes a vertex outside [0, %d)", nv); goto done; }
-    WCHK(hipMemcpyAsync(weight, d_w, sizeof(double) * nv, hipMemcpyDefault, st), "download");
-    WCHK(hipStreamSynchronize(st), "weights");
-done:
-    if (arena) (void)hipFree(arena);
-    return rc;
+    if (mem.status()[0]) {
+        mem.idle();
+        return fail(CVT_ERR_ARG, "a face indexes a vertex outside [0, %d)", nv);
+    }
+    if (!own_w) {
+        WCHK(hipMemcpyAsync(weight, d_w, 8 * nvs, hipMemcpyDefault, st), "download");
+        WCHK(hipStreamSynchronize(st), "weights");
+    }
+    mem.idle();
+    return CVT_OK;
 }

@@ -9,7 +9,7 @@ import ctypes as C
 import numpy as np
 
 from ._lib import call, lib
-from .engine import _out_ptr, _ptr
+from .engine import _out_ptr, _ptr, _torch_ready_all
 
 MARKER = -32768
 
@@ -53,16 +53,17 @@ def rasterize(points, weight, triangles, scale: float, n: int, out=None):
     numpy arrays or torch tensors in host or device memory.  out: an
     (n, n) float32 array or tensor to write (host or device), or None for a
     new numpy array."""
-    pp, kp = _ptr(points, np.float64)
-    pw, kw = _ptr(weight, np.float64)
-    pt, kt = _ptr(triangles, np.int32)
+    _torch_ready_all(points, weight, triangles, out)
+    pp, kp = _ptr(points, np.float64, True)
+    pw, kw = _ptr(weight, np.float64, True)
+    pt, kt = _ptr(triangles, np.int32, True)
     nv = int(np.prod(kp.shape)) // 2
     nf = int(np.prod(kt.shape)) // 3
     if int(np.prod(kw.shape)) != nv:
         raise ValueError("weight must hold one value per point")
     if out is None:
         out = np.empty((n, n), np.float32)
-    po = _out_ptr(out, np.float32, n * n)
+    po = _out_ptr(out, np.float32, n * n, ready=True)
     call("cvt_rasterize", pp, pw, nv, pt, nf, po, float(scale), int(n))
     return out
 

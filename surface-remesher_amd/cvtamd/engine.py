@@ -23,10 +23,20 @@ def _torch_ready(a):
         torch.cuda.current_stream(a.device).synchronize()
 
 
-def _ptr(a, dtype=None):
+def _torch_ready_all(*arrays):
+    """_torch_ready once per device of the tensors among arrays, for a call
+    with several (a wait on an idle stream is 3 us of a call's 60)."""
+    seen = set()
+    for a in arrays:
+        if hasattr(a, "data_ptr") and getattr(a, "is_cuda", False) and a.device not in seen:
+            seen.add(a.device)
+            _torch_ready(a)
+
+
+def _ptr(a, dtype=None, ready=False):
     """(pointer, keep-alive) for an input: a numpy array (converted to a
     contiguous copy of dtype when needed) or a contiguous torch tensor of
-    that dtype."""
+    that dtype.  ready: the caller has waited for the tensor's stream."""
     if a is None:
         return None, None
     if hasattr(a, "data_ptr"):
@@ -36,13 +46,14 @@ def _ptr(a, dtype=None):
             got, want = str(a.dtype).replace("torch.", ""), np.dtype(dtype).name
             if got != want and not (got == "bool" and want == "uint8"):
                 raise TypeError(f"tensor dtype {a.dtype}, expected {want}")
-        _torch_ready(a)
+        if not ready:
+            _torch_ready(a)
         return C.c_void_p(a.data_ptr()), a
     arr = np.ascontiguousarray(a, dtype=dtype)
     return arr.ctypes.data_as(C.c_void_p), arr
 
 
-def _out_ptr(a, dtype, count, torch_dtypes=()):
+def _out_ptr(a, dtype, count, torch_dtypes=(), ready=False):
     """Pointer to an output the library writes in place: a numpy array or
     torch tensor of exactly dtype (or, for a tensor, one of torch_dtypes,
     e.g. bfloat16 for raw 16-bit words), C-contiguous, writable and holding
@@ -57,7 +68,8 @@ def _out_ptr(a, dtype, count, torch_dtypes=()):
             raise ValueError("out tensor must be contiguous")
         if a.numel() != count:
             raise ValueError(f"out tensor holds {a.numel()} values, expected {count}")
-        _torch_ready(a)
+        if not ready:
+            _torch_ready(a)
         return C.c_void_p(a.data_ptr())
     if not isinstance(a, np.ndarray):
         raise TypeError("out must be a numpy array or a torch tensor")

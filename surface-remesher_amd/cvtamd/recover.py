@@ -17,7 +17,7 @@ from __future__ import annotations
 import numpy as np
 
 from ._lib import call
-from .engine import _out_ptr, _ptr
+from .engine import _out_ptr, _ptr, _torch_ready_all
 
 
 def locate_points(uv, tri, q, p3=None, out=None):
@@ -30,10 +30,11 @@ def locate_points(uv, tri, q, p3=None, out=None):
     (host or device memory) are accepted.  out: None for new numpy arrays,
     or the arrays/tensors to write (host or device memory), (face, w) or,
     with p3, (face, w, xyz)."""
-    uvp, k0 = _ptr(uv, np.float64)
-    trp, k1 = _ptr(tri, np.int32)
-    qp, k2 = _ptr(q, np.float64)
-    p3p, k3 = _ptr(p3, np.float64)
+    _torch_ready_all(uv, tri, q, p3, *(out or ()))
+    uvp, k0 = _ptr(uv, np.float64, True)
+    trp, k1 = _ptr(tri, np.int32, True)
+    qp, k2 = _ptr(q, np.float64, True)
+    p3p, k3 = _ptr(p3, np.float64, True)
     nv = int(np.prod(k0.shape)) // 2 if k0 is not None else 0
     nf = int(np.prod(k1.shape)) // 3 if k1 is not None else 0
     nq = int(np.prod(k2.shape)) // 2
@@ -46,9 +47,9 @@ def locate_points(uv, tri, q, p3=None, out=None):
             raise ValueError("out must be (face, w) or, with p3, (face, w, xyz)")
         face, w = out[0], out[1]
         out3 = out[2] if p3 is not None else None
-    pf = _out_ptr(face, np.int32, nq)
-    pw = _out_ptr(w, np.float64, 3 * nq)
-    po = None if out3 is None else _out_ptr(out3, np.float64, 3 * nq)
+    pf = _out_ptr(face, np.int32, nq, ready=True)
+    pw = _out_ptr(w, np.float64, 3 * nq, ready=True)
+    po = None if out3 is None else _out_ptr(out3, np.float64, 3 * nq, ready=True)
     call("cvt_locate_points", uvp, p3p, nv, trp, nf, qp, nq, pf, pw, po)
     return (face, w) if p3 is None else (face, w, out3)
 

@@ -12,7 +12,7 @@ from __future__ import annotations
 import numpy as np
 
 from ._lib import call
-from .engine import _out_ptr, _ptr
+from .engine import _out_ptr, _ptr, _torch_ready_all
 
 
 def vertex_weights(uv, p3, tri, out=None):
@@ -26,14 +26,15 @@ def vertex_weights(uv, p3, tri, out=None):
     float64 array or tensor to write (host or device; a device tensor keeps
     the weights on the GPU for the rasterizer), or None for a new numpy
     array."""
-    uvp, k0 = _ptr(uv, np.float64)
-    p3p, k1 = _ptr(p3, np.float64)
-    trp, k2 = _ptr(tri, np.int32)
+    _torch_ready_all(uv, p3, tri, out)
+    uvp, k0 = _ptr(uv, np.float64, True)
+    p3p, k1 = _ptr(p3, np.float64, True)
+    trp, k2 = _ptr(tri, np.int32, True)
     nv = int(np.prod(k0.shape)) // 2
     if int(np.prod(k1.shape)) != 3 * nv:
         raise ValueError("p3 must hold one 3D point per uv vertex")
     nf = int(np.prod(k2.shape)) // 3
     if out is None:
         out = np.empty(nv, np.float64)
-    call("cvt_vertex_weights", uvp, p3p, nv, trp, nf, _out_ptr(out, np.float64, nv))
+    call("cvt_vertex_weights", uvp, p3p, nv, trp, nf, _out_ptr(out, np.float64, nv, ready=True))
     return out
