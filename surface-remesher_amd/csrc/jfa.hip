@@ -573,24 +573,59 @@ __device__ __forceinline__ void run_of(const RunGeo &g, int u, int &y, int &seg)
 // redirected candidates duplicate the centre row's); a column quad that is
 // off the grid for every lane of the wave is skipped for the same reason,
 // and one that is off for some lanes holds the centre quad's labels there.
-template <int MODE, int TAB, int I>
+// SHIFT: the lanes of a wave are neighbours on the row (every lane on the
+// grid), so a position left or right of a lane's quad is a centre position
+// of the lane `shift` below or above, and its site is taken from there by a
+// cross-lane read; only the outermost `shift` lanes of each side look theirs
+// up.  For tables gathered from memory: a gather costs a cycle per distinct
+// line, of which a row of 256 pixels has about as many as sites.  4096^2 /
+// 65536 sites, us per pass: steps 64 .. 4 79.5 -> 56.0, step 2 43.0 -> 41.4,
+// step 1 42.1 -> 39.9.  With the whole table in LDS the reads cost more than
+// the lookups (2048^2 / 16384 sites 4.76 -> 5.01 ms per 40 iterations).
+template <int MODE, int TAB, int I, bool SHIFT>
 __device__ __forceinline__ void run_row(const RowData<MODE> &R, const SiteTab<TAB> &tab,
                                         const float (&px)[4], const float (&py)[4],
                                         double (&best)[4][4], bool lok, bool rok, bool left,
-                                        bool right)
+                                        bool right, int shift)
 {
     constexpr int j0 = I - 2 < 0 ? 0 : I - 2;
     constexpr int j1 = I > 3 ? 3 : I;
+    const int lane = threadIdx.x & 63;
+    const bool hl = lane < shift, hr = lane >= 64 - shift;
+    float2 own[SHIFT ? 4 : 1];                     // sites of the centre quad
+    if constexpr (SHIFT) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) own[jj] = tab(q_el(R.c, jj));
+    }
+    // the site of a position whose owner's centre site is `mine`, or `edge`
+    // for the outermost lanes
+    auto from_lane = [&](int lanes, float2 mine, bool outer, float2 edge) {
+        const int at = 4 * (lane + lanes);
+        const int x = __builtin_amdgcn_ds_bpermute(at, __float_as_int(mine.x));
+        const int y = __builtin_amdgcn_ds_bpermute(at, __float_as_int(mine.y));
+        return make_float2(outer ? edge.x : __int_as_float(x), outer ? edge.y : __int_as_float(y));
+    };
     if constexpr (MODE == STEP_ANY) {
+        float2 edge[SHIFT ? 4 : 1];
+        if constexpr (SHIFT) {
+            if (hl || hr) {
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) edge[jj] = tab(hl ? q_el(R.l, jj) : q_el(R.r, jj));
+            }
+        }
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            if (q == 0 && !left) continue;
-            if (q == 2 && !right) continue;
+            if (q == 0 && !left && !SHIFT) continue;
+            if (q == 2 && !right && !SHIFT) continue;
             const u32x4 &Q = q == 0 ? R.l : q == 1 ? R.c : R.r;
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
                 const uint32_t l = q_el(Q, jj);
-                const float2 st = tab(l);
+                float2 st;
+                if constexpr (!SHIFT) st = tab(l);
+                else if (q == 1) st = own[jj];
+                else if (q == 0) st = from_lane(-shift, own[jj], hl, edge[jj]);
+                else st = from_lane(shift, own[jj], hr, edge[jj]);
                 const float dx = st.x - px[jj];
                 const float dx2 = dx * dx;
                 // one key register per label: lo = label, hi = each use's d
@@ -621,9 +656,20 @@ __device__ __forceinline__ void run_row(const RowData<MODE> &R, const SiteTab<TA
             P[6] = rok ? R.r.x : c.z;
             P[7] = rok ? R.r.y : c.w;
         }
+        float2 edge[SHIFT ? MODE : 1];
+        if constexpr (SHIFT) {
+            if (hl || hr) {
+#pragma unroll
+                for (int e = 0; e < MODE; ++e) edge[e] = tab(hl ? P[e] : P[4 + MODE + e]);
+            }
+        }
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
-            const float2 st = tab(P[k]);
+            float2 st;
+            if constexpr (!SHIFT) st = tab(P[k]);
+            else if (k < MODE) st = from_lane(-1, own[4 - MODE + k], hl, edge[k]);
+            else if (k >= 4 + MODE) st = from_lane(1, own[k - 4 - MODE], hr, edge[k - 4 - MODE]);
+            else st = own[k - MODE];
             float dy[4];
 #pragma unroll
             for (int j = j0; j <= j1; ++j) dy[j] = st.y - py[j];
@@ -655,13 +701,14 @@ __device__ __forceinline__ double key_max() { return __hiloint2double(0x7f800000
 // first two.  Rows past the grid end their chain: their outputs are not
 // stored and their loads not issued.  With `stage` the site table is staged
 // after the wave's first loads are issued, so the two latencies overlap.
-template <int MODE, int TAB, class PRO = NoPrologue>
+template <int MODE, int TAB, bool SHIFT = false, class PRO = NoPrologue>
 __device__ __forceinline__ void wave_runs(const MapGeo &m, const SiteTab<TAB> &tab,
                                           const RunGeo &g, int u, int u_end, int stride,
                                           bool stage, const PRO &pro = PRO())
 {
     const int lane4 = 4 * (threadIdx.x & 63);
     const int k = m.step, H = m.H, W = m.W;
+    const int shift = !SHIFT ? 0 : MODE == STEP_ANY ? k >> 2 : 1;   // lanes
     RowData<MODE> R0, R1, R2;
     int y = 0, seg = 0;
     if (u < u_end) {
@@ -697,17 +744,23 @@ __device__ __forceinline__ void wave_runs(const MapGeo &m, const SiteTab<TAB> &t
             for (int jj = 0; jj < 4; ++jj) best[j][jj] = key_max();
 
         if (y + k < H) load_row<MODE>(R2, m, y + k, seg, lane4);
-        if (y - k >= 0) run_row<MODE, TAB, 0>(R0, tab, px, py, best, lok, rok, left, right);
+        if (y - k >= 0) run_row<MODE, TAB, 0, SHIFT>(R0, tab, px, py, best, lok, rok, left, right,
+                                                           shift);
         if (y + 2 * k < H) load_row<MODE>(R0, m, y + 2 * k, seg, lane4);
-        if (y < H) run_row<MODE, TAB, 1>(R1, tab, px, py, best, lok, rok, left, right);
+        if (y < H) run_row<MODE, TAB, 1, SHIFT>(R1, tab, px, py, best, lok, rok, left, right,
+                                                           shift);
         if (y + 3 * k < H) load_row<MODE>(R1, m, y + 3 * k, seg, lane4);
-        if (y + k < H) run_row<MODE, TAB, 2>(R2, tab, px, py, best, lok, rok, left, right);
+        if (y + k < H) run_row<MODE, TAB, 2, SHIFT>(R2, tab, px, py, best, lok, rok, left, right,
+                                                           shift);
         if (y + 4 * k < H) load_row<MODE>(R2, m, y + 4 * k, seg, lane4);
-        if (y + 2 * k < H) run_row<MODE, TAB, 3>(R0, tab, px, py, best, lok, rok, left, right);
+        if (y + 2 * k < H) run_row<MODE, TAB, 3, SHIFT>(R0, tab, px, py, best, lok, rok, left, right,
+                                                           shift);
         if (un < u_end && yn - k >= 0) load_row<MODE>(R0, m, yn - k, sn, lane4);
-        if (y + 3 * k < H) run_row<MODE, TAB, 4>(R1, tab, px, py, best, lok, rok, left, right);
+        if (y + 3 * k < H) run_row<MODE, TAB, 4, SHIFT>(R1, tab, px, py, best, lok, rok, left, right,
+                                                           shift);
         if (un < u_end && yn < H) load_row<MODE>(R1, m, yn, sn, lane4);
-        if (y + 4 * k < H) run_row<MODE, TAB, 5>(R2, tab, px, py, best, lok, rok, left, right);
+        if (y + 4 * k < H) run_row<MODE, TAB, 5, SHIFT>(R2, tab, px, py, best, lok, rok, left, right,
+                                                           shift);
 
         if (xb < W) {
             const uint32_t o1 = 4u * (uint32_t)xc;
@@ -734,13 +787,13 @@ __device__ __forceinline__ void wave_runs(const MapGeo &m, const SiteTab<TAB> &t
 }
 
 // Runs [u0, u1) of one map by all waves of the block, dealt round robin.
-template <int MODE, int TAB, class PRO>
+template <int MODE, int TAB, bool SHIFT, class PRO>
 __device__ __forceinline__ void quad_runs(const MapGeo &m, const SiteTab<TAB> &tab, int u0, int u1,
                                           const PRO &pro)
 {
     const int nwaves = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    wave_runs<MODE, TAB>(m, tab, run_geo(m), u0 + wave, u1, nwaves, true, pro);
+    wave_runs<MODE, TAB, SHIFT>(m, tab, run_geo(m), u0 + wave, u1, nwaves, true, pro);
 }
 
 // Single map, site table staged at LDS byte 0 in a static array of ENTRIES
@@ -751,15 +804,15 @@ __device__ __forceinline__ void quad_runs(const MapGeo &m, const SiteTab<TAB> &t
 #define JFA_THREADS(E) ((E) > 5120 || (E) < 0 ? 1024 : 256)
 #define JFA_MINB(E) ((E) > 5120 || (E) < 0 ? 1 : 4)
 
-template <int MODE, int TAB, class PRO>
+template <int MODE, int TAB, bool SHIFT, class PRO>
 __device__ __forceinline__ void quad_layout(const MapGeo &m, const SiteTab<TAB> &tab, bool runs,
                                             const PRO &pro)
 {
     int a, b;
-    if (runs) {
+    if (SHIFT || runs) {
         band_of(blockIdx.x, gridDim.x, run_geo(m).count, a, b);
-        quad_runs<MODE, TAB>(m, tab, a, b, pro);
-    } else {
+        quad_runs<MODE, TAB, SHIFT>(m, tab, a, b, pro);
+    } else if constexpr (!SHIFT) {
         band_of(blockIdx.x, gridDim.x, m.H, a, b);
         quad_rows<MODE, TAB>(m, tab, a, b, pro);
     }
@@ -819,7 +872,7 @@ struct SparseReset {
     }
 };
 
-template <int MODE, int ENTRIES, bool RUNS>
+template <int MODE, int ENTRIES, bool RUNS, bool SHIFT = false>
 __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa_quad(
     const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
     const float2 *__restrict__ sites, int table_f4, int W, int H, int step,
@@ -842,7 +895,7 @@ __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa
         tab.src = reinterpret_cast<const f32x4 *>(sites);
         tab.n4 = table_f4;
         tab.base = 0;
-        quad_layout<MODE, TAB_LDS0>(m, tab, RUNS, pro);
+        quad_layout<MODE, TAB_LDS0, false>(m, tab, RUNS, pro);
     } else if constexpr (ENTRIES < 0) {
         __shared__ float4 lds_tab[-ENTRIES / 2];
         // entries 0 .. -ENTRIES - 3 staged, then a zero pair; the rest of the
@@ -855,13 +908,13 @@ __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa
         tab.g = buf_rsrc(sites + kept, 8u * (uint32_t)(2 * table_f4 - kept));
         tab.split = 8u * (uint32_t)kept;
         tab.base = 0;
-        quad_layout<MODE, TAB_SPLIT>(m, tab, RUNS, pro);
+        quad_layout<MODE, TAB_SPLIT, SHIFT>(m, tab, RUNS, pro);
     } else {
         SiteTab<TAB_GLOBAL> tab;
         tab.g = buf_rsrc(sites, 16u * (uint32_t)table_f4);
         tab.base = 0;
         tab.n4 = 0;
-        quad_layout<MODE, TAB_GLOBAL>(m, tab, RUNS, pro);
+        quad_layout<MODE, TAB_GLOBAL, false>(m, tab, RUNS, pro);
     }
 }
 
@@ -1165,8 +1218,14 @@ static void launch_quad(hipStream_t st, const JfaPlan &p, const uint32_t *in, ui
                            p.table_f4, W, H, step, clear, none, nclear, rstep, stop);
         break;
     case -20480:
-        hipLaunchKernelGGL((k_jfa_quad<MODE, -20480, RUNS>), g, b, 0, st, in, out, sites,
-                           p.table_f4, W, H, step, clear, none, nclear, rstep, stop);
+        // whole 256-pixel segments, and a lane's neighbour positions within
+        // the wave on one side at least (step 128: half of them)
+        if (RUNS && W % 256 == 0 && step <= 128)
+            hipLaunchKernelGGL((k_jfa_quad<MODE, -20480, RUNS, RUNS>), g, b, 0, st, in, out, sites,
+                               p.table_f4, W, H, step, clear, none, nclear, rstep, stop);
+        else
+            hipLaunchKernelGGL((k_jfa_quad<MODE, -20480, RUNS>), g, b, 0, st, in, out, sites,
+                               p.table_f4, W, H, step, clear, none, nclear, rstep, stop);
         break;
     default:
         hipLaunchKernelGGL((k_jfa_quad<MODE, 0, RUNS>), g, b, 0, st, in, out, sites, p.table_f4, W,
