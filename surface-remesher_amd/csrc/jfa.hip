@@ -926,26 +926,39 @@ __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa
 // a kTailHalo-pixel halo of the step-16 map into LDS and runs the five
 // passes there, each over the tile grown by the steps still to come (8, 4,
 // 2, 1, 0 pixels), so every tap a pass reads was written by the pass before
-// it.  Taps off the grid are redirected to the pixel's own row or column,
-// as in the dense pass, so the grid edges need no halo.  Each pixel takes
+// it.  A thread evaluates runs of kTailRun pixels one step apart in a column:
+// a tap row serves up to three of them, so a run looks up 3 (kTailRun + 2)
+// sites instead of 9 kTailRun.  Taps off the grid are the pixel's own row
+// or column in the dense pass: their candidates repeat the centre's, so rows
+// are left out and columns read again.  Each pixel takes
 // the (d, label) minimum over its nine taps with the dense pass's distance
-// formula: the map equals the dense passes bit for bit.
+// formula: the map equals the dense passes bit for bit.  The last pass writes
+// the map.
+// Bound by the latency of its five dependent passes and by LDS reads:
+// 512^2 / 1024 sites 10.9 us (11.6 with nine lookups per
+// pixel), 1024^2 / 4096 sites 27.8 us (34.2); 12.6 and 27.8 with runs of three on 512
+// threads.
 // ---------------------------------------------------------------------------
 static constexpr int kTailT = 32, kTailHalo = 16, kTailP = kTailT + 2 * kTailHalo;
+static constexpr int kTailRun = 2, kTailThreads = 1024;
+
+static_assert((kTailT + kTailHalo) * (kTailT + kTailHalo) / kTailRun * (kTailT + kTailHalo) < 65536,
+              "item / width by multiplication");
 
 template <int ENTRIES>
-__global__ __launch_bounds__(1024) void k_jfa_tail(const uint32_t *__restrict__ in,
-                                                   uint32_t *__restrict__ out,
-                                                   const float2 *__restrict__ sites, int table_f4,
-                                                   int W, int H, int tilesX, int skip,
-                                                   uint32_t *__restrict__ clear, uint32_t none,
-                                                   int nclear, const int *__restrict__ stop)
+__global__ __launch_bounds__(kTailThreads) void k_jfa_tail(const uint32_t *__restrict__ in,
+                                                           uint32_t *__restrict__ out,
+                                                           const float2 *__restrict__ sites,
+                                                           int table_f4, int W, int H, int tilesX,
+                                                           int skip, uint32_t *__restrict__ clear,
+                                                           uint32_t none, int nclear,
+                                                           const int *__restrict__ stop)
 {
     // the site table at LDS byte 0, then the two tile buffers
     __shared__ float4 lds_all[ENTRIES / 2 + kTailP * kTailP / 2];
     uint32_t *const buf0 = reinterpret_cast<uint32_t *>(lds_all + ENTRIES / 2);
     uint32_t *const buf1 = buf0 + kTailP * kTailP;
-    const int tid = threadIdx.x, nt = blockDim.x;
+    const int tid = threadIdx.x;
     const int tY = blockIdx.x / tilesX, tX = blockIdx.x - tY * tilesX;
     const int X0 = tX * kTailT, Y0 = tY * kTailT;
     const int bx = X0 - kTailHalo, by = Y0 - kTailHalo;   // the buffers' origin on the grid
@@ -958,56 +971,94 @@ __global__ __launch_bounds__(1024) void k_jfa_tail(const uint32_t *__restrict__ 
     pro.nclear = nclear;
     pro.rstep = 0;
     pro.none = none;
-    {
-        const int halo = kTailHalo >> skip;
-        const int x0 = max(X0 - halo, 0), x1 = min(X0 + kTailT + halo, W);
-        const int y0 = max(Y0 - halo, 0), y1 = min(Y0 + kTailT + halo, H);
-        const int w = x1 - x0, n = w * (y1 - y0);
-        for (int i = tid; i < n; i += nt) {
-            const int r = i / w, x = x0 + (i - r * w), y = y0 + r;
-            buf0[(y - by) * kTailP + (x - bx)] = in[(long)y * W + x];
-        }
-    }
     SiteTab<TAB_LDS0> tab;
     tab.lds = (lds_cchar *)lds_all;
     tab.src = reinterpret_cast<const f32x4 *>(sites);
     tab.n4 = table_f4;
     tab.base = 0;
-    tab.stage();                     // ends with a barrier: buf0 is complete too
+    {
+        // the tile and the table: every load is issued before the first wait.
+        // The buffer's row r is grid row by + r; a thread takes one column.
+        const int halo = kTailHalo >> skip;
+        const int c = tid % kTailP, x = bx + c;
+        const bool col = x >= max(X0 - halo, 0) && x < min(X0 + kTailT + halo, W);
+        const int y0 = max(Y0 - halo, 0), y1 = min(Y0 + kTailT + halo, H);
+        constexpr int RS = kTailThreads / kTailP, N = kTailP / RS;
+        constexpr int NT = (ENTRIES / 2 + kTailThreads - 1) / kTailThreads;
+        uint32_t v[N];
+        u32x4 e[NT];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int y = by + tid / kTailP + RS * k;
+            v[k] = col && y >= y0 && y < y1 ? in[(long)y * W + x] : 0u;
+        }
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(sites, 16u * (uint32_t)table_f4);
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+            e[k] = __builtin_amdgcn_raw_buffer_load_b128(r, 16u * (uint32_t)(tid + k * kTailThreads), 0, 0);
+#pragma unroll
+        for (int k = 0; k < N; ++k) buf0[(tid / kTailP + RS * k) * kTailP + c] = v[k];
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+            if ((k + 1) * kTailThreads <= ENTRIES / 2 || tid + k * kTailThreads < ENTRIES / 2)
+                reinterpret_cast<u32x4 *>(lds_all)[tid + k * kTailThreads] = e[k];
+        __syncthreads();
+    }
     if (pro()) return;
     uint32_t *cur = buf0, *nxt = buf1;
 #pragma unroll 1
     for (int k = skip; k < 5; ++k) {
-        const int s = k == 0 ? 8 : k == 1 ? 4 : k == 2 ? 2 : 1;
-        const int g = k == 0 ? 8 : k == 1 ? 4 : k == 2 ? 2 : k == 3 ? 1 : 0;   // halo after
+        const int ls = k < 3 ? 3 - k : 0, s = 1 << ls;         // step 8, 4, 2, 1, 1
+        const int g = k < 3 ? s : k == 3 ? 1 : 0;               // halo after
         const int x0 = max(X0 - g, 0), x1 = min(X0 + kTailT + g, W);
         const int y0 = max(Y0 - g, 0), y1 = min(Y0 + kTailT + g, H);
-        const int w = x1 - x0, n = w * (y1 - y0);
-        for (int i = tid; i < n; i += nt) {
-            const int r = i / w, x = x0 + (i - r * w), y = y0 + r;
-            // tap columns and rows, off-grid ones redirected to the pixel's own
-            const int cx[3] = {x - s >= 0 ? x - s : x, x, x + s < W ? x + s : x};
-            const int cy[3] = {y - s >= 0 ? y - s : y, y, y + s < H ? y + s : y};
-            const float px = (float)x + 0.5f, py = (float)y + 0.5f;
-            double best = 0.0;
+        const int w = x1 - x0, nq = (((y1 - y0 + s - 1) >> ls) + kTailRun - 1) / kTailRun;
+        // column of item i: x0 + i % w (exact: i w < 2^16, as w <= 48 and an
+        // item has kTailRun of at most 48 rows)
+        const uint32_t inv = 65536u / (uint32_t)w + 1u;
+        for (int i = tid; i < w * (nq << ls); i += kTailThreads) {
+            const int r = (int)(((uint32_t)i * inv) >> 16), x = x0 + (i - r * w);
+            const int y = y0 + (r & (s - 1)) + kTailRun * ((r >> ls) << ls);   // first row
+            const int cl = x - s >= 0 ? -s : 0, cr = x + s < W ? s : 0;
+            const float px = (float)x + 0.5f;
+            float py[kTailRun];
+            double best[kTailRun];
 #pragma unroll
-            for (int t = 0; t < 9; ++t) {
-                const uint32_t l = cur[(cy[t / 3] - by) * kTailP + (cx[t % 3] - bx)];
-                const double key = cand(tab(l), l, px, py);
-                best = (t == 0) ? key : __builtin_fmin(best, key);
+            for (int j = 0; j < kTailRun; ++j) {
+                py[j] = (float)(y + j * s) + 0.5f;
+                best[j] = key_max();
             }
-            nxt[(y - by) * kTailP + (x - bx)] = (uint32_t)__double2loint(best);
+            const uint32_t *at = cur + (y - s - by) * kTailP + (x - bx);
+#pragma unroll
+            for (int t = 0; t < kTailRun + 2; ++t, at += s * kTailP) {
+                const int yt = y + (t - 1) * s;
+                if (yt < 0 || yt >= H || yt - s >= y1) continue;
+                const uint32_t l3[3] = {at[cl], at[0], at[cr]};
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    const float2 st = tab(l3[q]);
+                    const float dx = st.x - px, dx2 = dx * dx;
+#pragma unroll
+                    for (int j = 0; j < kTailRun; ++j) {
+                        if (j < t - 2 || j > t) continue;
+                        const float dy = st.y - py[j];
+                        best[j] = __builtin_fmin(best[j], jfa_key(__builtin_fmaf(dy, dy, dx2), l3[q]));
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kTailRun; ++j) {
+                const int yj = y + j * s;
+                if (yj >= y1) break;
+                const uint32_t l = (uint32_t)__double2loint(best[j]);
+                if (k == 4) out[(long)yj * W + x] = l;
+                else nxt[(yj - by) * kTailP + (x - bx)] = l;
+            }
         }
         __syncthreads();
         uint32_t *const t = cur;
         cur = nxt;
         nxt = t;
-    }
-    const int x1 = min(X0 + kTailT, W), y1 = min(Y0 + kTailT, H);
-    const int w = x1 - X0, n = w * (y1 - Y0);
-    for (int i = tid; i < n; i += nt) {
-        const int r = i / w, x = X0 + (i - r * w), y = Y0 + r;
-        out[(long)y * W + x] = cur[(y - by) * kTailP + (x - bx)];
     }
 }
 
@@ -1026,10 +1077,10 @@ void launch_jfa_tail(hipStream_t st, const JfaPlan &p, int passes, const uint32_
 {
     const int tx = (W + kTailT - 1) / kTailT, ty = (H + kTailT - 1) / kTailT;
     if (p.tail_entries == 2048)
-        hipLaunchKernelGGL(k_jfa_tail<2048>, dim3(tx * ty), dim3(1024), 0, st, in, out, sites,
+        hipLaunchKernelGGL(k_jfa_tail<2048>, dim3(tx * ty), dim3(kTailThreads), 0, st, in, out, sites,
                            p.table_f4, W, H, tx, 5 - passes, clear, none, nclear, stop);
     else
-        hipLaunchKernelGGL(k_jfa_tail<5120>, dim3(tx * ty), dim3(1024), 0, st, in, out, sites,
+        hipLaunchKernelGGL(k_jfa_tail<5120>, dim3(tx * ty), dim3(kTailThreads), 0, st, in, out, sites,
                            p.table_f4, W, H, tx, 5 - passes, clear, none, nclear, stop);
 }
 
