@@ -72,7 +72,8 @@ struct Schedule {
 // source/gcvt.cu:1033).  The level runs at least one iteration (do ...
 // while, source/gcvt.cu:1111-1142).
 static int run_level(Ctx *c, const float *rho, const uint8_t *mask, int max_iter, bool finest,
-                     Schedule &sc, int S0, float *domega, int *tgt, uint32_t *owner, double escale)
+                     Schedule &sc, int S0, float *domega, int *tgt, int *cnt, uint32_t *owner,
+                     double escale)
 {
     const double threshold = finest ? 1e-5 : 3e-1;   // source/gcvt.cu:1131-1137
     int nst[1] = {S0};
@@ -90,10 +91,15 @@ static int run_level(Ctx *c, const float *rho, const uint8_t *mask, int max_iter
         return fail(CVT_ERR_HIP, "capture");
     int rc = c->enqueue_jfa();
     if (!rc) rc = c->enqueue_moments();
-    if (!rc) rc = c->enqueue_update(UPD_COMPAT | UPD_DEV_S, sc.omega, nullptr, 1, nullptr, domega, ca);
     if (!rc)
-        hipLaunchKernelGGL(k_compat_compact, dim3(1), dim3(1024), 0, c->stream, c->sites, tgt, owner,
-                           c->seed, c->W, c->dstate);
+        rc = c->enqueue_update(UPD_COMPAT | UPD_DEV_S, sc.omega, nullptr, 1, nullptr, domega, ca, 1);
+    if (!rc) {
+        const int nb = std::max(1, (S0 + 255) / 256);
+        hipLaunchKernelGGL(k_compat_count, dim3(nb + 1), dim3(256), 0, c->stream, tgt, owner, cnt, nb,
+                           c->dstate, c->blockpart, c->final_args(1, nullptr));
+        hipLaunchKernelGGL(k_compat_compact, dim3(nb), dim3(256), 0, c->stream, c->sites, tgt, owner,
+                           c->seed, c->W, cnt, nb, c->dstate);
+    }
     const hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
     if (e != hipSuccess || hipGraphInstantiate(&gx, g, nullptr, nullptr, 0) != hipSuccess) {
@@ -184,7 +190,7 @@ extern "C" int cvt_compat_gcvt(int16_t *voronoi, const float *density, const uin
     std::vector<float *> lrho(levels, nullptr);
     uint8_t *dmask = nullptr;
     float *domega = nullptr;
-    int *tgt = nullptr;
+    int *tgt = nullptr, *cnt = nullptr;            // targets, then the merge's counts
     uint32_t *owner = nullptr;
     short2 *dcoords = nullptr;
     std::vector<float> cur;
@@ -222,7 +228,8 @@ extern "C" int cvt_compat_gcvt(int16_t *voronoi, const float *density, const uin
     if (mask) CCHK(hipMemcpyAsync(dmask, mask, np, hipMemcpyDefault, c->stream), "mask upload");
     else CCHK(hipMemsetAsync(dmask, 0, np, c->stream), "mask clear");
     CCHK(hipMalloc(&domega, sizeof(float)), "alloc");
-    CCHK(hipMalloc(&tgt, sizeof(int) * std::max(S, 1)), "alloc");
+    CCHK(hipMalloc(&tgt, sizeof(int) * ((size_t)std::max(S, 1) + (S + 255) / 256 + 2)), "alloc");
+    cnt = tgt + std::max(S, 1);
     CCHK(hipMalloc(&owner, sizeof(uint32_t) * np), "alloc");
     hipLaunchKernelGGL(k_fill_u32, dim3(1024), dim3(256), 0, c->stream, owner, (uint32_t)CVT_NONE, np);
     CCHK(hipStreamSynchronize(c->stream), "setup");
@@ -242,7 +249,7 @@ extern "C" int cvt_compat_gcvt(int16_t *voronoi, const float *density, const uin
         const int Sl = (int)(cur.size() / 2);
         if (!rc) rc = cvt_set_sites(hl, cur.data(), nullptr, Sl);
         if (!rc)
-            rc = run_level(cl, cl->rho, dmask, max_iter, l == 0, sc, Sl, domega, tgt, owner,
+            rc = run_level(cl, cl->rho, dmask, max_iter, l == 0, sc, Sl, domega, tgt, cnt, owner,
                            ldexp(1.0, 2 * l));
         if (!rc && l > 0) {
             int nst = 0;
