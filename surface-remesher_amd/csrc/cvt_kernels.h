@@ -687,7 +687,7 @@ static __global__ void k_until(int *__restrict__ dstate, double *__restrict__ un
 // their seeds; the owner map is cleared again.  Two launches of a block per 256
 // sites: the first counts each block's survivors (and marks the others by the
 // complement of their target), the second adds the counts before its block and
-// moves the sites.  8192 sites 8.8 us together (18.2 us in one workgroup,
+// moves the sites.  4096 sites 8.8 us together (18.2 us in one workgroup,
 // bound by the scattered stores of a single CU).  cnt: a count per block, then
 // the number of sites before the merge.  The first launch has one more block,
 // which finalizes the update that set the targets (deferred to here: the
