@@ -50,6 +50,7 @@
 #include "../../include/cvt.h"
 #include "cvt_engine.h"
 #include "dt_predicates.h"
+#include "scan.h"
 
 namespace cvt {
 
@@ -600,12 +601,32 @@ __global__ __launch_bounds__(1024) void k_dt_vote_lds(Pts P, int n, int T,
     }
 }
 
-__global__ void k_dt_split_flags(const unsigned long long *__restrict__ vote, int T,
-                                 int *__restrict__ flag)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < T) flag[t] = vote[t] != NO_BID;
-}
+// the scan that ranks the triangles to split counts those with a bid ...
+struct BidLoad {
+    const unsigned long long *vote;
+    __device__ __forceinline__ int4 operator()(long base, int n) const
+    {
+        int4 c;
+        c.x = base < n && vote[base] != NO_BID;
+        c.y = base + 1 < n && vote[base + 1] != NO_BID;
+        c.z = base + 2 < n && vote[base + 2] != NO_BID;
+        c.w = base + 3 < n && vote[base + 3] != NO_BID;
+        return c;
+    }
+};
+// ... and hands the counters and the count to the host's pinned memory; the
+// next round counts its uninserted points from zero
+struct PublishVote {
+    int *cnt, *host;
+    __device__ __forceinline__ void operator()(int total) const
+    {
+        const int i = threadIdx.x;
+        if (i >= NUM_C) return;
+        host[i] = i == C_SPLITS ? total : cnt[i];
+        if (i == C_UNINS) cnt[i] = 0;
+        __threadfence_system();
+    }
+};
 
 // the point whose bid won; place: where the point of each caller's index is
 // kept (null: at it)
@@ -626,9 +647,11 @@ __global__ void k_dt_split(Pts P, int n, int T, int *__restrict__ tv,
                            int *__restrict__ to, const unsigned long long *__restrict__ vote,
                            const int *__restrict__ base, int *__restrict__ loc,
                            const int *__restrict__ place, int *__restrict__ chk, int next_pass,
-                           int *__restrict__ list, int *__restrict__ cnt)
+                           int *__restrict__ list, int *__restrict__ cnt,
+                           unsigned long long *__restrict__ next_vote)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < T) next_vote[t] = NO_BID;      // of the next round, and of the children below
     if (t == 0) {                          // the flip run that follows checks the children
         cnt[C_LIST] = 3 * base[T];
         cnt[C_LIST + 1] = cnt[C_CAND] = cnt[C_CAND + 1] = cnt[C_PASSES] = cnt[C_CONV] = 0;
@@ -649,6 +672,7 @@ __global__ void k_dt_split(Pts P, int n, int T, int *__restrict__ tv,
     for (int i = 0; i < 3; ++i) {
         const int s = slot[i];
         chk[s] = next_pass;
+        next_vote[s] = NO_BID;
         list[3 * base[t] + i] = s;
         tv[3 * s] = v[(i + 1) % 3];
         tv[3 * s + 1] = v[(i + 2) % 3];
@@ -1321,7 +1345,7 @@ struct DtCtx {
     Pts pts() const { return Pts{P, sorted ? ids : nullptr}; }
     const int *places() const { return sorted ? place : nullptr; }
     int *tv = nullptr, *to = nullptr;      // [Tmax][3]
-    unsigned long long *vote = nullptr;    // [Tmax]
+    unsigned long long *vote[2] = {nullptr, nullptr};   // [Tmax], of this round and the next
     int *flag = nullptr, *pos = nullptr;   // [Tmax], [Tmax + 1]
     int *fvote = nullptr, *fstamp = nullptr, *fwd = nullptr, *chk = nullptr;
     int *list[2] = {nullptr, nullptr};     // [Tmax] triangles a flip pass looks at
@@ -1388,7 +1412,7 @@ extern "C" int cvt_dt_create(cvt_dt **out, int max_points)
         carve(c->P, N + 1, set); carve(c->in, N, set); carve(c->ids, N + 1, set);
         carve(c->place, N, set); carve(c->bounds, 4 * kParts, set);
         carve(c->tv, 3 * T, set); carve(c->to, 3 * T, set);
-        carve(c->vote, T, set); carve(c->flag, T, set); carve(c->pos, T + 1, set);
+        carve(c->vote[0], T, set); carve(c->vote[1], T, set); carve(c->flag, T, set); carve(c->pos, T + 1, set);
         carve(c->fvote, T, set); carve(c->fstamp, T, set); carve(c->fwd, 3 * T, set);
         carve(c->chk, T, set);
         carve(c->list[0], T, set); carve(c->list[1], T, set); carve(c->cand, 3 * T / 2 + 1, set);
@@ -1625,30 +1649,27 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
     if (h[C_ERR]) return fail(CVT_ERR_ARG, "degenerate input: all points collinear or coincident");
     hipLaunchKernelGGL(k_dt_locate0, dim3(nb(n)), dim3(256), 0, st, c->pts(), n, c->loc, c->cnt);
     hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_CONV, 1, 1L);
+    hipLaunchKernelGGL(k_dt_fill<unsigned long long>, dim3(1), dim3(64), 0, st, c->vote[0], NO_BID, 4L);
     int T = 4, round = 0, done = 0;
     int first = 1;                     // first pass of the latest flip run
     // Each round inserts at least one point.  A round's bids are enqueued
     // behind the flips of the round before and do nothing while those go on
     // (C_CONV): the host reads the counters once per round.
     for (int guard = 0; guard <= n; ++guard) {
+        unsigned long long *const vote = c->vote[guard & 1];
         for (;;) {
-            hipLaunchKernelGGL(k_dt_fill<unsigned long long>, dim3(nb(T)), dim3(256), 0, st,
-                               c->vote, NO_BID, (long)T);
-            hipLaunchKernelGGL(k_dt_fill<int>, dim3(1), dim3(64), 0, st, c->cnt + C_UNINS, 0, 1L);
             if (T <= kVoteLds)
                 hipLaunchKernelGGL(k_dt_vote_lds,
                                    dim3((unsigned)std::min<long>(256, (n + 1023) / 1024)),
                                    dim3(1024), 0, st, c->pts(), n, T, c->tv, c->to, c->fstamp,
                                    first,
-                                   c->loc, c->vote, c->cnt);
+                                   c->loc, vote, c->cnt);
             else
                 hipLaunchKernelGGL(k_dt_vote, dim3(nb(n)), dim3(256), 0, st, c->pts(), n, T, c->tv,
-                                   c->to, c->fstamp, first, c->loc, c->vote, c->cnt);
-            hipLaunchKernelGGL(k_dt_split_flags, dim3(nb(T)), dim3(256), 0, st, c->vote, T,
-                               c->flag);
-            launch_exclusive_scan(st, c->flag, T, c->pos);
-            const int rc = read_counters(c, c->pos + T, "vote");
-            if (rc) return rc;
+                                   c->to, c->fstamp, first, c->loc, vote, c->cnt);
+            launch_scan(st, BidLoad{vote}, T, c->pos, PublishVote{c->cnt, c->hcnt});
+            DCHK(hipGetLastError(), "vote");
+            DCHK(hipStreamSynchronize(st), "vote");
             if (guard == 0) break;
             const int left = flips_left(c, done, round);
             if (left == 0) break;
@@ -1660,9 +1681,10 @@ static int dt_run(cvt_dt *dt, const double *points, int num_points, const int *s
         const int splits = h[C_SPLITS];
         if (T + 2 * splits > c->Tmax) return fail(CVT_ERR_CAPACITY, "triangle capacity");
         hipLaunchKernelGGL(k_dt_split, dim3(nb(T)), dim3(256), 0, st, c->pts(), n, T, c->tv, c->to,
-                           c->vote, c->pos, c->loc, c->places(), c->chk, round + 1, c->list[0], c->cnt);
+                           vote, c->pos, c->loc, c->places(), c->chk, round + 1, c->list[0], c->cnt,
+                           c->vote[(guard + 1) & 1]);
         hipLaunchKernelGGL(k_dt_relocate_split, dim3(nb(n)), dim3(256), 0, st, c->pts(), n, T, c->tv,
-                           c->vote, c->pos, c->loc, c->places(), c->cnt);
+                           vote, c->pos, c->loc, c->places(), c->cnt);
         T += 2 * splits;
         ++c->stats[0];
         done = 0;

@@ -32,6 +32,7 @@
 #include "../../include/cvt.h"
 #include "cvt_engine.h"
 #include "mesh_scratch.h"
+#include "scan.h"
 
 namespace cvt {
 
@@ -157,124 +158,6 @@ __global__ void k_face_boxes(const double *__restrict__ uv, int nv, const int *_
     box[i] = bx;
     for (int y = bx.y0; y <= bx.y1; ++y)
         for (int x = bx.x0; x <= bx.x1; ++x) atomicAdd(&count[y * g.G + x], 1);
-}
-
-// Exclusive prefix sum of n counts into start[0 .. n] over tiles of 4096
-// counts (1024 threads x 4 consecutive counts).  Up to kScanOne counts one
-// workgroup walks over the tiles (k_scan_one: 4.5 us for 6 000 counts, where
-// three launches take 7.4 us and their gaps; 11 us for 16 384, where they take
-// 8.2); beyond that in three launches:
-//   k_scan_tiles        each tile's total, parked in start[tile * 4096];
-//   k_scan_tile_totals  one workgroup turns the parked totals into the tiles'
-//                       offsets in place and writes start[n];
-//   k_scan_apply        each tile reads its offset, then writes its starts
-//                       (its first entry, the parked offset, last).
-constexpr int kScanTile = 4096, kScanOne = 8192;
-
-// exclusive prefix sum over a 1024-thread workgroup of one value per thread;
-// total receives the workgroup's sum (lds: 32 ints)
-__device__ __forceinline__ int wg_exclusive_scan(int v, int *lds, int &total)
-{
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    __syncthreads();                       // lds is free (a previous call has read it)
-    if (lane == 63) lds[wv] = x;
-    __syncthreads();
-    if (wv == 0) {
-        int t = (lane < 16) ? lds[lane] : 0;
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) {
-            const int y = __shfl_up(t, o, 64);
-            if (lane >= o) t += y;
-        }
-        if (lane < 16) lds[16 + lane] = t;
-    }
-    __syncthreads();
-    total = lds[31];
-    return (wv > 0 ? lds[15 + wv] : 0) + x - v;
-}
-
-// the thread's 4 counts (0 past n)
-__device__ __forceinline__ int4 tile_counts(const int *__restrict__ count, long base, int n)
-{
-    if (base + 3 < n) return *reinterpret_cast<const int4 *>(count + base);
-    int4 c = {0, 0, 0, 0};
-    if (base < n) c.x = count[base];
-    if (base + 1 < n) c.y = count[base + 1];
-    if (base + 2 < n) c.z = count[base + 2];
-    return c;
-}
-
-__global__ __launch_bounds__(1024) void k_scan_tiles(const int *__restrict__ count, int n,
-                                                     int *__restrict__ start)
-{
-    __shared__ int lds[32];
-    const long tile0 = (long)blockIdx.x * kScanTile;
-    const int4 c = tile_counts(count, tile0 + 4 * threadIdx.x, n);
-    int total;
-    wg_exclusive_scan(c.x + c.y + c.z + c.w, lds, total);
-    if (threadIdx.x == 0) start[tile0] = total;
-}
-
-__global__ __launch_bounds__(1024) void k_scan_tile_totals(int *__restrict__ start, int n,
-                                                           int ntiles)
-{
-    __shared__ int lds[32];
-    int carry = 0;
-    for (int c = 0; c < ntiles; c += 1024) {
-        const int b = c + (int)threadIdx.x;
-        const long at = (long)b * kScanTile;
-        const int v = (b < ntiles) ? start[at] : 0;
-        int total;
-        const int ex = wg_exclusive_scan(v, lds, total);
-        if (b < ntiles) start[at] = carry + ex;
-        carry += total;
-    }
-    if (threadIdx.x == 0) start[n] = carry;
-}
-
-__global__ __launch_bounds__(1024) void k_scan_apply(const int *__restrict__ count, int n,
-                                                     int *__restrict__ start)
-{
-    __shared__ int lds[32];
-    const long tile0 = (long)blockIdx.x * kScanTile;
-    const int off = start[tile0];          // read by every thread before the scan's barriers
-    const long base = tile0 + 4 * threadIdx.x;
-    const int4 c = tile_counts(count, base, n);
-    int total;
-    int run = off + wg_exclusive_scan(c.x + c.y + c.z + c.w, lds, total);
-    const int v[4] = {c.x, c.y, c.z, c.w};
-    for (int k = 0; k < 4; ++k)
-        if (base + k < n) {
-            start[base + k] = run;
-            run += v[k];
-        }
-}
-
-__global__ __launch_bounds__(1024) void k_scan_one(const int *__restrict__ count, int n,
-                                                   int *__restrict__ start)
-{
-    __shared__ int lds[32];
-    int carry = 0;
-    for (int tile0 = 0; tile0 < n; tile0 += kScanTile) {
-        const long base = tile0 + 4 * (long)threadIdx.x;
-        const int4 c = tile_counts(count, base, n);
-        int total;
-        int run = carry + wg_exclusive_scan(c.x + c.y + c.z + c.w, lds, total);
-        const int v[4] = {c.x, c.y, c.z, c.w};
-        for (int k = 0; k < 4; ++k)
-            if (base + k < n) {
-                start[base + k] = run;
-                run += v[k];
-            }
-        carry += total;
-    }
-    if (threadIdx.x == 0) start[n] = carry;
 }
 
 // (face, bin) pairs: each face writes its index into the lists of its bins;
@@ -412,14 +295,7 @@ void launch_zero(hipStream_t st, void *p, size_t bytes)
 
 void launch_exclusive_scan(hipStream_t st, const int *count, int n, int *start)
 {
-    if (n <= kScanOne) {
-        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, st, count, n, start);
-        return;
-    }
-    const int ntiles = (int)(((long)n + kScanTile - 1) / kScanTile);
-    hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(1024), 0, st, count, n, start);
-    hipLaunchKernelGGL(k_scan_tile_totals, dim3(1), dim3(1024), 0, st, start, n, ntiles);
-    hipLaunchKernelGGL(k_scan_apply, dim3(ntiles), dim3(1024), 0, st, count, n, start);
+    launch_scan(st, CountLoad{count}, n, start, ScanDone());
 }
 
 }  // namespace cvt
