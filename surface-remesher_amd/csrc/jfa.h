@@ -9,19 +9,20 @@
 namespace cvt {
 
 // Launch shape of a JFA pass for one grid: the quad kernel (4 pixels per
-// lane, persistent workgroups over runs or bands of rows) when W % 4 == 0,
+// lane, persistent workgroups over runs or bands of rows) when W % 4 == 0
+// (quad), and on the steps that take runs at other widths from 9 up (ragged),
 // with the site table in a static LDS array of lds_entries float2 (16, 40 or
 // 160 KB) when it fits, or, for larger tables, lds_entries = -20480: the
 // first 20478 entries and a zero entry in LDS, the rest gathered from global
 // memory;
 // otherwise one pixel per lane.  tail_entries: the array (16 or 40 KB) that
 // launch_jfa_tail stages the table in, at any width; 0 when it is larger.
-// runs_mask < 0 (JFA_AUTO): runs where every wave of the launch gets one,
-// bands of rows elsewhere; otherwise bit k set = runs at step 2^k, clear =
+// runs_mask < 0 (JFA_AUTO): runs where every wave of the launch gets one (on
+// ragged plans from 1.5 per CU), bands of rows (one pixel per lane) elsewhere; otherwise bit k set = runs at step 2^k, clear =
 // bands (the labels do not depend on it).
 enum { JFA_AUTO = -1 };
 struct JfaPlan {
-    bool quad = false, lds = false;
+    bool quad = false, ragged = false, lds = false;
     int grid = 0, threads = 0, table_f4 = 0, lds_entries = 0, tail_entries = 0;
     size_t lds_bytes = 0;
     int runs_mask = JFA_AUTO, blocks_per_cu = 0;
@@ -35,7 +36,7 @@ int jfa_runs_mask(const JfaPlan &p, int W, int H);
 
 // One JFA pass over a W x H map of byte-offset labels (8 * site index, `none`
 // for no site): out(p) = best of the 9 labels at p + step * {-1, 0, 1}^2.
-// If clear is non-null it is reset to `none`: with nclear > 0 on quad plans
+// If clear is non-null it is reset to `none`: with nclear > 0 in the quad kernel
 // only where it can hold entries, the seed pixels q of sites [0, nclear)
 // (rstep == 0) or q + rstep * {-1, 0, 1}^2 (rstep > 0); otherwise pixel by
 // pixel.  The site table must hold capS + 1 entries rounded up to an even

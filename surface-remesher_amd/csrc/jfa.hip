@@ -274,10 +274,12 @@ __device__ __forceinline__ void load_row(RowData<MODE> &d, const MapGeo &m, int 
     const uint32_t s = row_off(m, y);
     if constexpr (MODE == STEP_ANY) {
         // a tap column outside the grid is redirected to the centre column
-        // (for step >= 4 the whole quad is in or out together)
+        // (for step >= 4 and a width in fours the whole quad is in or out
+        // together; otherwise the right quad that crosses the row's end is
+        // the row's last four labels, sorted out by end_quad)
         const int st = m.step;
         const uint32_t o0 = (xc - st >= 0) ? o1 - 4u * (uint32_t)st : o1;
-        const uint32_t o2 = (xc + 3 + st < m.W) ? o1 + 4u * (uint32_t)st : o1;
+        const uint32_t o2 = (xc + st < m.W) ? 4u * (uint32_t)min(xc + st, m.W - 4) : o1;
         d.l = __builtin_amdgcn_raw_buffer_load_b128(m.rin, o0, s, 0);
         d.c = __builtin_amdgcn_raw_buffer_load_b128(m.rin, o1, s, 0);
         d.r = __builtin_amdgcn_raw_buffer_load_b128(m.rin, o2, s, 0);
@@ -285,7 +287,8 @@ __device__ __forceinline__ void load_row(RowData<MODE> &d, const MapGeo &m, int 
         // side words: the one (two) labels left of the quad and right of it;
         // unused (and replaced by the centre labels) at the grid's edges
         const uint32_t oL = (xc > 0) ? o1 - 4u * MODE : o1;
-        const uint32_t oR = (xc + 4 < m.W) ? o1 + 16u : o1;
+        // (step 2: with one label left of them, the centre's last and it)
+        const uint32_t oR = (xc + 3 + MODE < m.W) ? o1 + 16u : (xc + 4 < m.W) ? o1 + 12u : o1;
         d.c = __builtin_amdgcn_raw_buffer_load_b128(m.rin, o1, s, 0);
         if constexpr (MODE == STEP_1) {
             d.l = __builtin_amdgcn_raw_buffer_load_b32(m.rin, oL, s, 0);
@@ -564,6 +567,16 @@ __device__ __forceinline__ void run_of(const RunGeo &g, int u, int &y, int &seg)
     seg = __builtin_amdgcn_readfirstlane(seg);
 }
 
+// the right quad of a lane whose taps cross the row's end by `over` pixels
+// (1 .. 3): r holds the row's last four labels, and the taps off the grid
+// take the centre's
+__device__ __forceinline__ u32x4 end_quad(const u32x4 &r, const u32x4 &c, int over)
+{
+    return u32x4{over == 1 ? r.y : over == 2 ? r.z : over == 3 ? r.w : r.x,
+                 over == 1 ? r.z : over == 2 ? r.w : over == 3 ? c.y : r.y,
+                 over == 1 ? r.w : over >= 2 ? c.z : r.z, over >= 1 ? c.w : r.w};
+}
+
 // One tap row of a run, evaluated as it streams in.  A run's output rows are
 // y + j*k (j = 0..3) and its tap rows y + (i - 1)*k (i = 0..5); tap row I is
 // the down tap of output row I - 2, the centre of I - 1 and the up tap of I.
@@ -586,7 +599,7 @@ template <int MODE, int TAB, int I, bool SHIFT>
 __device__ __forceinline__ void run_row(const RowData<MODE> &R, const SiteTab<TAB> &tab,
                                         const float (&px)[4], const float (&py)[4],
                                         double (&best)[4][4], bool lok, bool rok, bool left,
-                                        bool right, int shift)
+                                        bool right, int shift, int over, bool ragged)
 {
     constexpr int j0 = I - 2 < 0 ? 0 : I - 2;
     constexpr int j1 = I > 3 ? 3 : I;
@@ -617,7 +630,8 @@ __device__ __forceinline__ void run_row(const RowData<MODE> &R, const SiteTab<TA
         for (int q = 0; q < 3; ++q) {
             if (q == 0 && !left && !SHIFT) continue;
             if (q == 2 && !right && !SHIFT) continue;
-            const u32x4 &Q = q == 0 ? R.l : q == 1 ? R.c : R.r;
+            u32x4 Q = q == 0 ? R.l : q == 1 ? R.c : R.r;
+            if (q == 2 && !SHIFT && ragged) Q = end_quad(R.r, R.c, over);
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
                 const uint32_t l = q_el(Q, jj);
@@ -653,8 +667,8 @@ __device__ __forceinline__ void run_row(const RowData<MODE> &R, const SiteTab<TA
             P[0] = lok ? R.l.x : c.x;
             P[1] = lok ? R.l.y : c.y;
             P[2] = c.x; P[3] = c.y; P[4] = c.z; P[5] = c.w;
-            P[6] = rok ? R.r.x : c.z;
-            P[7] = rok ? R.r.y : c.w;
+            P[6] = right ? R.r.x : rok ? R.r.y : c.z;
+            P[7] = right ? R.r.y : c.w;
         }
         float2 edge[SHIFT ? MODE : 1];
         if constexpr (SHIFT) {
@@ -732,10 +746,15 @@ __device__ __forceinline__ void wave_runs(const MapGeo &m, const SiteTab<TAB> &t
             py[j] = __int_as_float(
                 __builtin_amdgcn_readfirstlane(__float_as_int((float)(y + j * k) + 0.5f)));
         const bool lok = xc > 0, rok = xc + 4 < W;
-        bool left = true, right = true;
+        bool left = true, right = true, ragged = false;
+        int over = 0;
         if constexpr (MODE == STEP_ANY) {
             left = __ballot(xc - k >= 0) != 0ull;
-            right = __ballot(xc + 3 + k < W) != 0ull;
+            right = __ballot(xc + k < W) != 0ull;
+            over = xc + k < W ? max(xc + k + 4 - W, 0) : 0;
+            ragged = __ballot(over > 0) != 0ull;
+        } else if constexpr (MODE == STEP_2) {
+            right = xc + 5 < W;
         }
         double best[4][4];
 #pragma unroll
@@ -745,22 +764,22 @@ __device__ __forceinline__ void wave_runs(const MapGeo &m, const SiteTab<TAB> &t
 
         if (y + k < H) load_row<MODE>(R2, m, y + k, seg, lane4);
         if (y - k >= 0) run_row<MODE, TAB, 0, SHIFT>(R0, tab, px, py, best, lok, rok, left, right,
-                                                           shift);
+                                                           shift, over, ragged);
         if (y + 2 * k < H) load_row<MODE>(R0, m, y + 2 * k, seg, lane4);
         if (y < H) run_row<MODE, TAB, 1, SHIFT>(R1, tab, px, py, best, lok, rok, left, right,
-                                                           shift);
+                                                           shift, over, ragged);
         if (y + 3 * k < H) load_row<MODE>(R1, m, y + 3 * k, seg, lane4);
         if (y + k < H) run_row<MODE, TAB, 2, SHIFT>(R2, tab, px, py, best, lok, rok, left, right,
-                                                           shift);
+                                                           shift, over, ragged);
         if (y + 4 * k < H) load_row<MODE>(R2, m, y + 4 * k, seg, lane4);
         if (y + 2 * k < H) run_row<MODE, TAB, 3, SHIFT>(R0, tab, px, py, best, lok, rok, left, right,
-                                                           shift);
+                                                           shift, over, ragged);
         if (un < u_end && yn - k >= 0) load_row<MODE>(R0, m, yn - k, sn, lane4);
         if (y + 3 * k < H) run_row<MODE, TAB, 4, SHIFT>(R1, tab, px, py, best, lok, rok, left, right,
-                                                           shift);
+                                                           shift, over, ragged);
         if (un < u_end && yn < H) load_row<MODE>(R1, m, yn, sn, lane4);
         if (y + 4 * k < H) run_row<MODE, TAB, 5, SHIFT>(R2, tab, px, py, best, lok, rok, left, right,
-                                                           shift);
+                                                           shift, over, ragged);
 
         if (xb < W) {
             const uint32_t o1 = 4u * (uint32_t)xc;
@@ -797,9 +816,8 @@ __device__ __forceinline__ void quad_runs(const MapGeo &m, const SiteTab<TAB> &t
 }
 
 // Single map, site table staged at LDS byte 0 in a static array of ENTRIES
-// float2 (the kernel's only LDS), gathered from global memory when
-// ENTRIES == 0, or split when ENTRIES < 0: the first -ENTRIES sites staged
-// in LDS, the rest gathered.  RUNS picks the work layout: runs down chains
+// float2 (the kernel's only LDS), or split when ENTRIES < 0: the first
+// -ENTRIES sites staged in LDS, the rest gathered.  RUNS picks the work layout: runs down chains
 // of rows, or bands of rows (quad_rows).
 #define JFA_THREADS(E) ((E) > 5120 || (E) < 0 ? 1024 : 256)
 #define JFA_MINB(E) ((E) > 5120 || (E) < 0 ? 1 : 4)
@@ -896,7 +914,7 @@ __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa
         tab.n4 = table_f4;
         tab.base = 0;
         quad_layout<MODE, TAB_LDS0, false>(m, tab, RUNS, pro);
-    } else if constexpr (ENTRIES < 0) {
+    } else {
         __shared__ float4 lds_tab[-ENTRIES / 2];
         // entries 0 .. -ENTRIES - 3 staged, then a zero pair; the rest of the
         // table (from entry -ENTRIES - 2) is gathered
@@ -909,12 +927,6 @@ __global__ __launch_bounds__(JFA_THREADS(ENTRIES), JFA_MINB(ENTRIES)) void k_jfa
         tab.split = 8u * (uint32_t)kept;
         tab.base = 0;
         quad_layout<MODE, TAB_SPLIT, SHIFT>(m, tab, RUNS, pro);
-    } else {
-        SiteTab<TAB_GLOBAL> tab;
-        tab.g = buf_rsrc(sites, 16u * (uint32_t)table_f4);
-        tab.base = 0;
-        tab.n4 = 0;
-        quad_layout<MODE, TAB_GLOBAL, false>(m, tab, RUNS, pro);
     }
 }
 
@@ -1215,6 +1227,7 @@ JfaPlan plan_jfa(int W, int H, int capS, int runs_mask, int blocks_per_cu)
     }
     JfaPlan p;
     p.quad = (W % 4 == 0) && W >= 8;
+    p.ragged = (W % 4 != 0) && W >= 8;
     // sites and the sentinel (index capS), as whole float4 pairs; the site
     // buffer holds capS + 2 entries, so the last pair is always inside it
     p.table_f4 = (capS + 2) / 2;
@@ -1223,7 +1236,7 @@ JfaPlan plan_jfa(int W, int H, int capS, int runs_mask, int blocks_per_cu)
     p.tail_entries = entries <= kLdsEntries[0]   ? kLdsEntries[0]
                      : entries <= kLdsEntries[1] ? kLdsEntries[1]
                                                  : 0;
-    if (p.quad) {
+    if (p.quad || p.ragged) {
         for (int e : kLdsEntries)
             if (entries <= e) { p.lds_entries = e; break; }
         // too large for LDS: the first 20480 entries there, the rest gathered
@@ -1268,7 +1281,7 @@ static void launch_quad(hipStream_t st, const JfaPlan &p, const uint32_t *in, ui
         hipLaunchKernelGGL((k_jfa_quad<MODE, 20480, RUNS>), g, b, 0, st, in, out, sites,
                            p.table_f4, W, H, step, clear, none, nclear, rstep, stop);
         break;
-    case -20480:
+    default:      // -20480
         // whole 256-pixel segments, and a lane's neighbour positions within
         // the wave on one side at least (step 128: half of them)
         if (RUNS && W % 256 == 0 && step <= 128)
@@ -1277,10 +1290,6 @@ static void launch_quad(hipStream_t st, const JfaPlan &p, const uint32_t *in, ui
         else
             hipLaunchKernelGGL((k_jfa_quad<MODE, -20480, RUNS>), g, b, 0, st, in, out, sites,
                                p.table_f4, W, H, step, clear, none, nclear, rstep, stop);
-        break;
-    default:
-        hipLaunchKernelGGL((k_jfa_quad<MODE, 0, RUNS>), g, b, 0, st, in, out, sites, p.table_f4, W,
-                           H, step, clear, none, nclear, rstep, stop);
         break;
     }
 }
@@ -1293,12 +1302,24 @@ static void launch_quad(hipStream_t st, const JfaPlan &p, const uint32_t *in, ui
 // 6510 iter/s.  Runs need work for every wave, though: a run is four rows of
 // a 256-pixel segment, so on small grids (512^2: 256 runs at step 1 for 1024
 // waves) bands keep more waves busy (15 870 against 13 170 iter/s with runs
-// whenever they fill a quarter of the waves).
+// whenever they fill a quarter of the waves).  Where the width is no multiple
+// of four the other side is the kernel of one pixel per lane, which looks up
+// nine sites per pixel from L1: runs from 1.5 per CU (50 iterations with every
+// pass dense, one pixel per lane -> runs: 509 x 511 / 17339 sites, 256 runs,
+// 3.9 -> 4.8 ms; 766 x 509 / 2599, 384 runs, 3.57 -> 3.43; 767 x 767 / 9804,
+// 576, 6.9 -> 5.0; 1533 x 1021 / 17391 13.5 -> 6.0; 2050 x 1500 / 12300, the
+// first five passes by the lattice, 19.8 -> 6.7; 3001 x 2000 / 20006, 43
+// iterations, 32.4 -> 8.3).
 static bool use_runs(const JfaPlan &p, int W, int H, int step)
 {
+    if (!p.quad && !p.ragged) return false;
+    // (a ragged row's last quad, which starts at W - 4, must not have its left
+    // taps partly off the grid)
+    if (p.ragged && step > W - 4 && step < W) return false;
     if (p.runs_mask >= 0) return (p.runs_mask >> __builtin_ctz((unsigned)step)) & 1;
     const long n = (H + step - 1) / step;
     const long runs = (long)std::min(step, H) * ((n + 3) / 4) * ((W + 255) / 256);
+    if (p.ragged) return 2 * runs >= 3 * (long)g_num_cu;
     return runs >= (long)p.grid * (p.threads / 64);
 }
 
@@ -1306,11 +1327,10 @@ int jfa_runs_mask(const JfaPlan &p, int W, int H)
 {
     // steps 1, 2, 4 .. the first step (the largest power of two below max(W, H))
     int mask = 0;
-    if (p.quad)
-        for (int k = 0;; ++k) {
-            if (use_runs(p, W, H, 1 << k)) mask |= 1 << k;
-            if ((2 << k) >= std::max(W, H)) break;
-        }
+    for (int k = 0;; ++k) {
+        if (use_runs(p, W, H, 1 << k)) mask |= 1 << k;
+        if ((2 << k) >= std::max(W, H)) break;
+    }
     return mask;
 }
 
@@ -1318,15 +1338,13 @@ void launch_jfa_pass(hipStream_t st, const JfaPlan &p, const uint32_t *in, uint3
                      const float2 *sites, int W, int H, int step, uint32_t *clear, uint32_t none,
                      int nclear, int rstep, const int *stop)
 {
-    if (p.quad) {
-        const bool runs = use_runs(p, W, H, step);
+    const bool runs = use_runs(p, W, H, step);
+    if (p.quad || runs) {
         if (step == 1 && runs)
             launch_quad<STEP_1, true>(st, p, in, out, sites, W, H, step, clear, none, nclear, rstep, stop);
         else if (step == 1)
             launch_quad<STEP_1, false>(st, p, in, out, sites, W, H, step, clear, none, nclear, rstep, stop);
-        // (step 2 with the all-global table keeps bands: six buffers of it
-        // spill)
-        else if (step == 2 && runs && p.lds_entries != 0)
+        else if (step == 2 && runs)
             launch_quad<STEP_2, true>(st, p, in, out, sites, W, H, step, clear, none, nclear, rstep, stop);
         else if (step == 2) launch_quad<STEP_2, false>(st, p, in, out, sites, W, H, step, clear, none, nclear, rstep, stop);
         else if (runs)
