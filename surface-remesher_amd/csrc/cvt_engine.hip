@@ -67,29 +67,26 @@ int Ctx::enqueue_moments() { return launch_moments_on(this, labels_map()); }
 static int launch_moments_on(Ctx *c, const uint32_t *lab)
 {
     const float rs = (float)ldexp(1.0, -c->rho_exp);
-    dim3 grid(c->tilesX * c->tilesY), block(c->tile >= 64 ? 512 : 256);
+    const dim3 grid(c->tilesX * c->tilesY);
+    // tiles that are all resident at three workgroups of eight waves per CU
+    const bool ahead = grid.x <= 768u;
+#define CVT_MOMENTS(T, NW, AHEAD)                                                                 \
+    hipLaunchKernelGGL((k_moments<T, NW, AHEAD>), grid, dim3(64 * NW), 0, c->stream, lab, c->rho, \
+                       c->sites, c->S, c->W, c->H, rs, c->tilesX, c->tilesY, c->slots,            \
+                       (long)c->capS, c->ovf, c->ovf_cap, c->ovf_head, c->dflags, c->dstate)
     switch (c->tile) {
-    case 32:
-        hipLaunchKernelGGL(k_moments<32>, grid, block, 0, c->stream, lab, c->rho, c->sites, c->S,
-                           c->W, c->H, rs, c->tilesX, c->tilesY, c->slots, (long)c->capS, c->ovf, c->ovf_cap,
-                           c->ovf_head, c->dflags, c->dstate);
-        break;
+    case 32: CVT_MOMENTS(32, 4, false); break;
     case 64:
-        hipLaunchKernelGGL(k_moments<64>, grid, block, 0, c->stream, lab, c->rho, c->sites, c->S,
-                           c->W, c->H, rs, c->tilesX, c->tilesY, c->slots, (long)c->capS, c->ovf, c->ovf_cap,
-                           c->ovf_head, c->dflags, c->dstate);
+        if (ahead) CVT_MOMENTS(64, 8, true);
+        else CVT_MOMENTS(64, 8, false);
         break;
     case 128:
-        hipLaunchKernelGGL(k_moments<128>, grid, block, 0, c->stream, lab, c->rho, c->sites, c->S,
-                           c->W, c->H, rs, c->tilesX, c->tilesY, c->slots, (long)c->capS, c->ovf, c->ovf_cap,
-                           c->ovf_head, c->dflags, c->dstate);
+        if (ahead) CVT_MOMENTS(128, 8, true);
+        else CVT_MOMENTS(128, 8, false);
         break;
-    default:
-        hipLaunchKernelGGL(k_moments<256>, grid, block, 0, c->stream, lab, c->rho, c->sites, c->S,
-                           c->W, c->H, rs, c->tilesX, c->tilesY, c->slots, (long)c->capS, c->ovf, c->ovf_cap,
-                           c->ovf_head, c->dflags, c->dstate);
-        break;
+    default: CVT_MOMENTS(256, 8, true); break;   // (two workgroups per CU by their LDS)
     }
+#undef CVT_MOMENTS
     return hipGetLastError() == hipSuccess ? CVT_OK : fail(CVT_ERR_HIP, "moment launch failed");
 }
 

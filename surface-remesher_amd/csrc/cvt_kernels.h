@@ -174,10 +174,10 @@ struct TailRec {
 
 // LDS of one tile: a hash of HC labels (a power of two <= CVT_HASH_CAP) with
 // their fixed-point sums, and the waves' run-end queues
-template <int HC> struct TileLds {
+template <int HC, int NW> struct TileLds {
     int keys[HC];
     unsigned long long acc[HC][4];
-    TailRec q[8][CVT_TAILQ];   // one queue per wave, up to 8 waves
+    TailRec q[NW][CVT_TAILQ];  // one queue per wave
     int full;
 };
 
@@ -187,8 +187,8 @@ template <int T> struct TileHash {
     static constexpr int HC = T == 64 ? 256 : T == 128 ? 512 : CVT_HASH_CAP;
 };
 
-template <int HC>
-__device__ __forceinline__ void tile_lds_init(TileLds<HC> &L)
+template <int HC, int NW>
+__device__ __forceinline__ void tile_lds_init(TileLds<HC, NW> &L)
 {
     for (int j = threadIdx.x; j < HC; j += blockDim.x) {
         L.keys[j] = -1;
@@ -214,9 +214,13 @@ struct MomLoad {
 // map.  A wave's first label and density loads are issued before the hash is
 // cleared.  stop (may be null): the stop word of cvt_lloyd_until, read with
 // those loads; when it is set the routine returns true before adding
-// anything.
-template <int SEG, int HC>
-__device__ __forceinline__ bool tile_moments(TileLds<HC> &L, const uint32_t *__restrict__ lab,
+// anything.  AHEAD: the next step's pixels are loaded while a step is
+// evaluated and a queue is drained when it is full and at the end, not after
+// every step (fuller drains; the sums are integers, so the order does not
+// matter); it takes 68 registers instead of 58, seven waves per SIMD instead
+// of eight.
+template <int SEG, bool AHEAD, int HC, int NW>
+__device__ __forceinline__ bool tile_moments(TileLds<HC, NW> &L, const uint32_t *__restrict__ lab,
                                              const float *__restrict__ rho,
                                              const float2 *__restrict__ sites, int key_base,
                                              int S, int W, int H, float rho_scale, int tx0,
@@ -271,9 +275,48 @@ __device__ __forceinline__ bool tile_moments(TileLds<HC> &L, const uint32_t *__r
     tile_lds_init(L);
     if (halt) return true;
 
-    const int nw = blockDim.x >> 6;
-    for (int g = wave; g < steps; g += nw) {
-        if (g > wave) step_load(g, ld);
+    int base = 0;                            // records in the wave's queue
+    auto drain = [&](int nrec) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // one lane per record: site-relative fp64 sums into the hash
+        for (int e = lane; e < nrec; e += 64) {
+            const TailRec t = q[e];
+            const float2 sv = sites[t.key];
+            const double A = t.a, B = t.b, Cc = t.c;
+            const double ox = ((double)(t.xy & 0xffff) + 0.5) - (double)sv.x;
+            const double oy = ((double)(t.xy >> 16) + 0.5) - (double)sv.y;
+            const double DX = B + A * ox;
+            const double DY = A * oy;
+            const double E = Cc + 2.0 * ox * B + A * (ox * ox + oy * oy);
+            const unsigned hsh = ((unsigned)t.key * 2654435761u) >> (32 - __builtin_ctz(HC));
+            int slot = -1;
+            for (int probe = 0; probe < HC; ++probe) {
+                const int h = (hsh + probe) & (HC - 1);
+                const int old = atomicCAS(&L.keys[h], -1, t.key);
+                if (old == -1 || old == t.key) { slot = h; break; }
+            }
+            if (slot >= 0) {
+                atomicAdd(&L.acc[slot][0], (unsigned long long)cvt_fix(A, MOM_FW));
+                atomicAdd(&L.acc[slot][1], (unsigned long long)cvt_fix(DX, MOM_FX));
+                atomicAdd(&L.acc[slot][2], (unsigned long long)cvt_fix(DY, MOM_FX));
+                atomicAdd(&L.acc[slot][3], (unsigned long long)cvt_fix(E, MOM_FE));
+            } else {
+                L.full = 1;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    for (int g = wave; g < steps; g += NW) {
+        MomLoad next;
+        if constexpr (AHEAD) {
+            if (g + NW < steps) step_load(g + NW, next);
+        } else {
+            if (g > wave) step_load(g, ld);
+        }
         int x0, y;
         step_pos(g, x0, y);
         int key[4];
@@ -353,42 +396,7 @@ __device__ __forceinline__ bool tile_moments(TileLds<HC> &L, const uint32_t *__r
         tl[1] = key[2] != key[1];
         tl[2] = key[3] != key[2];
         tl[3] = (seg_lane == SL - 1) || (knext != key[3]);
-        auto drain = [&](int nrec) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // one lane per record: site-relative fp64 sums into the hash
-            for (int e = lane; e < nrec; e += 64) {
-                const TailRec t = q[e];
-                const float2 sv = sites[t.key];
-                const double A = t.a, B = t.b, Cc = t.c;
-                const double ox = ((double)(t.xy & 0xffff) + 0.5) - (double)sv.x;
-                const double oy = ((double)(t.xy >> 16) + 0.5) - (double)sv.y;
-                const double DX = B + A * ox;
-                const double DY = A * oy;
-                const double E = Cc + 2.0 * ox * B + A * (ox * ox + oy * oy);
-                const unsigned hsh = ((unsigned)t.key * 2654435761u) >> (32 - __builtin_ctz(HC));
-                int slot = -1;
-                for (int probe = 0; probe < HC; ++probe) {
-                    const int h = (hsh + probe) & (HC - 1);
-                    const int old = atomicCAS(&L.keys[h], -1, t.key);
-                    if (old == -1 || old == t.key) { slot = h; break; }
-                }
-                if (slot >= 0) {
-                    atomicAdd(&L.acc[slot][0], (unsigned long long)cvt_fix(A, MOM_FW));
-                    atomicAdd(&L.acc[slot][1], (unsigned long long)cvt_fix(DX, MOM_FX));
-                    atomicAdd(&L.acc[slot][2], (unsigned long long)cvt_fix(DY, MOM_FX));
-                    atomicAdd(&L.acc[slot][3], (unsigned long long)cvt_fix(E, MOM_FE));
-                } else {
-                    L.full = 1;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        };
         // queue the run ends: records ordered by (j, lane)
-        int base = 0;
         bool first_piece = true;                 // no head yet in this lane at <= j
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -413,8 +421,14 @@ __device__ __forceinline__ bool tile_moments(TileLds<HC> &L, const uint32_t *__r
             }
             base += __popcll(bal);
         }
-        drain(base);
+        if constexpr (AHEAD) {
+            ld = next;
+        } else {
+            drain(base);
+            base = 0;
+        }
     }
+    if constexpr (AHEAD) drain(base);
     return false;
 }
 
@@ -423,8 +437,8 @@ __device__ __forceinline__ bool tile_moments(TileLds<HC> &L, const uint32_t *__r
 // its 3 x 3 window, tagged with the epoch; otherwise a record is chained to
 // the site (integer atomics only to allocate records).  site_off: index of
 // this map's first site in slots / ovf_head / sites.
-template <int HC>
-__device__ __forceinline__ void tile_flush(TileLds<HC> &L, const float2 *__restrict__ sites,
+template <int HC, int NW>
+__device__ __forceinline__ void tile_flush(TileLds<HC, NW> &L, const float2 *__restrict__ sites,
                                            int site_off, int T, int tX, int tY, int tilesX,
                                            int tilesY, int epoch, Slot *__restrict__ slots, long nrows,
                                            OvfRec *__restrict__ ovf, int ovf_cap,
@@ -466,18 +480,22 @@ __device__ __forceinline__ void tile_flush(TileLds<HC> &L, const float2 *__restr
 // moments (reference replacement for pbaCVDComputeCentroid + the energy
 // texture, source/gcvt.cu:562-732, :788-802): one workgroup per T x T tile,
 // eight waves for tiles of 64 pixels or more (four for 32: a 32-pixel tile
-// has four wave steps)
-template <int T>
-static __global__ __launch_bounds__(512) void k_moments(
+// has four wave steps).  Bound by vector instructions (about 350 per wave step
+// of 256 pixels) where every SIMD has eight waves, by a wave's chain of steps
+// on fewer: there AHEAD (512^2 / 1024 sites 5.8 -> 5.1 us; at 2048^2 / 16384
+// and 4096^2 / 65536, where the eighth wave counts, 11.2 -> 12.8 and
+// 32.5 -> 34.9: not taken).
+template <int T, int NW, bool AHEAD>
+static __global__ __launch_bounds__(64 * NW) void k_moments(
     const uint32_t *__restrict__ lab, const float *__restrict__ rho,
     const float2 *__restrict__ sites, int S, int W, int H, float rho_scale, int tilesX,
     int tilesY, Slot *__restrict__ slots, long nrows, OvfRec *__restrict__ ovf, int ovf_cap,
     int *__restrict__ ovf_head, int *__restrict__ dflags, int *__restrict__ dstate)
 {
-    __shared__ TileLds<TileHash<T>::HC> L;
+    __shared__ TileLds<TileHash<T>::HC, NW> L;
     const int tile = blockIdx.x;
     const int tX = tile % tilesX, tY = tile / tilesX;
-    if (tile_moments<(T < 64 ? T : 64)>(L, lab, rho, sites, 0, S, W, H, rho_scale, tX * T, tY * T,
+    if (tile_moments<(T < 64 ? T : 64), AHEAD>(L, lab, rho, sites, 0, S, W, H, rho_scale, tX * T, tY * T,
                                         T, dstate + ST_STOP))
         return;   // a stop rule held (cvt_lloyd_until)
     tile_flush(L, sites, 0, T, tX, tY, tilesX, tilesY, dstate[ST_EPOCH], slots, nrows, ovf, ovf_cap,
