@@ -480,7 +480,7 @@ __device__ __forceinline__ void tile_flush(TileLds<HC, NW> &L, const float2 *__r
 // moments (reference replacement for pbaCVDComputeCentroid + the energy
 // texture, source/gcvt.cu:562-732, :788-802): one workgroup per T x T tile,
 // eight waves for tiles of 64 pixels or more (four for 32: a 32-pixel tile
-// has four wave steps).  Bound by vector instructions (about 350 per wave step
+// has four wave steps).  Bound by vector instructions (about 270 per wave step
 // of 256 pixels) where every SIMD has eight waves, by a wave's chain of steps
 // on fewer: there AHEAD (512^2 / 1024 sites 5.8 -> 5.1 us; at 2048^2 / 16384
 // and 4096^2 / 65536, where the eighth wave counts, 11.2 -> 12.8 and
