@@ -360,7 +360,7 @@ unsigned Batch::pass_modes(int k) const
 
 void Batch::enqueue_jfa()
 {
-    launch_jfa_batch_lattice(stream, d_patch, d_lat_patch, (int)lat_patch.size(), seed, first, lab0,
+    launch_jfa_batch_lattice(stream, d_patch, d_lat_patch, (int)lat_patch.size(), seed, first,
                              sites);
     for (int k = 0; k < pmax; ++k) {
         const unsigned modes = pass_modes(k);

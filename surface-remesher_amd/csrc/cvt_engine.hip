@@ -177,12 +177,9 @@ int Ctx::enqueue_jfa(hipEvent_t after_first)
     const int tail = use_tail ? jfa_tail_passes(jplan, np, done) : 0;
     int k = 0;
     if (done) {
-        // the JFA's last launch writes the map whose parity is the count of
-        // launches that follow; the other one is free
-        const int after = tail ? np - done - tail + 1 : np - done;
         first_clean = false;
-        launch_jfa_lattice(stream, seed, first, lab[after & 1], sites, W, H, none(),
-                           dstate + ST_STOP, blockpart, dstate, &fa);
+        launch_jfa_lattice(stream, seed, first, sites, W, H, none(), dstate + ST_STOP, blockpart,
+                           dstate, &fa);
         if (after_first) hipEventRecord(after_first, stream);
         in = first;
         step >>= done;

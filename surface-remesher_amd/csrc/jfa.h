@@ -62,11 +62,10 @@ void launch_jfa_tail(hipStream_t st, const JfaPlan &plan, int passes, const uint
 // The first passes of a JFA in one launch over residue classes
 // (jfa_lattice.hip): how many a map of W x H pixels and S sites takes that way
 // (0: none), and the launch, which reads the seed map and writes the map after
-// those passes to `out`, every pixel of it.  scratch: a map that nothing else
-// reads or writes meanwhile.  The seed map is left as it is.  stop, blockpart,
-// dstate and fa as in launch_jfa_seed_pass.
+// those passes to `out`, every pixel of it.  The seed map is left as it is.
+// stop, blockpart, dstate and fa as in launch_jfa_seed_pass.
 int jfa_lattice_passes(int W, int H, int S);
-void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out, uint32_t *scratch,
+void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out,
                         const float2 *sites, int W, int H, uint32_t none,
                         const int *stop = nullptr, const double *blockpart = nullptr,
                         int *dstate = nullptr, const FinalArgs *fa = nullptr);
@@ -133,7 +132,7 @@ void launch_jfa_batch_seeds(hipStream_t st, const BatchPatch *patches, const int
 int jfa_batch_lattice_passes(int W, int H, int S);
 int jfa_batch_lattice_groups(int W, int H);
 void launch_jfa_batch_lattice(hipStream_t st, const BatchPatch *patches, const int *group_patch,
-                              int groups, const uint32_t *seed, uint32_t *first, uint32_t *scratch,
+                              int groups, const uint32_t *seed, uint32_t *first,
                               const float2 *sites);
 
 }  // namespace cvt

@@ -174,19 +174,28 @@ __device__ __forceinline__ void lat_nearest(uint32_t (&m)[8], uint32_t seeds, fl
 }
 
 // A class with more seeds than the mask path takes (sites in step with the
-// class stride; otherwise one class in 10^5 at 200 pixels per site): its five
-// passes through memory by the whole workgroup, one dense evaluation per
-// lattice point.  The class's pixels of the maps are this workgroup's alone.
-// Passes alternate between out and scratch and end in out.
-__device__ __forceinline__ void lattice_class_dense(const uint32_t *seed, uint32_t *out,
-                                                    uint32_t *scratch, const float2 *sites, int W,
-                                                    int s, int x0, int y0, int nx, int ny)
+// class stride, or by chance: see jfa_lattice_passes): its five passes by the
+// whole workgroup, one dense evaluation per lattice point, between two label
+// arrays in the LDS of the masks (which the caller is done with).  1024^2 /
+// 6512 sites, where a launch meets such a class most of the time: 50
+// iterations 5.10 ms with these passes through the maps, 4.16 in LDS.
+template <int NW>
+__device__ __forceinline__ void lattice_class_dense(LatLds<NW> &L, const uint32_t *seed,
+                                                    const __amdgpu_buffer_rsrc_t rout,
+                                                    const float2 *sites, int W, int s, int x0,
+                                                    int y0, int nx, int ny)
 {
+    static_assert(sizeof(L.mask) >= 2 * kLat * kLat * sizeof(uint32_t), "two label arrays");
     const char *sb = reinterpret_cast<const char *>(sites);
+    uint32_t *lab[2] = {L.mask, L.mask + kLat * kLat};
+    __syncthreads();
+    for (int q = threadIdx.x; q < nx * ny; q += blockDim.x)
+        lab[0][q] = seed[(size_t)(y0 + s * (q / nx)) * W + (x0 + s * (q % nx))];
+    __syncthreads();
 #pragma unroll 1
     for (int p = 0; p < kLatPasses; ++p) {
-        const uint32_t *in = p == 0 ? seed : (p & 1) ? out : scratch;
-        uint32_t *dst = (p & 1) ? scratch : out;
+        const uint32_t *in = lab[p & 1];
+        uint32_t *dst = lab[~p & 1];
         const int t = 16 >> p;
 #pragma unroll 1
         for (int q = threadIdx.x; q < nx * ny; q += blockDim.x) {
@@ -199,8 +208,7 @@ __device__ __forceinline__ void lattice_class_dense(const uint32_t *seed, uint32
                 int jj = j + (a / 3 - 1) * t, ii = i + (a % 3 - 1) * t;
                 jj = jj < 0 || jj >= ny ? j : jj;
                 ii = ii < 0 || ii >= nx ? i : ii;
-                l[a] = __hip_atomic_load(in + (size_t)(y0 + s * jj) * W + (x0 + s * ii),
-                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                l[a] = in[nx * jj + ii];
             }
             double best = __hiloint2double(0x7f800000, -1);
 #pragma unroll
@@ -210,11 +218,14 @@ __device__ __forceinline__ void lattice_class_dense(const uint32_t *seed, uint32
                 const float d = __builtin_fmaf(dy, dy, dx * dx);
                 best = __builtin_fmin(best, __hiloint2double(__float_as_int(d), (int)l[a]));
             }
-            __hip_atomic_store(dst + (size_t)(y0 + s * j) * W + (x0 + s * i),
-                               (uint32_t)__double2loint(best), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t lb = (uint32_t)__double2loint(best);
+            if (p < kLatPasses - 1)
+                dst[q] = lb;
+            else
+                __builtin_amdgcn_raw_buffer_store_b32(
+                    lb, rout, 4u * ((uint32_t)(y0 + s * j) * (uint32_t)W + (uint32_t)(x0 + s * i)),
+                    0, 16);
         }
-        __threadfence();
         __syncthreads();
     }
 }
@@ -222,7 +233,7 @@ __device__ __forceinline__ void lattice_class_dense(const uint32_t *seed, uint32
 // The classes (rx0 .. rx0 + NW - 1, ry) modulo s of one W x H map.
 template <int NW>
 __device__ __forceinline__ void lattice_group(LatLds<NW> &L, const uint32_t *seed, uint32_t *out,
-                                              uint32_t *scratch, const float2 *sites, int W, int H,
+                                              const float2 *sites, int W, int H,
                                               int s, int rx0, int ry, uint32_t none,
                                               const int *stop)
 {
@@ -416,7 +427,7 @@ __device__ __forceinline__ void lattice_group(LatLds<NW> &L, const uint32_t *see
     for (int cc = 0; cc < NW; ++cc) {
         const int xc = rx0 + cc;
         if (L.cnt[cc] > kLatCap)       // (its pixels lie on the grid: xc < W)
-            lattice_class_dense(seed, out, scratch, sites, W, s, xc, ry, (W - xc + s - 1) / s, ny);
+            lattice_class_dense<NW>(L, seed, rout, sites, W, s, xc, ry, (W - xc + s - 1) / s, ny);
     }
 }
 
@@ -430,8 +441,8 @@ __device__ __forceinline__ int lattice_unit(int b, int n)
 
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_jfa_lattice(
-    const uint32_t *seed, uint32_t *out, uint32_t *scratch, const float2 *__restrict__ sites, int W,
-    int H, int s, uint32_t none, const int *__restrict__ stop, int fin,
+    const uint32_t *seed, uint32_t *out, const float2 *__restrict__ sites, int W, int H,
+    int s, uint32_t none, const int *__restrict__ stop, int fin,
     const double *__restrict__ blockpart, int *__restrict__ dstate, FinalArgs fa)
 {
     __shared__ LatLds<NW> L;
@@ -446,14 +457,14 @@ __global__ __launch_bounds__(64 * NW) void k_jfa_lattice(
     const int gx = s / NW;
     const int ry = u / gx, rx0 = NW * (u - gx * ry);
     if (rx0 >= W) return;
-    lattice_group<NW>(L, seed, out, scratch, sites, W, H, s, rx0, ry, none, stop);
+    lattice_group<NW>(L, seed, out, sites, W, H, s, rx0, ry, none, stop);
 }
 
 static constexpr int kBatchNW = 8;   // classes per workgroup of the batched launch
 
 __global__ __launch_bounds__(64 * kBatchNW) void k_jfa_batch_lattice(
     const BatchPatch *__restrict__ patches, const int *__restrict__ group_patch,
-    const uint32_t *seed, uint32_t *first, uint32_t *scratch, const float2 *__restrict__ sites)
+    const uint32_t *seed, uint32_t *first, const float2 *__restrict__ sites)
 {
     __shared__ LatLds<kBatchNW> L;
     const BatchPatch P = patches[group_patch[blockIdx.x]];
@@ -461,8 +472,8 @@ __global__ __launch_bounds__(64 * kBatchNW) void k_jfa_batch_lattice(
     const int u = lattice_unit((int)blockIdx.x - P.lat_off, gx * s);
     const int ry = u / gx, rx0 = kBatchNW * (u - gx * ry);
     if (rx0 >= P.W) return;
-    lattice_group<kBatchNW>(L, seed + P.pix_off, first + P.pix_off, scratch + P.pix_off, sites,
-                            P.W, P.H, s, rx0, ry, 8u * (uint32_t)(P.site_off + P.cap), nullptr);
+    lattice_group<kBatchNW>(L, seed + P.pix_off, first + P.pix_off, sites, P.W, P.H, s, rx0, ry,
+                            8u * (uint32_t)(P.site_off + P.cap), nullptr);
 }
 
 static int first_step(int W, int H)
@@ -478,13 +489,17 @@ int jfa_lattice_passes(int W, int H, int S)
     // steps of 64 and more (a group of four classes is a quad of pixels), a
     // shorter side of at least half the first step (a class is 32 points long
     // and a wave's work does not shrink with its width), and few enough seeds
-    // per class: at 200 pixels per site a class of 1024 points holds 5.1 on
-    // average, and more than the mask path's 16 once in 4e4 classes
+    // per class: with 8 on average one class in 300 holds more than the mask
+    // path's 16, and one or more of them add about 6 us to the launch.  Measured
+    // against the dense passes, 50 iterations: 512^2 / 2016 sites (7.9 per
+    // class) 2.50 -> 2.42 ms, / 1638 (6.4) 2.46 -> 2.03, 2048^2 / 32263 (7.9)
+    // 11.1 -> 9.4, / 26052 (6.4) 10.1 -> 8.2, 1100^2 / 26888 (6.6) 10.4 -> 7.9.
     if (first < 64 || 2 * std::min(W, H) < first) return 0;
-    return (long)W * H >= 200L * S ? kLatPasses : 0;
+    const long classes = (long)(first / 16) * (first / 16);
+    return S <= 8 * classes ? kLatPasses : 0;
 }
 
-void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out, uint32_t *scratch,
+void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out,
                         const float2 *sites, int W, int H, uint32_t none, const int *stop,
                         const double *blockpart, int *dstate, const FinalArgs *fa)
 {
@@ -492,7 +507,7 @@ void launch_jfa_lattice(hipStream_t st, const uint32_t *seed, uint32_t *out, uin
     const FinalArgs f = fa ? *fa : FinalArgs();
 #define CVT_LATTICE(NW)                                                                        \
     hipLaunchKernelGGL(k_jfa_lattice<NW>, dim3(s / NW * s + fin), dim3(64 * NW), 0, st, seed, \
-                       out, scratch, sites, W, H, s, none, stop, fin, blockpart, dstate, f)
+                       out, sites, W, H, s, none, stop, fin, blockpart, dstate, f)
     // s^2 classes, one per wave.  Wide groups write whole cache lines, narrow
     // ones spread the waves over the CUs and wait for fewer others.  Measured
     // back to back with 4 / 8 / 16 waves: 512^2 11.8 / 14.2 / 20.0 us, 1024^2
@@ -519,12 +534,11 @@ int jfa_batch_lattice_groups(int W, int H)
 }
 
 void launch_jfa_batch_lattice(hipStream_t st, const BatchPatch *patches, const int *group_patch,
-                              int groups, const uint32_t *seed, uint32_t *first, uint32_t *scratch,
-                              const float2 *sites)
+                              int groups, const uint32_t *seed, uint32_t *first, const float2 *sites)
 {
     if (groups > 0)
         hipLaunchKernelGGL(k_jfa_batch_lattice, dim3(groups), dim3(64 * kBatchNW), 0, st, patches,
-                           group_patch, seed, first, scratch, sites);
+                           group_patch, seed, first, sites);
 }
 
 }  // namespace cvt

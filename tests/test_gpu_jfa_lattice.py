@@ -30,6 +30,11 @@ def random_sites(seed, W, H, S):
     (2048, 1030, 10000), # sixteen-wave groups, ragged rows
     (4096, 2051, 9000),  # eight-wave groups
     (512, 512, 1),       # one site
+    (512, 512, 2048),    # eight sites per class, the most that take it; dense classes likely
+    (1024, 1024, 8192),
+    (1100, 700, 32768),  # the same on classes of 18 x 11 points
+    (2048, 2048, 32768),
+    (2047, 2048, 32769), # one site too many
 ])
 def test_labels_equal_oracle(gpu, orc, W, H, S):
     xy = random_sites(W + H + S, W, H, S)

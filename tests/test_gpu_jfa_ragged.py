@@ -21,6 +21,9 @@ pytestmark = pytest.mark.gpu
     (765, 512, 18000),      # the fewest runs that are taken (1.5 per CU), a table of 160 KB
     (67, 8191, 900),        # step 64 (of the row's last quad) between W - 4 and W
     (9, 8191, 300),         # the smallest width
+    (2049, 2051, 140000),   # more than eight sites per class of the first passes: every step dense,
+                            # step 2048 between W - 4 and W
+    (1025, 1024, 40000),
 ])
 def test_labels_equal_oracle(gpu, orc, W, H, S):
     xy = random_sites(W + H + S, W, H, S)
