@@ -28,3 +28,17 @@ pytestmark = pytest.mark.gpu
 def test_labels_equal_oracle(gpu, orc, W, H, S):
     xy = random_sites(W + H + S, W, H, S)
     assert np.array_equal(labels(W, H, xy), orc.jfa(W, H, xy))
+
+
+@pytest.mark.parametrize("W,H,S", [(9, 12, 5), (11, 70, 40), (13, 40, 20), (98, 77, 150),
+                                   (259, 130, 5000), (67, 300, 30000)])
+def test_forced_runs_equal_oracle(gpu, orc, W, H, S):
+    """runs asked for at every step, on grids of any size"""
+    import cvtamd
+    xy = random_sites(W + H + S, W, H, S)
+    with cvtamd.Engine(W, H, S) as e:
+        e.jfa_shape = (1 << 13) - 1, 0
+        e.set_sites(xy)
+        e.voronoi()
+        lab = e.labels()
+    assert np.array_equal(lab, orc.jfa(W, H, xy))
