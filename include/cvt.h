@@ -195,7 +195,8 @@ int cvt_ref_init_sites(int16_t *voronoi, const float *density, const uint8_t *ma
  * (x*scale, y*scale) is the float64 barycentric interpolation of weight over
  * the first triangle (index order) containing it, 0 outside every triangle.
  * points holds num_point (x, y) pairs already shifted to the origin,
- * triangle 3 vertex indices per triangle. */
+ * triangle 3 vertex indices per triangle.  CVT_ERR_CAPACITY where the
+ * triangles' boxes meet 16x16-pixel tiles 2^31 times or more. */
 int cvt_rasterize(const double *points, const double *weight, int num_point, const int *triangle,
                   int num_tri, float *density, double scale, int n);
 /* cvt_rasterize for callers that cannot allocate device memory (code under
@@ -239,6 +240,8 @@ int cvt_extract_points(const int16_t *voronoi, const uint8_t *mask, int n, doubl
  * (1 - w1 - w2, w1, w2 as recover() stores them; -1 where face is -1); with
  * p3 [nv][3] (the 3D vertices), out3 [nq][3] receives sum_j w_j p3[v_j]
  * summed in j order from 0.0 (source/recover.h:117-123; 0 where face is -1).
+ * CVT_ERR_CAPACITY where the faces' boxes meet the search grid's bins (about
+ * two faces each, at most 1024 x 1024) 2^31 times or more.
  * Host or device pointers; the call returns when the results are written. */
 int cvt_locate_points(const double *uv, const double *p3, int nv, const int *tri, int nf,
                       const double *q, int nq, int *face, double *w, double *out3);

@@ -114,24 +114,27 @@ struct FaceXY {
     double x1, y1, x2, y2, x3, y3;
 };
 
-// per face: index validation, the corner record, the conservative bin box
-// and its (face, bin) pairs counted per bin.  Faces to test everywhere are
-// appended to alw in any order (a query keeps the lowest-index hit).
-// status: {a face indexes outside, pairs beyond the list, faces in alw}
-__global__ void k_face_boxes(const double *__restrict__ uv, int nv, const int *__restrict__ tri,
-                             int nf, const unsigned long long *__restrict__ bb, int G,
-                             FaceXY *__restrict__ xy, FaceBox *__restrict__ box,
-                             int *__restrict__ alw, int *__restrict__ count,
-                             int *__restrict__ status)
+// status: {a face indexes outside, pairs beyond the list, faces in alw, -, and
+// the (face, bin) pairs in 64 bits}
+constexpr int kStatus = 8;
+__device__ __forceinline__ unsigned long long *pair_total(int *status)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nf) return;
+    return reinterpret_cast<unsigned long long *>(status + 4);
+}
+
+// face i: index validation, the corner record and the conservative bin box.
+// Faces to test everywhere are appended to alw in any order (a query keeps the
+// lowest-index hit).
+__device__ __forceinline__ FaceBox face_box(const double *__restrict__ uv, int nv,
+                                            const int *__restrict__ tri, int i, const BinGrid &g,
+                                            FaceXY *__restrict__ xy, int *__restrict__ alw,
+                                            int *__restrict__ status)
+{
     const int a = tri[3 * i], b = tri[3 * i + 1], c = tri[3 * i + 2];
     FaceBox bx = {1, 0, 1, 0};
     if ((unsigned)a >= (unsigned)nv || (unsigned)b >= (unsigned)nv || (unsigned)c >= (unsigned)nv) {
         status[0] = 1;
-        box[i] = bx;
-        return;
+        return bx;
     }
     const double x1 = uv[2 * a], y1 = uv[2 * a + 1];
     const double x2 = uv[2 * b], y2 = uv[2 * b + 1];
@@ -141,13 +144,11 @@ __global__ void k_face_boxes(const double *__restrict__ uv, int nv, const int *_
     const double d00 = v0x * v0x + v0y * v0y, d11 = v1x * v1x + v1y * v1y;
     const double d01 = v0x * v1x + v0y * v1y;
     const double den = d00 * d11 - d01 * d01;
-    if (den == 0) { box[i] = bx; return; }          // holds no point
+    if (den == 0) return bx;                         // holds no point
     if (!(den > 1e-12 * d00 * d11)) {                // thin or non-finite: test everywhere
         alw[atomicAdd(&status[2], 1)] = i;
-        box[i] = bx;
-        return;
+        return bx;
     }
-    const BinGrid g = bin_grid(bb, G);
     const double xmin = fmin(x1, fmin(x2, x3)), xmax = fmax(x1, fmax(x2, x3));
     const double ymin = fmin(y1, fmin(y2, y3)), ymax = fmax(y1, fmax(y2, y3));
     const double eps = 1e-9 * fmax(xmax - xmin, ymax - ymin) + 1e-300;
@@ -155,9 +156,28 @@ __global__ void k_face_boxes(const double *__restrict__ uv, int nv, const int *_
     bx.x1 = bin_of(xmax + eps, g.ox, g.inv, g.G);
     bx.y0 = bin_of(ymin - eps, g.oy, g.inv, g.G);
     bx.y1 = bin_of(ymax + eps, g.oy, g.inv, g.G);
-    box[i] = bx;
-    for (int y = bx.y0; y <= bx.y1; ++y)
-        for (int x = bx.x0; x <= bx.x1; ++x) atomicAdd(&count[y * g.G + x], 1);
+    return bx;
+}
+
+// per face: its record and box, and its (face, bin) pairs counted per bin and
+// in all
+__global__ void k_face_boxes(const double *__restrict__ uv, int nv, const int *__restrict__ tri,
+                             int nf, const unsigned long long *__restrict__ bb, int G,
+                             FaceXY *__restrict__ xy, FaceBox *__restrict__ box,
+                             int *__restrict__ alw, int *__restrict__ count,
+                             int *__restrict__ status)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    int pairs = 0;
+    if (i < nf) {
+        const BinGrid g = bin_grid(bb, G);
+        const FaceBox bx = face_box(uv, nv, tri, i, g, xy, alw, status);
+        box[i] = bx;
+        for (int y = bx.y0; y <= bx.y1; ++y)
+            for (int x = bx.x0; x <= bx.x1; ++x) atomicAdd(&count[y * g.G + x], 1);
+        pairs = (bx.x1 - bx.x0 + 1) * (bx.y1 - bx.y0 + 1);
+    }
+    add_pairs(pairs, pair_total(status));
 }
 
 // (face, bin) pairs: each face writes its index into the lists of its bins;
@@ -169,7 +189,7 @@ __global__ void k_bin_fill(const FaceBox *__restrict__ box, int nf,
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nf) return;
-    if (start[grid * grid] > cap) {
+    if (*pair_total(status) > (unsigned long long)cap) {
         if (i == 0) status[1] = 1;
         return;
     }
@@ -202,14 +222,13 @@ __global__ __launch_bounds__(256) void k_locate(const FaceXY *__restrict__ xy,
                                                 const double *__restrict__ q, int nq,
                                                 int *__restrict__ face, double *__restrict__ w,
                                                 double *__restrict__ out3,
-                                                const int *__restrict__ status,
-                                                int *__restrict__ host)
+                                                int *__restrict__ status, int *__restrict__ host)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k == 0) {
         host[0] = status[0];
         host[1] = status[1];
-        host[2] = start[G * G];
+        host[2] = pairs_word(*pair_total(status));
     }
     if (k >= nq || status[0] || status[1]) return;
     const int nalw = status[2];
@@ -353,7 +372,7 @@ extern "C" int cvt_locate_points(const double *uv, const double *p3, int nv, con
         carve.base = mem.base();
         carve.at = 0;
         carve(d_bb, 4);                          // zeroed from here
-        carve(d_status, 4); carve(d_count, nb); carve(d_cursor, nb);
+        carve(d_status, kStatus); carve(d_count, nb); carve(d_cursor, nb);
         zeroed = (carve.at + 255) & ~(size_t)255;
         carve(d_start, nb + 1); carve(d_box, nfa); carve(d_xy, nfa); carve(d_alw, nfa);
         if (!own_uv) carve(d_uv, 2 * nva);
@@ -404,6 +423,10 @@ extern "C" int cvt_locate_points(const double *uv, const double *p3, int nv, con
             return fail(CVT_ERR_ARG, "a face indexes a vertex outside [0, %d)", nv);
         }
         if (!host[1]) break;
+        if (host[2] < 0) {
+            mem.idle();
+            return fail(CVT_ERR_CAPACITY, "2^31 or more (face, bin) pairs");
+        }
         cap = (size_t)host[2];
         LCHK(more.take(sizeof(int) * cap), "alloc");
         d_list = reinterpret_cast<int *>(more.base());

@@ -82,6 +82,21 @@ __device__ __forceinline__ bool inside_exact(double n2, double n3, double den)
     return !(b1 < 0 || b2 < 0 || b3 < 0);
 }
 
+// Adds the (face, cell) pairs of a wave's lanes, at most 2^20 each, to a
+// call's total; called by every lane of the wave.  The lists' starts are 32-bit
+// sums, which wrap beyond 2^31 - 1 pairs: whether the lists hold all pairs is
+// decided from this total.
+__device__ __forceinline__ void add_pairs(int pairs, unsigned long long *total)
+{
+    for (int o = 32; o > 0; o >>= 1) pairs += __shfl_xor(pairs, o, 64);
+    if ((threadIdx.x & 63) == 0 && pairs > 0) atomicAdd(total, (unsigned long long)pairs);
+}
+// the total as the host reads it: -1 where no list of 32-bit starts holds it
+__device__ __forceinline__ int pairs_word(unsigned long long total)
+{
+    return total > 0x7fffffffull ? -1 : (int)total;
+}
+
 // positions of a call's buffers in its scratch, each at a 256-byte boundary:
 // run once to size it and once to place them
 struct Carver {

@@ -42,24 +42,25 @@ __device__ __forceinline__ void tile_range(const TriBox &b, int &tx0, int &tx1, 
     ty0 = b.y0 / RT; ty1 = b.y1 / RT;
 }
 
-// words of a call's status
-enum { ST_BAD, ST_OVERFLOW, ST_ALWAYS };
-
-// per triangle: index validation, the conservative pixel box, and its
-// (triangle, tile) pairs counted per tile.  Triangles to test everywhere are
-// appended to alw in any order (a pixel keeps the lowest-index hit).
-__global__ void k_tri_boxes(const double *__restrict__ pts, int nv, const int *__restrict__ tri,
-                            int nt, double scale, int n, int tiles_x, TriBox *__restrict__ box,
-                            int *__restrict__ alw, int *__restrict__ count, int *__restrict__ status)
+// words of a call's status; from ST_PAIRS the (triangle, tile) pairs in 64 bits
+enum { ST_BAD, ST_OVERFLOW, ST_ALWAYS, ST_PAIRS = 4, ST_WORDS = 8 };
+__device__ __forceinline__ unsigned long long *pair_total(int *status)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nt) return;
+    return reinterpret_cast<unsigned long long *>(status + ST_PAIRS);
+}
+
+// triangle i: index validation and the conservative pixel box.  Triangles to
+// test everywhere are appended to alw in any order (a pixel keeps the
+// lowest-index hit).
+__device__ __forceinline__ TriBox tri_box(const double *__restrict__ pts, int nv,
+                                          const int *__restrict__ tri, int i, double scale, int n,
+                                          int *__restrict__ alw, int *__restrict__ status)
+{
     const int a = tri[3 * i], b = tri[3 * i + 1], c = tri[3 * i + 2];
     TriBox bx = {1, 0, 1, 0};
     if ((unsigned)a >= (unsigned)nv || (unsigned)b >= (unsigned)nv || (unsigned)c >= (unsigned)nv) {
         status[ST_BAD] = 1;
-        box[i] = bx;
-        return;
+        return bx;
     }
     const double x1 = pts[2 * a], y1 = pts[2 * a + 1];
     const double x2 = pts[2 * b], y2 = pts[2 * b + 1];
@@ -68,11 +69,10 @@ __global__ void k_tri_boxes(const double *__restrict__ pts, int nv, const int *_
     const double d00 = v0x * v0x + v0y * v0y, d11 = v1x * v1x + v1y * v1y;
     const double d01 = v0x * v1x + v0y * v1y;
     const double den = d00 * d11 - d01 * d01;
-    if (den == 0) { box[i] = bx; return; }          // never hits
+    if (den == 0) return bx;                         // never hits
     if (!(den > 1e-12 * d00 * d11)) {                // thin or non-finite: test everywhere
         alw[atomicAdd(&status[ST_ALWAYS], 1)] = i;
-        box[i] = bx;
-        return;
+        return bx;
     }
     const double xmin = fmin(x1, fmin(x2, x3)), xmax = fmax(x1, fmax(x2, x3));
     const double ymin = fmin(y1, fmin(y2, y3)), ymax = fmax(y1, fmax(y2, y3));
@@ -85,24 +85,41 @@ __global__ void k_tri_boxes(const double *__restrict__ pts, int nv, const int *_
     bx.y1 = (int)fmin((double)(n - 1), ceil(hi_y));
     if (!(hi_x >= 0.0) || !(hi_y >= 0.0) || !(lo_x <= n - 1.0) || !(lo_y <= n - 1.0))
         bx = TriBox{1, 0, 1, 0};
-    box[i] = bx;
-    if (bx.x0 > bx.x1 || bx.y0 > bx.y1) return;
-    int tx0, tx1, ty0, ty1;
-    tile_range(bx, tx0, tx1, ty0, ty1);
-    for (int y = ty0; y <= ty1; ++y)
-        for (int x = tx0; x <= tx1; ++x) atomicAdd(&count[y * tiles_x + x], 1);
+    return bx;
+}
+
+// per triangle: its box, and its (triangle, tile) pairs counted per tile and
+// in all
+__global__ void k_tri_boxes(const double *__restrict__ pts, int nv, const int *__restrict__ tri,
+                            int nt, double scale, int n, int tiles_x, TriBox *__restrict__ box,
+                            int *__restrict__ alw, int *__restrict__ count, int *__restrict__ status)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    int pairs = 0;
+    if (i < nt) {
+        const TriBox bx = tri_box(pts, nv, tri, i, scale, n, alw, status);
+        box[i] = bx;
+        if (bx.x0 <= bx.x1 && bx.y0 <= bx.y1) {
+            int tx0, tx1, ty0, ty1;
+            tile_range(bx, tx0, tx1, ty0, ty1);
+            for (int y = ty0; y <= ty1; ++y)
+                for (int x = tx0; x <= tx1; ++x) atomicAdd(&count[y * tiles_x + x], 1);
+            pairs = (tx1 - tx0 + 1) * (ty1 - ty0 + 1);
+        }
+    }
+    add_pairs(pairs, pair_total(status));
 }
 
 // (triangle, tile) pairs: each triangle writes its index into its tiles'
 // lists; with more pairs than the `cap` the list holds, nothing is written and
 // the overflow word is raised.
-__global__ void k_tile_fill(const TriBox *__restrict__ box, int nt, int tiles_x, int ntiles,
+__global__ void k_tile_fill(const TriBox *__restrict__ box, int nt, int tiles_x,
                             const int *__restrict__ start, int *__restrict__ cursor,
                             int *__restrict__ list, int cap, int *__restrict__ status)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nt) return;
-    if (start[ntiles] > cap) {
+    if (*pair_total(status) > (unsigned long long)cap) {
         if (i == 0) status[ST_OVERFLOW] = 1;
         return;
     }
@@ -144,8 +161,7 @@ __global__ __launch_bounds__(256) void k_raster(const double *__restrict__ pts,
                                                 const int *__restrict__ alw, int tiles_x,
                                                 int ntiles, double scale, int n,
                                                 float *__restrict__ density,
-                                                const int *__restrict__ status,
-                                                int *__restrict__ host)
+                                                int *__restrict__ status, int *__restrict__ host)
 {
     struct Cand {
         double x1, y1, v0x, v0y, v1x, v1y, d00, d01, d11, den;
@@ -155,7 +171,7 @@ __global__ __launch_bounds__(256) void k_raster(const double *__restrict__ pts,
     if (host && blockIdx.x == 0 && threadIdx.x == 0) {
         host[0] = status[ST_BAD];
         host[1] = status[ST_OVERFLOW];
-        host[2] = start[ntiles];
+        host[2] = pairs_word(*pair_total(status));
     }
     if (status[ST_BAD] || status[ST_OVERFLOW]) return;
     const int wave = threadIdx.x >> 6, t = threadIdx.x & 63;
@@ -275,7 +291,7 @@ extern "C" int cvt_rasterize(const double *points, const double *weight, int num
     auto layout = [&]() {
         carve.base = mem.base();
         carve.at = 0;
-        carve(d_status, 4);                      // zeroed from here
+        carve(d_status, ST_WORDS);               // zeroed from here
         carve(d_count, ntiles); carve(d_cursor, ntiles);
         zeroed = (carve.at + 255) & ~(size_t)255;
         carve(d_start, (size_t)ntiles + 1); carve(d_box, nta); carve(d_alw, nta);
@@ -308,8 +324,8 @@ extern "C" int cvt_rasterize(const double *points, const double *weight, int num
     int *host = mem.status();
     for (int round = 0; round < 2; ++round) {
         if (num_tri > 0)
-            hipLaunchKernelGGL(k_tile_fill, gt, blk, 0, st, d_box, num_tri, tiles_x, ntiles, d_start,
-                               d_cursor, d_list, (int)cap, d_status);
+            hipLaunchKernelGGL(k_tile_fill, gt, blk, 0, st, d_box, num_tri, tiles_x, d_start, d_cursor,
+                               d_list, (int)cap, d_status);
         hipLaunchKernelGGL(k_raster, dim3((ntiles + 3) / 4), blk, 0, st, d_pts, d_wt, d_tri, d_list,
                            d_start, d_alw, tiles_x, ntiles, scale, n, d_den, d_status, host);
         RCHK(hipGetLastError(), "raster launch");
@@ -319,6 +335,10 @@ extern "C" int cvt_rasterize(const double *points, const double *weight, int num
             return fail(CVT_ERR_ARG, "a triangle indexes a vertex outside [0, %d)", num_point);
         }
         if (!host[1]) break;
+        if (host[2] < 0) {
+            mem.idle();
+            return fail(CVT_ERR_CAPACITY, "2^31 or more (triangle, tile) pairs");
+        }
         cap = (size_t)host[2];
         RCHK(more.take(sizeof(int) * cap), "alloc");
         d_list = reinterpret_cast<int *>(more.base());
@@ -336,7 +356,7 @@ extern "C" int cvt_rasterize(const double *points, const double *weight, int num
 // ---------------------------------------------------------------------------
 // cvt_rasterize_noalloc: cvt_rasterize for callers that cannot allocate.  All
 // of its working memory (triangle boxes, the thin-triangle list, per-tile
-// counts and list starts, the (triangle, tile) lists and three status words)
+// counts and list starts, the (triangle, tile) lists and the status words)
 // lives in one static device array, so the call allocates nothing.  Each
 // device holds its own copy of the array; its address is looked up once per
 // device with hipGetSymbolAddress.  Every call on a device shares that
@@ -442,14 +462,14 @@ extern "C" int cvt_rasterize_noalloc(const double *points, const double *weight,
     // the counts, cursors and status words left by the last call start at zero
     hipLaunchKernelGGL(k_zero_i32, dim3(256), dim3(256), 0, st, count, (long)ntiles);
     hipLaunchKernelGGL(k_zero_i32, dim3(256), dim3(256), 0, st, cursor, (long)ntiles);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, status, 4L);
+    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, st, status, (long)ST_WORDS);
     if (num_tri > 0)
         hipLaunchKernelGGL(k_tri_boxes, dim3((num_tri + 255) / 256), dim3(256), 0, st, points,
                            num_point, triangle, num_tri, scale, n, tiles_x, box, alw, count, status);
     launch_exclusive_scan(st, count, ntiles, start);
     if (num_tri > 0)
         hipLaunchKernelGGL(k_tile_fill, dim3((num_tri + 255) / 256), dim3(256), 0, st, box,
-                           num_tri, tiles_x, ntiles, start, cursor, list, NOALLOC_MAX_PAIRS, status);
+                           num_tri, tiles_x, start, cursor, list, NOALLOC_MAX_PAIRS, status);
     hipLaunchKernelGGL(k_raster, dim3((ntiles + 3) / 4), dim3(256), 0, st, points, weight, triangle,
                        list, start, alw, tiles_x, ntiles, scale, n, density, status, nullptr);
     int h[3] = {0, 0, 0};
