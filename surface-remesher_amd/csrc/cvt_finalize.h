@@ -24,7 +24,8 @@ __device__ __forceinline__ double wave_tree_sum(double v)
     return v;
 }
 
-// Run by all 256 threads of one workgroup (red_e, red_g: 256 doubles of LDS
+// Run by every thread of one workgroup of 256 threads or more, of which the
+// first 256 work and all meet the barriers (red_e, red_g: 256 doubles of LDS
 // each).  Thread t sums partials t, t + 256, ... of the nblocks blocks, then
 // the tree of 256 (steps 128 and 64 in LDS, 32 .. 1 in wave 0).  Then, on
 // thread 0: E and |grad E| appended to the history, the stop rule tested,
@@ -34,13 +35,15 @@ __device__ __forceinline__ void cvt_finalize_block(const double *__restrict__ bl
                                                    const FinalArgs &fa, double *red_e,
                                                    double *red_g)
 {
-    double te = 0.0, tg = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += 256) {
-        te += __hip_atomic_load(&blockpart[2 * b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        tg += __hip_atomic_load(&blockpart[2 * b + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < 256) {
+        double te = 0.0, tg = 0.0;
+        for (int b = threadIdx.x; b < nblocks; b += 256) {
+            te += __hip_atomic_load(&blockpart[2 * b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            tg += __hip_atomic_load(&blockpart[2 * b + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        red_e[threadIdx.x] = te;
+        red_g[threadIdx.x] = tg;
     }
-    red_e[threadIdx.x] = te;
-    red_g[threadIdx.x] = tg;
     __syncthreads();
     for (int o = 128; o >= 64; o >>= 1) {
         if (threadIdx.x < o) {
@@ -77,3 +80,12 @@ __device__ __forceinline__ void cvt_finalize_block(const double *__restrict__ bl
     }
 }
 
+// A deferred finalize, when one is pending: run by every thread of one
+// workgroup of 256 threads or more.
+__device__ __forceinline__ void cvt_finalize_pending(const double *__restrict__ blockpart,
+                                                     int *__restrict__ dstate, const FinalArgs &fa,
+                                                     double *red_e, double *red_g)
+{
+    const int nblocks = dstate[ST_PEND];
+    if (nblocks > 0) cvt_finalize_block(blockpart, nblocks, dstate, fa, red_e, red_g);
+}

@@ -675,8 +675,7 @@ static __global__ __launch_bounds__(256) void k_finalize_pending(const double *_
                                                                  FinalArgs fa)
 {
     __shared__ double red_e[256], red_g[256];
-    const int nb = dstate[ST_PEND];
-    if (nb > 0) cvt_finalize_block(blockpart, nb, dstate, fa, red_e, red_g);
+    cvt_finalize_pending(blockpart, dstate, fa, red_e, red_g);
 }
 
 // cvt_lloyd_until: arm the stop rule (relative decrease over `window`
@@ -720,8 +719,7 @@ static __global__ __launch_bounds__(256) void k_compat_count(int *__restrict__ t
     __shared__ double red_e[256], red_g[256];
     __shared__ int part[4];
     if ((int)blockIdx.x == nblocks) {
-        const int pending = dstate[ST_PEND];
-        if (pending > 0) cvt_finalize_block(blockpart, pending, dstate, fa, red_e, red_g);
+        cvt_finalize_pending(blockpart, dstate, fa, red_e, red_g);
         return;
     }
     const int S = dstate[ST_NSITES], i = blockIdx.x * 256 + threadIdx.x;

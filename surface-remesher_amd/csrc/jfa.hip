@@ -1383,8 +1383,7 @@ __global__ __launch_bounds__(256) void k_jfa_seeds(const uint32_t *__restrict__ 
     if (fin && blockIdx.x == 0) {
         // the previous iteration's deferred finalize, beside the scatter
         __shared__ double red_e[256], red_g[256];
-        const int nb = dstate[ST_PEND];
-        if (nb > 0) cvt_finalize_block(blockpart, nb, dstate, fa, red_e, red_g);
+        cvt_finalize_pending(blockpart, dstate, fa, red_e, red_g);
         return;
     }
     const int halt = stop_word(stop);   // tested once the site's load is in flight

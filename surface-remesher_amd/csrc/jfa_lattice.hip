@@ -449,8 +449,7 @@ __global__ __launch_bounds__(64 * NW) void k_jfa_lattice(
     if (fin && blockIdx.x == 0) {
         // the previous iteration's deferred finalize, beside the passes
         __shared__ double red_e[256], red_g[256];
-        const int nb = dstate[ST_PEND];
-        if (nb > 0 && threadIdx.x < 256) cvt_finalize_block(blockpart, nb, dstate, fa, red_e, red_g);
+        cvt_finalize_pending(blockpart, dstate, fa, red_e, red_g);
         return;
     }
     const int u = lattice_unit((int)blockIdx.x - fin, (int)gridDim.x - fin);
