@@ -216,7 +216,9 @@ int cvt_rasterize_noalloc(const double *points, const double *weight, int num_po
 /* Gives back the device memory that cvt_rasterize, cvt_locate_points and
  * cvt_vertex_weights keep from call to call: at most four blocks and 64 MB
  * per device (larger ones are freed by the call that needed them).  Blocks in
- * use by a call of another thread stay with it. */
+ * use by a call of another thread stay with it.  A program that resets a
+ * device need not call it first: blocks that the reset has freed are neither
+ * used nor freed again. */
 int cvt_release_scratch(void);
 
 /* CDT input points (the site scan of delaunayInput, source/delaunay.h:48-58):

@@ -14,12 +14,29 @@ namespace cvt {
 
 namespace {
 
+// Between two calls a program may reset the device, which frees what lies in the
+// store, and the addresses may then hold allocations of its own.  Each
+// allocation has an id that no other of the process ever gets, so a block is
+// used, and freed, only while its ids still stand for its addresses (0.06 us
+// an id).
 struct Block {
     int device;
     char *dev;
     size_t bytes;
     int *pinned;
+    uint64_t dev_id, pinned_id;
 };
+
+// the id of the allocation at p, 0 where there is none
+uint64_t allocation_id(void *p)
+{
+    uint64_t id = 0;
+    if (hipPointerGetAttribute(&id, HIP_POINTER_ATTRIBUTE_BUFFER_ID, p) == hipSuccess) return id;
+    (void)hipGetLastError();
+    return 0;
+}
+bool holds(void *p, uint64_t id) { return id && allocation_id(p) == id; }
+bool whole(const Block &b) { return holds(b.dev, b.dev_id) && holds(b.pinned, b.pinned_id); }
 
 std::mutex g_mutex;
 std::vector<Block> &store()
@@ -29,10 +46,11 @@ std::vector<Block> &store()
     return *s;
 }
 
+// frees a block that has lain in the store
 void drop(const Block &b)
 {
-    (void)hipFree(b.dev);
-    (void)hipHostFree(b.pinned);
+    if (holds(b.dev, b.dev_id)) (void)hipFree(b.dev);
+    if (holds(b.pinned, b.pinned_id)) (void)hipHostFree(b.pinned);
 }
 
 }  // namespace
@@ -52,21 +70,27 @@ hipError_t MeshScratch::take(size_t bytes)
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        std::vector<Block> &s = store();
-        auto best = s.end();
-        for (auto i = s.begin(); i != s.end(); ++i)
-            if (i->device == device && i->bytes >= bytes && (best == s.end() || i->bytes < best->bytes))
-                best = i;
-        if (best != s.end()) {
-            device_ = device;
-            dev_ = best->dev;
-            bytes_ = best->bytes;
-            pinned_ = best->pinned;
+    for (;;) {
+        Block b;
+        {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            std::vector<Block> &s = store();
+            auto best = s.end();
+            for (auto i = s.begin(); i != s.end(); ++i)
+                if (i->device == device && i->bytes >= bytes && (best == s.end() || i->bytes < best->bytes))
+                    best = i;
+            if (best == s.end()) break;
+            b = *best;
             s.erase(best);
+        }
+        if (whole(b)) {
+            device_ = device;
+            dev_ = b.dev;
+            bytes_ = b.bytes;
+            pinned_ = b.pinned;
             return hipSuccess;
         }
+        drop(b);
     }
     // whole megabytes, so that a slightly larger mesh fits the same block
     const size_t mb = (size_t)1 << 20, want = std::max(mb, (bytes + mb - 1) / mb * mb);
@@ -94,7 +118,12 @@ MeshScratch::~MeshScratch()
 {
     if (!dev_) return;
     if (!idle_) (void)hipStreamSynchronize(nullptr);
-    Block b{device_, dev_, bytes_, pinned_};
+    Block b{device_, dev_, bytes_, pinned_, allocation_id(dev_), allocation_id(pinned_)};
+    if (!b.dev_id || !b.pinned_id) {               // could not be told from another's later
+        (void)hipFree(dev_);
+        (void)hipHostFree(pinned_);
+        return;
+    }
     Block out{};
     try {
         std::lock_guard<std::mutex> lock(g_mutex);

@@ -18,7 +18,8 @@ constexpr int kStatusWords = 16;
 // 245 us to locate 49152 points in an 11858-face mesh and 400 us for its vertex
 // weights and 2048^2 raster, for 60 and 130 us of kernels; now 72 and 154 us.
 // A block belongs to one call at a time, whatever thread makes it, and is
-// released only after the call has waited for its work.  The store holds at
+// released only after the call has waited for its work.  A block that a reset
+// of the device has freed since is left alone.  The store holds at
 // most kScratchBlocks blocks and kScratchBytes bytes per device; larger ones
 // are freed at once, and all of them when a device allocation here fails or
 // cvt_release_scratch is called.

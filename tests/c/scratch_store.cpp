@@ -1,0 +1,167 @@
+// The mesh calls' store of working memory (mesh_scratch.cpp) over a runtime of
+// its own: addresses are numbers that are given out again as soon as they are
+// free, every allocation has a new id, and a reset of a device frees all that
+// it holds.  Ends with status 1 where the store hands out or frees memory that
+// is not its own.
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <map>
+#include <vector>
+
+#include "../../surface-remesher_amd/csrc/mesh_scratch.h"
+
+struct Alloc {
+    size_t bytes;
+    uint64_t id;
+    int device;                 // -1: pinned
+    bool program;               // the program's own
+};
+static std::map<uintptr_t, Alloc> g_mem;
+static uint64_t g_id = 0;
+static int g_device = 0, g_mallocs = 0;
+static bool g_program = false;
+
+static void check(bool ok, const char *what)
+{
+    if (ok) return;
+    printf("%s\n", what);
+    exit(1);
+}
+
+static void *place(size_t bytes, int device)
+{
+    uintptr_t at = (uintptr_t)1 << 32;
+    for (const auto &m : g_mem) {          // the lowest gap that is large enough
+        if (m.first - at >= bytes && m.first > at) break;
+        at = m.first + ((m.second.bytes + 4095) & ~(size_t)4095);
+    }
+    g_mem[at] = Alloc{bytes, ++g_id, device, g_program};
+    return (void *)at;
+}
+
+static hipError_t give_back(void *p)
+{
+    const auto i = g_mem.find((uintptr_t)p);
+    if (i == g_mem.end()) return hipErrorInvalidValue;
+    check(i->second.program == g_program, "freed what is not its own");
+    g_mem.erase(i);
+    return hipSuccess;
+}
+
+static void reset(int device)
+{
+    for (auto i = g_mem.begin(); i != g_mem.end();)
+        i = i->second.device == device || i->second.device < 0 ? g_mem.erase(i) : std::next(i);
+}
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t bytes)
+{
+    ++g_mallocs;
+    *p = place(bytes, g_device);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
+{
+    *p = place(bytes, -1);
+    return hipSuccess;
+}
+hipError_t hipFree(void *p) { return give_back(p); }
+hipError_t hipHostFree(void *p) { return give_back(p); }
+hipError_t hipGetDevice(int *d) { *d = g_device; return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *, const void *) { return hipErrorInvalidValue; }
+hipError_t hipPointerGetAttribute(void *data, hipPointer_attribute which, hipDeviceptr_t p)
+{
+    const auto i = g_mem.upper_bound((uintptr_t)p);
+    if (which != HIP_POINTER_ATTRIBUTE_BUFFER_ID || i == g_mem.begin()) return hipErrorInvalidValue;
+    const auto m = std::prev(i);
+    if ((uintptr_t)p >= m->first + m->second.bytes) return hipErrorInvalidValue;
+    *static_cast<uint64_t *>(data) = m->second.id;
+    return hipSuccess;
+}
+int cvt_release_scratch(void);
+}
+namespace cvt {
+void clear_error() {}
+}
+
+// a mesh call: a block of `bytes`, and whether it lies in memory of the store
+static void call(size_t bytes)
+{
+    cvt::MeshScratch m;
+    check(m.take(bytes) == hipSuccess, "take");
+    for (void *p : {(void *)m.base(), (void *)m.status()}) {
+        const auto i = g_mem.find((uintptr_t)p);
+        check(i != g_mem.end(), "a block that no longer exists");
+        check(!i->second.program, "a block in the program's memory");
+    }
+    check(g_mem[(uintptr_t)m.base()].bytes >= bytes, "a block that is too small");
+    m.idle();
+}
+
+static void *program(size_t bytes)
+{
+    g_program = true;
+    void *p = nullptr;
+    (void)hipMalloc(&p, bytes);
+    g_program = false;
+    return p;
+}
+
+static size_t held(int device)
+{
+    size_t n = 0;
+    for (const auto &m : g_mem) n += m.second.program || m.second.device != device ? 0 : m.second.bytes;
+    return n;
+}
+
+int main(int argc, char **argv)
+{
+    const char *what = argc > 1 ? argv[1] : "";
+    const size_t mb = (size_t)1 << 20;
+    if (!strcmp(what, "reuse")) {
+        call(3 * mb);
+        const int n = g_mallocs;
+        call(3 * mb);
+        call(mb);
+        check(g_mallocs == n, "a second call allocates");
+        g_device = 1;                              // another device, its own blocks
+        call(mb);
+        check(g_mallocs == n + 1, "a block of another device");
+        check(cvt_release_scratch() == 0 && g_mem.empty(), "memory kept after the release");
+    } else if (!strcmp(what, "reset")) {
+        call(3 * mb);
+        reset(0);
+        call(3 * mb);                              // nothing at the old address
+        reset(0);
+        program(3 * mb);                           // the program's memory there
+        call(3 * mb);
+        reset(0);
+        program(64 * mb);                          // ... and around it
+        program(mb);
+        call(2 * mb);
+    } else if (!strcmp(what, "reset-release")) {
+        call(3 * mb);
+        reset(0);
+        program(3 * mb);
+        program(sizeof(int) * cvt::kStatusWords);
+        const size_t n = g_mem.size();
+        check(cvt_release_scratch() == 0 && g_mem.size() == n, "the program's memory freed");
+    } else if (!strcmp(what, "reset-evict")) {
+        call(40 * mb);
+        call(60 * mb);
+        reset(0);
+        program(40 * mb);
+        program(60 * mb);
+        for (int k = 1; k < 8; ++k) call(8 * k * mb);
+    } else {
+        return 2;
+    }
+    for (int d = 0; d < 2; ++d) check(held(d) <= cvt::kScratchBytes, "more than the store's bound");
+    printf("ok\n");
+    return 0;
+}
