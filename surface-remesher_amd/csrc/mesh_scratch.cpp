@@ -124,31 +124,39 @@ MeshScratch::~MeshScratch()
         (void)hipHostFree(pinned_);
         return;
     }
-    Block out{};
+    // the newest block stays, for the next call like this one, and the oldest
+    // leave until the others fit beside it (were this one to leave, a mesh that
+    // has grown past half the bound would be allocated anew on every call)
+    if (bytes_ > kScratchBytes) {
+        drop(b);
+        return;
+    }
     try {
         std::lock_guard<std::mutex> lock(g_mutex);
-        std::vector<Block> &s = store();
-        s.push_back(b);
-        b.dev = nullptr;
-        size_t held = 0, count = 0;
-        auto least = s.end();
-        for (auto i = s.begin(); i != s.end(); ++i)
-            if (i->device == device_) {
-                held += i->bytes;
-                ++count;
-                if (least == s.end() || i->bytes < least->bytes) least = i;
-            }
-        // over the bounds: too many bytes, this block leaves; too many blocks,
-        // the smallest
-        if (held > kScratchBytes || count > (size_t)kScratchBlocks) {
-            auto i = held > kScratchBytes ? s.end() - 1 : least;
-            out = *i;
-            s.erase(i);
-        }
+        store().push_back(b);
     } catch (...) {
-        if (b.dev) out = b;
+        drop(b);
+        return;
     }
-    if (out.dev) drop(out);
+    for (;;) {
+        Block out{};
+        {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            std::vector<Block> &s = store();
+            size_t held = 0, count = 0;
+            auto oldest = s.end();
+            for (auto i = s.begin(); i != s.end(); ++i)
+                if (i->device == device_) {
+                    held += i->bytes;
+                    ++count;
+                    if (oldest == s.end()) oldest = i;
+                }
+            if (held <= kScratchBytes && count <= (size_t)kScratchBlocks) return;
+            out = *oldest;
+            s.erase(oldest);
+        }
+        drop(out);
+    }
 }
 
 bool in_place(const void *p, size_t align)

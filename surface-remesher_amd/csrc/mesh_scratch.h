@@ -19,9 +19,9 @@ constexpr int kStatusWords = 16;
 // weights and 2048^2 raster, for 60 and 130 us of kernels; now 72 and 154 us.
 // A block belongs to one call at a time, whatever thread makes it, and is
 // released only after the call has waited for its work.  A block that a reset
-// of the device has freed since is left alone.  The store holds at
-// most kScratchBlocks blocks and kScratchBytes bytes per device; larger ones
-// are freed at once, and all of them when a device allocation here fails or
+// of the device has freed since is left alone.  The store holds the newest
+// blocks, at most kScratchBlocks and kScratchBytes bytes per device; larger
+// ones are freed at once, and all of them when a device allocation here fails or
 // cvt_release_scratch is called.
 constexpr int kScratchBlocks = 4;
 constexpr size_t kScratchBytes = (size_t)64 << 20;

@@ -158,6 +158,31 @@ int main(int argc, char **argv)
         program(40 * mb);
         program(60 * mb);
         for (int k = 1; k < 8; ++k) call(8 * k * mb);
+    } else if (!strcmp(what, "growth")) {
+        // meshes that grow past half the bound, each size called twice
+        for (size_t size : {20, 33, 40, 41, 50, 63, 64}) {
+            call(size * mb);
+            const int n = g_mallocs;
+            call(size * mb);
+            check(g_mallocs == n, "a repeated call allocates");
+            check(held(0) <= cvt::kScratchBytes, "more than the store's bound");
+        }
+        call(65 * mb);                             // too large to keep
+        const int n = g_mallocs;
+        call(64 * mb);
+        check(g_mallocs == n, "a larger call drops what fits");
+    } else if (!strcmp(what, "count")) {
+        {
+            cvt::MeshScratch m[6];                 // six calls at once
+            for (int k = 0; k < 6; ++k) {
+                check(m[k].take((k + 1) * mb) == hipSuccess, "take");
+                m[k].idle();
+            }
+        }
+        check(g_mem.size() == 2 * cvt::kScratchBlocks, "blocks kept");
+        const int n = g_mallocs;
+        call(mb);
+        check(g_mallocs == n, "a call on the smallest mesh allocates");
     } else {
         return 2;
     }

@@ -29,7 +29,7 @@ def harness(tmp_path_factory):
     return d / "h"
 
 
-@pytest.mark.parametrize("case", ["reuse", "reset", "reset-release", "reset-evict"])
+@pytest.mark.parametrize("case", ["reuse", "reset", "reset-release", "reset-evict", "growth", "count"])
 def test_store(harness, case):
     r = subprocess.run([str(harness), case], capture_output=True, text=True, timeout=60)
     assert (r.returncode, r.stdout) == (0, "ok\n"), r.stderr
