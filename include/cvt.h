@@ -321,8 +321,8 @@ int cvt_batch_synchronize(cvt_batch *batch);
  * general position (no three points collinear, no four cocircular) it is
  * the unique one.  Exact duplicate points are dropped (cvt_dt_stats counts
  * them).  CVT_ERR_ARG for non-finite points, for inputs whose points are
- * all collinear, and for coordinates whose magnitudes span more than 2^71
- * units of their finest bit.  Arrays may be host or device memory; the
+ * all collinear, and where a sign that float64 leaves open is asked of
+ * coordinates whose lowest set bits lie more than 71 binary places apart.  Arrays may be host or device memory; the
  * call returns when the output is written.
  * --------------------------------------------------------------------- */
 typedef struct cvt_dt cvt_dt;
@@ -346,7 +346,8 @@ int cvt_dt_destroy(cvt_dt *dt);
 /* orient[i] = sign of orient2d(a, b, c) and incircle[i] = sign of
  * incircle(a, b, c, d) for count 8-double records (ax ay bx by cx cy dx dy),
  * evaluated on the device by the triangulation's exact predicates (gDel2D's
- * orient2dFastExact / incircleExact, source/gDel2D/gDel2D/GPU/KerShewchuk.h:636,726) */
+ * orient2dFastExact / incircleExact, source/gDel2D/gDel2D/GPU/KerShewchuk.h:636,726);
+ * CVT_ERR_ARG as in cvt_dt_compute */
 int cvt_dt_predicates(const double *quads, int count, int *orient, int *incircle);
 
 typedef struct cvt_unet cvt_unet;

@@ -286,6 +286,22 @@ DT_HD_COLD int orient_exact(double ax, double ay, double bx, double by, double c
     return orient_wide(x, err);
 }
 
+// Whether the coordinates' highest bits are near enough that their lowest set
+// bits, at most 52 below, lie within the 71 that to_integers takes: what is
+// decided without the integer stages is left to them otherwise, which refuse a
+// wider span.
+template <int K> DT_HD bool near_exponents(const double (&x)[K])
+{
+    uint32_t lo = ~0u, hi = 0;
+    for (int i = 0; i < K; ++i) {
+        const uint32_t u = (uint32_t)(__builtin_bit_cast(uint64_t, x[i]) >> 32) & 0x7fffffffu;
+        const uint32_t v = x[i] == 0.0 ? ~0u : u;
+        hi = u > hi ? u : hi;
+        lo = v < lo ? v : lo;
+    }
+    return lo == ~0u || (hi >> 20) - (lo >> 20) <= 19;
+}
+
 // whether a - b = d exactly (the rounding error of the difference is zero)
 DT_HD bool exact_diff(double a, double b, double d)
 {
@@ -304,6 +320,8 @@ DT_HD int orient_products(double ax, double ay, double bx, double by, double cx,
 {
     const double u = ax - cx, v = by - cy, s = ay - cy, t = bx - cx;
     const double l = u * v, r = s * t;
+    const double x[6] = {ax, ay, bx, by, cx, cy};
+    if (!near_exponents<6>(x)) return 2;
     if (bound == 0.0 && (u == 0.0 || v == 0.0) && (s == 0.0 || t == 0.0)) return 0;
     if (!(bound > 1e-270 && bound < 1e270) || !exact_diff(ax, cx, u) || !exact_diff(by, cy, v) ||
         !exact_diff(ay, cy, s) || !exact_diff(bx, cx, t))
@@ -389,13 +407,13 @@ DT_HD int incircle(double ax, double ay, double bx, double by, double cx, double
     const double bound = 2.3e-15 * perm;
     if ((det > bound || -det > bound) && bound > 1e-290 && bound < 1e290)
         return det > 0 ? 1 : -1;
+    const double x[8] = {ax, ay, bx, by, cx, cy, dx, dy};
     // four points on one horizontal or vertical line: every product has a
     // factor that is zero (a difference is zero only for equal numbers)
     if (perm == 0.0 && (ady == 0.0 || bdx == 0.0) && (bdy == 0.0 || adx == 0.0) &&
         (bdy == 0.0 || cdx == 0.0) && (cdy == 0.0 || bdx == 0.0) &&
-        (cdy == 0.0 || adx == 0.0) && (ady == 0.0 || cdx == 0.0))
+        (cdy == 0.0 || adx == 0.0) && (ady == 0.0 || cdx == 0.0) && near_exponents<8>(x))
         return 0;
-    const double x[8] = {ax, ay, bx, by, cx, cy, dx, dy};
     return incircle_exact(x, bound, err);
 }
 
