@@ -603,6 +603,7 @@ __global__ __launch_bounds__(1024) void k_dt_vote_lds(Pts P, int n, int T,
 
 // the scan that ranks the triangles to split counts those with a bid ...
 struct BidLoad {
+    static constexpr int kOne = 8192;
     const unsigned long long *vote;
     __device__ __forceinline__ int4 operator()(long base, int n) const
     {

@@ -10,17 +10,21 @@ namespace cvt {
 // over tiles of 4096 counts (1024 threads x 4 consecutive counts).  A count
 // comes from load(base, n), the four from `base` (a multiple of 4; 0 past n),
 // and done(total) runs in the workgroup that knows the sum, with all of its
-// 1024 threads.  Up to kScanOne counts one
-// workgroup does it, a thread taking up to 32 consecutive counts whose loads
-// are in flight together (k_scan_one: 2.7 us for 6 000 counts, 5.4 us for
-// 16 384, 9.8 us for 32 768, where three launches take 7.4, 8.2 and 10.8 us and
-// their gaps); beyond that in three launches:
+// 1024 threads.  Up to Load::kOne counts one workgroup does it, a thread taking
+// up to 32 consecutive counts whose loads are in flight together (k_scan_one);
+// beyond that in three launches:
 //   k_scan_tiles        each tile's total, parked in start[tile * 4096];
 //   k_scan_tile_totals  one workgroup turns the parked totals into the tiles'
 //                       offsets in place and writes start[n];
 //   k_scan_apply        each tile reads its offset, then writes its starts
 //                       (its first entry, the parked offset, last).
-constexpr int kScanTile = 4096, kScanOne = 32768;
+// The single workgroup is bound by the lines its strided loads fetch, so the
+// line between the two depends on the width of what is loaded.  us behind the
+// kernel that writes it, gaps included, one workgroup / three launches:
+//               8192        12000       16384        24576        32768
+//   counts      2.7 / 7.5   3.1 / 7.6   3.7 / 7.5    6.8 / 7.5    8.7 / 7.6
+//   64-bit bids 4.2 / 7.8   8.5 / 7.8   10.7 / 7.8   16.5 / 8.3   21.5 / 8.5
+constexpr int kScanTile = 4096;
 
 // exclusive prefix sum over a 1024-thread workgroup of one value per thread;
 // total receives the workgroup's sum (lds: 32 ints)
@@ -51,6 +55,7 @@ __device__ __forceinline__ int wg_exclusive_scan(int v, int *lds, int &total)
 }
 
 struct CountLoad {
+    static constexpr int kOne = 24576;
     const int *count;
     __device__ __forceinline__ int4 operator()(long base, int n) const
     {
@@ -148,21 +153,24 @@ __global__ __launch_bounds__(1024) void k_scan_one(Load load, int n, int *__rest
 template <class Load, class Done>
 void launch_scan(hipStream_t st, Load load, int n, int *start, Done done)
 {
+    static_assert(Load::kOne <= 32768, "eight quads per thread");
     const dim3 b(1024);
-    if (n <= 4096)
-        hipLaunchKernelGGL((k_scan_one<1, Load, Done>), dim3(1), b, 0, st, load, n, start, done);
-    else if (n <= 8192)
-        hipLaunchKernelGGL((k_scan_one<2, Load, Done>), dim3(1), b, 0, st, load, n, start, done);
-    else if (n <= 16384)
-        hipLaunchKernelGGL((k_scan_one<4, Load, Done>), dim3(1), b, 0, st, load, n, start, done);
-    else if (n <= kScanOne)
-        hipLaunchKernelGGL((k_scan_one<8, Load, Done>), dim3(1), b, 0, st, load, n, start, done);
-    else {
-        const int ntiles = (int)(((long)n + kScanTile - 1) / kScanTile);
-        hipLaunchKernelGGL((k_scan_tiles<Load>), dim3(ntiles), b, 0, st, load, n, start);
-        hipLaunchKernelGGL((k_scan_tile_totals<Done>), dim3(1), b, 0, st, start, n, ntiles, done);
-        hipLaunchKernelGGL((k_scan_apply<Load>), dim3(ntiles), b, 0, st, load, n, start);
+#define CVT_SCAN_ONE(Q) \
+    hipLaunchKernelGGL((k_scan_one<Q, Load, Done>), dim3(1), b, 0, st, load, n, start, done)
+    if (n <= Load::kOne) {
+        if (n <= 4096) CVT_SCAN_ONE(1);
+        else if (Load::kOne <= 8192 || n <= 8192) CVT_SCAN_ONE(2);
+        else if constexpr (Load::kOne > 8192) {
+            if (n <= 16384) CVT_SCAN_ONE(4);
+            else CVT_SCAN_ONE(8);
+        }
+#undef CVT_SCAN_ONE
+        return;
     }
+    const int ntiles = (int)(((long)n + kScanTile - 1) / kScanTile);
+    hipLaunchKernelGGL((k_scan_tiles<Load>), dim3(ntiles), b, 0, st, load, n, start);
+    hipLaunchKernelGGL((k_scan_tile_totals<Done>), dim3(1), b, 0, st, start, n, ntiles, done);
+    hipLaunchKernelGGL((k_scan_apply<Load>), dim3(ntiles), b, 0, st, load, n, start);
 }
 
 }  // namespace cvt
