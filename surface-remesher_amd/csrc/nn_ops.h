@@ -30,6 +30,12 @@ struct NnConv {
     const uint16_t *mask;
 };
 void nn_conv3x3(hipStream_t s, const NnConv &p, int N, int H, int W, int Cin, int Cout);
+// the kernel that it takes for a size: k_conv3x3_keep<8, 2, 2, 1>,
+// <4, 2, 2, 1>, <2, 1, 4, 1> and <4, 2, 2, 3>, k_conv3x3<4, 2, 2, 6, 9>,
+// <4, 2, 2, 4, 9>, <2, 1, 2, 2, 9>, <4, 2, 2, 2, 3> and <4, 2, 2, 2, 9>
+enum NnConvKernel { NN_KEEP_8, NN_KEEP_4, NN_KEEP_2, NN_KEEP_3SLICES, NN_CONV_96, NN_CONV_64,
+                    NN_CONV_SMALL, NN_CONV_CIN64, NN_CONV_32, NN_CONV_KERNELS };
+int nn_conv3x3_kernel(int N, int H, int W, int Cin, int Cout);
 // gradients dw[9][Cout][Cin] and then db[Cout] of the convolution p (its
 // inputs) from the out-gradient g; work holds
 // nn_dw_max_splits(Cin, Cout) * Cout * (9 * Cin + 1) floats

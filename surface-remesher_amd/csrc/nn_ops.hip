@@ -919,6 +919,19 @@ static inline unsigned nblk(long n, int b = 256) { return (unsigned)((n + b - 1)
 // CUs a block.  Blocks that keep their weights: two per CU, or one where those
 // of three slices take the registers; each then walks its tiles and loads
 // ahead (16 images forward, one slice: 0.47 ms, 0.55 with half the blocks).
+int nn_conv3x3_kernel(int N, int H, int W, int Cin, int Cout)
+{
+    const int NC = Cout / 32;
+    auto tiles = [&](int tw, int th) { return (long)N * ((W + tw - 1) / tw) * ((H + th - 1) / th); };
+    const long t8 = tiles(32, 8);
+    if (Cin == 32) return tiles(32, 16) * NC >= 384 ? NN_KEEP_8 : t8 * NC >= 192 ? NN_KEEP_4 : NN_KEEP_2;
+    if (Cin == 96 && t8 * NC >= 1024) return NN_KEEP_3SLICES;
+    if (Cin >= 128 && Cout % 96 == 0 && t8 * (Cout / 96) >= 192) return NN_CONV_96;
+    if (Cin >= 128 && Cout % 64 == 0 && t8 * (Cout / 64) >= 192) return NN_CONV_64;
+    if (t8 * NC < 256) return NN_CONV_SMALL;
+    return Cin == 64 ? NN_CONV_CIN64 : NN_CONV_32;
+}
+
 void nn_conv3x3(hipStream_t s, const NnConv &p, int N, int H, int W, int Cin, int Cout)
 {
     const int NC = Cout / 32;
@@ -926,13 +939,13 @@ void nn_conv3x3(hipStream_t s, const NnConv &p, int N, int H, int W, int Cin, in
         const int tx = (W + tw - 1) / tw, ty = (H + th - 1) / th;
         return ConvShape{H, W, Cin, Cout, tx, ty, N * tx * ty};
     };
-    auto tiles = [&](int tw, int th) { return (long)shape(tw, th).tiles; };
 #define NN_KEEP(R, WX, WY, NS)                                                                     \
     {                                                                                              \
         const ConvShape q = shape(16 * WX, R * WY);                                                \
         const int per = (q.tiles + 7) / 8, most = std::max(1, (NS == 1 ? 64 : 32) / NC);           \
         hipLaunchKernelGGL((k_conv3x3_keep<R, WX, WY, NS>), dim3(8 * NC * std::min(per, most)),    \
                            dim3(64 * WX * WY), 0, s, p, q);                                        \
+        break;                                                                                     \
     }
 #define NN_CONV(R, WX, WY, NT, WD)                                                                 \
     {                                                                                              \
@@ -940,26 +953,19 @@ void nn_conv3x3(hipStream_t s, const NnConv &p, int N, int H, int W, int Cin, in
         const int per = (q.tiles + 7) / 8;                                                         \
         hipLaunchKernelGGL((k_conv3x3<R, WX, WY, NT, WD>), dim3(8 * per * (2 * NC / NT)),          \
                            dim3(64 * WX * WY), (16 * WX + 2) * (R * WY + 2) * 2 * Cin, s, p, q);   \
+        break;                                                                                     \
     }
-    const long t8 = tiles(32, 8);
-    if (Cin == 32 && tiles(32, 16) * NC >= 384)
-        NN_KEEP(8, 2, 2, 1)
-    else if (Cin == 32 && t8 * NC >= 192)
-        NN_KEEP(4, 2, 2, 1)
-    else if (Cin == 32)
-        NN_KEEP(2, 1, 4, 1)
-    else if (Cin == 96 && t8 * NC >= 1024)
-        NN_KEEP(4, 2, 2, 3)
-    else if (Cin >= 128 && Cout % 96 == 0 && t8 * (Cout / 96) >= 192)
-        NN_CONV(4, 2, 2, 6, 9)
-    else if (Cin >= 128 && Cout % 64 == 0 && t8 * (Cout / 64) >= 192)
-        NN_CONV(4, 2, 2, 4, 9)
-    else if (t8 * NC < 256)
-        NN_CONV(2, 1, 2, 2, 9)
-    else if (Cin == 64)
-        NN_CONV(4, 2, 2, 2, 3)
-    else
-        NN_CONV(4, 2, 2, 2, 9)
+    switch (nn_conv3x3_kernel(N, H, W, Cin, Cout)) {
+    case NN_KEEP_8: NN_KEEP(8, 2, 2, 1)
+    case NN_KEEP_4: NN_KEEP(4, 2, 2, 1)
+    case NN_KEEP_2: NN_KEEP(2, 1, 4, 1)
+    case NN_KEEP_3SLICES: NN_KEEP(4, 2, 2, 3)
+    case NN_CONV_96: NN_CONV(4, 2, 2, 6, 9)
+    case NN_CONV_64: NN_CONV(4, 2, 2, 4, 9)
+    case NN_CONV_SMALL: NN_CONV(2, 1, 2, 2, 9)
+    case NN_CONV_CIN64: NN_CONV(4, 2, 2, 2, 3)
+    default: NN_CONV(4, 2, 2, 2, 9)
+    }
 #undef NN_CONV
 #undef NN_KEEP
 }
