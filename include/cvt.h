@@ -340,7 +340,9 @@ int cvt_dt_compute_constrained(cvt_dt *dt, const double *points, int num_points,
                                const int *segments, int num_segments, int *tri, int *opp,
                                int capacity, int *num_tri);
 /* stats[4]: insertion rounds, flip passes, flips and dropped duplicates of
- * the last cvt_dt_compute (gDel2D's Statistics, CommonTypes.h:532) */
+ * the last cvt_dt_compute (gDel2D's Statistics, CommonTypes.h:532).  Passes
+ * are counted in fours: p passes that flip, in one round, add 4 (p / 4 + 1),
+ * whatever the launches they run in; a round of constraint insertion adds 1. */
 int cvt_dt_stats(cvt_dt *dt, int *stats);
 int cvt_dt_destroy(cvt_dt *dt);
 /* orient[i] = sign of orient2d(a, b, c) and incircle[i] = sign of

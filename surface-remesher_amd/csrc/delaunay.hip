@@ -1491,7 +1491,8 @@ static int flips_left(DtCtx *c, int &done, int &round)
     done += c->hcnt[C_RAN];
     round += c->hcnt[C_RAN];
     if (c->hcnt[C_CONV] || c->hcnt[C_ERR]) {
-        // passes are counted in fours, as a run read its flips back once did
+        // what cvt_dt_stats has always reported: the run's passes in whole
+        // fours, up to the first four that begin with nothing left to flip
         c->stats[1] += 4 * (c->hcnt[C_PASSES] / 4 + 1);
         return 0;
     }

@@ -23,7 +23,7 @@
 // It replaced a seed scatter and four dense passes, each with its launch, the
 // site table staged into every CU's LDS, a map read and a map written.  At 256
 // pixels per site the five passes took 23.5 us at 512^2, 52.7 at 2048^2 and
-// 350 at 4096^2; the launch takes 11.8, 20.6 and 65 us.  It executes 1574 wave
+// 350 at 4096^2; the launch takes 12.3, 21.7 and 75 us in an iteration.  It executes 1574 wave
 // VALU instructions per class (10.5 us of issue at 2048^2, 42 at 4096^2) and
 // is bound by those and, on small grids, by the chain of its latencies (seed
 // map load, LDS atomics, site gather, label stores).

@@ -5,7 +5,8 @@
 // channels, K = 9 taps x input channels, on v_mfma_f32_16x16x32_bf16 (A:
 // lane i + 16 (k / 8) holds A[i][k], element k % 8; B: lane j + 16 (k / 8)
 // holds B[k][j]; C: lane j + 16 (i / 4) holds C[i][j], element i % 4).
-// Weights: [9][Cout][Cin] (tap = 3 ky + kx).  The data gradient of a conv is a
+// Weights: fp32 masters and gradients [9][Cout][Cin] (tap = 3 ky + kx), bf16
+// copies in operand order (conv_weight_index).  The data gradient of a conv is a
 // forward conv of the output gradient with the flipped, transposed weights;
 // the weight gradient is a split-K GEMM over pixels whose partials are summed
 // in a fixed order (deterministic).
@@ -569,8 +570,6 @@ __global__ __launch_bounds__(512) void k_sum_splits(const float *__restrict__ pa
     }
 }
 
-// fp32 master [9][Cout][Cin] -> bf16 forward copy (same layout) and the
-// flipped, transposed copy for the data gradient: [9][Cin][Cout], tap -> 8 - tap
 // position of a convolution weight in k_conv3x3's operand order: blocks
 // [Cout / 32][9 taps][Cin / 32][2 row operands][64 lanes][8 channels of ci];
 // lane l, operand b holds row co = 8 ((l & 15) / 4) + 4 b + l % 4 of its
@@ -582,6 +581,9 @@ __device__ __forceinline__ long conv_weight_index(int tap, int co, int ci, int C
     return ((((long)(co >> 5) * 9 + tap) * (Cin >> 5) + (ci >> 5)) * 2 + b) * 512 + lane * 8 + (i & 7);
 }
 
+// fp32 master [9][Cout][Cin] -> the bf16 forward copy and the flipped, transposed
+// copy for the data gradient (Cin and Cout exchanged, tap -> 8 - tap), both in
+// the order of conv_weight_index
 __global__ void k_weights_bf16(const float *__restrict__ w, int Cin, int Cout,
                                uint16_t *__restrict__ wf, uint16_t *__restrict__ wb)
 {

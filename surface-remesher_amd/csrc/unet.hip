@@ -205,7 +205,6 @@ int cvt_unet_create(cvt_unet **out, int R, int max_batch, unsigned long long see
     memset(u->wf, 0, sizeof u->wf); memset(u->wb, 0, sizeof u->wb);
     memset(u->a, 0, sizeof u->a); memset(u->ga, 0, sizeof u->ga);
     memset(u->pool, 0, sizeof u->pool); memset(u->gpool, 0, sizeof u->gpool);
-   
     u->R = R;
     u->maxb = max_batch;
     long off = 0;
