@@ -1410,8 +1410,11 @@ extern "C" int cvt_dt_create(cvt_dt **out, int max_points)
     };
     auto layout = [&](bool set) {
         at = 0;
-        carve(c->P, N + 1, set); carve(c->in, N, set); carve(c->ids, N + 1, set);
-        carve(c->place, N, set); carve(c->bounds, 4 * kParts, set);
+        carve(c->P, N + 1, set);
+        if (max_points >= kSortMin) {              // (fewer points are never sorted)
+            carve(c->in, N, set); carve(c->ids, N + 1, set); carve(c->place, N, set);
+            carve(c->bounds, 4 * kParts, set);
+        }
         carve(c->tv, 3 * T, set); carve(c->to, 3 * T, set);
         carve(c->vote[0], T, set); carve(c->vote[1], T, set); carve(c->flag, T, set); carve(c->pos, T + 1, set);
         carve(c->fvote, T, set); carve(c->fstamp, T, set); carve(c->fwd, 3 * T, set);
